@@ -271,3 +271,119 @@ def tolerance(case):
         # a loss is a mean of signed terms that nearly cancel
         return {"rel": 1e-4 if "grpo" in case["path"] else 1e-5}
     return {"rel": 1e-2} if case["dtype"] == "bf16" else {"rel": 2e-3}
+
+
+def _exact_head(hidden, weight, bias, ids, temperature, upstream=None):
+    """float64 log-probs of ``ids`` (``IGNORE`` rows: 0) and, given ``upstream(logp) -> d loss / d logp``
+    (or its values), the gradients w.r.t. hidden, weight and bias."""
+    h, w = hidden.detach().double(), weight.detach().double()
+    b = bias.detach().double() if bias is not None else None
+    live = ids != IGNORE
+    safe = torch.where(live, ids, torch.zeros_like(ids))
+    blocks = [slice(lo, min(lo + 1024, h.size(0))) for lo in range(0, h.size(0), 1024)]
+
+    def scaled(rows):
+        z = h[rows] @ w.t()
+        return (z if b is None else z + b).div_(temperature)
+
+    logp, lse = torch.empty_like(h[:, 0]), torch.empty_like(h[:, 0])
+    for rows in blocks:
+        z = scaled(rows)
+        lse[rows] = torch.logsumexp(z, 1)
+        logp[rows] = torch.where(live[rows], z.gather(1, safe[rows, None])[:, 0] - lse[rows], torch.zeros_like(lse[rows]))
+        del z
+    if upstream is None:
+        return logp, None
+    g = upstream(logp) if callable(upstream) else upstream.double()
+    g = torch.where(live, g, torch.zeros_like(g)) / temperature
+    dh, dw, db = torch.empty_like(h), torch.zeros_like(w), torch.zeros_like(w[:, 0])
+    for rows in blocks:
+        dz = scaled(rows).sub_(lse[rows, None]).exp_().mul_(-g[rows, None])
+        dz.scatter_add_(1, safe[rows, None], g[rows, None])
+        dh[rows] = dz @ w
+        dw.addmm_(dz.t(), h[rows])
+        db += dz.sum(0)
+        del dz
+    return logp, (dh, dw, db)
+
+
+def _exact_grpo(cur, old, ref, rewards, mask, group, beta, clip=0.2):
+    """float64 ``(loss, policy, kl)`` of the masked mean of the clipped ratio terms and k3 KL."""
+    r = rewards.double().view(-1, group)
+    std = ((r * r).mean(1, keepdim=True) - r.mean(1, keepdim=True) ** 2).clamp_min(1e-12).sqrt()
+    adv = ((r - r.mean(1, keepdim=True)) / std).view(-1, 1)
+    keep, zero = mask.bool(), torch.zeros_like(cur)
+    ratio = torch.exp(torch.where(keep, cur - old.double(), zero))
+    policy = -torch.minimum(ratio * adv, ratio.clamp(1 - clip, 1 + clip) * adv)
+    diff = torch.where(keep, ref.double() - cur, zero)
+    count = keep.sum()
+    policy = torch.where(keep, policy, zero).sum() / count
+    kl = torch.where(keep, diff.exp() - diff - 1, zero).sum() / count
+    return policy + beta * kl, policy, kl
+
+
+def exact(case, seed):
+    """What ``run`` returns for these inputs, by plain torch in float64."""
+    state = prepare(case, seed)
+    path = case["path"]
+    if path.startswith("logits"):
+        def selected(logits, ids):
+            return torch.cat([z.double().gather(1, i[:, None])[:, 0] - torch.logsumexp(z.double(), 1)
+                              for z, i in zip(logits.split(512), ids.split(512))])
+
+        logits, ids = state["logits"].detach().view(-1, case["vocab"]), state["ids"].reshape(-1)
+        cur = selected(logits, ids)
+        if path == "logits_logp":
+            return cur
+        cur.requires_grad_(True)
+        ref = selected(state["ref"].view(-1, case["vocab"]), ids)
+        shape = state["ids"].shape
+        out = _exact_grpo(cur.view(shape), state["old"], ref.view(shape), state["rewards"], state["mask"],
+                          case["group"], 0.04)
+        g, = torch.autograd.grad(out[0], [cur])
+        grad = torch.empty(logits.shape, device=logits.device, dtype=torch.float64)
+        for lo in range(0, len(cur), 512):
+            rows = slice(lo, lo + 512)
+            dz = torch.softmax(logits[rows].double(), 1).mul_(-g[rows, None])
+            grad[rows] = dz.scatter_add_(1, ids[rows, None], g[rows, None])
+        return (*(x.detach() for x in out), grad.view(state["logits"].shape))
+    if path == "score":
+        args = (state["ids"], case["temperature"])
+        logp = _exact_head(state["hidden"], state["weight"], state["bias"], *args)[0]
+        if not case["reference"]:
+            return logp
+        return logp, _exact_head(state["hidden"], state["ref_weight"], state["ref_bias"], *args)[0]
+    if path == "train":
+        x = state["hidden"].detach().double()
+        if case["norm"]:
+            gain = state["gain"].detach().double()
+            rstd = (x.square().mean(1, keepdim=True) + 1e-6).rsqrt()
+            y = x * rstd * gain
+        else:
+            y = x
+        logp, (dh, dw, db) = _exact_head(y, state["weight"], state["bias"], state["ids"], case["temperature"],
+                                         state["upstream"])
+        grads = [dh]
+        if case["norm"]:
+            d = dh * gain
+            grads[0] = rstd * (d - x * rstd * rstd * (d * x).mean(1, keepdim=True))
+        if not case["main_grad"]:
+            grads.append(dw)
+        if case["norm"]:
+            grads.append((dh * x * rstd).sum(0))
+        if case["bias"]:
+            grads.append(db)
+        return (logp, *grads, dw if case["main_grad"] else None)
+    shape = state["ids"].shape
+    ids = torch.where(state["mask"], state["ids"], torch.full_like(state["ids"], IGNORE)).view(-1)
+    values = []
+
+    def upstream(logp):
+        cur = logp.detach().view(shape).requires_grad_(True)
+        out = _exact_grpo(cur, state["old"], state["ref"], state["rewards"], state["mask"], case["group"], 0.04)
+        values.extend(x.detach() for x in out)
+        return torch.autograd.grad(out[0], [cur])[0].view(-1)
+
+    logp, (dh, dw, db) = _exact_head(state["hidden"].view(-1, case["hidden"]), state["head"].weight, state["bias"],
+                                     ids, case["temperature"], upstream)
+    return (*values, logp.view(shape), dh.view(state["hidden"].shape), dw) + ((db,) if case["bias"] else ())
