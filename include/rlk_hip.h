@@ -41,8 +41,9 @@ enum {
     RLK_ERR_LAUNCH = -3       /* HIP refused the launch */
 };
 
-/* ABI version of this header (major * 100 + minor): 101 (100 + rlk_device_info and
- * rlk_linear_logp_fwd_plan). */
+/* ABI version of this header (major * 100 + minor): 102 (100 + rlk_device_info,
+ * rlk_linear_logp_fwd_plan and the typed weight gradients, rlk_linear_logp_bwd_typed and
+ * rlk_linear_logp_rmsnorm_bwd_typed). */
 int rlk_version(void);
 
 /* Message of the last error returned on the calling thread ("" if none). Host pointer, valid
@@ -196,6 +197,22 @@ int rlk_linear_logp_bwd_accum(const float* grad_logp, const void* hidden, const 
                               int64_t ignore_index, int32_t use_ignore, int32_t accumulate,
                               rlk_stream_t stream);
 
+/* rlk_linear_logp_bwd with d_weight [V, H] in the type of `weight` (bf16 / f16), as autograd returns it:
+ * the sum over the tokens is fp32 as there and is rounded once, by the launch that finishes it, so the
+ * values are those of rlk_linear_logp_bwd followed by a cast, without the [V, H] fp32 round trip.  With
+ * several token chunks the running fp32 sum of the earlier ones lies in the workspace.  d_weight must
+ * start on a 16-byte boundary; fp32 heads, H % 8 != 0 and misaligned matrices are
+ * RLK_ERR_UNSUPPORTED (use rlk_linear_logp_bwd). */
+int rlk_linear_logp_bwd_typed_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype,
+                                              size_t dz_budget_bytes, size_t* bytes);
+
+int rlk_linear_logp_bwd_typed(const float* grad_logp, const void* hidden, const void* weight,
+                              const float* bias, const int64_t* targets, const float* lse,
+                              void* d_hidden, void* d_weight, float* d_bias, void* workspace,
+                              size_t workspace_bytes, size_t dz_budget_bytes, int64_t N, int32_t H,
+                              int64_t V, int64_t vocab_start, int32_t dtype, float temperature,
+                              int64_t ignore_index, int32_t use_ignore, rlk_stream_t stream);
+
 /* ------------------------------------------------------------------------------------------ *
  * Final RMSNorm in front of the head (the step before the path).
  *
@@ -252,6 +269,19 @@ int rlk_linear_logp_rmsnorm_bwd(const float* grad_logp, const void* x, const flo
                                 size_t dz_budget_bytes, int64_t N, int32_t H, int64_t V,
                                 int64_t vocab_start, int32_t dtype, float temperature,
                                 int64_t ignore_index, int32_t use_ignore, rlk_stream_t stream);
+
+/* rlk_linear_logp_rmsnorm_bwd with d_weight in the type of `weight`, as rlk_linear_logp_bwd_typed (same
+ * restrictions; `weight` 16-byte aligned). */
+int rlk_linear_logp_rmsnorm_bwd_typed_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype,
+                                                      size_t dz_budget_bytes, size_t* bytes);
+
+int rlk_linear_logp_rmsnorm_bwd_typed(const float* grad_logp, const void* x, const float* gain, float eps,
+                                      const void* weight, const float* bias, const int64_t* targets,
+                                      const float* lse, void* d_x, float* d_gain, void* d_weight,
+                                      float* d_bias, void* workspace, size_t workspace_bytes,
+                                      size_t dz_budget_bytes, int64_t N, int32_t H, int64_t V,
+                                      int64_t vocab_start, int32_t dtype, float temperature,
+                                      int64_t ignore_index, int32_t use_ignore, rlk_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------ *
  * Selected-token log-prob from materialised logits (the `fused_logp` family).

@@ -37,6 +37,10 @@ SIGNATURES = {
                                        _i64, _i32, _i64, _i64, _i32, _f32, _i64, _i32, _vp]),
     "rlk_linear_logp_bwd_accum": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _sz,
                                              _i64, _i32, _i64, _i64, _i32, _f32, _i64, _i32, _i32, _vp]),
+    "rlk_linear_logp_bwd_typed_workspace_bytes": (_c.c_int, [_i64, _i32, _i64, _i32, _sz,
+                                                             _c.POINTER(_sz)]),
+    "rlk_linear_logp_bwd_typed": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _sz,
+                                             _i64, _i32, _i64, _i64, _i32, _f32, _i64, _i32, _vp]),
     "rlk_rmsnorm_fwd": (_c.c_int, [_vp, _vp, _f32, _vp, _vp, _i64, _i32, _i32, _vp]),
     "rlk_rmsnorm_bwd_workspace_bytes": (_c.c_int, [_i64, _i32, _c.POINTER(_sz)]),
     "rlk_rmsnorm_bwd": (_c.c_int, [_vp, _vp, _f32, _vp, _vp, _vp, _vp, _sz, _i64, _i32, _i32, _vp]),
@@ -50,6 +54,11 @@ SIGNATURES = {
     "rlk_linear_logp_rmsnorm_bwd": (_c.c_int, [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                                _vp, _vp, _sz, _sz, _i64, _i32, _i64, _i64, _i32, _f32,
                                                _i64, _i32, _vp]),
+    "rlk_linear_logp_rmsnorm_bwd_typed_workspace_bytes": (_c.c_int, [_i64, _i32, _i64, _i32, _sz,
+                                                                     _c.POINTER(_sz)]),
+    "rlk_linear_logp_rmsnorm_bwd_typed": (_c.c_int, [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _vp,
+                                                     _vp, _vp, _vp, _sz, _sz, _i64, _i32, _i64, _i64,
+                                                     _i32, _f32, _i64, _i32, _vp]),
     "rlk_logp_from_logits": (_c.c_int, [_vp, _i32, _vp, _vp, _i32, _vp, _vp, _i64, _i64, _i64, _vp]),
     "rlk_logp_from_logits_pair": (_c.c_int, [_vp, _vp, _i32, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i64,
                                              _i64, _i64, _vp]),

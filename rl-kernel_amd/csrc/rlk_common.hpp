@@ -37,11 +37,13 @@ int wide_bwd(const float* grad_logp, const void* hidden, const void* weight, con
              int32_t use_ignore, int32_t accumulate, hipStream_t stream);
 // rlk_linear_logp_bwd with one more switch: accumulate != 0 adds d_weight / d_bias to what the
 // buffers already hold (callers that feed the tokens in several blocks).
+// d_weight_cast (16-bit kernels only): the finished weight gradient goes there in the weight's type, and
+// d_weight is only the running fp32 sum of earlier token chunks (unused, may be null, when there are none).
 int linear_logp_bwd_accumulating(const float* grad_logp, const void* hidden, const void* weight,
                                  const float* bias, const int64_t* targets, const float* lse,
                                  void* d_hidden, float* d_weight, float* d_bias, void* workspace,
                                  size_t workspace_bytes, size_t dz_budget_bytes, int64_t N, int32_t H,
                                  int64_t V, int64_t vocab_start, int32_t dtype, float temperature,
                                  int64_t ignore_index, int32_t use_ignore, int32_t accumulate,
-                                 hipStream_t stream);
+                                 hipStream_t stream, void* d_weight_cast = nullptr);
 }  // namespace rlk

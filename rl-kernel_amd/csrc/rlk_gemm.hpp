@@ -262,7 +262,7 @@ struct TileIO {
     }
 };
 
-template <class T, bool A_KMAJOR, bool B_KMAJOR, int BK, int WIN>
+template <class T, bool A_KMAJOR, bool B_KMAJOR, int BK, int WIN, bool TAIL = false>
 struct TileGemmDtl;
 
 // Workgroup tile contraction for any K.  acc[i][j] (+)= A rows x B rows over k in [0, K).
@@ -416,7 +416,16 @@ constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) |
 // cover ((k >> 3) & 1) by 2 chunks, so those 32 lanes hit 32 different 8-byte bank pairs.
 __device__ inline int kmajor_swizzle(int k) { return ((k & 3) << 2) ^ (((k >> 3) & 1) << 1); }
 
-template <bool KMAJOR, int ROWS, int BK>
+// Where the K steps of a contraction whose last 256-wide K tile is ragged find their operands (TAIL
+// loops): the ragged tile of a tensor is shifted back so that it ends at the tensor's edge, so from
+// K step `from` on the byte address is `a` / `b` away from the regular advance.  The entries of the
+// shifted tile that its left neighbour owns are zeros in the dZ operand, so they add nothing.
+struct KTail {
+    int from = 0x7fffffff;
+    int64_t a = 0, b = 0;
+};
+
+template <bool KMAJOR, int ROWS, int BK, bool TAIL = false>
 struct DtlIO {
     static_assert(BK == 64 && ROWS == 256, "direct-to-LDS layout is written for 256 x 64 tiles");
     static constexpr int kBytes = ROWS * BK * 2;            // 32 KiB, dense
@@ -431,6 +440,8 @@ struct DtlIO {
     uint32_t step;           // uniform byte advance per K step
     int nk;                  // K steps per tile
     int wave;                // uniform wavefront index
+    int tail_from;           // TAIL: first K step of the shifted last K tile
+    int64_t tail_adj;        // TAIL: uniform byte adjustment of those steps
 
     __device__ inline void init(const Operand& op, int K)
     {
@@ -469,6 +480,7 @@ struct DtlIO {
         const bool over = kt >= nk;
         const int rel = over ? (kt - nk < nk ? kt - nk : nk - 1) : kt;
         const char* src = (over ? next : base) + static_cast<size_t>(rel) * step;
+        if constexpr (TAIL) src += rel >= tail_from ? tail_adj : 0;  // uniform
         const uint32_t dst = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
                                  (RLK_LDS char*)(lds))) + static_cast<uint32_t>((wave + kWaves * p) * 1024);
         asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
@@ -506,15 +518,15 @@ struct DtlIO {
 // WIN: MFMA slots (of the 32 of the second slice) over which the 8 loads of a K step are spread.
 // 32 spaces them evenly over the slice; 16 sends them all out in its first half, which the
 // persistent dZ and dH kernels prefer (they stall more on operand loads than the forward).
-template <class T, bool A_KMAJOR, bool B_KMAJOR, int BK, int WIN>
+template <class T, bool A_KMAJOR, bool B_KMAJOR, int BK, int WIN, bool TAIL>
 struct TileGemmDtl {
     using AT = Acc16;
     static constexpr int TM = AT::TM;
     static constexpr int TN = AT::TN;
     static constexpr int KK = BK / 32;
     static_assert(KK == 2, "the loop is written for two 32-wide slices per K step");
-    using IOA = DtlIO<A_KMAJOR, 256, BK>;
-    using IOB = DtlIO<B_KMAJOR, 256, BK>;
+    using IOA = DtlIO<A_KMAJOR, 256, BK, TAIL>;
+    using IOB = DtlIO<B_KMAJOR, 256, BK, TAIL>;
     using Plan = FragPlan<TM, TN>;
     static constexpr int PA = IOA::kPasses;
     static constexpr int PB = IOB::kPasses;
@@ -586,13 +598,16 @@ struct TileGemmDtl {
     // Fill the pipeline for the first tile: K step 0 in LDS and published, the fragments of its
     // first slice in registers, K step 1 in flight.
     __device__ static inline void begin(Stream& st, const Operand& A, const Operand& B, int K,
-                                        char* smem)
+                                        char* smem, const KTail& tail = KTail())
     {
         const int wave = threadIdx.x >> 6;
         st.wm = wave / kWN;
         st.wn = wave % kWN;
         st.la.init(A, K);
         st.lb.init(B, K);
+        st.la.tail_from = st.lb.tail_from = tail.from;
+        st.la.tail_adj = tail.a;
+        st.lb.tail_adj = tail.b;
         st.nk = K / BK;
         st.phase = 0;
         static_for<0, PA>([&](auto pc) { st.la.load_one(0, smem, decltype(pc)::value); });
@@ -660,10 +675,10 @@ struct TileGemmDtl {
     }
 
     __device__ static inline void run(const Operand& A, const Operand& B, int K,
-                                      f32x4_t (&acc)[TM][TN], char* smem)
+                                      f32x4_t (&acc)[TM][TN], char* smem, const KTail& tail = KTail())
     {
         Stream st;
-        begin(st, A, B, K, smem);
+        begin(st, A, B, K, smem, tail);
         tile(st, A.base, B.base, acc, smem);
         end(st);
     }

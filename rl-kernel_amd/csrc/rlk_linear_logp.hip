@@ -60,12 +60,18 @@ struct FwdArgs {
 };
 
 // One workgroup = one block of 256 tokens x one contiguous range of vocab tiles.
-// GENERAL = false covers only full vocab tiles [0, vtiles) split n_split ways (a bias is added to
-// the finished tile before the softmax update); GENERAL = true handles masked rows over tiles
-// [tile_lo, tile_lo+vtiles).
-template <class T, int BK, bool GENERAL>
+// GENERAL = false covers vocab tiles [0, vtiles) split n_split ways, every one of 256 valid rows (a
+// bias is added to the finished tile before the softmax update); GENERAL = true handles masked rows
+// over tiles [tile_lo, tile_lo+vtiles).  When V is not a multiple of 256 the last tile of the chained
+// walk is shifted back to rows [V - 256, V) and the rows of its left neighbour are masked, so it runs
+// in the same launch and pipeline as all others.  A launch of its own for the ragged tile kept
+// row_blocks workgroups busy for a whole tile while the other CUs waited: 70 of 750 us at 4096 x
+// 2048 x 50257, 48 of 458 us at 1000 x 1536 x 151936.
+// CHAIN (!GENERAL, H a multiple of BK and >= 2 BK, V >= 256): all tiles run through one pipeline.
+template <class T, int BK, bool GENERAL, bool CHAIN>
 __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
 {
+    static_assert(!(GENERAL && CHAIN), "the chained variant covers full tiles only");
     using AT = Acc16;
     constexpr int TM = AT::TM, TN = AT::TN;
     using Gemm = TileGemm<T, false, false, BK>;
@@ -159,11 +165,13 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
 
     const int n_heads = a.weight2 != nullptr ? 2 : 1;
     Operand B{a.hidden + static_cast<int64_t>(tok0) * a.H, a.H, tok_valid};
+    // first vocab row of a tile; only the chained walk is ever given a tile that has to move back
+    auto tile_row = [&](int vt) { return CHAIN ? min(vt * 256, a.V - 256) : vt * 256; };
     auto tile_origin = [&](int head, int vt) {
-        return (head == 0 ? a.weight : a.weight2) + static_cast<int64_t>(vt) * 256 * a.H;
+        return (head == 0 ? a.weight : a.weight2) + static_cast<int64_t>(tile_row(vt)) * a.H;
     };
-    if (!GENERAL && a.H % BK == 0 && a.H >= 2 * BK && t0 < t1) {
-        // every tile is full: one pipeline runs through all tiles of the range (and then through
+    if constexpr (CHAIN) {
+        // every tile is full (or moved back) and every split has a tile (n_split <= vtiles): one pipeline runs through all tiles of the range (and then through
         // the same range of the second head), the K loop of a tile already fetching the head of the
         // next one while the softmax update runs (the pipeline looks two K steps ahead, which stays
         // within the next tile from two steps up)
@@ -172,6 +180,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
         for (int head = 0; head < n_heads; ++head) {
             reset_state();
             for (int vt = t0; vt < t1; ++vt) {
+                const int row0 = tile_row(vt);
                 f32x4_t acc[TM][TN];
                 zero_acc(acc);
                 const void* next = vt + 1 < t1 ? tile_origin(head, vt + 1)
@@ -179,8 +188,9 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
                                                                      : tile_origin(head, vt));
                 Dtl::template tile<true>(st, next, B.base, acc, smem);
                 const float* bias = head == 0 ? a.bias : a.bias2;
-                if (bias != nullptr) add_bias<AT>(acc, bias, vt * 256 + wm * (TM * 16), lane);  // uniform
-                fwd_epilogue<GENERAL, AT>(acc, a, nullptr, vt * 256 + wm * (TM * 16), lane, tgt, m, s, zt);
+                if (bias != nullptr) add_bias<AT>(acc, bias, row0 + wm * (TM * 16), lane);  // uniform
+                mask_rows<T>(acc, wm * (TM * 16), vt * 256 - row0, lane);
+                fwd_epilogue<GENERAL, AT>(acc, a, nullptr, row0 + wm * (TM * 16), vt * 256, lane, tgt, m, s, zt);
             }
             if (head == 0)
                 flush_state(a.part_m, a.part_s, a.part_z);
@@ -199,7 +209,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
                 zero_acc(acc);
                 Gemm::run(A, B, a.H, acc, smem);
                 if (!GENERAL && bias != nullptr) add_bias<AT>(acc, bias, v0 + wm * (TM * 16), lane);  // uniform
-                fwd_epilogue<GENERAL, AT>(acc, a, bias, v0 + wm * (TM * 16), lane, tgt, m, s, zt);
+                fwd_epilogue<GENERAL, AT>(acc, a, bias, v0 + wm * (TM * 16), v0, lane, tgt, m, s, zt);
             }
             if (head == 0)
                 flush_state(a.part_m, a.part_s, a.part_z);
@@ -324,6 +334,8 @@ struct DzArgs {
     int tok_tiles;
     int v_tiles;        // vocab tiles of this launch
     int v_tile_lo;      // first vocab tile of this launch
+    int tok_shift;      // rows / vocab rows by which the last token / vocab tile is moved back (see
+    int v_shift;        // BwdShift; 0 in the unchained kernels)
     int64_t v_global0;  // global id of the piece's first vocab row
     int64_t ignore_index;
     int use_ignore;
@@ -341,19 +353,24 @@ constexpr int kDzStageBytes = 64 * 64;
 // workgroup barrier.  The 8-byte units of a row are XOR-swizzled with 2 * ((token / 4) & 3), which
 // makes both the writes (16 tokens x 2 lane groups per pass) and the reads (4 rows x 8 units)
 // conflict-free.
+//
+// A tile that is shifted back (tok_back rows, v_back vocab rows) is still stored at its own place of
+// the block; what its neighbour owns is stored as zeros (token rows here through gs = 0, vocab rows
+// by the caller through mask_rows).
 template <class T, bool GENERAL>
 __device__ inline void dz_epilogue(const f32x4_t (&acc)[Acc16::TM][Acc16::TN], const DzArgs& a, int vt, int tt,
-                                   char* stage)
+                                   int v_back, int tok_back, char* stage)
 {
     using AT = Acc16;
     constexpr int TM = AT::TM, TN = AT::TN;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int wm = wave / kWN, wn = wave % kWN;
-    const int tok0 = tt * 256, v0 = vt * 256;
+    const int tok0 = tt * 256 - tok_back;
     const int tok_rows = min(256, a.tok_valid - tok0);
     const float gscale = a.scales[0];
-    const int vw = v0 + wm * (TM * 16);
+    const int vd = vt * 256 + wm * (TM * 16);  // column of the block
+    const int vw = vd - v_back;                // vocab row of the piece
     const int grp = lane >> 4;  // this lane holds rows 4 * grp + 0..3 of every 16-row tile
 
     float gs[TN], nlse2[TN];
@@ -364,17 +381,17 @@ __device__ inline void dz_epilogue(const f32x4_t (&acc)[Acc16::TM][Acc16::TN], c
         const int tl = wn * (TN * 16) + AT::col(j, lane);
         const int tc = tok0 + (tl < tok_rows ? tl : tok_rows - 1);
         const int64_t tg = a.targets[tc];
-        const bool live = tl < tok_rows && !(a.use_ignore && tg == a.ignore_index);
+        const bool live = tl >= tok_back && tl < tok_rows && !(a.use_ignore && tg == a.ignore_index);
         gs[j] = live ? a.grad[tc] * gscale : 0.f;
         nlse2[j] = -a.lse[tc] * kLog2e;
-        const int64_t trel = tg - a.v_global0 - vw;
-        etgt[j] = (trel >= 0 && trel < TM * 16) ? AT::reg_of_row(static_cast<int>(trel), lane) : -1;
+        const int64_t tv = tg - a.v_global0, trel = tv - vw;
+        etgt[j] = (trel >= 0 && trel < TM * 16 && tv >= vt * 256) ? AT::reg_of_row(static_cast<int>(trel), lane) : -1;
         any_target = any_target || etgt[j] >= 0;
     }
     // the one-hot term is added only when some lane of the wavefront owns its target row here
     const bool hot = __builtin_amdgcn_ballot_w64(any_target) != 0;  // uniform
 
-    uint16_t* dtile = a.dz + static_cast<int64_t>(tok0 + wn * (TN * 16)) * a.ldz + vw;
+    uint16_t* dtile = a.dz + static_cast<int64_t>(tt * 256 + wn * (TN * 16)) * a.ldz + vd;
     auto stage_rows = [&](auto ipc, auto hot_c) {
         constexpr int ip = decltype(ipc)::value;  // 32-row group = MFMA tiles 2 ip and 2 ip + 1
         constexpr bool HOT = decltype(hot_c)::value;
@@ -433,9 +450,10 @@ __device__ inline void dz_epilogue(const f32x4_t (&acc)[Acc16::TM][Acc16::TN], c
 }
 
 // GENERAL = false: every vocab tile of the launch is full (a bias is added to the finished tile).
-// CHAIN (needs !GENERAL, full token tiles, H a multiple of BK and >= 2 BK): the workgroup walks
-// its tiles through one pipeline; while a tile's epilogue runs, the first K steps of the next
-// tile are already on their way into LDS.
+// CHAIN (needs !GENERAL, H a multiple of BK and >= 2 BK, and 256 rows to read for every tile: the last
+// token tile and the last vocab tile may be shifted back by a.tok_shift / a.v_shift rows): the
+// workgroup walks its tiles through one pipeline; while a tile's epilogue runs, the first K steps of
+// the next tile are already on their way into LDS.
 template <class T, int BK, bool GENERAL, bool CHAIN>
 __global__ __launch_bounds__(kThreads) void linear_logp_dz_kernel(DzArgs a)
 {
@@ -449,8 +467,12 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dz_kernel(DzArgs a)
     if (!walk.valid()) return;
     int vt, tt;
     walk.coords(false, vt, tt);
-    auto w_origin = [&](int v) { return a.weight + static_cast<int64_t>(v + a.v_tile_lo) * 256 * a.H; };
-    auto h_origin = [&](int t) { return a.hidden + static_cast<int64_t>(t) * 256 * a.H; };
+    auto v_back = [&](int v) { return CHAIN && v == a.v_tiles - 1 ? a.v_shift : 0; };
+    auto tok_back = [&](int t) { return CHAIN && t == a.tok_tiles - 1 ? a.tok_shift : 0; };
+    auto w_origin = [&](int v) {
+        return a.weight + static_cast<int64_t>((v + a.v_tile_lo) * 256 - v_back(v)) * a.H;
+    };
+    auto h_origin = [&](int t) { return a.hidden + static_cast<int64_t>(t * 256 - tok_back(t)) * a.H; };
     f32x4_t acc[AT::TM][AT::TN];
     if constexpr (CHAIN) {
         char* stage = smem + Dtl::kSmemBytes + wave * kDzStageBytes;
@@ -460,11 +482,13 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dz_kernel(DzArgs a)
             const bool more = walk.has_next();
             int nvt = vt, ntt = tt;
             if (more) walk.coords(true, nvt, ntt);
+            const int vb = v_back(vt);
             zero_acc(acc);
             Dtl::template tile<true>(st, w_origin(nvt), h_origin(ntt), acc, smem);
             if (a.bias != nullptr)  // uniform
-                add_bias<AT>(acc, a.bias, (vt + a.v_tile_lo) * 256 + (wave / kWN) * (AT::TM * 16), threadIdx.x & 63);
-            dz_epilogue<T, GENERAL>(acc, a, vt + a.v_tile_lo, tt, stage);
+                add_bias<AT>(acc, a.bias, (vt + a.v_tile_lo) * 256 - vb + (wave / kWN) * (AT::TM * 16), threadIdx.x & 63);
+            mask_rows<T>(acc, (wave / kWN) * (AT::TM * 16), vb, threadIdx.x & 63);
+            dz_epilogue<T, GENERAL>(acc, a, vt + a.v_tile_lo, tt, vb, tok_back(tt), stage);
             if (!more) break;
             walk.advance();
             vt = nvt;
@@ -481,7 +505,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dz_kernel(DzArgs a)
             Gemm::run(A, B, a.H, acc, smem);  // ends with a barrier: LDS is free
             if (!GENERAL && a.bias != nullptr)  // uniform
                 add_bias<AT>(acc, a.bias, v0 + (wave / kWN) * (AT::TM * 16), threadIdx.x & 63);
-            dz_epilogue<T, GENERAL>(acc, a, vt + a.v_tile_lo, tt, smem + wave * kDzStageBytes);
+            dz_epilogue<T, GENERAL>(acc, a, vt + a.v_tile_lo, tt, 0, 0, smem + wave * kDzStageBytes);
             if (!walk.has_next()) break;
             walk.advance();
             walk.coords(false, vt, tt);
@@ -510,6 +534,9 @@ struct DhArgs {
     int ksplit;           // > 1: the vocab range is cut into ksplit parts computed by separate
     float* part;          //      workgroups, each writing its own fp32 slot [ksplit][rows][H]
     int64_t part_stride;  //      (elements per slot); linear_logp_dh_reduce_kernel adds them up
+    int nk;               // K steps (of 64 vocab rows) of the piece, the shifted tile's among them;
+    KTail tail;           //      0: the block has no shifted tiles, K runs over [0, v_valid)
+    int tok_shift;        // rows by which the last token tile is moved back
 };
 
 // Epilogue of one dH tile.  The read-modify-write of the running fp32 partial is latency-bound, so
@@ -529,7 +556,8 @@ __device__ inline void dh_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int wm = wave / kWN, wn = wave % kWN;
-    const int tok0 = tt * 256;
+    const int tok_min = tt * 256;  // first token row this tile owns
+    const int tok0 = tok_min - (!FULL && tt == a.tok_tiles - 1 ? a.tok_shift : 0);
     const float oscale = a.scales[1];
     const int hbase = h0 + wm * (TM * 16) + 4 * (lane >> 4);  // + i * 16
     const uint32_t ldh = static_cast<uint32_t>(a.H);
@@ -548,7 +576,7 @@ __device__ inline void dh_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
         for (int jj = 0; jj < 2; ++jj) {
             const int j = jb + jj;
             const int tl = tok0 + wn * (TN * 16) + AT::col(j, lane);
-            tok_ok[jj] = FULL || tl < a.tok_valid;
+            tok_ok[jj] = FULL || (tl >= tok_min && tl < a.tok_valid);
             trow[jj] = static_cast<int64_t>(tok_ok[jj] ? tl : a.tok_valid - 1) * a.H;
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
@@ -596,6 +624,7 @@ template <class T>
 __device__ inline bool dh_epilogue(const f32x4_t (&acc)[Acc16::TM][Acc16::TN], const DhArgs& a, int tt, int h0,
                                    int h_min, float* acc_dst, bool first, bool last)
 {
+    // (a token tile that is moved back is short of 256 rows of its own)
     const bool full = tt * 256 + 256 <= a.tok_valid && h0 + 256 <= a.H && h_min == h0;  // uniform
     if (full)
         dh_epilogue_impl<T, true>(acc, a, tt, h0, h_min, acc_dst, first, last);
@@ -604,13 +633,13 @@ __device__ inline bool dh_epilogue(const f32x4_t (&acc)[Acc16::TM][Acc16::TN], c
     return full;
 }
 
-// CHAIN (needs ksplit == 1, H >= 256, v_valid a multiple of BK and >= 2 BK): the workgroup walks
-// its tiles through one pipeline.
+// CHAIN (needs ksplit == 1, H >= 256 and a.nk >= 2): the workgroup walks its tiles through one
+// pipeline.
 template <class T, int BK, bool CHAIN>
 __global__ __launch_bounds__(kThreads) void linear_logp_dh_kernel(DhArgs a)
 {
     using Gemm = TileGemm<T, true, false, BK>;
-    using Dtl = TileGemmDtl<T, true, false, BK, kWinDh>;
+    using Dtl = TileGemmDtl<T, true, false, BK, kWinDh, true>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     f32x4_t acc[Acc16::TM][Acc16::TN];
     if constexpr (CHAIN) {
@@ -624,7 +653,8 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dh_kernel(DhArgs a)
         auto z_origin = [&](int t) { return a.dz + static_cast<int64_t>(t) * 256 * a.ldz; };
         typename Dtl::Stream st;
         bool counted = false;
-        Dtl::begin(st, Operand{w_origin(ht), a.H, 256}, Operand{z_origin(tt), a.ldz, 256}, a.v_valid, smem);
+        Dtl::begin(st, Operand{w_origin(ht), a.H, 256}, Operand{z_origin(tt), a.ldz, 256}, a.nk * BK, smem,
+                   a.tail);
         for (;;) {
             const bool more = walk.has_next();
             int ntt = tt, nht = ht;
@@ -650,16 +680,16 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dh_kernel(DhArgs a)
         if (a.ksplit > 1) {  // uniform
             ks = ht % a.ksplit;
             ht /= a.ksplit;
-            const int steps = (a.v_valid + BK - 1) / BK;
+            const int steps = a.nk > 0 ? a.nk : (a.v_valid + BK - 1) / BK;
             const int base = steps / a.ksplit, extra = steps % a.ksplit;
             const int s0 = ks * base + (ks < extra ? ks : extra);
             const int s1 = s0 + base + (ks < extra ? 1 : 0);
             k0 = s0 * BK;
-            kn = min(a.v_valid, s1 * BK) - k0;
+            kn = (a.nk > 0 ? s1 * BK : min(a.v_valid, s1 * BK)) - k0;
             if (kn <= 0) {  // a short last piece can leave a part without K steps: it computes one
                 empty_part = true;  // step of the piece's head and discards it
                 k0 = 0;
-                kn = min(a.v_valid, BK);
+                kn = a.nk > 0 ? BK : min(a.v_valid, BK);
             }
             acc_dst = a.part + static_cast<int64_t>(ks) * a.part_stride;
             first = true;
@@ -669,7 +699,13 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dh_kernel(DhArgs a)
         Operand A{a.weight + static_cast<int64_t>(k0) * a.H + h0, a.H, min(256, a.H - h0)};
         Operand B{a.dz + static_cast<int64_t>(tok0) * a.ldz + k0, a.ldz, 256};
         zero_acc(acc);
-        Gemm::run(A, B, kn, acc, smem);
+        if (a.nk > 0) {  // uniform
+            KTail tail = a.tail;
+            tail.from = max(0, tail.from - k0 / BK);
+            Dtl::run(A, B, a.ksplit > 1 ? kn : a.nk * BK, acc, smem, tail);
+        } else {
+            Gemm::run(A, B, kn, acc, smem);
+        }
         if (empty_part) zero_acc(acc);  // uniform: this part's slot must hold zeros
         dh_epilogue<T>(acc, a, tt, h0, h0, acc_dst, first, last);
     }
@@ -712,6 +748,11 @@ struct DwArgs {
     int v_tiles;
     int h_tiles;
     int accumulate;  // 1: dw += ..., 0: dw = ...
+    uint16_t* out;   // piece origin [v][H]: the finished sum leaves in the weight's type, dw is only
+                     // read (accumulate); null: the sum goes to dw
+    int nk;          // K steps (of 64 tokens) of the chunk, the shifted tile's among them; 0: the block
+    KTail tail;      // has no shifted tiles, K runs over [0, tok_valid)
+    int v_shift;     // vocab rows by which the last vocab tile is moved back
 };
 
 // Epilogue of one dW tile.  Orientation: M (accumulator registers) = hidden column, N (lane) =
@@ -722,7 +763,7 @@ struct DwArgs {
 // piece and inside H): a uniform tile origin plus a 32-bit lane offset, no predicates; otherwise
 // clamped reads and predicated stores.
 // The tile covers hidden columns [h0, h0 + 256) and owns those from h_min on (see dh_epilogue_impl).
-template <bool FULL>
+template <class T, bool FULL>
 __device__ inline void dw_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::TN], const DwArgs& a, int vt,
                                         int h0, int h_min)
 {
@@ -731,12 +772,14 @@ __device__ inline void dw_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int wm = wave / kWN, wn = wave % kWN;
-    const int v0 = vt * 256;
+    const int v_min = vt * 256;  // first vocab row this tile owns
+    const int v0 = v_min - (!FULL && vt == a.v_tiles - 1 ? a.v_shift : 0);
     const float oscale = a.scales[1];
     const int hbase = h0 + wm * (TM * 16) + 4 * (lane >> 4);  // + i * 16
     const uint32_t ldw = static_cast<uint32_t>(a.H);
     // FULL: byte offsets inside the tile stay below 256 * H * 4 (32 bits)
     char* tile = reinterpret_cast<char*>(a.dw + static_cast<int64_t>(v0) * a.H + h0);
+    char* otile = reinterpret_cast<char*>(a.out + static_cast<int64_t>(v0) * a.H + h0);
     const uint32_t lane_el = static_cast<uint32_t>(wn * (TN * 16) + (lane & 15)) * ldw +
                              static_cast<uint32_t>(wm * (TM * 16) + 4 * (lane >> 4));
 #pragma unroll
@@ -748,7 +791,7 @@ __device__ inline void dw_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
         for (int jj = 0; jj < 2; ++jj) {
             const int j = jb + jj;
             const int v = v0 + wn * (TN * 16) + AT::col(j, lane);
-            v_ok[jj] = FULL || v < a.v_valid;
+            v_ok[jj] = FULL || (v >= v_min && v < a.v_valid);
             vrow[jj] = static_cast<int64_t>(v_ok[jj] ? v : a.v_valid - 1) * a.H;
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
@@ -771,11 +814,19 @@ __device__ inline void dw_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
             for (int i = 0; i < TM; ++i) {
                 const int h = hbase + i * 16;
                 const f32x4_t val = acc[i][j] * oscale + old[jj][i];
-                if (FULL) {
-                    char* rowp = tile + (static_cast<size_t>(j * 16) * ldw + i * 16) * 4u;
-                    *reinterpret_cast<f32x4_t*>(rowp + lane_el * 4u) = val;
-                } else if (v_ok[jj] && h >= h_min && h < a.H) {  // H % 8 == 0: a quad is all-in or all-out
-                    *reinterpret_cast<f32x4_t*>(a.dw + vrow[jj] + h) = val;
+                const bool mine = FULL || (v_ok[jj] && h >= h_min && h < a.H);  // H % 8 == 0: a quad is all-in or all-out
+                const size_t uni = static_cast<size_t>(j * 16) * ldw + i * 16;  // uniform
+                if (a.out != nullptr) {  // uniform
+                    const u32x2_t pk{T::pack2(val.x, val.y), T::pack2(val.z, val.w)};
+                    if (FULL)
+                        *reinterpret_cast<u32x2_t*>(otile + uni * 2u + lane_el * 2u) = pk;
+                    else if (mine)
+                        *reinterpret_cast<u32x2_t*>(a.out + vrow[jj] + h) = pk;
+                } else {
+                    if (FULL)
+                        *reinterpret_cast<f32x4_t*>(tile + uni * 4u + lane_el * 4u) = val;
+                    else if (mine)
+                        *reinterpret_cast<f32x4_t*>(a.dw + vrow[jj] + h) = val;
                 }
             }
         }
@@ -783,24 +834,24 @@ __device__ inline void dw_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
 }
 
 // Returns whether the tile was full (then every wavefront issued all its stores unconditionally).
+template <class T>
 __device__ inline bool dw_epilogue(const f32x4_t (&acc)[Acc16::TM][Acc16::TN], const DwArgs& a, int vt, int h0,
                                    int h_min)
 {
     const bool full = vt * 256 + 256 <= a.v_valid && h0 + 256 <= a.H && h_min == h0;  // uniform
     if (full)
-        dw_epilogue_impl<true>(acc, a, vt, h0, h_min);
+        dw_epilogue_impl<T, true>(acc, a, vt, h0, h_min);
     else
-        dw_epilogue_impl<false>(acc, a, vt, h0, h_min);
+        dw_epilogue_impl<T, false>(acc, a, vt, h0, h_min);
     return full;
 }
 
-// CHAIN (needs H >= 256, tok_valid a multiple of BK and >= 2 BK): the workgroup walks its tiles
-// through one pipeline.
+// CHAIN (needs H >= 256 and a.nk >= 2): the workgroup walks its tiles through one pipeline.
 template <class T, int BK, bool CHAIN>
 __global__ __launch_bounds__(kThreads) void linear_logp_dw_kernel(DwArgs a)
 {
     using Gemm = TileGemm<T, true, true, BK>;
-    using Dtl = TileGemmDtl<T, true, true, BK, kWinDw>;
+    using Dtl = TileGemmDtl<T, true, true, BK, kWinDw, true>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     TileWalk walk(a.v_tiles * a.h_tiles, a.v_tiles, a.h_tiles);
     if (!walk.valid()) return;
@@ -814,7 +865,8 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dw_kernel(DwArgs a)
         auto h_origin = [&](int h) { return a.hidden + h_col(h); };  // M rows
         typename Dtl::Stream st;
         bool counted = false;
-        Dtl::begin(st, Operand{h_origin(ht), a.H, 256}, Operand{z_origin(vt), a.ldz, 256}, a.tok_valid, smem);
+        Dtl::begin(st, Operand{h_origin(ht), a.H, 256}, Operand{z_origin(vt), a.ldz, 256}, a.nk * BK, smem,
+                   a.tail);
         for (;;) {
             const bool more = walk.has_next();
             int nvt = vt, nht = ht;
@@ -822,7 +874,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dw_kernel(DwArgs a)
             zero_acc(acc);
             // a full tile's epilogue issues TM * TN unconditional stores per wavefront
             Dtl::template tile<true, Acc16::TM * Acc16::TN / 2>(st, h_origin(nht), z_origin(nvt), acc, smem, counted);
-            counted = dw_epilogue(acc, a, vt, h_col(ht), ht * 256);
+            counted = dw_epilogue<T>(acc, a, vt, h_col(ht), ht * 256);
             if (!more) break;
             walk.advance();
             vt = nvt;
@@ -835,12 +887,24 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dw_kernel(DwArgs a)
             Operand B{z_origin(vt), a.ldz, 256};
             zero_acc(acc);
             Gemm::run(A, B, a.tok_valid, acc, smem);
-            dw_epilogue(acc, a, vt, ht * 256, ht * 256);
+            dw_epilogue<T>(acc, a, vt, ht * 256, ht * 256);
             if (!walk.has_next()) break;
             walk.advance();
             walk.coords(false, vt, ht);
         }
     }
+}
+
+// Fewer tokens than a tile: the rows of `hidden` followed by rows of zeros up to one 256-row tile, so
+// that dZ and dW run on the full-tile pipeline (at most 256 x H x 2 bytes, a few us against the
+// register-staged loop that a K tail of the whole dW contraction would need: 12 to 20 % of a
+// backward at 160 tokens).  16 bytes per thread.
+__global__ void linear_logp_pad_rows_kernel(const uint16_t* src, uint16_t* dst, int64_t valid8, int64_t total8)
+{
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= total8) return;
+    reinterpret_cast<u32x4_t*>(dst)[i] =
+        i < valid8 ? reinterpret_cast<const u32x4_t*>(src)[i] : u32x4_t{0u, 0u, 0u, 0u};
 }
 
 // db[v] (+)= sum_tok dZ[tok][v] in two fixed-order levels.  Level 1: one workgroup per (256
@@ -875,13 +939,15 @@ __global__ __launch_bounds__(256) void linear_logp_db_partial_kernel(const uint1
 }
 
 // Level 2: the token tiles of the block in ascending order, times 1 / loss_scale.
+// v_shift: the last vocab tile's columns start that many vocab rows earlier than its place says.
 __global__ void linear_logp_db_finish_kernel(const float* part, int64_t part_ld, int tok_tiles, int v_valid,
-                                             const float* scales, float* db, int accumulate)
+                                             int v_shift, const float* scales, float* db, int accumulate)
 {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= v_valid) return;
-    float sum = part[v];
-    for (int t = 1; t < tok_tiles; ++t) sum += part[static_cast<int64_t>(t) * part_ld + v];
+    const int c = v < v_valid / 256 * 256 ? v : v + v_shift;
+    float sum = part[c];
+    for (int t = 1; t < tok_tiles; ++t) sum += part[static_cast<int64_t>(t) * part_ld + c];
     sum *= scales[1];
     db[v] = accumulate ? db[v] + sum : sum;
 }
@@ -934,8 +1000,9 @@ namespace {
 constexpr int kBK = RLK_BK;
 
 // Forward launch plan: a pure function of (N, H, V, which kernels run).
-//   fast launch   : full vocab tiles [0, full_tiles) split n_fast ways
-//   general launch: the ragged last tile (all tiles for the fp32 kernels) split n_gen ways
+//   fast launch   : vocab tiles split n_fast ways: all of them when the chained walk runs (it moves a
+//                   ragged last tile back), otherwise the full ones
+//   general launch: the ragged last tile of the other sizes (all tiles for the fp32 kernels), n_gen ways
 struct FwdPlan {
     int row_blocks;
     int patch_rows;
@@ -991,6 +1058,9 @@ int split_count(int row_blocks, int tiles, int patch_rows)
     return best;
 }
 
+// Sizes whose vocab tiles all run through the forward's one pipeline.
+bool fwd_chained(int H, int64_t V) { return H % kBK == 0 && H >= 2 * kBK && V >= 256; }
+
 FwdPlan fwd_plan(int64_t N, int H, int64_t V, bool all_general)
 {
     FwdPlan p;
@@ -998,7 +1068,7 @@ FwdPlan fwd_plan(int64_t N, int H, int64_t V, bool all_general)
     p.patch_rows = patch_rows_for(H);
     const int all = static_cast<int>((V + 255) / 256);
     const int full = static_cast<int>(V / 256);
-    p.fast_tiles = all_general ? 0 : full;
+    p.fast_tiles = all_general ? 0 : (fwd_chained(H, V) ? all : full);
     p.gen_tiles = all - p.fast_tiles;
     p.n_fast = split_count(p.row_blocks, p.fast_tiles, p.patch_rows);
     p.n_gen = split_count(p.row_blocks, p.gen_tiles, p.patch_rows);
@@ -1031,7 +1101,8 @@ struct BwdPlan {
     size_t acc_bytes;
     size_t part_bytes;
     size_t db_bytes;
-    size_t scales_off, dz_off, acc_off, part_off, db_off, total;
+    size_t pad_bytes;  // rows of one token tile when there are fewer tokens than that
+    size_t scales_off, dz_off, acc_off, part_off, db_off, pad_off, total;
 };
 
 // Cost of the three launches of one dZ block of ct x pt tiles, in K steps of one CU: a launch of
@@ -1148,7 +1219,9 @@ BwdPlan bwd_plan(int64_t N, int H, int64_t V, size_t budget)
     // per-token-tile column sums of the dZ block (d_bias): 1 KiB per dZ tile
     p.db_bytes = static_cast<size_t>(best_ct) * p.v_piece * 4;
     p.db_off = p.part_off + align_up(p.part_bytes, 256);
-    p.total = p.db_off + align_up(p.db_bytes, 256);
+    p.pad_bytes = N < 256 ? static_cast<size_t>(256) * H * 2 : 0;
+    p.pad_off = p.db_off + align_up(p.db_bytes, 256);
+    p.total = p.pad_off + align_up(p.pad_bytes, 256);
     memo = Key{N, V, H, budget, p};
     return p;
 }
@@ -1247,6 +1320,8 @@ struct BwdCall {
     int32_t use_ignore;
     hipStream_t stream;
     int accumulate;  // 1: d_weight / d_bias already hold the sums of earlier tokens, add to them
+    void* d_weight_cast;  // [V][H] of the weight's type or null: the finished d_weight sum goes here and
+                          // d_weight only holds the running sums of earlier chunks
 };
 
 // Grid of a chained launch: one workgroup per compute unit, rounded down to a multiple of 8 so
@@ -1279,6 +1354,22 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
     const uint16_t* w = static_cast<const uint16_t*>(c.weight);
     uint16_t* dh = static_cast<uint16_t*>(c.d_hidden);
     const int h_tiles = (H + 255) / 256;
+    // Ragged token counts and vocabularies on the full-tile pipelines: the last token tile and the last
+    // vocab tile are moved back so that they end at N and V (rows that exist whenever there are 256 of
+    // them) and what their neighbours own is zero in the dZ block; fewer than 256 tokens are padded.
+    // Device time against a launch for the ragged vocab tile, register-staged loops for K tails and
+    // unchained dZ / dW launches for ragged token counts (the dW figures with the typed gradient):
+    // 1000 x 1536 x 151936 dZ 599 -> 498 us, dW and its cast 1197 -> 515 us; 4096 x 2048 x 50257 dZ
+    // 789 -> 732 us, dH 732 -> 658 us.
+    const bool shifted = H % kBK == 0 && H >= 256 && V >= 256;
+    const bool padded = shifted && N < 256;
+    if (padded) {
+        uint16_t* pad = reinterpret_cast<uint16_t*>(ws + p.pad_off);
+        const int64_t total8 = 256LL * H / 8;
+        hipLaunchKernelGGL(linear_logp_pad_rows_kernel, dim3(static_cast<unsigned>((total8 + 255) / 256)), dim3(256),
+                           0, stream, hid, pad, N * H / 8, total8);
+        hid = pad;
+    }
 
     hipLaunchKernelGGL(linear_logp_scales_kernel, dim3(1), dim3(1024), 0, stream, c.grad_logp,
                        static_cast<int>(N), 1.f / c.temperature, c.dtype, scales);
@@ -1303,6 +1394,20 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
             if (v_valid <= 0) break;
             const int v_tiles = (v_valid + 255) / 256;
             const bool last_piece = (v_lo + p.v_piece >= V);
+            const int tok_rag = tok_valid % 256, v_rag = v_valid % 256;
+            const int tok_shift = shifted && !padded && tok_rag != 0 ? 256 - tok_rag : 0;
+            const int v_shift = shifted && v_rag != 0 ? 256 - v_rag : 0;
+            // K steps of dW (tokens) and dH (vocab rows): four per full tile, and of a shifted tile those
+            // that hold rows of its own (two at least where it is the only one: the pipeline's minimum)
+            auto k_steps = [](int valid, int shift) {
+                const int full = valid / 256, rag = valid % 256;
+                if (shift == 0) return full > 0 ? 4 * full : std::max(2, (rag + kBK - 1) / kBK);
+                const int own = (rag + kBK - 1) / kBK;
+                return 4 * full + (full == 0 ? std::max(2, own) : own);
+            };
+            // byte offset of those steps: past the tile's leading steps, and for the operand that is read
+            // from the tensor itself `shift` rows back (the dZ block has the tile in its place)
+            auto k_skip = [&](int valid, int shift) { return 4 * (valid / 256) + 4 - k_steps(valid, shift); };
 
             DzArgs z;
             z.hidden = hid + tok_lo * H;
@@ -1318,6 +1423,8 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
             z.v_valid = v_valid;
             z.H = H;
             z.tok_tiles = tok_tiles;
+            z.tok_shift = tok_shift;
+            z.v_shift = v_shift;
             z.v_global0 = c.vocab_start + v_lo;
             z.ignore_index = c.ignore_index;
             z.use_ignore = c.use_ignore;
@@ -1342,12 +1449,22 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
             h.ksplit = ksplit;
             h.part = ksplit > 1 ? reinterpret_cast<float*>(ws + p.part_off) : nullptr;
             h.part_stride = static_cast<int64_t>(tok_tiles) * 256 * H;
+            const bool dh_chain = ksplit == 1 && H >= 256 && (shifted || (v_valid % kBK == 0 && v_valid >= 2 * kBK));
+            h.nk = shifted ? k_steps(v_valid, v_shift) : (dh_chain ? v_valid / kBK : 0);
+            h.tok_shift = tok_shift;
+            h.tail = KTail();
+            if (v_shift != 0) {
+                const int64_t skip = static_cast<int64_t>(k_skip(v_valid, v_shift)) * kBK;
+                h.tail = KTail{v_valid / 256 * 4, (skip - v_shift) * H * 2, skip * 2};
+            }
 
             DwArgs d;
             d.dz = dz;
             d.hidden = hid + tok_lo * H;
             d.scales = scales;
             d.dw = c.d_weight ? c.d_weight + v_lo * H : nullptr;
+            d.out = c.d_weight_cast && ci == p.n_chunks - 1
+                        ? static_cast<uint16_t*>(c.d_weight_cast) + v_lo * H : nullptr;
             d.ldz = p.ldz;
             d.H = H;
             d.v_valid = v_valid;
@@ -1355,17 +1472,25 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
             d.v_tiles = v_tiles;
             d.h_tiles = h_tiles;
             d.accumulate = ci > 0 || c.accumulate != 0;
+            const bool dw_chain = H >= 256 && (shifted || (tok_valid % kBK == 0 && tok_valid >= 2 * kBK));
+            d.nk = shifted ? k_steps(tok_valid, tok_shift) : (dw_chain ? tok_valid / kBK : 0);
+            d.v_shift = v_shift;
+            d.tail = KTail();
+            if (tok_shift != 0) {
+                const int64_t skip = static_cast<int64_t>(k_skip(tok_valid, tok_shift)) * kBK;
+                d.tail = KTail{tok_valid / 256 * 4, (skip - tok_shift) * H * 2, skip * p.ldz * 2};
+            }
 
-            // dZ block: full vocab tiles through the fast variant (chained through one pipeline
-            // when the token tiles are full too), the ragged last one through the general one
-            const int fast_tiles = v_valid / 256;
+            // dZ block: chained through one pipeline when every tile can read 256 rows; otherwise the
+            // full vocab tiles through the fast variant and the ragged last one through the general one
+            const int fast_tiles = shifted ? v_tiles : v_valid / 256;
             const int gen_tiles = v_tiles - fast_tiles;
             const bool k_ok = H % kBK == 0 && H >= 2 * kBK;
             if (fast_tiles > 0) {
                 z.v_tiles = fast_tiles;
                 z.v_tile_lo = 0;
                 const int tiles = tok_tiles * fast_tiles;
-                if (k_ok && tok_valid % 256 == 0)
+                if (shifted || (k_ok && tok_valid % 256 == 0))
                     hipLaunchKernelGGL((linear_logp_dz_kernel<T, kBK, false, true>),
                                        dim3(chain_grid(tiles, n_cu)), dim3(kThreads), kDzChainSmem,
                                        stream, z);
@@ -1382,7 +1507,7 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
             }
             if (dh) {
                 const int tiles = tok_tiles * h_tiles;
-                if (ksplit == 1 && H >= 256 && v_valid % kBK == 0 && v_valid >= 2 * kBK) {
+                if (dh_chain) {
                     hipLaunchKernelGGL((linear_logp_dh_kernel<T, kBK, true>),
                                        dim3(chain_grid(tiles, n_cu)), dim3(kThreads), kChainSmem,
                                        stream, h);
@@ -1398,9 +1523,9 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
                     }
                 }
             }
-            if (c.d_weight) {
+            if (c.d_weight || c.d_weight_cast) {
                 const int tiles = v_tiles * h_tiles;
-                if (H >= 256 && tok_valid % kBK == 0 && tok_valid >= 2 * kBK)
+                if (dw_chain)
                     hipLaunchKernelGGL((linear_logp_dw_kernel<T, kBK, true>),
                                        dim3(chain_grid(tiles, n_cu)), dim3(kThreads), kChainSmem,
                                        stream, d);
@@ -1414,7 +1539,7 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
                                    stream, dz, p.ldz, db_part, static_cast<int64_t>(p.v_piece));
                 hipLaunchKernelGGL(linear_logp_db_finish_kernel, dim3((v_valid + 255) / 256), dim3(256), 0,
                                    stream, db_part, static_cast<int64_t>(p.v_piece), tok_tiles, v_valid,
-                                   scales, c.d_bias + v_lo, (ci > 0 || c.accumulate != 0) ? 1 : 0);
+                                   v_shift, scales, c.d_bias + v_lo, (ci > 0 || c.accumulate != 0) ? 1 : 0);
             }
             if (int rc = check_launch("linear_logp backward launch failed")) return rc;
         }
@@ -1423,21 +1548,21 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
 }
 
 // One forward contraction launch: a.row_blocks x a.n_split workgroups of the given variant.
-template <class T, bool GENERAL>
+template <class T, bool GENERAL, bool CHAIN>
 int launch_fwd_as(const FwdArgs& a, hipStream_t stream)
 {
     using G = TileGemm<T, false, false, kBK>;
-    if (int rc = set_smem(linear_logp_fwd_kernel<T, kBK, GENERAL>, G::kSmemBytes)) return rc;
-    hipLaunchKernelGGL((linear_logp_fwd_kernel<T, kBK, GENERAL>), dim3(a.row_blocks * a.n_split),
+    if (int rc = set_smem(linear_logp_fwd_kernel<T, kBK, GENERAL, CHAIN>, G::kSmemBytes)) return rc;
+    hipLaunchKernelGGL((linear_logp_fwd_kernel<T, kBK, GENERAL, CHAIN>), dim3(a.row_blocks * a.n_split),
                        dim3(kThreads), G::kSmemBytes, stream, a);
     return 0;
 }
 
-template <bool GENERAL>
+template <bool GENERAL, bool CHAIN>
 int launch_fwd(const FwdArgs& a, int32_t dtype, hipStream_t stream)
 {
-    return dtype == RLK_DTYPE_BF16 ? launch_fwd_as<Bf16, GENERAL>(a, stream)
-                                   : launch_fwd_as<F16, GENERAL>(a, stream);
+    return dtype == RLK_DTYPE_BF16 ? launch_fwd_as<Bf16, GENERAL, CHAIN>(a, stream)
+                                   : launch_fwd_as<F16, GENERAL, CHAIN>(a, stream);
 }
 
 // A second head over the same hidden states and targets (a frozen reference model).
@@ -1698,14 +1823,16 @@ int fwd_enqueue(const void* hidden, const void* weight, const float* bias, const
         a.split_lo = 0;
         a.tile_lo = 0;
         a.vtiles = plan.fast_tiles;
-        if (int rc = launch_fwd<false>(a, dtype, stream)) return rc;
+        if (int rc = fwd_chained(H, V) ? launch_fwd<false, true>(a, dtype, stream)
+                                       : launch_fwd<false, false>(a, dtype, stream))
+            return rc;
     }
     if (mfma && plan.n_gen > 0) {
         a.n_split = plan.n_gen;
         a.split_lo = plan.n_fast;
         a.tile_lo = plan.fast_tiles;
         a.vtiles = plan.gen_tiles;
-        if (int rc = launch_fwd<true>(a, dtype, stream)) return rc;
+        if (int rc = launch_fwd<true, false>(a, dtype, stream)) return rc;
     }
     if (int rc = check_launch("linear_logp_fwd_kernel launch failed")) return rc;
 
@@ -1812,6 +1939,42 @@ int rlk_linear_logp_bwd_accum(const float* grad_logp, const void* hidden, const 
                                              ignore_index, use_ignore, accumulate != 0 ? 1 : 0, stream);
 }
 
+int rlk_linear_logp_bwd_typed_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype,
+                                              size_t dz_budget_bytes, size_t* bytes)
+{
+    if (dtype != RLK_DTYPE_BF16 && dtype != RLK_DTYPE_F16)
+        return rlk_fail(RLK_ERR_UNSUPPORTED, "the typed weight gradient is for bf16 and f16 heads");
+    if (int rc = rlk_linear_logp_bwd_workspace_bytes(N, H, V, dtype, dz_budget_bytes, bytes)) return rc;
+    const BwdPlan p = bwd_plan(N, H, V, clamp_dz_budget(dz_budget_bytes));
+    // the running fp32 sum of all token chunks but the last
+    if (p.n_chunks > 1) *bytes = align_up(*bytes, 256) + static_cast<size_t>(V) * H * 4;
+    return 0;
+}
+
+int rlk_linear_logp_bwd_typed(const float* grad_logp, const void* hidden, const void* weight,
+                              const float* bias, const int64_t* targets, const float* lse,
+                              void* d_hidden, void* d_weight, float* d_bias, void* workspace,
+                              size_t workspace_bytes, size_t dz_budget_bytes, int64_t N, int32_t H,
+                              int64_t V, int64_t vocab_start, int32_t dtype, float temperature,
+                              int64_t ignore_index, int32_t use_ignore, hipStream_t stream)
+{
+    if (int rc = check_common(N, H, V, dtype)) return rc;
+    if (!grad_logp || !hidden || !weight || !targets || !lse || !d_weight)
+        return rlk_fail(RLK_ERR_ARG, "null pointer");
+    if (!use_mfma(hidden, weight, H, dtype) || (reinterpret_cast<uintptr_t>(d_weight) & 15) != 0)
+        return rlk_fail(RLK_ERR_UNSUPPORTED,
+                        "rlk_linear_logp_bwd_typed takes bf16 / f16, H % 8 == 0 and 16-byte aligned matrices");
+    size_t need = 0, base = 0;
+    if (int rc = rlk_linear_logp_bwd_typed_workspace_bytes(N, H, V, dtype, dz_budget_bytes, &need)) return rc;
+    if (int rc = rlk_linear_logp_bwd_workspace_bytes(N, H, V, dtype, dz_budget_bytes, &base)) return rc;
+    if (!workspace || workspace_bytes < need) return rlk_fail(RLK_ERR_ARG, "workspace too small");
+    float* running = need > base
+                         ? reinterpret_cast<float*>(static_cast<char*>(workspace) + align_up(base, 256)) : nullptr;
+    return rlk::linear_logp_bwd_accumulating(grad_logp, hidden, weight, bias, targets, lse, d_hidden, running,
+                                             d_bias, workspace, base, dz_budget_bytes, N, H, V, vocab_start,
+                                             dtype, temperature, ignore_index, use_ignore, 0, stream, d_weight);
+}
+
 }  // extern "C"
 
 int rlk::linear_logp_bwd_accumulating(const float* grad_logp, const void* hidden, const void* weight,
@@ -1820,12 +1983,13 @@ int rlk::linear_logp_bwd_accumulating(const float* grad_logp, const void* hidden
                                       size_t workspace_bytes, size_t dz_budget_bytes, int64_t N,
                                       int32_t H, int64_t V, int64_t vocab_start, int32_t dtype,
                                       float temperature, int64_t ignore_index, int32_t use_ignore,
-                                      int32_t accumulate, hipStream_t stream)
+                                      int32_t accumulate, hipStream_t stream, void* d_weight_cast)
 {
     if (int rc = check_common(N, H, V, dtype)) return rc;
     if (!(temperature > 0.f)) return rlk_fail(RLK_ERR_ARG, "temperature must be greater than zero");
     if (!grad_logp || !hidden || !weight || !targets || !lse) return rlk_fail(RLK_ERR_ARG, "null pointer");
-    if (!d_hidden && !d_weight && !d_bias) return rlk_fail(RLK_ERR_ARG, "no gradient requested");
+    if (!d_hidden && !d_weight && !d_bias && !d_weight_cast)
+        return rlk_fail(RLK_ERR_ARG, "no gradient requested");
     if (bias == nullptr && d_bias != nullptr) return rlk_fail(RLK_ERR_ARG, "d_bias given without bias");
     dz_budget_bytes = clamp_dz_budget(dz_budget_bytes);
     size_t need = 0;
@@ -1833,14 +1997,18 @@ int rlk::linear_logp_bwd_accumulating(const float* grad_logp, const void* hidden
     if (!workspace || workspace_bytes < need) return rlk_fail(RLK_ERR_ARG, "workspace too small");
     if (reinterpret_cast<uintptr_t>(workspace) & 255)
         return rlk_fail(RLK_ERR_ARG, "workspace must be 256-byte aligned");
+    if (!use_mfma(hidden, weight, H, dtype) && d_weight_cast != nullptr)
+        return rlk_fail(RLK_ERR_UNSUPPORTED, "the fp32 matrix-core kernels write fp32 weight gradients only");
     if (!use_mfma(hidden, weight, H, dtype))
         return wide_bwd(grad_logp, hidden, weight, bias, targets, lse, d_hidden, d_weight, d_bias,
                         workspace, dz_budget_bytes, N, H, V, vocab_start, dtype, temperature,
                         ignore_index, use_ignore, accumulate, stream);
     const BwdPlan p = bwd_plan(N, H, V, dz_budget_bytes);
+    if (d_weight_cast != nullptr && d_weight == nullptr && (p.n_chunks > 1 || accumulate))
+        return rlk_fail(RLK_ERR_ARG, "several token chunks need a running fp32 weight gradient");
     int n_cu = 0;
     if (int rc = compute_units(&n_cu)) return rc;
     BwdCall c{grad_logp, hidden, weight, bias, targets, lse, d_hidden, d_weight, d_bias, workspace,
-              N, H, V, vocab_start, dtype, temperature, ignore_index, use_ignore, stream, accumulate};
+              N, H, V, vocab_start, dtype, temperature, ignore_index, use_ignore, stream, accumulate, d_weight_cast};
     return dtype == RLK_DTYPE_BF16 ? bwd_enqueue<Bf16>(c, p, n_cu) : bwd_enqueue<F16>(c, p, n_cu);
 }

@@ -314,8 +314,11 @@ int rlk_linear_logp_rmsnorm_fwd_workspace_bytes(int64_t N, int32_t H, int64_t V,
 {
     if (!bytes || N <= 0 || H <= 0 || V <= 0) return rlk_fail(RLK_ERR_ARG, "bad workspace query");
     const int64_t nb = block_tokens(N);
-    size_t fwd = 0;
+    size_t fwd = 0, tail = 0;
     if (int rc = rlk_linear_logp_fwd_workspace_bytes(nb, H, V, dtype, &fwd)) return rc;
+    if (N % nb != 0)  // a short last block has a plan of its own
+        if (int rc = rlk_linear_logp_fwd_workspace_bytes(N % nb, H, V, dtype, &tail)) return rc;
+    fwd = fwd > tail ? fwd : tail;
     *bytes = up256(static_cast<size_t>(nb) * H * elt_bytes(dtype)) + up256(fwd);
     return 0;
 }
@@ -358,7 +361,13 @@ int rlk_linear_logp_rmsnorm_bwd_workspace_bytes(int64_t N, int32_t H, int64_t V,
     if (!bytes || N <= 0 || H <= 0 || V <= 0) return rlk_fail(RLK_ERR_ARG, "bad workspace query");
     const int64_t nb = block_tokens(N);
     size_t bwd = 0;
-    if (int rc = rlk_linear_logp_bwd_workspace_bytes(nb, H, V, dtype, dz_budget_bytes, &bwd)) return rc;
+    const int64_t half = (nb + 1) / 2;  // block length without d_x, see rlk_linear_logp_rmsnorm_bwd
+    for (int64_t n : {nb, N % nb, half, N % half}) {  // short last blocks have plans of their own
+        if (n == 0) continue;
+        size_t one = 0;
+        if (int rc = rlk_linear_logp_bwd_workspace_bytes(n, H, V, dtype, dz_budget_bytes, &one)) return rc;
+        bwd = bwd > one ? bwd : one;
+    }
     // one block of normalised rows (+ 256 bytes so that it can be cut into two aligned halves, see
     // rlk_linear_logp_rmsnorm_bwd); the gradient w.r.t. the normalised rows goes straight into d_x
     const size_t rows = up256(static_cast<size_t>(nb) * H * elt_bytes(dtype)) + 256;
@@ -366,17 +375,20 @@ int rlk_linear_logp_rmsnorm_bwd_workspace_bytes(int64_t N, int32_t H, int64_t V,
     return 0;
 }
 
-int rlk_linear_logp_rmsnorm_bwd(const float* grad_logp, const void* x, const float* gain, float eps,
-                                const void* weight, const float* bias, const int64_t* targets,
-                                const float* lse, void* d_x, float* d_gain, float* d_weight,
-                                float* d_bias, void* workspace, size_t workspace_bytes,
-                                size_t dz_budget_bytes, int64_t N, int32_t H, int64_t V,
-                                int64_t vocab_start, int32_t dtype, float temperature,
-                                int64_t ignore_index, int32_t use_ignore, hipStream_t stream)
+}  // extern "C"
+
+namespace {
+
+// d_weight_cast: see linear_logp_bwd_accumulating; the last block of tokens writes it.
+int norm_bwd(const float* grad_logp, const void* x, const float* gain, float eps, const void* weight,
+             const float* bias, const int64_t* targets, const float* lse, void* d_x, float* d_gain,
+             float* d_weight, void* d_weight_cast, float* d_bias, void* workspace, size_t workspace_bytes,
+             size_t dz_budget_bytes, int64_t N, int32_t H, int64_t V, int64_t vocab_start, int32_t dtype,
+             float temperature, int64_t ignore_index, int32_t use_ignore, hipStream_t stream)
 {
     if (int rc = check_norm(x, gain, N, H, dtype)) return rc;
     if (!grad_logp || !weight || !targets || !lse) return rlk_fail(RLK_ERR_ARG, "null pointer");
-    if (!d_x && !d_gain && !d_weight && !d_bias) return rlk_fail(RLK_ERR_ARG, "no gradient requested");
+    if (!d_x && !d_gain && !d_weight && !d_weight_cast && !d_bias) return rlk_fail(RLK_ERR_ARG, "no gradient requested");
     size_t need = 0;
     if (int rc = rlk_linear_logp_rmsnorm_bwd_workspace_bytes(N, H, V, dtype, dz_budget_bytes, &need)) return rc;
     if (!workspace || workspace_bytes < need) return rlk_fail(RLK_ERR_ARG, "workspace too small");
@@ -414,7 +426,8 @@ int rlk_linear_logp_rmsnorm_bwd(const float* grad_logp, const void* x, const flo
                                                   lse + t0, need_norm_bwd ? dxb : nullptr,
                                                   d_weight, d_bias, bwd_ws, bwd_bytes, dz_budget_bytes,
                                                   n, H, V, vocab_start, dtype, temperature,
-                                                  ignore_index, use_ignore, t0 > 0 ? 1 : 0, stream))
+                                                  ignore_index, use_ignore, t0 > 0 ? 1 : 0, stream,
+                                                  t0 + n == N ? d_weight_cast : nullptr))
             return rc;
         if (need_norm_bwd) {
             if (int rc = rmsnorm_bwd_enqueue(xb, gain, eps, dxb, dxb, d_gain, t0 > 0 ? 1 : 0, gain_ws,
@@ -423,6 +436,58 @@ int rlk_linear_logp_rmsnorm_bwd(const float* grad_logp, const void* x, const flo
         }
     }
     return 0;
+}
+
+}  // namespace
+
+extern "C" {
+
+int rlk_linear_logp_rmsnorm_bwd(const float* grad_logp, const void* x, const float* gain, float eps,
+                                const void* weight, const float* bias, const int64_t* targets,
+                                const float* lse, void* d_x, float* d_gain, float* d_weight,
+                                float* d_bias, void* workspace, size_t workspace_bytes,
+                                size_t dz_budget_bytes, int64_t N, int32_t H, int64_t V,
+                                int64_t vocab_start, int32_t dtype, float temperature,
+                                int64_t ignore_index, int32_t use_ignore, hipStream_t stream)
+{
+    return norm_bwd(grad_logp, x, gain, eps, weight, bias, targets, lse, d_x, d_gain, d_weight, nullptr, d_bias,
+                    workspace, workspace_bytes, dz_budget_bytes, N, H, V, vocab_start, dtype, temperature,
+                    ignore_index, use_ignore, stream);
+}
+
+int rlk_linear_logp_rmsnorm_bwd_typed_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype,
+                                                      size_t dz_budget_bytes, size_t* bytes)
+{
+    if (dtype != RLK_DTYPE_BF16 && dtype != RLK_DTYPE_F16)
+        return rlk_fail(RLK_ERR_UNSUPPORTED, "the typed weight gradient is for bf16 and f16 heads");
+    if (int rc = rlk_linear_logp_rmsnorm_bwd_workspace_bytes(N, H, V, dtype, dz_budget_bytes, bytes)) return rc;
+    int64_t plan[5];
+    if (int rc = rlk_linear_logp_bwd_plan(block_tokens(N), H, V, dtype, dz_budget_bytes, plan)) return rc;
+    // the running fp32 sum of all blocks and chunks but the last
+    if (N > kNormBlockTokens || plan[2] > 1) *bytes = up256(*bytes) + static_cast<size_t>(V) * H * 4;
+    return 0;
+}
+
+int rlk_linear_logp_rmsnorm_bwd_typed(const float* grad_logp, const void* x, const float* gain, float eps,
+                                      const void* weight, const float* bias, const int64_t* targets,
+                                      const float* lse, void* d_x, float* d_gain, void* d_weight,
+                                      float* d_bias, void* workspace, size_t workspace_bytes,
+                                      size_t dz_budget_bytes, int64_t N, int32_t H, int64_t V,
+                                      int64_t vocab_start, int32_t dtype, float temperature,
+                                      int64_t ignore_index, int32_t use_ignore, hipStream_t stream)
+{
+    if (int rc = check_norm(x, gain, N, H, dtype)) return rc;
+    if (V <= 0 || !d_weight || !d_x) return rlk_fail(RLK_ERR_ARG, "d_x and d_weight are both written");
+    if (H % 8 != 0 || (reinterpret_cast<uintptr_t>(weight) & 15) != 0 || (reinterpret_cast<uintptr_t>(d_weight) & 15) != 0)
+        return rlk_fail(RLK_ERR_UNSUPPORTED, "the typed weight gradient takes H % 8 == 0 and 16-byte aligned matrices");
+    size_t need = 0, base = 0;
+    if (int rc = rlk_linear_logp_rmsnorm_bwd_typed_workspace_bytes(N, H, V, dtype, dz_budget_bytes, &need)) return rc;
+    if (int rc = rlk_linear_logp_rmsnorm_bwd_workspace_bytes(N, H, V, dtype, dz_budget_bytes, &base)) return rc;
+    if (!workspace || workspace_bytes < need) return rlk_fail(RLK_ERR_ARG, "workspace too small");
+    float* running = need > base ? reinterpret_cast<float*>(static_cast<char*>(workspace) + up256(base)) : nullptr;
+    return norm_bwd(grad_logp, x, gain, eps, weight, bias, targets, lse, d_x, d_gain, running, d_weight, d_bias,
+                    workspace, base, dz_budget_bytes, N, H, V, vocab_start, dtype, temperature, ignore_index,
+                    use_ignore, stream);
 }
 
 }  // extern "C"

@@ -15,10 +15,11 @@ constexpr float kLn2 = 0.6931471805599453f;
 // (log2(e) / temperature).
 // GENERAL = false: no bias and no masked vocab rows (every tile full), the common case.
 // The target logit is picked up in the same pass that feeds the sum, so the captured value is
-// the very fp32 number that entered the softmax.
+// the very fp32 number that entered the softmax.  `vw` is the slab's first vocab row; targets below
+// `v_own` belong to another tile (a last tile that is shifted back overlaps its neighbour).
 template <bool GENERAL, class AT, class Args>
 __device__ inline void fwd_epilogue(const typename AT::vec (&acc)[AT::TM][AT::TN], const Args& a,
-                                    const float* bias, int vw, int lane, const int (&tgt)[AT::TN],
+                                    const float* bias, int vw, int v_own, int lane, const int (&tgt)[AT::TN],
                                     float (&m)[AT::TN], float (&s)[AT::TN], float (&zt)[AT::TN])
 {
     constexpr int TM = AT::TM, TN = AT::TN, R = AT::kRegs;
@@ -43,7 +44,7 @@ __device__ inline void fwd_epilogue(const typename AT::vec (&acc)[AT::TM][AT::TN
         const float mnew = fmaxf(m[j], tmax);
         const float mref = mnew == -INFINITY ? 0.f : mnew;
         // register index (i * R + r) of the target row in this lane, or -1
-        const int etgt = AT::reg_of_row(tgt[j] - vw, lane);
+        const int etgt = AT::reg_of_row(tgt[j] >= v_own ? tgt[j] - vw : -1, lane);
         // four partial sums (fixed association) keep the exp results off a single add chain; the
         // target capture runs only when some lane of the wavefront owns a target row in this slab
         float ps[4] = {0.f, 0.f, 0.f, 0.f};
@@ -92,6 +93,26 @@ __device__ inline void add_bias(typename AT::vec (&acc)[AT::TM][AT::TN], const f
                 acc[i][j][q * 4 + 3] += b3;
             }
         }
+}
+
+// Rows below `skip` of a finished 256-row tile (M index) become -inf: they belong to the left neighbour
+// of a tile that was shifted back to end at the vocabulary's edge, and exp2 makes them exact zeros, in
+// the softmax sum and in dZ alike.  One more product does it: A holds -inf in k = 0 of those rows, B
+// holds 1 there, everything else is zero.  (Selecting in the accumulators, on a branch or before the
+// first product, cost the forward 28 to 497 spilled registers and 2 % of its time.)
+template <class T>
+__device__ inline void mask_rows(f32x4_t (&acc)[Acc16::TM][Acc16::TN], int slab_row0, int skip, int lane)
+{
+    if (skip <= __builtin_amdgcn_readfirstlane(slab_row0)) return;  // uniform
+    const bool k0 = lane < 16;  // lanes 0 .. 15 hold k = 0 .. 7 of an operand fragment, k = 0 in the low half
+    const u32x4_t one{k0 ? static_cast<uint32_t>(T::from_float(1.f)) : 0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < Acc16::TM; ++i) {
+        const bool out = k0 && slab_row0 + i * 16 + lane < skip;
+        const u32x4_t low{out ? static_cast<uint32_t>(T::from_float(-INFINITY)) : 0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int j = 0; j < Acc16::TN; ++j) acc[i][j] = T::mfma(low, one, acc[i][j]);
+    }
 }
 
 // Tiles of a launch are handed out round by round: workgroup b computes the tiles with linear ids

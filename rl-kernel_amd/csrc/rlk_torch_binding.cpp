@@ -123,6 +123,7 @@ std::vector<at::Tensor> fused_linear_logp_forward_ex(at::Tensor hidden, at::Tens
 // Backward: [d_hidden (input dtype), d_weight (f32), d_bias (f32)], an undefined tensor for every
 // gradient that is not wanted.  weight_grad_out / bias_grad_out: caller-owned fp32 buffers that
 // receive (accumulate: are added) the gradients and are what the call returns in their place.
+// typed_weight: d_weight is a fresh tensor of the weight's type (rlk_linear_logp_bwd_typed).
 std::vector<at::Tensor> fused_linear_logp_backward(at::Tensor grad_logp, at::Tensor hidden, at::Tensor weight,
                                                    at::Tensor target, at::Tensor lse,
                                                    c10::optional<at::Tensor> bias, double temperature,
@@ -130,7 +131,8 @@ std::vector<at::Tensor> fused_linear_logp_backward(at::Tensor grad_logp, at::Ten
                                                    bool need_hidden, bool need_weight, bool need_bias,
                                                    int64_t dz_budget_bytes,
                                                    c10::optional<at::Tensor> weight_grad_out,
-                                                   c10::optional<at::Tensor> bias_grad_out, bool accumulate)
+                                                   c10::optional<at::Tensor> bias_grad_out, bool accumulate,
+                                                   bool typed_weight)
 {
     TORCH_CHECK(hidden.dim() == 2 && weight.dim() == 2, "hidden and weight must be 2D tensors");
     TORCH_CHECK(hidden.is_cuda() && weight.is_cuda(), "hidden and weight must be CUDA tensors");
@@ -151,10 +153,15 @@ std::vector<at::Tensor> fused_linear_logp_backward(at::Tensor grad_logp, at::Ten
     const bool want_bias = has_bias && need_bias;
     at::Tensor d_hidden, d_weight, d_bias, bias_f;
     if (need_hidden) d_hidden = at::empty_like(hidden);
-    if (need_weight) d_weight = weight_grad_out.has_value() && weight_grad_out->defined() ? *weight_grad_out
+    TORCH_CHECK(!typed_weight || (need_weight && !weight_grad_out.has_value() && !bias_grad_out.has_value() &&
+                                  !accumulate),
+                "a typed weight gradient takes no gradient buffers");
+    if (typed_weight)
+        d_weight = at::empty_like(weight);
+    else if (need_weight) d_weight = weight_grad_out.has_value() && weight_grad_out->defined() ? *weight_grad_out
                                                                                           : at::empty({v, hd}, f32);
     if (want_bias) d_bias = bias_grad_out.has_value() && bias_grad_out->defined() ? *bias_grad_out : at::empty({v}, f32);
-    if (d_weight.defined())
+    if (d_weight.defined() && !typed_weight)
         TORCH_CHECK(d_weight.scalar_type() == at::kFloat && d_weight.is_contiguous() && d_weight.numel() == v * hd,
                     "weight_grad_out must be contiguous float32 [V, H]");
     if (d_bias.defined())
@@ -166,9 +173,19 @@ std::vector<at::Tensor> fused_linear_logp_backward(at::Tensor grad_logp, at::Ten
         bias_p = bias_f.data_ptr<float>();
     }
     size_t ws_bytes = 0;
-    TORCH_CHECK(rlk_linear_logp_bwd_workspace_bytes(n, hd, v, dt, static_cast<size_t>(dz_budget_bytes), &ws_bytes) == 0,
-                rlk_last_error());
+    const auto query = typed_weight ? rlk_linear_logp_bwd_typed_workspace_bytes : rlk_linear_logp_bwd_workspace_bytes;
+    TORCH_CHECK(query(n, hd, v, dt, static_cast<size_t>(dz_budget_bytes), &ws_bytes) == 0, rlk_last_error());
     auto ws = at::empty({static_cast<int64_t>(ws_bytes)}, hidden.options().dtype(at::kByte));
+    if (typed_weight) {
+        const int rc = rlk_linear_logp_bwd_typed(
+            g.data_ptr<float>(), hidden.data_ptr(), weight.data_ptr(), bias_p, target.data_ptr<int64_t>(),
+            lse.data_ptr<float>(), d_hidden.defined() ? d_hidden.data_ptr() : nullptr, d_weight.data_ptr(),
+            d_bias.defined() ? d_bias.data_ptr<float>() : nullptr, ws.data_ptr(), static_cast<size_t>(ws.numel()),
+            static_cast<size_t>(dz_budget_bytes), n, hd, v, vocab_start, dt, static_cast<float>(temperature),
+            ignore_index.value_or(0), ignore_index.has_value() ? 1 : 0, current_stream(hidden));
+        TORCH_CHECK(rc == 0, "rlk_linear_logp_bwd_typed: ", rlk_last_error());
+        return {d_hidden, d_weight, d_bias};
+    }
     const int rc = rlk_linear_logp_bwd_accum(
         g.data_ptr<float>(), hidden.data_ptr(), weight.data_ptr(), bias_p, target.data_ptr<int64_t>(),
         lse.data_ptr<float>(), d_hidden.defined() ? d_hidden.data_ptr() : nullptr,
@@ -275,7 +292,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
           pybind11::arg("vocab_start") = 0, pybind11::arg("need_hidden") = true,
           pybind11::arg("need_weight") = true, pybind11::arg("need_bias") = true,
           pybind11::arg("dz_budget_bytes") = 0, pybind11::arg("weight_grad_out") = pybind11::none(),
-          pybind11::arg("bias_grad_out") = pybind11::none(), pybind11::arg("accumulate") = false);
+          pybind11::arg("bias_grad_out") = pybind11::none(), pybind11::arg("accumulate") = false,
+          pybind11::arg("typed_weight") = false);
     m.def("fused_logp_forward_out", &fused_logp_forward_out, "Fused logp out");
     m.def("fused_logp_forward_fp32", &fused_logp_forward_fp32, "Fused logp fp32");
     m.def("fused_logp_forward_indexed_out", &fused_logp_forward_indexed_out, "Fused logp indexed out");

@@ -108,7 +108,7 @@ class _FusedGRPOStepFunction(torch.autograd.Function):
         d_h, d_w, d_b = LL.fused_linear_logp_backward(
             upstream, hidden_2d, w, target_1d, lse, bias_t if ctx.has_bias else None,
             temperature=ctx.temperature, ignore_index=IGNORE_INDEX, need_hidden=need_h,
-            need_weight=need_w, need_bias=need_b)
+            need_weight=need_w, need_bias=need_b, typed_weight=True)
         grad_hidden = d_h.reshape(tuple(ctx.lead_shape) + (hidden_2d.size(1),)) if need_h else None
         grad_weight = d_w.to(ctx.weight_dtype) if need_w else None
         grad_bias = d_b.to(ctx.bias_dtype) if need_b else None

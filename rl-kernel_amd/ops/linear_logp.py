@@ -254,6 +254,13 @@ def fused_norm_linear_logp_forward(
     return logp, lse, err
 
 
+def _typed_weight_ok(hidden_2d: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether the library can write the weight gradient in the weight's own 16-bit type (the sizes and
+    alignments its 16-bit kernels take); otherwise it is fp32 and the caller casts it."""
+    return (weight.dtype in (torch.bfloat16, torch.float16) and weight.size(1) % 8 == 0
+            and hidden_2d.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
+
 @_native.on_tensor_device
 def fused_norm_linear_logp_backward(
     grad_logp: torch.Tensor,
@@ -272,9 +279,11 @@ def fused_norm_linear_logp_backward(
     need_weight: bool = True,
     need_bias: bool = True,
     dz_budget_bytes: int = 0,
+    typed_weight: bool = False,
 ):
     """Raw backward: ``(d_x [N,H] input dtype, d_gain [H] fp32, d_weight [V,H] fp32, d_bias [V]
-    fp32)``; ``d_x`` is the gradient w.r.t. the UN-normalised hidden states."""
+    fp32)``; ``d_x`` is the gradient w.r.t. the UN-normalised hidden states.  ``typed_weight``:
+    ``d_weight`` in the weight's type where the library can write it (see ``_typed_weight_ok``)."""
     lib = _native.load()
     n, h = x_2d.shape
     v = weight.size(0)
@@ -284,16 +293,20 @@ def fused_norm_linear_logp_backward(
     g = grad_logp.reshape(-1).to(torch.float32).contiguous()
     d_x = torch.empty_like(x_2d) if need_x else None
     d_gain = torch.empty(h, device=dev, dtype=torch.float32) if need_gain else None
-    d_weight = torch.empty(v, h, device=dev, dtype=torch.float32) if need_weight else None
+    typed = typed_weight and need_weight and need_x and _typed_weight_ok(x_2d, weight)
+    d_weight = torch.empty(v, h, device=dev, dtype=weight.dtype if typed else torch.float32) \
+        if need_weight else None
     want_bias = bias is not None and need_bias
     d_bias = torch.empty(v, device=dev, dtype=torch.float32) if want_bias else None
     bias_f = None if bias is None else bias.detach().to(torch.float32).contiguous()
     need = _native.ctypes.c_size_t(0)
-    _native.check(lib.rlk_linear_logp_rmsnorm_bwd_workspace_bytes(n, h, v, dt, int(dz_budget_bytes),
-                                                                  _native.ctypes.byref(need)),
+    query = lib.rlk_linear_logp_rmsnorm_bwd_typed_workspace_bytes if typed else \
+        lib.rlk_linear_logp_rmsnorm_bwd_workspace_bytes
+    _native.check(query(n, h, v, dt, int(dz_budget_bytes), _native.ctypes.byref(need)),
                   "norm + linear_logp backward workspace query")
     ws = torch.empty(max(need.value, 256), device=dev, dtype=torch.uint8)
-    rc = lib.rlk_linear_logp_rmsnorm_bwd(
+    call = lib.rlk_linear_logp_rmsnorm_bwd_typed if typed else lib.rlk_linear_logp_rmsnorm_bwd
+    rc = call(
         _ptr(g), _ptr(x_2d), _ptr(gain), float(eps), _ptr(weight), _ptr(bias_f), _ptr(target_1d),
         _ptr(lse), _ptr(d_x), _ptr(d_gain), _ptr(d_weight), _ptr(d_bias), _ptr(ws), ws.numel(),
         int(dz_budget_bytes), n, h, v, 0, dt, float(temperature),
@@ -321,6 +334,7 @@ def fused_linear_logp_backward(
     weight_grad_out: Optional[torch.Tensor] = None,
     bias_grad_out: Optional[torch.Tensor] = None,
     accumulate: bool = False,
+    typed_weight: bool = False,
 ):
     """Raw backward: ``(d_hidden [N,H] input dtype, d_weight [V,H] fp32, d_bias [V] fp32)``.
 
@@ -332,6 +346,9 @@ def fused_linear_logp_backward(
     receive the gradients instead of fresh tensors (they are what the call returns);
     ``accumulate`` adds to what they hold instead of overwriting it, as the reference keeps one
     fp32 ``grad_w`` over its token chunks (same file :404,423-437).
+
+    ``typed_weight``: ``d_weight`` in the weight's type, rounded once from the fp32 sum by the kernel
+    that finishes it, where the library can write it (see ``_typed_weight_ok``; fp32 otherwise).
     """
     lib = _native.load()
     n, h = hidden_2d.shape
@@ -345,6 +362,8 @@ def fused_linear_logp_backward(
         _check_grad_buffer("bias_grad_out", bias_grad_out, (v,), dev)
     if accumulate and ((need_weight and weight_grad_out is None) or (want_bias and bias_grad_out is None)):
         raise ValueError("accumulate=True needs the buffers to add to (weight_grad_out / bias_grad_out)")
+    typed = typed_weight and need_weight and weight_grad_out is None and bias_grad_out is None \
+        and not accumulate and _typed_weight_ok(hidden_2d, weight)
     compiled = _compiled.module()
     if compiled is not None and hidden_2d.is_contiguous() and weight.is_contiguous() \
             and target_1d.dtype == torch.long and target_1d.is_contiguous() \
@@ -352,24 +371,32 @@ def fused_linear_logp_backward(
         d_hidden, d_weight, d_bias = compiled.fused_linear_logp_backward(
             grad_logp, hidden_2d, weight, target_1d, lse, bias, float(temperature), ignore_index,
             int(vocab_start), bool(need_hidden), bool(need_weight), bool(want_bias),
-            int(dz_budget_bytes), weight_grad_out, bias_grad_out, bool(accumulate))
+            int(dz_budget_bytes), weight_grad_out, bias_grad_out, bool(accumulate), typed)
         return d_hidden, d_weight, d_bias
     g = grad_logp.reshape(-1).to(torch.float32).contiguous()
     d_hidden = torch.empty_like(hidden_2d) if need_hidden else None
     d_weight = None
     if need_weight:
         d_weight = weight_grad_out if weight_grad_out is not None else \
-            torch.empty(v, h, device=dev, dtype=torch.float32)
+            torch.empty(v, h, device=dev, dtype=weight.dtype if typed else torch.float32)
     d_bias = None
     if want_bias:
         d_bias = bias_grad_out if bias_grad_out is not None else \
             torch.empty(v, device=dev, dtype=torch.float32)
     bias_f = None if bias is None else bias.detach().to(torch.float32).contiguous()
     need = _native.ctypes.c_size_t(0)
-    _native.check(lib.rlk_linear_logp_bwd_workspace_bytes(n, h, v, dt, int(dz_budget_bytes),
-                                                          _native.ctypes.byref(need)),
+    query = lib.rlk_linear_logp_bwd_typed_workspace_bytes if typed else lib.rlk_linear_logp_bwd_workspace_bytes
+    _native.check(query(n, h, v, dt, int(dz_budget_bytes), _native.ctypes.byref(need)),
                   "linear_logp backward workspace query")
     ws = torch.empty(need.value, device=dev, dtype=torch.uint8)
+    if typed:
+        rc = lib.rlk_linear_logp_bwd_typed(
+            _ptr(g), _ptr(hidden_2d), _ptr(weight), _ptr(bias_f), _ptr(target_1d), _ptr(lse),
+            _ptr(d_hidden), _ptr(d_weight), _ptr(d_bias), _ptr(ws), ws.numel(), int(dz_budget_bytes),
+            n, h, v, int(vocab_start), dt, float(temperature),
+            0 if ignore_index is None else int(ignore_index), int(ignore_index is not None), _stream(dev))
+        _native.check(rc, "rlk_linear_logp_bwd_typed")
+        return d_hidden, d_weight, d_bias
     rc = lib.rlk_linear_logp_bwd_accum(
         _ptr(g), _ptr(hidden_2d), _ptr(weight), _ptr(bias_f), _ptr(target_1d), _ptr(lse),
         _ptr(d_hidden), _ptr(d_weight), _ptr(d_bias), _ptr(ws), ws.numel(), int(dz_budget_bytes),
@@ -446,7 +473,7 @@ class _FusedLinearLogpFunction(torch.autograd.Function):
             grad_logp, hidden_2d, w, target_1d, lse, bias_t if ctx.has_bias else None,
             temperature=ctx.temperature, ignore_index=ctx.ignore_index,
             need_hidden=need_h, need_weight=want_w, need_bias=want_b,
-            weight_grad_out=w_buf, bias_grad_out=b_buf, accumulate=adding)
+            weight_grad_out=w_buf, bias_grad_out=b_buf, accumulate=adding, typed_weight=w_out is None)
         grad_hidden = d_h.reshape(tuple(ctx.lead_shape) + (hidden_2d.size(1),)) if need_h else None
         grad_weight = d_w.to(ctx.weight_dtype) if need_w and w_out is None else None
         grad_bias = d_b.to(ctx.bias_dtype) if need_b and b_out is None else None
@@ -491,7 +518,7 @@ class _FusedNormLinearLogpFunction(torch.autograd.Function):
         d_x, d_g, d_w, d_b = fused_norm_linear_logp_backward(
             grad_logp, x_2d, g, w, target_1d, lse, bias_t if ctx.has_bias else None, eps=ctx.eps,
             temperature=ctx.temperature, ignore_index=ctx.ignore_index, need_x=need_x,
-            need_gain=need_g, need_weight=need_w, need_bias=need_b)
+            need_gain=need_g, need_weight=need_w, need_bias=need_b, typed_weight=True)
         return (d_x.reshape(tuple(ctx.lead_shape) + (x_2d.size(1),)) if need_x else None,
                 d_g.to(ctx.gain_dtype) if need_g else None,
                 d_w.to(ctx.weight_dtype) if need_w else None,
