@@ -260,6 +260,50 @@ __device__ inline float combine_token(const CombineArgs& a, int64_t n)
     return lp;
 }
 
+// Many splits (few tokens): 16 tokens x 16 split groups per workgroup fetch the partial states side by
+// side, then one thread per token adds the rescaled sums in split order, as combine_token would; the
+// merged state replaces the token's slot 0, which the combine kernels read as their only split.  One
+// thread walking all splits of a token through memory is a chain of dependent loads: 37 us for 160
+// tokens x 62 splits.  LDS: the terms [2][n_split][16] behind the group maxima [16][16].
+constexpr int kMergeTokens = 16, kMergeGroups = 16;
+inline size_t merge_smem(int n_split) { return static_cast<size_t>(kMergeGroups + 2 * n_split) * kMergeTokens * 4; }
+__global__ __launch_bounds__(256) void linear_logp_merge_kernel(float* part_m, float* part_s, float* part_z, int N,
+                                                                int n_split)
+{
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    float* gmax = reinterpret_cast<float*>(smem);
+    float* term_s = gmax + kMergeGroups * kMergeTokens;
+    float* term_z = term_s + n_split * kMergeTokens;
+    const int tx = threadIdx.x % kMergeTokens, g = threadIdx.x / kMergeTokens;
+    const int n = blockIdx.x * kMergeTokens + tx;
+    const bool live = n < N;
+    float mm = -INFINITY;
+    if (live)
+        for (int sp = g; sp < n_split; sp += kMergeGroups) mm = fmaxf(mm, part_m[static_cast<int64_t>(sp) * N + n]);
+    gmax[g * kMergeTokens + tx] = mm;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kMergeGroups; ++k) mm = fmaxf(mm, gmax[k * kMergeTokens + tx]);
+    if (live)
+        for (int sp = g; sp < n_split; sp += kMergeGroups) {
+            const int64_t o = static_cast<int64_t>(sp) * N + n;
+            term_s[sp * kMergeTokens + tx] = part_s[o] * exp2f(part_m[o] - mm);
+            term_z[sp * kMergeTokens + tx] = part_z[o];
+        }
+    __syncthreads();  // also: every read of slot 0 of these tokens is behind us
+    if (g == 0 && live) {
+        float ss = 0.f, zz = 0.f;
+#pragma unroll 8
+        for (int sp = 0; sp < n_split; ++sp) {
+            ss += term_s[sp * kMergeTokens + tx];
+            zz += term_z[sp * kMergeTokens + tx];
+        }
+        part_m[n] = mm;
+        part_s[n] = ss;
+        part_z[n] = zz;
+    }
+}
+
 __global__ void linear_logp_combine_kernel(CombineArgs a)
 {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1029,7 +1073,10 @@ int patch_rows_for(int H)
 // wins, a smaller one when it is within 1.5 %, among the counts that leave every workgroup a run of
 // at least 8 tiles and keep the split partials (12 bytes per token and split) within the 8 MiB the
 // allocation-free entry point has; measured over 4 - 32 splits at 48 - 243 token blocks, this
-// choice is within 1.5 % of the best count tried.
+// choice is within 1.5 % of the best count tried.  As long as the launch does not fill one round of
+// the chip, shorter runs are taken too (from 64 tiles on; smaller vocabularies keep the runs and with
+// them one grouping of the sums for a batch and its micro-batches): one block of 160 tokens x 501 tiles at H = 4096 ran 62
+// workgroups of 8 - 9 tiles in 741 us and runs 251 of two in 250 us.
 int split_count(int row_blocks, int tiles, int patch_rows)
 {
     if (tiles <= 0) return 0;
@@ -1039,14 +1086,15 @@ int split_count(int row_blocks, int tiles, int patch_rows)
     // token blocks, 2 or 3 splits ran at 1160 - 1190 TFLOP/s where 4 ran at 1383.
     const int want = 32 / patch_rows;
     const int lo = tiles >= want * 16 ? want : 1;
-    int hi = tiles < 64 ? tiles : 64;
+    const int most = row_blocks < 4 ? 256 / row_blocks : 64;
+    int hi = tiles < most ? tiles : most;
     const int64_t fit = static_cast<int64_t>(RLK_STATIC_SCRATCH_BYTES) / (3072LL * row_blocks);
     if (hi > fit) hi = fit > lo ? static_cast<int>(fit) : lo;
     int best = lo;
     int64_t best_cost = -1;
     for (int s = lo; s <= hi; ++s) {
         const int64_t run = (tiles + s - 1) / s;
-        if (s > lo && run < 8) break;
+        if (s > lo && run < 8 && (tiles < 64 || static_cast<int64_t>(row_blocks) * s > 256)) break;
         const int64_t rounds = (static_cast<int64_t>(row_blocks) * s + 255) / 256;
         const int64_t cost = rounds * (2 * run + 1);
         // a larger count has to be 1.5 % better than the best smaller one to replace it
@@ -1851,6 +1899,18 @@ int fwd_enqueue(const void* hidden, const void* weight, const float* bias, const
     c.ignore_index = ignore_index;
     c.use_ignore = use_ignore;
     c.strict = strict_targets;
+    // from 16 splits on the partials are merged by a launch of their own (up to there one thread per
+    // token takes at most as long as that launch)
+    if (plan.total_splits >= 16) {
+        const dim3 blocks((a.N + kMergeTokens - 1) / kMergeTokens);
+        const size_t lds = merge_smem(plan.total_splits);  // at most 256 splits: 33 KiB
+        hipLaunchKernelGGL(linear_logp_merge_kernel, blocks, dim3(256), lds, stream, a.part_m, a.part_s, a.part_z, a.N,
+                           plan.total_splits);
+        if (second != nullptr)
+            hipLaunchKernelGGL(linear_logp_merge_kernel, blocks, dim3(256), lds, stream, a.part2_m, a.part2_s,
+                               a.part2_z, a.N, plan.total_splits);
+        c.n_split = 1;
+    }
     if (second != nullptr) {  // the reference head: same merge, never strict
         CombineArgs c2 = c;
         c2.part_m = a.part2_m;
