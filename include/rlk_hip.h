@@ -76,8 +76,9 @@ int rlk_device_info(int32_t device, int32_t* compute_units, int32_t* max_clock_k
  *            With strict_targets == 0 such a row yields logp = -lse (z_t = 0), which is what a
  *            vocab-parallel shard must return (csrc/cuda/fused_linear_logp_sm90.cu:256-280).
  *   dtype: RLK_DTYPE_BF16 / RLK_DTYPE_F16 with H % 8 == 0 and 16-byte aligned matrices run on the
- *   16-bit MFMA tiles; RLK_DTYPE_F32, other H or misaligned matrices run on the fp32 matrix
- *   instruction (operands widened to fp32 on the way into LDS, same tiling, any N, H, V >= 1) --
+ *   16-bit MFMA tiles; RLK_DTYPE_F32, other H or misaligned matrices run on the fp32
+ *   kernels (operands widened to fp32 on the way into LDS and multiplied to fp32 accuracy, same tiling,
+ *   any N, H, V >= 1) --
  *   the counterpart of the reference's "unsupported dtype/shape falls back to the portable op"
  *   (rl_engine/kernels/ops/cuda/loss/linear_logp.py:45-55,350-351), except that here the
  *   portable op is a matrix-core HIP kernel too.  Every forward entry point below (static

@@ -1,8 +1,9 @@
 // fp32 matrix-core kernels of the fused linear-logprob path for inputs the 16-bit MFMA tiles do
 // not take: fp32 tensors, hidden sizes that are not a multiple of 8, matrices that do not start on
 // a 16-byte boundary.  Every operand is widened to fp32 on its way into LDS (exact for bf16 and
-// f16) and multiplied with v_mfma_f32_32x32x2_f32, so products and sums are plain fp32 and the
-// results follow the reference's fp32 arithmetic.  Same workgroup tile (256 x 256, 2 x 4
+// f16) and multiplied as three bf16 pieces (SplitGemm below; v_mfma_f32_32x32x2_f32 where an infinity or
+// NaN is in the way), so products are fp32 to the last bit or two, sums are fp32, and the results follow
+// the reference's fp32 arithmetic.  Same workgroup tile (256 x 256, 2 x 4
 // wavefronts), same accumulator layout and same split / combine structure as the 16-bit kernels;
 // dZ stays fp32.  All loads are clamped or masked element by element, so any N, H, V >= 1 and any
 // element alignment is accepted.  All reductions run in a fixed order: same input, same bits.
@@ -305,6 +306,203 @@ struct WideGemm {
     }
 };
 
+// The same contraction on the 16-bit matrix instruction, to fp32 accuracy.  Every element is cut into
+// three bf16 pieces on its way into LDS, x = hi + mid + lo exactly (8 bits each: hi by truncation, so it
+// cannot overflow, mid and lo by rounding the remainders), and a product is the sum of the six piece
+// products down to 2^-16 of it; the three that are left out stay below 2^-22 of a product, most of
+// them far below and with random sign, so the roundings of the running fp32 sums decide the error, and
+// one instruction adds 16 products where the fp32 one adds two: error against 64 bits, start of the
+// comparison = v_mfma_f32_32x32x2_f32, 2048 x 2048 x 32768: logp 6.7e-7 -> 5.7e-7, dH 1.6e-6 -> 1.0e-6, dW
+// 8.1e-7 -> 5.0e-7.  (The five small products in a sum of their own: 7e-7, but 300 spilled registers
+// and 13 % slower.)  Bound: the matrix pipe under the board's power limit at six 16-bit products (1450
+// TFLOP/s sustained / 6 = 240) against 157 TFLOP/s peak of the fp32 instruction; the same shape
+// forward + backward 8.35 -> 5.04 ms.
+// An infinity or NaN in an operand tile has no such pieces (inf * 0 in the small products): the
+// workgroup sees it while it converts and computes that tile again on the fp32 instruction.
+//
+//   K-contiguous: LDS [256 rows][3 pieces][16 k]; rows 96 bytes apart: eight rows start in eight
+//                 different 16-byte chunks of the 256-byte bank line
+//   K-major:      LDS [3 pieces][16 k][256 rows], chunks of k-line k moved by 4 (k & 3): the four k-lines
+//                 x 64 bytes of a transposing read cover every bank once
+struct Pieces {
+    u32x2_t hi, mid, lo;  // four elements each
+};
+
+__device__ inline Pieces split3(f32x4_t v, float& bad)
+{
+    Pieces p;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const float x0 = v[2 * h], x1 = v[2 * h + 1];
+        // 0 * finite = 0: stays 0 until the first infinity or NaN
+        bad = fmaf(x0, 0.f, bad);
+        bad = fmaf(x1, 0.f, bad);
+        const uint32_t b0 = __builtin_bit_cast(uint32_t, x0), b1 = __builtin_bit_cast(uint32_t, x1);
+        const uint32_t hi = (b0 >> 16) | (b1 & 0xffff0000u);
+        const float r0 = x0 - __builtin_bit_cast(float, b0 & 0xffff0000u);
+        const float r1 = x1 - __builtin_bit_cast(float, b1 & 0xffff0000u);
+        const uint32_t mid = Bf16::pack2(r0, r1);
+        const float q0 = r0 - __builtin_bit_cast(float, mid << 16);
+        const float q1 = r1 - __builtin_bit_cast(float, mid & 0xffff0000u);
+        p.hi[h] = hi;
+        p.mid[h] = mid;
+        p.lo[h] = Bf16::pack2(q0, q1);
+    }
+    return p;
+}
+
+template <bool KMAJOR>
+struct SplitLds {
+    static constexpr int kPiece = KMAJOR ? kWBK * 512 : 32;  // bytes between the pieces of an element
+    static constexpr int kBytes = 256 * 3 * kWBK * 2;
+
+    __device__ static inline void store(char* lds, const Pieces& v, int g)
+    {
+        const int idx = g * kThreads + static_cast<int>(threadIdx.x);
+        const int k = idx >> 6, q = idx & 63;  // K-major: k-line, group of four rows
+        char* at = lds + (KMAJOR ? k * 512 + ((q >> 1) ^ ((k & 3) << 2)) * 16 + (q & 1) * 8
+                                 : (idx >> 2) * 96 + (idx & 3) * 8);
+        *reinterpret_cast<u32x2_t*>(at) = v.hi;
+        *reinterpret_cast<u32x2_t*>(at + kPiece) = v.mid;
+        *reinterpret_cast<u32x2_t*>(at + 2 * kPiece) = v.lo;
+    }
+
+    // MFMA 32x32x16 operand fragment: lane l holds row (row0 + l % 32), k = 8 (l / 32) + 0..7
+    // (row0 a multiple of 32).
+    __device__ static inline bf16x8_t frag(const char* lds, int row0, int piece)
+    {
+        const int l = threadIdx.x & 63;
+        if (KMAJOR) {
+            const int a = (l & 15) >> 2, b = l & 3;  // see TileIO::frag
+            const int c = (row0 >> 3) + 2 * ((l >> 4) & 1) + (b >> 1);
+            const char* p0 = lds + piece * kPiece + (8 * (l >> 5) + a) * 512 + (c ^ (a << 2)) * 16 + (b & 1) * 8;
+            const s16x4_t x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((RLK_LDS s16x4_t*)(p0));
+            const s16x4_t y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((RLK_LDS s16x4_t*)(p0 + 4 * 512));
+            const u32x2_t x2 = __builtin_bit_cast(u32x2_t, x), y2 = __builtin_bit_cast(u32x2_t, y);
+            return __builtin_bit_cast(bf16x8_t, u32x4_t{x2.x, x2.y, y2.x, y2.y});
+        } else {
+            return *reinterpret_cast<const bf16x8_t*>(lds + (row0 + (l & 31)) * 96 + piece * kPiece + 16 * (l >> 5));
+        }
+    }
+};
+
+template <int DTA, int DTB, bool A_KMAJOR, bool B_KMAJOR>
+struct SplitGemm {
+    using Exact = WideGemm<DTA, DTB, A_KMAJOR, B_KMAJOR>;
+    using IOA = typename Exact::IOA;
+    using IOB = typename Exact::IOB;
+    using LA = SplitLds<A_KMAJOR>;
+    using LB = SplitLds<B_KMAJOR>;
+    static constexpr int kStageBytes = LA::kBytes + LB::kBytes;
+    static constexpr int kStages = 3;
+    static constexpr int kSmemBytes = kStages * kStageBytes;
+    static_assert(kSmemBytes >= Exact::kSmemBytes, "the fp32 loop runs in the same LDS");
+    typedef bf16x8_t Frag[3];  // hi, mid, lo
+
+    __device__ static inline void run(const WideOperand& A, const WideOperand& B, int K,
+                                      f32x16_t (&acc)[kTM][kTN], char* smem)
+    {
+        float bad;
+        if (IOA::fast_ok(A, K) && IOB::fast_ok(B, K))  // uniform
+            bad = run_impl<true>(A, B, K, acc, smem);
+        else
+            bad = run_impl<false>(A, B, K, acc, smem);
+        if (__syncthreads_or(bad != bad)) {
+            zero_acc(acc);
+            Exact::template run_impl<false>(A, B, K, acc, smem);
+        }
+    }
+
+    // One 32 x 32 tile's share of a stage.
+    __device__ static inline void product(const Frag& a, const Frag& b, f32x16_t& acc)
+    {
+        auto mul = [](bf16x8_t x, bf16x8_t y, f32x16_t c) {
+            return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0);
+        };
+        acc = mul(a[2], b[0], acc);
+        acc = mul(a[0], b[2], acc);
+        acc = mul(a[1], b[1], acc);
+        acc = mul(a[1], b[0], acc);
+        acc = mul(a[0], b[1], acc);
+        acc = mul(a[0], b[0], acc);
+    }
+
+    // Stage kt multiplies while stage kt + 2 is converted into the LDS stage that kt - 1 has left and
+    // the first fragments of stage kt + 1 (published by the last barrier) are read, so that neither
+    // conversions nor LDS latency stand in front of the matrix work behind a barrier.
+    // Returns a value that is NaN when this thread met an infinity or NaN.
+    template <bool FAST>
+    __device__ static inline float run_impl(const WideOperand& A, const WideOperand& B, int K,
+                                            f32x16_t (&acc)[kTM][kTN], char* smem)
+    {
+        IOA la;
+        IOB lb;
+        la.init(A, K, FAST);
+        lb.init(B, K, FAST);
+        const int wave = threadIdx.x >> 6;
+        const int ra0 = (wave / kWN) * (kTM * 32), rb0 = (wave % kWN) * (kTN * 32);
+        const int nk = (K + kWBK - 1) / kWBK;
+        float bad = 0.f;
+        f32x4_t reg[4];  // groups 0, 1 of A and 0, 1 of B
+        auto fetch = [&](int kt, int n) {
+            reg[n] = n < 2 ? la.template load<FAST>(kt, n) : lb.template load<FAST>(kt, n - 2);
+        };
+        auto convert = [&](char* stage, int n) {
+            if (n < 2)
+                LA::store(stage, split3(reg[n], bad), n);
+            else
+                LB::store(stage + LA::kBytes, split3(reg[n], bad), n - 2);
+        };
+        auto stage_at = [&](int st) { return smem + st * kStageBytes; };
+        // stages 0 and 1 in LDS, stage 2 on its way (past the last stage: the last one again)
+        for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+            for (int n = 0; n < 4; ++n) fetch(min(kt, nk - 1), n);
+#pragma unroll
+            for (int n = 0; n < 4; ++n) convert(stage_at(kt), n);
+        }
+#pragma unroll
+        for (int n = 0; n < 4; ++n) fetch(min(2, nk - 1), n);
+        __syncthreads();
+        Frag fa[2], fb[kTN];
+        auto read_a = [&](Frag& f, const char* stage, int i) {
+#pragma unroll
+            for (int p = 0; p < 3; ++p) f[p] = LA::frag(stage, ra0 + i * 32, p);
+        };
+        auto read_b = [&](Frag& f, const char* stage, int j) {
+#pragma unroll
+            for (int p = 0; p < 3; ++p) f[p] = LB::frag(stage + LA::kBytes, rb0 + j * 32, p);
+        };
+#pragma unroll
+        for (int j = 0; j < kTN; ++j) read_b(fb[j], stage_at(0), j);
+        read_a(fa[0], stage_at(0), 0);
+        int cur = 0;
+        for (int kt = 0; kt < nk; ++kt) {
+            const int nxt = cur + 1 == kStages ? 0 : cur + 1, dst = nxt + 1 == kStages ? 0 : nxt + 1;
+            const int ahead = min(kt + 3, nk - 1);
+            static_for<0, kTM>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                if constexpr (i + 1 < kTM)
+                    read_a(fa[(i + 1) & 1], stage_at(cur), i + 1);
+                else
+                    read_a(fa[(i + 1) & 1], stage_at(nxt), 0);
+                static_for<0, kTN>([&](auto jc) {
+                    constexpr int j = decltype(jc)::value;
+                    product(fa[i & 1], fb[j], acc[i][j]);
+                    if constexpr (i + 1 == kTM) read_b(fb[j], stage_at(nxt), j);
+                    if constexpr (j == 0) {
+                        convert(stage_at(dst), i);
+                        fetch(ahead, i);
+                    }
+                });
+            });
+            __syncthreads();
+            cur = nxt;
+        }
+        return bad;
+    }
+};
+
 // ------------------------------------------------------------------------------------------- //
 // Forward: partial softmax states of one (256-token block) x (range of vocab tiles)
 // ------------------------------------------------------------------------------------------- //
@@ -330,7 +528,7 @@ struct WideFwdArgs {
 template <int DT>
 __global__ __launch_bounds__(kThreads) void wide_fwd_kernel(WideFwdArgs a)
 {
-    using Gemm = WideGemm<DT, DT, false, false>;
+    using Gemm = SplitGemm<DT, DT, false, false>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     int tb, sp;
     xcd_tile(blockIdx.x, a.row_blocks * a.n_split, a.row_blocks, a.n_split, 8, tb, sp);
@@ -437,7 +635,7 @@ struct WideDzArgs {
 template <int DT>
 __global__ __launch_bounds__(kThreads) void wide_dz_kernel(WideDzArgs a)
 {
-    using Gemm = WideGemm<DT, DT, false, false>;
+    using Gemm = SplitGemm<DT, DT, false, false>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -515,7 +713,7 @@ struct WideDhArgs {
 template <int DT>
 __global__ __launch_bounds__(kThreads) void wide_dh_kernel(WideDhArgs a)
 {
-    using Gemm = WideGemm<DT, RLK_DTYPE_F32, true, false>;
+    using Gemm = SplitGemm<DT, RLK_DTYPE_F32, true, false>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tiles = a.h_tiles * a.tok_tiles;
     const int slot = blockIdx.x / tiles;
@@ -592,7 +790,7 @@ struct WideDwArgs {
 template <int DT>
 __global__ __launch_bounds__(kThreads) void wide_dw_kernel(WideDwArgs a)
 {
-    using Gemm = WideGemm<DT, RLK_DTYPE_F32, true, true>;
+    using Gemm = SplitGemm<DT, RLK_DTYPE_F32, true, true>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -712,7 +910,7 @@ WidePlan wide_plan(int64_t N, int32_t H, int64_t V, size_t budget)
 template <int DT>
 int wide_fwd_launch(const WideFwdArgs& a, hipStream_t stream)
 {
-    using G = WideGemm<DT, DT, false, false>;
+    using G = SplitGemm<DT, DT, false, false>;
     if (int rc = wide_smem(wide_fwd_kernel<DT>, G::kSmemBytes)) return rc;
     hipLaunchKernelGGL(wide_fwd_kernel<DT>, dim3(a.row_blocks * a.n_split), dim3(kThreads), G::kSmemBytes,
                        stream, a);
@@ -726,9 +924,9 @@ int wide_bwd_launch(const float* grad_logp, const void* hidden, const void* weig
                     int64_t vocab_start, float temperature, int64_t ignore_index, int32_t use_ignore,
                     int32_t accumulate, hipStream_t stream)
 {
-    using GZ = WideGemm<DT, DT, false, false>;
-    using GH = WideGemm<DT, RLK_DTYPE_F32, true, false>;
-    using GW = WideGemm<DT, RLK_DTYPE_F32, true, true>;
+    using GZ = SplitGemm<DT, DT, false, false>;
+    using GH = SplitGemm<DT, RLK_DTYPE_F32, true, false>;
+    using GW = SplitGemm<DT, RLK_DTYPE_F32, true, true>;
     if (int rc = wide_smem(wide_dz_kernel<DT>, GZ::kSmemBytes)) return rc;
     if (int rc = wide_smem(wide_dh_kernel<DT>, GH::kSmemBytes)) return rc;
     if (int rc = wide_smem(wide_dw_kernel<DT>, GW::kSmemBytes)) return rc;
