@@ -42,8 +42,8 @@ enum {
 };
 
 /* ABI version of this header (major * 100 + minor): 102 (100 + rlk_device_info,
- * rlk_linear_logp_fwd_plan and the typed weight gradients, rlk_linear_logp_bwd_typed and
- * rlk_linear_logp_rmsnorm_bwd_typed). */
+ * rlk_linear_logp_fwd_plan, the typed weight gradients rlk_linear_logp_bwd_typed and
+ * rlk_linear_logp_rmsnorm_bwd_typed, and rlk_check_targets). */
 int rlk_version(void);
 
 /* Message of the last error returned on the calling thread ("" if none). Host pointer, valid
@@ -283,6 +283,13 @@ int rlk_linear_logp_rmsnorm_bwd_typed(const float* grad_logp, const void* x, con
                                       size_t dz_budget_bytes, int64_t N, int32_t H, int64_t V,
                                       int64_t vocab_start, int32_t dtype, float temperature,
                                       int64_t ignore_index, int32_t use_ignore, rlk_stream_t stream);
+
+/* Range check of token ids ahead of a launch that uses them: *out_of_range = 1 when some id lies outside
+ * [0, vocab) and is neither the ignore index (use_ignore != 0) nor at a position whose mask is 0 (mask
+ * uint8 [n] or NULL), else 0.  out_of_range may be pinned host memory: a caller that waits for this
+ * launch alone can raise while the contraction behind it is still running. */
+int rlk_check_targets(const int64_t* targets, const uint8_t* mask, int64_t n, int64_t vocab,
+                      int64_t ignore_index, int32_t use_ignore, int32_t* out_of_range, rlk_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------ *
  * Selected-token log-prob from materialised logits (the `fused_logp` family).

@@ -59,6 +59,7 @@ SIGNATURES = {
     "rlk_linear_logp_rmsnorm_bwd_typed": (_c.c_int, [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _vp,
                                                      _vp, _vp, _vp, _sz, _sz, _i64, _i32, _i64, _i64,
                                                      _i32, _f32, _i64, _i32, _vp]),
+    "rlk_check_targets": (_c.c_int, [_vp, _vp, _i64, _i64, _i64, _i32, _vp, _vp]),
     "rlk_logp_from_logits": (_c.c_int, [_vp, _i32, _vp, _vp, _i32, _vp, _vp, _i64, _i64, _i64, _vp]),
     "rlk_logp_from_logits_pair": (_c.c_int, [_vp, _vp, _i32, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i64,
                                              _i64, _i64, _vp]),
@@ -122,6 +123,36 @@ def check(rc: int, what: str) -> None:
     if rc == -2:
         raise NotImplementedError(f"{what}: {msg}")
     raise RuntimeError(f"{what}: {msg} (code {rc})")
+
+
+class TargetCheck:
+    """Range check of token ids that a caller raises on without waiting for the launches behind it: the
+    check is the first launch of the call and writes pinned host memory, the contraction follows, and
+    ``out_of_range()`` waits for the check alone, so that whatever the caller enqueues next (the
+    backward, as a rule) is on its way while the contraction runs.  ``out_of_range()`` has to be called
+    on every path: it is also what keeps the host word alive until the launch has written it."""
+
+    def __init__(self, ids, vocab, *, mask=None, ignore_index=None):
+        import torch
+
+        self._event = None
+        if ids.numel() == 0:
+            return
+        with torch.cuda.device(ids.device):
+            stream = torch.cuda.current_stream(ids.device)
+            self._flag = torch.empty(1, dtype=torch.int32, pin_memory=True)
+            check(load().rlk_check_targets(
+                ids.data_ptr(), None if mask is None else mask.data_ptr(), ids.numel(), int(vocab),
+                0 if ignore_index is None else int(ignore_index), int(ignore_index is not None),
+                self._flag.data_ptr(), stream.cuda_stream), "rlk_check_targets")
+            self._event = torch.cuda.Event()
+            self._event.record(stream)
+
+    def out_of_range(self) -> bool:
+        if self._event is None:
+            return False
+        self._event.synchronize()
+        return bool(self._flag[0])
 
 
 def on_tensor_device(fn):

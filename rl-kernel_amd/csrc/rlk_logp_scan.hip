@@ -216,9 +216,37 @@ __global__ __launch_bounds__(kScanThreads) void logp_scan_bwd_kernel(
     for (int64_t v = tail0 + t; v < vocab; v += kScanThreads) g[v] = value(v, x[v]);
 }
 
+// One workgroup: token ids are a few hundred KiB at most and are read once.
+constexpr int kCheckThreads = 1024;
+__global__ __launch_bounds__(kCheckThreads) void check_targets_kernel(const int64_t* ids, const uint8_t* mask,
+                                                                      int64_t n, int64_t vocab, int64_t ignore_index,
+                                                                      int use_ignore, int32_t* out)
+{
+    int bad = 0;
+#pragma unroll 8
+    for (int64_t i = threadIdx.x; i < n; i += kCheckThreads) {
+        const int64_t id = ids[i];
+        const bool on = mask == nullptr || mask[i] != 0;
+        bad |= on && !(use_ignore && id == ignore_index) && (id < 0 || id >= vocab);
+    }
+    bad = __syncthreads_or(bad);
+    if (threadIdx.x == 0) *out = bad ? 1 : 0;
+}
+
 }  // namespace rlk
 
 using namespace rlk;
+
+extern "C" int rlk_check_targets(const int64_t* targets, const uint8_t* mask, int64_t n, int64_t vocab,
+                                 int64_t ignore_index, int32_t use_ignore, int32_t* out_of_range, hipStream_t stream)
+{
+    if (!targets || !out_of_range) return rlk_fail(RLK_ERR_ARG, "null pointer");
+    if (n < 0 || vocab <= 0) return rlk_fail(RLK_ERR_ARG, "bad sizes");
+    hipLaunchKernelGGL(check_targets_kernel, dim3(1), dim3(kCheckThreads), 0, stream, targets, mask, n, vocab,
+                       ignore_index, use_ignore, out_of_range);
+    if (hipGetLastError() != hipSuccess) return rlk_fail(RLK_ERR_LAUNCH, "target check launch failed");
+    return 0;
+}
 
 extern "C" int rlk_logp_from_logits_bwd(const void* logits, int32_t logits_dtype, const int64_t* ids,
                                         const float* lse, const float* coeff, void* grad_logits,

@@ -81,11 +81,10 @@ class _FusedGRPOStepFunction(torch.autograd.Function):
         w = LL._aligned_contiguous(weight)
         target_1d = marked_ids.reshape(-1).to(device=hidden_2d.device, dtype=torch.long).contiguous()
         seq_len = hidden.shape[-2] if hidden.dim() >= 2 else 1
-        logp, lse, err, out3, _, _, dcur, dkl = fused_linear_logp_grpo_forward(
-            hidden_2d, w, target_1d, bias, old, ref, adv, mask, seq_len=seq_len, clip_eps=clip_eps,
-            beta=beta, temperature=temperature, ignore_index=IGNORE_INDEX)
-        if check_targets and bool(err.item()):
-            raise LL._out_of_range_error(target_1d, w.size(0), IGNORE_INDEX)
+        with LL._checked_targets(target_1d, w.size(0), IGNORE_INDEX, check_targets):
+            logp, lse, _, out3, _, _, dcur, dkl = fused_linear_logp_grpo_forward(
+                hidden_2d, w, target_1d, bias, old, ref, adv, mask, seq_len=seq_len, clip_eps=clip_eps,
+                beta=beta, temperature=temperature, ignore_index=IGNORE_INDEX)
         ctx.save_for_backward(hidden_2d, w, bias if bias is not None else hidden_2d, target_1d, lse,
                               dcur, dkl)
         ctx.has_bias = bias is not None

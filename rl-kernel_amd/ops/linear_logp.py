@@ -10,6 +10,7 @@ conventions of rl_engine/testing/reference_ops.py:15-47 into the kernel: ``tempe
 
 from __future__ import annotations
 
+import contextlib
 from typing import Any, Optional
 
 import torch
@@ -43,6 +44,22 @@ def _out_of_range_error(target_1d: torch.Tensor, vocab: int, ignore_index: Optio
         f"target_ids out of range: expected [0, {vocab - 1}], got [{t_min}, {t_max}]. "
         "Mask or filter padding / ignore-index values (e.g. -100) before this op."
     )
+
+
+@contextlib.contextmanager
+def _checked_targets(target_1d: torch.Tensor, vocab: int, ignore_index: Optional[int], enabled: bool):
+    """Around the launches of a forward: the range check goes in front of them, and its answer is waited
+    for (and raised) behind them, on the host only."""
+    if not enabled:
+        yield
+        return
+    pending = _native.TargetCheck(target_1d, vocab, ignore_index=ignore_index)
+    try:
+        yield
+    finally:
+        bad = pending.out_of_range()
+    if bad:
+        raise _out_of_range_error(target_1d, vocab, ignore_index)
 
 
 def _check_grad_buffer(name: str, buf: torch.Tensor, shape, device) -> None:
@@ -424,10 +441,9 @@ class _FusedLinearLogpFunction(torch.autograd.Function):
             ctx.weight_dtype = weight.dtype
             ctx.bias_dtype = bias.dtype if bias is not None else None
             return hidden_2d.new_zeros(hidden.shape[:-1], dtype=torch.float32)
-        logp, lse, err = fused_linear_logp_forward(
-            hidden_2d, w, target_1d, bias, temperature=temperature, ignore_index=ignore_index)
-        if check_targets and bool(err.item()):
-            raise _out_of_range_error(target_1d, w.size(0), ignore_index)
+        with _checked_targets(target_1d, w.size(0), ignore_index, check_targets):
+            logp, lse, _ = fused_linear_logp_forward(
+                hidden_2d, w, target_1d, bias, temperature=temperature, ignore_index=ignore_index)
         ctx.save_for_backward(hidden_2d, w, bias if bias is not None else hidden_2d, target_1d, lse)
         ctx.has_bias = bias is not None
         ctx.lead_shape = hidden.shape[:-1]
@@ -490,11 +506,10 @@ class _FusedNormLinearLogpFunction(torch.autograd.Function):
         g = _aligned_contiguous(gain.detach().to(torch.float32))  # the reference multiplies by weight.float()
         w = _aligned_contiguous(weight)
         target_1d = target_ids.reshape(-1).to(device=x_2d.device, dtype=torch.long).contiguous()
-        logp, lse, err = fused_norm_linear_logp_forward(
-            x_2d, g, w, target_1d, bias, eps=eps, temperature=temperature, ignore_index=ignore_index)
         ctx.empty = x_2d.size(0) == 0
-        if check_targets and not ctx.empty and bool(err.item()):
-            raise _out_of_range_error(target_1d, w.size(0), ignore_index)
+        with _checked_targets(target_1d, w.size(0), ignore_index, check_targets):
+            logp, lse, _ = fused_norm_linear_logp_forward(
+                x_2d, g, w, target_1d, bias, eps=eps, temperature=temperature, ignore_index=ignore_index)
         ctx.save_for_backward(x_2d, g, w, bias if bias is not None else x_2d, target_1d, lse)
         ctx.has_bias = bias is not None
         ctx.lead_shape = x.shape[:-1]
@@ -535,11 +550,10 @@ class _FusedLinearLogpPairFunction(torch.autograd.Function):
         w = _aligned_contiguous(weight)
         w_ref = _aligned_contiguous(ref_weight.detach())
         target_1d = target_ids.reshape(-1).to(device=hidden_2d.device, dtype=torch.long).contiguous()
-        logp, lse, ref_logp, _, err = fused_linear_logp_forward_pair(
-            hidden_2d, w, w_ref, target_1d, bias, ref_bias, temperature=temperature,
-            ignore_index=ignore_index)
-        if check_targets and hidden_2d.size(0) > 0 and bool(err.item()):
-            raise _out_of_range_error(target_1d, w.size(0), ignore_index)
+        with _checked_targets(target_1d, w.size(0), ignore_index, check_targets):
+            logp, lse, ref_logp, _, _ = fused_linear_logp_forward_pair(
+                hidden_2d, w, w_ref, target_1d, bias, ref_bias, temperature=temperature,
+                ignore_index=ignore_index)
         ctx.empty = hidden_2d.size(0) == 0
         ctx.save_for_backward(hidden_2d, w, bias if bias is not None else hidden_2d, target_1d, lse)
         ctx.has_bias = bias is not None
