@@ -43,7 +43,8 @@ enum {
 
 /* ABI version of this header (major * 100 + minor): 102 (100 + rlk_device_info,
  * rlk_linear_logp_fwd_plan, the typed weight gradients rlk_linear_logp_bwd_typed and
- * rlk_linear_logp_rmsnorm_bwd_typed, and rlk_check_targets). */
+ * rlk_linear_logp_rmsnorm_bwd_typed, rlk_check_targets and
+ * rlk_logp_from_logits_pair_masked). */
 int rlk_version(void);
 
 /* Message of the last error returned on the calling thread ("" if none). Host pointer, valid
@@ -316,6 +317,13 @@ int rlk_logp_from_logits_pair(const void* logits, const void* ref_logits, int32_
                               const int64_t* ids, void* out, void* ref_out, int32_t out_dtype,
                               float* lse_out, float* ref_lse_out, const int64_t* row_indices,
                               int64_t n_launch, int64_t n_rows, int64_t vocab, rlk_stream_t stream);
+
+/* The pair over all rows, without the rows whose mask is 0 (uint8 [n_rows]; prompt and padding positions
+ * of a loss over written logits): those are not read, their outputs and lse are 0. */
+int rlk_logp_from_logits_pair_masked(const void* logits, const void* ref_logits, int32_t logits_dtype,
+                                     const int64_t* ids, const uint8_t* mask, void* out, void* ref_out,
+                                     int32_t out_dtype, float* lse_out, float* ref_lse_out, int64_t n_rows,
+                                     int64_t vocab, rlk_stream_t stream);
 
 /* Backward of the above w.r.t. the logits:
  *   grad_logits[n][v] = coeff[n] * (onehot(ids[n])[v] - exp(logits[n][v] - lse[n]))

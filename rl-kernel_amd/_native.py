@@ -63,6 +63,8 @@ SIGNATURES = {
     "rlk_logp_from_logits": (_c.c_int, [_vp, _i32, _vp, _vp, _i32, _vp, _vp, _i64, _i64, _i64, _vp]),
     "rlk_logp_from_logits_pair": (_c.c_int, [_vp, _vp, _i32, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i64,
                                              _i64, _i64, _vp]),
+    "rlk_logp_from_logits_pair_masked": (_c.c_int, [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _i64,
+                                                    _i64, _vp]),
     "rlk_logp_from_logits_bwd": (_c.c_int, [_vp, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _vp]),
     "rlk_grpo_loss_workspace_bytes": (_c.c_int, [_i64, _c.POINTER(_sz)]),
     "rlk_grpo_loss_from_logp": (_c.c_int, [_vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _f32, _f32,

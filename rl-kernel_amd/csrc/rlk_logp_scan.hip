@@ -70,6 +70,7 @@ struct ScanSecond {
     const void* logits;
     void* out;
     float* lse_out;
+    const uint8_t* mask;  // [n_rows] or null: rows whose mask is 0 are not read, their results are 0
 };
 
 template <int DT>
@@ -87,6 +88,13 @@ __global__ __launch_bounds__(kScanThreads) void logp_scan_kernel(
     constexpr int kPer = 16 / sizeof(E);  // elements per 16-byte load
     const int64_t row = row_indices ? row_indices[blockIdx.x] : static_cast<int64_t>(blockIdx.x);
     if (row < 0 || row >= n_rows) return;  // uniform: rows outside the tensor are skipped
+    if (second.mask != nullptr && second.mask[row] == 0) {  // uniform
+        if (threadIdx.x == 0) {
+            store_out(out, out_dtype, row, 0.f);
+            if (lse_out) lse_out[row] = 0.f;
+        }
+        return;
+    }
     const E* x = static_cast<const E*>(logits_v) + row * vocab;
     const int t = threadIdx.x;
 
@@ -166,7 +174,8 @@ __global__ __launch_bounds__(kScanThreads) void logp_scan_kernel(
 }
 
 // grad_logits[n][v] = coeff[n] * (onehot(ids[n])[v] - exp(logits[n][v] - lse[n])); rows whose id
-// is outside [0, V) (the forward returned 0 for them) get a zero gradient.
+// is outside [0, V) (the forward returned 0 for them) get a zero gradient.  A row with coefficient 0
+// (a masked position) is written without being read.
 template <int DT>
 __global__ __launch_bounds__(kScanThreads) void logp_scan_bwd_kernel(
     const void* __restrict__ logits_v, const int64_t* __restrict__ ids,
@@ -204,6 +213,11 @@ __global__ __launch_bounds__(kScanThreads) void logp_scan_bwd_kernel(
     for (int64_t v = t; v < head; v += kScanThreads) g[v] = value(v, x[v]);
     const u32x4* xv = reinterpret_cast<const u32x4*>(x + head);
     u32x4* gv = reinterpret_cast<u32x4*>(g + head);
+    if (c == 0.f) {  // uniform
+        for (int64_t i = t; i < nvec; i += kScanThreads) gv[i] = u32x4{0u, 0u, 0u, 0u};
+        for (int64_t v = tail0 + t; v < vocab; v += kScanThreads) g[v] = E(0);
+        return;
+    }
     for (int64_t i = t; i < nvec; i += kScanThreads) {
         const u32x4 in = __builtin_nontemporal_load(xv + i);
         u32x4 o;
@@ -291,7 +305,7 @@ int scan_enqueue(const void* logits, int32_t logits_dtype, const int64_t* ids, v
         return rlk_fail(RLK_ERR_UNSUPPORTED, "output dtype must be bf16, f16, f32 or f64");
     if (n_launch == 0 || n_rows == 0) return 0;
     const dim3 grid(static_cast<unsigned>(n_launch), second ? 2u : 1u), block(kScanThreads);
-    const ScanSecond s2 = second ? *second : ScanSecond{nullptr, nullptr, nullptr};
+    const ScanSecond s2 = second ? *second : ScanSecond{nullptr, nullptr, nullptr, nullptr};
     switch (logits_dtype) {
         case RLK_DTYPE_BF16:
             hipLaunchKernelGGL(logp_scan_kernel<RLK_DTYPE_BF16>, grid, block, 0, stream, logits, ids,
@@ -331,7 +345,18 @@ extern "C" int rlk_logp_from_logits_pair(const void* logits, const void* ref_log
                                          hipStream_t stream)
 {
     if (!ref_logits || !ref_out) return rlk_fail(RLK_ERR_ARG, "null pointer");
-    const rlk::ScanSecond second{ref_logits, ref_out, ref_lse_out};
+    const rlk::ScanSecond second{ref_logits, ref_out, ref_lse_out, nullptr};
     return scan_enqueue(logits, logits_dtype, ids, out, out_dtype, lse_out, row_indices, n_launch,
                         n_rows, vocab, &second, stream);
+}
+
+extern "C" int rlk_logp_from_logits_pair_masked(const void* logits, const void* ref_logits, int32_t logits_dtype,
+                                                const int64_t* ids, const uint8_t* mask, void* out, void* ref_out,
+                                                int32_t out_dtype, float* lse_out, float* ref_lse_out,
+                                                int64_t n_rows, int64_t vocab, hipStream_t stream)
+{
+    if (!ref_logits || !ref_out || !mask) return rlk_fail(RLK_ERR_ARG, "null pointer");
+    const rlk::ScanSecond second{ref_logits, ref_out, ref_lse_out, mask};
+    return scan_enqueue(logits, logits_dtype, ids, out, out_dtype, lse_out, nullptr, n_rows, n_rows, vocab,
+                        &second, stream);
 }

@@ -199,6 +199,32 @@ class _RatioKLFromLogpFunction(torch.autograd.Function):
         return d_cur.view(ctx.shape), None, None, None
 
 
+def _active_logp_pair(policy_logits, ref_logits, action_ids, mask):
+    """Policy and reference log-probs of ``action_ids`` at the positions of ``mask``; ids out of range
+    there are a ``ValueError``."""
+    vocab = policy_logits.size(-1)
+    error = ValueError(f"action_ids at active (unmasked) positions must be in "
+                       f"[0, {vocab}); found out-of-range ids.")
+    if action_ids.device != policy_logits.device or mask.device != action_ids.device \
+            or mask.shape != action_ids.shape or action_ids.shape != policy_logits.shape[:-1] \
+            or not policy_logits.is_cuda or action_ids.is_floating_point():
+        # ids or mask elsewhere or of another shape: the general route
+        if bool((mask & ((action_ids < 0) | (action_ids >= vocab))).any()):
+            raise error
+        return differentiable_logp_pair_fp32(policy_logits, ref_logits, action_ids.masked_fill(~mask, 0))
+    ids = action_ids.reshape(-1).to(torch.long).contiguous()
+    flat_mask = mask.reshape(-1).contiguous()
+    pending = _native.TargetCheck(ids, vocab, mask=flat_mask)
+    try:
+        # an id out of range selects nothing in the kernels, so they may run ahead of the answer
+        pair = differentiable_logp_pair_fp32(policy_logits, ref_logits, ids, flat_mask)
+    finally:
+        bad = pending.out_of_range()
+    if bad:
+        raise error
+    return pair
+
+
 class RocmRatioKLOp:
     """Logits-fed ratio + k3 KL: mask-before-exp, so inactive positions give ratio 1 and kl 0
     (rl_engine/kernels/ops/pytorch/loss/ratio_kl.py:32-58 of the reference)."""
@@ -212,15 +238,9 @@ class RocmRatioKLOp:
     def forward(self, policy_logits, ref_logits, action_ids, attention_mask, old_logps
                 ) -> Tuple[torch.Tensor, torch.Tensor]:
         mask = attention_mask.to(torch.bool)
-        vocab = policy_logits.size(-1)
-        invalid = mask & ((action_ids < 0) | (action_ids >= vocab))
-        if bool(invalid.any()):
-            raise ValueError(f"action_ids at active (unmasked) positions must be in "
-                             f"[0, {vocab}); found out-of-range ids.")
-        safe_ids = action_ids.masked_fill(~mask, 0)
         # both logit tensors in one scan launch (the reference's program reads both rows too:
         # rl_engine/kernels/ops/triton/loss/ratio_kl.py:46-60)
-        logp_policy, logp_ref = differentiable_logp_pair_fp32(policy_logits, ref_logits, safe_ids)
+        logp_policy, logp_ref = _active_logp_pair(policy_logits, ref_logits, action_ids, mask)
         return _RatioKLFromLogpFunction.apply(logp_policy, logp_ref, old_logps, mask)
 
 
@@ -255,12 +275,7 @@ class RocmGRPOLossOp:
     def apply(self, policy_logits, ref_logits, action_ids, old_logps, sample_advantages,
               completion_mask, *, clip_eps: float = 0.2, beta: float = 0.0):
         mask = completion_mask.to(torch.bool)
-        vocab = policy_logits.size(-1)
-        if bool((mask & ((action_ids < 0) | (action_ids >= vocab))).any()):
-            raise ValueError(f"action_ids at active (unmasked) positions must be in "
-                             f"[0, {vocab}); found out-of-range ids.")
-        safe_ids = action_ids.masked_fill(~mask, 0)
-        cur, ref = differentiable_logp_pair_fp32(policy_logits, ref_logits, safe_ids)
+        cur, ref = _active_logp_pair(policy_logits, ref_logits, action_ids, mask)
         return self._from_logp(cur, old_logps, ref, sample_advantages.reshape(-1), mask,
                                clip_eps=clip_eps, beta=beta)
 

@@ -185,10 +185,11 @@ class _LogpFromLogitsFunction(torch.autograd.Function):
 
 class _LogpPairFromLogitsFunction(torch.autograd.Function):
     """fp32 selected log-probs of a policy and a reference logits tensor from ONE scan launch;
-    differentiable w.r.t. the policy logits only."""
+    differentiable w.r.t. the policy logits only.  Rows outside ``mask`` (bool, one per row, or None)
+    are not read and give 0."""
 
     @staticmethod
-    def forward(ctx, logits, ref_logits, ids):
+    def forward(ctx, logits, ref_logits, ids, mask=None):
         shape = logits.shape[:-1]
         logits_2d = logits.reshape(-1, logits.size(-1)).contiguous()
         ref_2d = ref_logits.reshape(-1, ref_logits.size(-1)).contiguous()
@@ -199,10 +200,16 @@ class _LogpPairFromLogitsFunction(torch.autograd.Function):
         lse = torch.empty(n, device=logits.device, dtype=torch.float32)
         if n > 0:
             with torch.cuda.device(logits_2d.device):
-                rc = _native.load().rlk_logp_from_logits_pair(
-                    logits_2d.data_ptr(), ref_2d.data_ptr(), _IN[logits_2d.dtype], ids_1d.data_ptr(),
-                    out.data_ptr(), ref_out.data_ptr(), _OUT[torch.float32], lse.data_ptr(), None, None,
-                    n, n, v, _stream(logits_2d.device))
+                if mask is not None:
+                    rc = _native.load().rlk_logp_from_logits_pair_masked(
+                        logits_2d.data_ptr(), ref_2d.data_ptr(), _IN[logits_2d.dtype], ids_1d.data_ptr(),
+                        mask.data_ptr(), out.data_ptr(), ref_out.data_ptr(), _OUT[torch.float32],
+                        lse.data_ptr(), None, n, v, _stream(logits_2d.device))
+                else:
+                    rc = _native.load().rlk_logp_from_logits_pair(
+                        logits_2d.data_ptr(), ref_2d.data_ptr(), _IN[logits_2d.dtype], ids_1d.data_ptr(),
+                        out.data_ptr(), ref_out.data_ptr(), _OUT[torch.float32], lse.data_ptr(), None, None,
+                        n, n, v, _stream(logits_2d.device))
             _native.check(rc, "rlk_logp_from_logits_pair")
         ctx.save_for_backward(logits_2d, ids_1d, lse)
         ctx.logits_shape = logits.shape
@@ -213,18 +220,20 @@ class _LogpPairFromLogitsFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out, _grad_ref):
         grad, _ = _LogpFromLogitsFunction.backward(ctx, grad_out)
-        return grad, None, None
+        return grad, None, None, None
 
 
 def differentiable_logp_pair_fp32(logits: torch.Tensor, ref_logits: torch.Tensor,
-                                  ids: torch.Tensor):
+                                  ids: torch.Tensor, mask: Optional[torch.Tensor] = None):
     """``(logp_policy, logp_ref)``; one launch when both tensors share shape, dtype and device,
-    two scans otherwise."""
+    two scans otherwise.  With ``mask`` (bool, shape of ``ids``, on the logits' device) the one launch
+    leaves masked rows unread and 0; what the two scans return there is not specified."""
     if logits.dtype not in _IN or ref_logits.dtype not in _IN:
         raise RuntimeError("logits dtype must be float32, float16 or bfloat16")
     if (logits.shape == ref_logits.shape and logits.dtype == ref_logits.dtype
             and logits.device == ref_logits.device):
-        return _LogpPairFromLogitsFunction.apply(logits, ref_logits.detach(), ids)
+        rows = None if mask is None else mask.reshape(-1).contiguous()
+        return _LogpPairFromLogitsFunction.apply(logits, ref_logits.detach(), ids, rows)
     with torch.no_grad():
         ref = _LogpFromLogitsFunction.apply(ref_logits.detach(), ids)
     return _LogpFromLogitsFunction.apply(logits, ids), ref
