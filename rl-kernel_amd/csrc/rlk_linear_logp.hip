@@ -260,12 +260,12 @@ __device__ inline float combine_token(const CombineArgs& a, int64_t n)
     return lp;
 }
 
-// Many splits (few tokens): 16 tokens x 16 split groups per workgroup fetch the partial states side by
+// Many splits (few tokens): 4 tokens x 64 split groups per workgroup fetch the partial states side by
 // side, then one thread per token adds the rescaled sums in split order, as combine_token would; the
 // merged state replaces the token's slot 0, which the combine kernels read as their only split.  One
 // thread walking all splits of a token through memory is a chain of dependent loads: 37 us for 160
-// tokens x 62 splits.  LDS: the terms [2][n_split][16] behind the group maxima [16][16].
-constexpr int kMergeTokens = 16, kMergeGroups = 16;
+// tokens x 62 splits.  LDS: the terms [2][n_split][4] behind the group maxima. (16 x 16 took 14 us for 160 tokens x 251 splits.)
+constexpr int kMergeTokens = 4, kMergeGroups = 64;
 inline size_t merge_smem(int n_split) { return static_cast<size_t>(kMergeGroups + 2 * n_split) * kMergeTokens * 4; }
 __global__ __launch_bounds__(256) void linear_logp_merge_kernel(float* part_m, float* part_s, float* part_z, int N,
                                                                 int n_split)
@@ -1173,6 +1173,20 @@ inline int dh_parts(int64_t ct, int64_t pt, int64_t ht)
     return parts;
 }
 
+// What a split dH launch really cuts its vocab range into: as many parts as give every CU a tile (at
+// least 16 K steps each; their slots stay within 256 tiles of fp32).  The powers of two above left the
+// launch on 64 to 192 CUs: 64 x 2048 x 32000 318 -> 239, 64 x 4096 x 128256
+// 1306 -> 1168, 1000 x 1536 x 151936 1910 -> 1838 us a pass.
+inline int dh_cuts(int64_t ct, int64_t pt, int64_t ht)
+{
+    const int parts = dh_parts(ct, pt, ht);
+    if (parts == 1) return 1;
+    int64_t cuts = 256 / (ct * ht);
+    if (cuts > pt / 4) cuts = pt / 4;
+    if (cuts > 32) cuts = 32;
+    return cuts > parts ? static_cast<int>(cuts) : parts;
+}
+
 inline int64_t block_cost(int64_t ct, int64_t pt, int64_t ht, int64_t hk)
 {
     const int64_t dz = (ct * pt + 255) / 256 * (hk + 3);
@@ -1259,7 +1273,7 @@ BwdPlan bwd_plan(int64_t N, int H, int64_t V, size_t budget)
     p.part_bytes = 0;
     for (int64_t ct : {best_ct, ct_last})
         for (int64_t pt : {best_pt, pt_last}) {
-            const int parts = dh_parts(ct, pt, ht);
+            const int parts = dh_cuts(ct, pt, ht);
             if (parts > 1)
                 p.part_bytes = std::max(p.part_bytes, static_cast<size_t>(parts) * ct * 256 * H * 4);
         }
@@ -1492,8 +1506,8 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
             h.h_tiles = h_tiles;
             h.first = pi == 0;
             h.last = last_piece;
-            // same rule as the plan's cost model: per (chunk, piece) kind
-            const int ksplit = dh_parts(tok_tiles, v_tiles, h_tiles);
+            // per (chunk, piece) kind
+            const int ksplit = dh_cuts(tok_tiles, v_tiles, h_tiles);
             h.ksplit = ksplit;
             h.part = ksplit > 1 ? reinterpret_cast<float*>(ws + p.part_off) : nullptr;
             h.part_stride = static_cast<int64_t>(tok_tiles) * 256 * H;
@@ -1903,7 +1917,7 @@ int fwd_enqueue(const void* hidden, const void* weight, const float* bias, const
     // token takes at most as long as that launch)
     if (plan.total_splits >= 16) {
         const dim3 blocks((a.N + kMergeTokens - 1) / kMergeTokens);
-        const size_t lds = merge_smem(plan.total_splits);  // at most 256 splits: 33 KiB
+        const size_t lds = merge_smem(plan.total_splits);  // at most 256 splits: 9 KiB
         hipLaunchKernelGGL(linear_logp_merge_kernel, blocks, dim3(256), lds, stream, a.part_m, a.part_s, a.part_z, a.N,
                            plan.total_splits);
         if (second != nullptr)
