@@ -91,9 +91,9 @@ int rlk_linear_logp_fwd_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t
 /* Schedule the forward will use for these sizes (the reference computes its own inside the host
  * function: 4 workgroups per SM divided by the token blocks, csrc/cuda/fused_linear_logp_sm90.cu:
  * 350-358,369, and does not expose it): out4 = { blocks of 256
- * tokens, vocab splits of the launch over the full vocab tiles, vocab splits of the launch over
- * the ragged last tile (all tiles for RLK_DTYPE_F32; 0 if there is no such launch), token blocks
- * per XCD patch }.  The contraction launches are blocks x splits workgroups.  Inputs whose rows
+ * tokens, vocab splits of the chained launch (all tiles when H % 64 == 0, H >= 128 and V >= 256, otherwise
+ * the full ones), vocab splits of the launch over the ragged last tile (all tiles for RLK_DTYPE_F32; 0 if
+ * there is no such launch), token blocks per XCD patch }.  The contraction launches are blocks x splits workgroups.  Inputs whose rows
  * do not start on 16-byte boundaries run the RLK_DTYPE_F32 schedule.  Host only; touches no
  * device. */
 int rlk_linear_logp_fwd_plan(int64_t N, int32_t H, int64_t V, int32_t dtype, int64_t* out4);

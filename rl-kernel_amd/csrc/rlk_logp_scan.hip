@@ -73,7 +73,9 @@ struct ScanSecond {
     const uint8_t* mask;  // [n_rows] or null: rows whose mask is 0 are not read, their results are 0
 };
 
-template <int DT>
+// MASKED: second.mask is given (a template so that the plain scan of a few rows, 13 us a call, does not
+// wait for one more argument).
+template <int DT, bool MASKED>
 __global__ __launch_bounds__(kScanThreads) void logp_scan_kernel(
     const void* __restrict__ logits_v, const int64_t* __restrict__ ids, void* __restrict__ out,
     int out_dtype, float* __restrict__ lse_out, const int64_t* __restrict__ row_indices,
@@ -88,7 +90,7 @@ __global__ __launch_bounds__(kScanThreads) void logp_scan_kernel(
     constexpr int kPer = 16 / sizeof(E);  // elements per 16-byte load
     const int64_t row = row_indices ? row_indices[blockIdx.x] : static_cast<int64_t>(blockIdx.x);
     if (row < 0 || row >= n_rows) return;  // uniform: rows outside the tensor are skipped
-    if (second.mask != nullptr && second.mask[row] == 0) {  // uniform
+    if (MASKED && second.mask[row] == 0) {  // uniform
         if (threadIdx.x == 0) {
             store_out(out, out_dtype, row, 0.f);
             if (lse_out) lse_out[row] = 0.f;
@@ -293,6 +295,21 @@ extern "C" int rlk_logp_from_logits_bwd(const void* logits, int32_t logits_dtype
 
 namespace {
 
+template <int DT>
+void scan_launch(const void* logits, const int64_t* ids, void* out, int32_t out_dtype, float* lse_out,
+                 const int64_t* row_indices, int64_t n_rows, int64_t vocab, const rlk::ScanSecond& s2, dim3 grid,
+                 hipStream_t stream)
+{
+    using namespace rlk;
+    const dim3 block(kScanThreads);
+    if (s2.mask != nullptr)
+        hipLaunchKernelGGL((logp_scan_kernel<DT, true>), grid, block, 0, stream, logits, ids, out, out_dtype, lse_out,
+                           row_indices, n_rows, vocab, s2);
+    else
+        hipLaunchKernelGGL((logp_scan_kernel<DT, false>), grid, block, 0, stream, logits, ids, out, out_dtype,
+                           lse_out, row_indices, n_rows, vocab, s2);
+}
+
 int scan_enqueue(const void* logits, int32_t logits_dtype, const int64_t* ids, void* out,
                  int32_t out_dtype, float* lse_out, const int64_t* row_indices, int64_t n_launch,
                  int64_t n_rows, int64_t vocab, const rlk::ScanSecond* second, hipStream_t stream)
@@ -304,20 +321,20 @@ int scan_enqueue(const void* logits, int32_t logits_dtype, const int64_t* ids, v
     if (out_dtype < RLK_DTYPE_BF16 || out_dtype > RLK_DTYPE_F64)
         return rlk_fail(RLK_ERR_UNSUPPORTED, "output dtype must be bf16, f16, f32 or f64");
     if (n_launch == 0 || n_rows == 0) return 0;
-    const dim3 grid(static_cast<unsigned>(n_launch), second ? 2u : 1u), block(kScanThreads);
+    const dim3 grid(static_cast<unsigned>(n_launch), second ? 2u : 1u);
     const ScanSecond s2 = second ? *second : ScanSecond{nullptr, nullptr, nullptr, nullptr};
     switch (logits_dtype) {
         case RLK_DTYPE_BF16:
-            hipLaunchKernelGGL(logp_scan_kernel<RLK_DTYPE_BF16>, grid, block, 0, stream, logits, ids,
-                               out, out_dtype, lse_out, row_indices, n_rows, vocab, s2);
+            scan_launch<RLK_DTYPE_BF16>(logits, ids, out, out_dtype, lse_out, row_indices, n_rows, vocab, s2, grid,
+                                      stream);
             break;
         case RLK_DTYPE_F16:
-            hipLaunchKernelGGL(logp_scan_kernel<RLK_DTYPE_F16>, grid, block, 0, stream, logits, ids,
-                               out, out_dtype, lse_out, row_indices, n_rows, vocab, s2);
+            scan_launch<RLK_DTYPE_F16>(logits, ids, out, out_dtype, lse_out, row_indices, n_rows, vocab, s2, grid,
+                                      stream);
             break;
         case RLK_DTYPE_F32:
-            hipLaunchKernelGGL(logp_scan_kernel<RLK_DTYPE_F32>, grid, block, 0, stream, logits, ids,
-                               out, out_dtype, lse_out, row_indices, n_rows, vocab, s2);
+            scan_launch<RLK_DTYPE_F32>(logits, ids, out, out_dtype, lse_out, row_indices, n_rows, vocab, s2, grid,
+                                      stream);
             break;
         default:
             return rlk_fail(RLK_ERR_UNSUPPORTED, "logits dtype must be bf16, f16 or f32");
