@@ -1116,6 +1116,9 @@ int patch_rows_for(int H)
 int split_count(int row_blocks, int tiles, int patch_rows)
 {
     if (tiles <= 0) return 0;
+    // tiny heads: one tile per workgroup side by side (128 x 64 x 1000: 53 us of two launches that walk
+    // 3 + 1 tiles, 31 us as one launch of 4)
+    if (static_cast<int64_t>(tiles) * row_blocks <= 32) return tiles;
     // At least 32 / patch_rows splits when each still gets a long run of tiles: the 32 workgroups
     // resident on one XCD then form a compact (token blocks x splits) patch that fetches 12 distinct
     // operand streams into its L2 (8 x 4 or 4 x 8) instead of 18 (16 x 2) or 33 (32 x 1); with 243
@@ -1152,7 +1155,9 @@ FwdPlan fwd_plan(int64_t N, int H, int64_t V, bool all_general)
     p.patch_rows = patch_rows_for(H);
     const int all = static_cast<int>((V + 255) / 256);
     const int full = static_cast<int>(V / 256);
-    p.fast_tiles = all_general ? 0 : (fwd_chained(H, V) ? all : full);
+    // a ragged vocabulary of a tiny unchained head is not worth a second launch
+    const bool tiny = V % 256 != 0 && static_cast<int64_t>(p.row_blocks) * all <= 32;
+    p.fast_tiles = all_general ? 0 : (fwd_chained(H, V) ? all : (tiny ? 0 : full));
     p.gen_tiles = all - p.fast_tiles;
     p.n_fast = split_count(p.row_blocks, p.fast_tiles, p.patch_rows);
     p.n_gen = split_count(p.row_blocks, p.gen_tiles, p.patch_rows);
@@ -1581,7 +1586,9 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
 
             // dZ block: chained through one pipeline when every tile can read 256 rows; otherwise the
             // full vocab tiles through the fast variant and the ragged last one through the general one
-            const int fast_tiles = shifted ? v_tiles : v_valid / 256;
+            // (all through the general one when the launch is tiny)
+            const bool tiny = v_rag != 0 && tok_tiles * v_tiles <= 32;
+            const int fast_tiles = shifted ? v_tiles : (tiny ? 0 : v_valid / 256);
             const int gen_tiles = v_tiles - fast_tiles;
             const bool k_ok = H % kBK == 0 && H >= 2 * kBK;
             if (fast_tiles > 0) {
