@@ -975,16 +975,19 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dw_kernel(DwArgs a)
     }
 }
 
-// Fewer tokens than a tile: the rows of `hidden` followed by rows of zeros up to one 256-row tile, so
-// that dZ and dW run on the full-tile pipeline (at most 256 x H x 2 bytes, a few us against the
-// register-staged loop that a K tail of the whole dW contraction would need: 12 to 20 % of a
-// backward at 160 tokens).  16 bytes per thread.
-__global__ void linear_logp_pad_rows_kernel(const uint16_t* src, uint16_t* dst, int64_t valid8, int64_t total8)
+// Fewer tokens than a tile: the rows of `hidden`, the last one repeated up to one 256-row tile, so that dZ
+// and dW run on the full-tile pipeline (at most 256 x H x 2 bytes, a few us against the register-staged
+// loop that a K tail of the whole dW contraction would need: 12 to 20 % of a backward at 160 tokens).
+// dZ evaluates a row past the end against the last token's log-sum-exp and a zero upstream gradient, so
+// that row has to hold that token's logits: a probability of at most 1 times 0.  (Rows of zeros have
+// logits of 0 or the bias; against a log-sum-exp below -88 their probability is inf and dZ NaN.)
+// One row per blockIdx.y, 16 bytes per thread.
+__global__ void linear_logp_pad_rows_kernel(const uint16_t* src, uint16_t* dst, int n_rows, int row8)
 {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= total8) return;
-    reinterpret_cast<u32x4_t*>(dst)[i] =
-        i < valid8 ? reinterpret_cast<const u32x4_t*>(src)[i] : u32x4_t{0u, 0u, 0u, 0u};
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= row8) return;
+    const int64_t row = blockIdx.y, from = row < n_rows ? row : n_rows - 1;
+    reinterpret_cast<u32x4_t*>(dst)[row * row8 + i] = reinterpret_cast<const u32x4_t*>(src)[from * row8 + i];
 }
 
 // db[v] (+)= sum_tok dZ[tok][v] in two fixed-order levels.  Level 1: one workgroup per (256
@@ -1468,9 +1471,9 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
     const bool padded = shifted && N < 256;
     if (padded) {
         uint16_t* pad = reinterpret_cast<uint16_t*>(ws + p.pad_off);
-        const int64_t total8 = 256LL * H / 8;
-        hipLaunchKernelGGL(linear_logp_pad_rows_kernel, dim3(static_cast<unsigned>((total8 + 255) / 256)), dim3(256),
-                           0, stream, hid, pad, N * H / 8, total8);
+        const int row8 = static_cast<int>(H / 8);
+        hipLaunchKernelGGL(linear_logp_pad_rows_kernel, dim3((row8 + 255) / 256, 256), dim3(256), 0, stream, hid, pad,
+                           static_cast<int>(N), row8);
         hid = pad;
     }
 
