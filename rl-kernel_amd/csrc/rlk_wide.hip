@@ -1,9 +1,9 @@
 // fp32 matrix-core kernels of the fused linear-logprob path for inputs the 16-bit MFMA tiles do
 // not take: fp32 tensors, hidden sizes that are not a multiple of 8, matrices that do not start on
 // a 16-byte boundary.  Every operand is widened to fp32 on its way into LDS (exact for bf16 and
-// f16) and multiplied as three bf16 pieces (SplitGemm below; v_mfma_f32_32x32x2_f32 where an infinity or
-// NaN is in the way), so products are fp32 to the last bit or two, sums are fp32, and the results follow
-// the reference's fp32 arithmetic.  Same workgroup tile (256 x 256, 2 x 4
+// f16) and multiplied as three bf16 pieces (SplitGemm below; v_mfma_f32_32x32x2_f32 where infinities, NaN or
+// rows of tiny elements are in the way), with an error at or below that of the fp32 instruction, sums
+// are fp32, and the results follow the reference's fp32 arithmetic.  Same workgroup tile (256 x 256, 2 x 4
 // wavefronts), same accumulator layout and same split / combine structure as the 16-bit kernels;
 // dZ stays fp32.  All loads are clamped or masked element by element, so any N, H, V >= 1 and any
 // element alignment is accepted.  All reductions run in a fixed order: same input, same bits.
@@ -306,19 +306,33 @@ struct WideGemm {
     }
 };
 
-// The same contraction on the 16-bit matrix instruction, to fp32 accuracy.  Every element is cut into
-// three bf16 pieces on its way into LDS, x = hi + mid + lo exactly (8 bits each: hi by truncation, so it
-// cannot overflow, mid and lo by rounding the remainders), and a product is the sum of the six piece
-// products down to 2^-16 of it; the three that are left out stay below 2^-22 of a product, most of
-// them far below and with random sign, so the roundings of the running fp32 sums decide the error, and
-// one instruction adds 16 products where the fp32 one adds two: error against 64 bits, start of the
-// comparison = v_mfma_f32_32x32x2_f32, 2048 x 2048 x 32768: logp 6.7e-7 -> 5.7e-7, dH 1.6e-6 -> 1.0e-6, dW
-// 8.1e-7 -> 5.0e-7.  (The five small products in a sum of their own: 7e-7, but 300 spilled registers
-// and 13 % slower.)  Bound: the matrix pipe under the board's power limit at six 16-bit products (1450
-// TFLOP/s sustained / 6 = 240) against 157 TFLOP/s peak of the fp32 instruction; the same shape
-// forward + backward 8.35 -> 5.04 ms.
-// An infinity or NaN in an operand tile has no such pieces (inf * 0 in the small products): the
-// workgroup sees it while it converts and computes that tile again on the fp32 instruction.
+// The same contraction on the 16-bit matrix instruction, at least as accurate as on the fp32 one.  Every
+// element is cut into three bf16 pieces on its way into LDS, x = hi + mid + lo exactly (8 bits and a sign
+// each, all by rounding to nearest), and a product is the sum of six of the nine piece products, the
+// method of Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations" (ARITH 2019).  The three left out are below 2^-24 of the product, most of
+// them far below and with random sign (by truncation hi and mid would leave 2^-22).
+//
+// The matrix instruction does not round its running sum to nearest: added straight into a long sum of
+// terms of one sign, the pieces fell 60 and 105 x 2^-24 of the sum short at K = 4096 and 16384.  So the six
+// products of a stage, smallest first, make a sum of their own from zero, whose last product alone
+// rounds at the size of the result, and one ordinary fp32 addition (to nearest) a stage takes it into the
+// accumulator, where the fp32 instruction rounds eight times.  Error of a dot product over sum |a b|, rms
+// in units of 2^-24, fp32 instruction -> here: random signs K = 16 0.41 -> 0.25, K = 4096 0.48 -> 0.14; one sign
+// K = 16 1.1 -> 0.7, K = 4096 14 -> 3.6, K = 16384 29 -> 7.0.
+//
+// Bound: the matrix pipe under the board's power limit at six 16-bit products (1450 TFLOP/s sustained / 6
+// = 240), next to 0.16 of that time in vector instructions for the pieces and as much again for the
+// additions, against 157 TFLOP/s peak of the fp32 instruction.  2048 x 2048 x 32768 forward + backward:
+// 8.35 ms on the fp32 instruction, 5.00 with the pieces added straight into the accumulator, 5.63 so (the
+// additions of a tile put behind the next tile's products, 32 registers instead of 16, spill: 5.60 against
+// 5.37 ms of kernel time).
+//
+// What pieces cannot hold: an infinity or NaN (they make the sum NaN), a sum that passes the largest
+// float on the way, and elements so small that mid and lo fall below bf16's smallest number.  The
+// workgroup then computes that tile again on the fp32 instruction: when a result is not finite, and
+// when all elements of a row that one thread converted, not all of them zero, are below 2^-95 (where a
+// row has larger ones too, what the small ones lose, 2^-126 at most, is nothing next to their sum).
 //
 //   K-contiguous: LDS [256 rows][3 pieces][16 k]; rows 96 bytes apart: eight rows start in eight
 //                 different 16-byte chunks of the 256-byte bank line
@@ -328,19 +342,15 @@ struct Pieces {
     u32x2_t hi, mid, lo;  // four elements each
 };
 
-__device__ inline Pieces split3(f32x4_t v, float& bad)
+__device__ inline Pieces split3(f32x4_t v)
 {
     Pieces p;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const float x0 = v[2 * h], x1 = v[2 * h + 1];
-        // 0 * finite = 0: stays 0 until the first infinity or NaN
-        bad = fmaf(x0, 0.f, bad);
-        bad = fmaf(x1, 0.f, bad);
-        const uint32_t b0 = __builtin_bit_cast(uint32_t, x0), b1 = __builtin_bit_cast(uint32_t, x1);
-        const uint32_t hi = (b0 >> 16) | (b1 & 0xffff0000u);
-        const float r0 = x0 - __builtin_bit_cast(float, b0 & 0xffff0000u);
-        const float r1 = x1 - __builtin_bit_cast(float, b1 & 0xffff0000u);
+        const uint32_t hi = Bf16::pack2(x0, x1);
+        const float r0 = x0 - __builtin_bit_cast(float, hi << 16);
+        const float r1 = x1 - __builtin_bit_cast(float, hi & 0xffff0000u);
         const uint32_t mid = Bf16::pack2(r0, r1);
         const float q0 = r0 - __builtin_bit_cast(float, mid << 16);
         const float q1 = r1 - __builtin_bit_cast(float, mid & 0xffff0000u);
@@ -350,6 +360,33 @@ __device__ inline Pieces split3(f32x4_t v, float& bad)
     }
     return p;
 }
+
+// The bits of all elements that this thread converted of a tile row, or-ed together (K-contiguous: one row
+// per group of four elements, K-major: the four rows of its groups).  An exponent of 32 or more, a
+// magnitude from 2^-95 on, shows in the exponent's upper three bits whatever else is or-ed in.
+template <bool KMAJOR>
+struct RowBits {
+    static constexpr int kRows = KMAJOR ? 4 : 2;
+    uint32_t bits[kRows];
+
+    __device__ inline void reset()
+    {
+#pragma unroll
+        for (uint32_t& b : bits) b = 0;
+    }
+    __device__ inline void note(f32x4_t v, int g)
+    {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bits[KMAJOR ? e % kRows : g] |= __builtin_bit_cast(uint32_t, v[e]);
+    }
+    __device__ inline bool too_small() const
+    {
+        bool small = false;
+#pragma unroll
+        for (uint32_t b : bits) small = small || ((b & 0x70000000u) == 0 && (b & 0x7fffffffu) != 0);
+        return small;
+    }
+};
 
 template <bool KMAJOR>
 struct SplitLds {
@@ -402,37 +439,39 @@ struct SplitGemm {
     __device__ static inline void run(const WideOperand& A, const WideOperand& B, int K,
                                       f32x16_t (&acc)[kTM][kTN], char* smem)
     {
-        float bad;
+        bool again;
         if (IOA::fast_ok(A, K) && IOB::fast_ok(B, K))  // uniform
-            bad = run_impl<true>(A, B, K, acc, smem);
+            again = run_impl<true>(A, B, K, acc, smem);
         else
-            bad = run_impl<false>(A, B, K, acc, smem);
-        if (__syncthreads_or(bad != bad)) {
+            again = run_impl<false>(A, B, K, acc, smem);
+        if (__syncthreads_or(again)) {
             zero_acc(acc);
             Exact::template run_impl<false>(A, B, K, acc, smem);
         }
     }
 
-    // One 32 x 32 tile's share of a stage.
-    __device__ static inline void product(const Frag& a, const Frag& b, f32x16_t& acc)
+    // One 32 x 32 tile's share of a stage, added to `out` as one number.
+    __device__ static inline void product(const Frag& a, const Frag& b, f32x16_t& out)
     {
         auto mul = [](bf16x8_t x, bf16x8_t y, f32x16_t c) {
             return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0);
         };
+        f32x16_t acc = {};
         acc = mul(a[2], b[0], acc);
         acc = mul(a[0], b[2], acc);
         acc = mul(a[1], b[1], acc);
         acc = mul(a[1], b[0], acc);
         acc = mul(a[0], b[1], acc);
         acc = mul(a[0], b[0], acc);
+        out += acc;
     }
 
     // Stage kt multiplies while stage kt + 2 is converted into the LDS stage that kt - 1 has left and
     // the first fragments of stage kt + 1 (published by the last barrier) are read, so that neither
     // conversions nor LDS latency stand in front of the matrix work behind a barrier.
-    // Returns a value that is NaN when this thread met an infinity or NaN.
+    // Returns whether this thread has a reason to compute the tile again on the fp32 instruction.
     template <bool FAST>
-    __device__ static inline float run_impl(const WideOperand& A, const WideOperand& B, int K,
+    __device__ static inline bool run_impl(const WideOperand& A, const WideOperand& B, int K,
                                             f32x16_t (&acc)[kTM][kTN], char* smem)
     {
         IOA la;
@@ -442,16 +481,22 @@ struct SplitGemm {
         const int wave = threadIdx.x >> 6;
         const int ra0 = (wave / kWN) * (kTM * 32), rb0 = (wave % kWN) * (kTN * 32);
         const int nk = (K + kWBK - 1) / kWBK;
-        float bad = 0.f;
+        RowBits<A_KMAJOR> pa;
+        RowBits<B_KMAJOR> pb;
+        pa.reset();
+        pb.reset();
         f32x4_t reg[4];  // groups 0, 1 of A and 0, 1 of B
         auto fetch = [&](int kt, int n) {
             reg[n] = n < 2 ? la.template load<FAST>(kt, n) : lb.template load<FAST>(kt, n - 2);
         };
         auto convert = [&](char* stage, int n) {
-            if (n < 2)
-                LA::store(stage, split3(reg[n], bad), n);
-            else
-                LB::store(stage + LA::kBytes, split3(reg[n], bad), n - 2);
+            if (n < 2) {
+                pa.note(reg[n], n);
+                LA::store(stage, split3(reg[n]), n);
+            } else {
+                pb.note(reg[n], n - 2);
+                LB::store(stage + LA::kBytes, split3(reg[n]), n - 2);
+            }
         };
         auto stage_at = [&](int st) { return smem + st * kStageBytes; };
         // stages 0 and 1 in LDS, stage 2 on its way (past the last stage: the last one again)
@@ -494,12 +539,21 @@ struct SplitGemm {
                         convert(stage_at(dst), i);
                         fetch(ahead, i);
                     }
+                    // the addition stays here (sunk below the next products it costs 300 registers)
+                    asm volatile("" : "+v"(acc[i][j]));
                 });
             });
             __syncthreads();
             cur = nxt;
         }
-        return bad;
+        float zero = 0.f;  // 0 * finite = 0; NaN once a result is infinite or NaN
+#pragma unroll
+        for (int i = 0; i < kTM; ++i)
+#pragma unroll
+            for (int j = 0; j < kTN; ++j)
+#pragma unroll
+                for (int r = 0; r < Acc32::kRegs; ++r) zero = fmaf(acc[i][j][r], 0.f, zero);
+        return zero != 0.f || pa.too_small() || pb.too_small();
     }
 };
 
