@@ -1112,16 +1112,16 @@ int patch_rows_for(int H)
 // wins, a smaller one when it is within 1.5 %, among the counts that leave every workgroup a run of
 // at least 8 tiles and keep the split partials (12 bytes per token and split) within the 8 MiB the
 // allocation-free entry point has; measured over 4 - 32 splits at 48 - 243 token blocks, this
-// choice is within 1.5 % of the best count tried.  As long as the launch does not fill one round of
-// the chip, shorter runs are taken too (from 64 tiles on; smaller vocabularies keep the runs and with
-// them one grouping of the sums for a batch and its micro-batches): one block of 160 tokens x 501 tiles at H = 4096 ran 62
-// workgroups of 8 - 9 tiles in 741 us and runs 251 of two in 250 us.
+// choice is within 1.5 % of the best count tried.  From 64 tiles on shorter runs are taken too as long as
+// the launch does not fill one round of the chip: one block of 160 tokens x 501 tiles at H = 4096 ran 62
+// workgroups of 8 - 9 tiles in 741 us and runs 251 of two in 250 us.  Below 64 tiles the runs of 8 stay, so
+// that a batch and its micro-batches sum in one grouping and give the same bits: whatever their sizes up
+// to 14 tiles (V <= 3584, one run per token block), up to 8192 tokens above.  (One tile per workgroup in
+// launches of up to 32 tiles took 200 x 64 x 3000 log-probs from 88 to 42 us and forward + backward of 160 x
+// 4096 x 8192 from 866 to 260, but grouped by the token count.)
 int split_count(int row_blocks, int tiles, int patch_rows)
 {
     if (tiles <= 0) return 0;
-    // tiny heads: one tile per workgroup side by side (128 x 64 x 1000: 53 us of two launches that walk
-    // 3 + 1 tiles, 31 us as one launch of 4)
-    if (static_cast<int64_t>(tiles) * row_blocks <= 32) return tiles;
     // At least 32 / patch_rows splits when each still gets a long run of tiles: the 32 workgroups
     // resident on one XCD then form a compact (token blocks x splits) patch that fetches 12 distinct
     // operand streams into its L2 (8 x 4 or 4 x 8) instead of 18 (16 x 2) or 33 (32 x 1); with 243
@@ -1158,9 +1158,7 @@ FwdPlan fwd_plan(int64_t N, int H, int64_t V, bool all_general)
     p.patch_rows = patch_rows_for(H);
     const int all = static_cast<int>((V + 255) / 256);
     const int full = static_cast<int>(V / 256);
-    // a ragged vocabulary of a tiny unchained head is not worth a second launch
-    const bool tiny = V % 256 != 0 && static_cast<int64_t>(p.row_blocks) * all <= 32;
-    p.fast_tiles = all_general ? 0 : (fwd_chained(H, V) ? all : (tiny ? 0 : full));
+    p.fast_tiles = all_general ? 0 : (fwd_chained(H, V) ? all : full);
     p.gen_tiles = all - p.fast_tiles;
     p.n_fast = split_count(p.row_blocks, p.fast_tiles, p.patch_rows);
     p.n_gen = split_count(p.row_blocks, p.gen_tiles, p.patch_rows);
