@@ -41,9 +41,9 @@ enum {
     RLK_ERR_LAUNCH = -3       /* HIP refused the launch */
 };
 
-/* ABI version of this header (major * 100 + minor): 102 (100 + rlk_device_info,
+/* ABI version of this header (major * 100 + minor): 103 (100 + rlk_device_info,
  * rlk_linear_logp_fwd_plan, the typed weight gradients rlk_linear_logp_bwd_typed and
- * rlk_linear_logp_rmsnorm_bwd_typed, rlk_check_targets and
+ * rlk_linear_logp_rmsnorm_bwd_typed, rlk_check_targets, rlk_mark_targets and
  * rlk_logp_from_logits_pair_masked). */
 int rlk_version(void);
 
@@ -293,6 +293,11 @@ int rlk_linear_logp_rmsnorm_bwd_typed(const float* grad_logp, const void* x, con
 int rlk_check_targets(const int64_t* targets, const uint8_t* mask, int64_t n, int64_t vocab,
                       int64_t ignore_index, int32_t use_ignore, int32_t* out_of_range, rlk_stream_t stream);
 
+/* The check, and a copy of the ids for kernels that know no mask: marked[i] = targets[i], or -1 where
+ * the mask is 0.  marked may be targets itself, or NULL (rlk_check_targets). */
+int rlk_mark_targets(const int64_t* targets, const uint8_t* mask, int64_t n, int64_t vocab, int64_t ignore_index,
+                     int32_t use_ignore, int64_t* marked, int32_t* out_of_range, rlk_stream_t stream);
+
 /* ------------------------------------------------------------------------------------------ *
  * Selected-token log-prob from materialised logits (the `fused_logp` family).
  *
@@ -320,7 +325,8 @@ int rlk_logp_from_logits_pair(const void* logits, const void* ref_logits, int32_
                               int64_t n_launch, int64_t n_rows, int64_t vocab, rlk_stream_t stream);
 
 /* The pair over all rows, without the rows whose mask is 0 (uint8 [n_rows]; prompt and padding positions
- * of a loss over written logits): those are not read, their outputs and lse are 0. */
+ * of a loss over written logits): those are not read, their outputs and lse are 0.  The backward below
+ * knows no mask: give it an id out of range (or the coefficient 0) for such a row. */
 int rlk_logp_from_logits_pair_masked(const void* logits, const void* ref_logits, int32_t logits_dtype,
                                      const int64_t* ids, const uint8_t* mask, void* out, void* ref_out,
                                      int32_t out_dtype, float* lse_out, float* ref_lse_out, int64_t n_rows,

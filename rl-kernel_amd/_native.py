@@ -60,6 +60,7 @@ SIGNATURES = {
                                                      _vp, _vp, _vp, _sz, _sz, _i64, _i32, _i64, _i64,
                                                      _i32, _f32, _i64, _i32, _vp]),
     "rlk_check_targets": (_c.c_int, [_vp, _vp, _i64, _i64, _i64, _i32, _vp, _vp]),
+    "rlk_mark_targets": (_c.c_int, [_vp, _vp, _i64, _i64, _i64, _i32, _vp, _vp, _vp]),
     "rlk_logp_from_logits": (_c.c_int, [_vp, _i32, _vp, _vp, _i32, _vp, _vp, _i64, _i64, _i64, _vp]),
     "rlk_logp_from_logits_pair": (_c.c_int, [_vp, _vp, _i32, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i64,
                                              _i64, _i64, _vp]),
@@ -132,9 +133,10 @@ class TargetCheck:
     check is the first launch of the call and writes pinned host memory, the contraction follows, and
     ``out_of_range()`` waits for the check alone, so that whatever the caller enqueues next (the
     backward, as a rule) is on its way while the contraction runs.  ``out_of_range()`` has to be called
-    on every path: it is also what keeps the host word alive until the launch has written it."""
+    on every path: it is also what keeps the host word alive until the launch has written it.
+    ``marked``: a tensor like ``ids`` that the same launch fills with the ids, -1 where ``mask`` is off."""
 
-    def __init__(self, ids, vocab, *, mask=None, ignore_index=None):
+    def __init__(self, ids, vocab, *, mask=None, ignore_index=None, marked=None):
         import torch
 
         self._event = None
@@ -143,10 +145,11 @@ class TargetCheck:
         with torch.cuda.device(ids.device):
             stream = torch.cuda.current_stream(ids.device)
             self._flag = torch.empty(1, dtype=torch.int32, pin_memory=True)
-            check(load().rlk_check_targets(
+            check(load().rlk_mark_targets(
                 ids.data_ptr(), None if mask is None else mask.data_ptr(), ids.numel(), int(vocab),
                 0 if ignore_index is None else int(ignore_index), int(ignore_index is not None),
-                self._flag.data_ptr(), stream.cuda_stream), "rlk_check_targets")
+                None if marked is None else marked.data_ptr(), self._flag.data_ptr(), stream.cuda_stream),
+                "rlk_mark_targets")
             self._event = torch.cuda.Event()
             self._event.record(stream)
 

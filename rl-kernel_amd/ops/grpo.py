@@ -214,10 +214,11 @@ def _active_logp_pair(policy_logits, ref_logits, action_ids, mask):
         return differentiable_logp_pair_fp32(policy_logits, ref_logits, action_ids.masked_fill(~mask, 0))
     ids = action_ids.reshape(-1).to(torch.long).contiguous()
     flat_mask = mask.reshape(-1).contiguous()
-    pending = _native.TargetCheck(ids, vocab, mask=flat_mask)
+    marked = torch.empty_like(ids)
+    pending = _native.TargetCheck(ids, vocab, mask=flat_mask, marked=marked)
     try:
         # an id out of range selects nothing in the kernels, so they may run ahead of the answer
-        pair = differentiable_logp_pair_fp32(policy_logits, ref_logits, ids, flat_mask)
+        pair = differentiable_logp_pair_fp32(policy_logits, ref_logits, marked, flat_mask, marked=True)
     finally:
         bad = pending.out_of_range()
     if bad:

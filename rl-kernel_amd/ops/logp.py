@@ -186,7 +186,8 @@ class _LogpFromLogitsFunction(torch.autograd.Function):
 class _LogpPairFromLogitsFunction(torch.autograd.Function):
     """fp32 selected log-probs of a policy and a reference logits tensor from ONE scan launch;
     differentiable w.r.t. the policy logits only.  Rows outside ``mask`` (bool, one per row, or None)
-    are not read and give 0."""
+    are not read and give 0; their ids are out of range, so they get a zero gradient whatever comes
+    from above."""
 
     @staticmethod
     def forward(ctx, logits, ref_logits, ids, mask=None):
@@ -224,12 +225,16 @@ class _LogpPairFromLogitsFunction(torch.autograd.Function):
 
 
 def differentiable_logp_pair_fp32(logits: torch.Tensor, ref_logits: torch.Tensor,
-                                  ids: torch.Tensor, mask: Optional[torch.Tensor] = None):
+                                  ids: torch.Tensor, mask: Optional[torch.Tensor] = None, *,
+                                  marked: bool = False):
     """``(logp_policy, logp_ref)``; one launch when both tensors share shape, dtype and device,
-    two scans otherwise.  With ``mask`` (bool, shape of ``ids``, on the logits' device) the one launch
-    leaves masked rows unread and 0; what the two scans return there is not specified."""
+    two scans otherwise.  With ``mask`` (bool, shape of ``ids``, on the logits' device) masked rows give 0
+    and get a zero gradient; the one launch does not read them.  ``marked``: ``ids`` is a copy of the
+    caller's ids with -1 at the masked rows (otherwise it is made here)."""
     if logits.dtype not in _IN or ref_logits.dtype not in _IN:
         raise RuntimeError("logits dtype must be float32, float16 or bfloat16")
+    if mask is not None and not marked:
+        ids = torch.where(mask.reshape(ids.shape), ids, -1)
     if (logits.shape == ref_logits.shape and logits.dtype == ref_logits.dtype
             and logits.device == ref_logits.device):
         rows = None if mask is None else mask.reshape(-1).contiguous()

@@ -42,3 +42,16 @@ def test_a_bad_target_raises_and_the_next_call_is_clean():
         out.sum().backward()
     torch.cuda.synchronize()
     assert torch.isfinite(out).all() and torch.isfinite(hidden.grad).all()
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1025, 9000])
+def test_marked_ids_are_a_copy_with_the_masked_ones_out_of_range(n):
+    from rl_kernel_amd import _native
+
+    dev = torch.device("cuda")
+    ids = torch.randint(0, 50, (n,), device=dev)
+    mask = torch.rand(n, device=dev) < 0.6
+    for m in (mask, None):
+        marked = torch.full_like(ids, 77)
+        assert not _native.TargetCheck(ids, 50, mask=m, marked=marked).out_of_range()
+        assert torch.equal(marked, ids if m is None else torch.where(m, ids, torch.full_like(ids, -1)))
