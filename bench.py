@@ -54,14 +54,14 @@ MEASURED_TRAFFIC = {
 }
 
 WORKLOADS = {
-    # BASELINE.json configs[1] shape; the metric is quoted on forward+backward at this shape
+    # the headline metric is quoted on forward+backward at this shape
     "llama3-8b-head": dict(tokens=32768, hidden=4096, vocab=128256, dtype="bf16",
                            temperature=1.0, ignore_frac=0.0),
     "llama3-8b-head-64k": dict(tokens=65536, hidden=4096, vocab=128256, dtype="bf16",
                                temperature=0.7, ignore_frac=0.0),
     "qwen3-head": dict(tokens=131072, hidden=2048, vocab=151936, dtype="f16",
                        temperature=1.0, ignore_frac=0.01),
-    # the configs[1] shape with the GRPO epilogue between forward and
+    # the headline shape with the GRPO epilogue between forward and
     # backward (one group of 64 responses x 512 positions, response lengths U{128..512})
     "llama3-8b-grpo-step": dict(tokens=32768, hidden=4096, vocab=128256, dtype="bf16",
                                 temperature=1.0, ignore_frac=0.0, grpo=dict(group=64, seq=512,
@@ -71,7 +71,7 @@ WORKLOADS = {
                         ignore_frac=0.0, scan=True),
     "small": dict(tokens=4096, hidden=1024, vocab=32768, dtype="bf16", temperature=1.0,
                   ignore_frac=0.0),
-    # fp32 hidden states and head on the fp32 matrix instruction (two shapes, see bench_fp32_inputs)
+    # fp32 hidden states and head (two shapes, see bench_fp32_inputs)
     "fp32-inputs": dict(tokens=4096, hidden=2048, vocab=32768, dtype="f32", temperature=1.0,
                         ignore_frac=0.0, fp32=True),
 }
@@ -736,11 +736,13 @@ def bench_reference_shapes(torch):
 
 def bench_fp32_inputs(torch):
     """fp32 hidden states and head (what the reference runs in its CPU tests and what callers that keep
-    an fp32 lm_head pass): the same entry points on the fp32 matrix instruction, priced against the
-    157.3 TFLOP/s fp32 matrix peak; a plain fp32 library GEMM of the forward's shape beside it."""
+    an fp32 lm_head pass): the same entry points on the fp32 kernels, which take an fp32 product as six
+    bf16 piece products on the 16-bit matrix instruction and are priced against a sixth of its peak;
+    a plain fp32 library GEMM of the forward's shape beside it."""
     from rl_kernel_amd.ops import linear_logp as LL
 
     dev = torch.device("cuda:0")
+    peak = PEAK_TFLOPS["bf16"] / 6.0
     rows = []
     for n, h, v in ((4096, 2048, 32768), (2048, 4096, 128256)):
         gen = torch.Generator(device=dev).manual_seed(v)
@@ -758,12 +760,13 @@ def bench_fp32_inputs(torch):
         flop = 2.0 * n * h * v
         rows.append({"shape": f"{n}x{h}x{v}", "fwd_ms": f_ms, "bwd_ms": b_ms,
                      "fwd_tflops": flop / f_ms / 1e9, "bwd_tflops": 3.0 * flop / b_ms / 1e9,
-                     "fwd_frac_of_fp32_peak": flop / f_ms / 1e9 / 157.3,
-                     "bwd_frac_of_fp32_peak": 3.0 * flop / b_ms / 1e9 / 157.3,
+                     "fwd_frac_of_peak": flop / f_ms / 1e9 / peak,
+                     "bwd_frac_of_peak": 3.0 * flop / b_ms / 1e9 / peak,
                      "library_fp32_gemm_tflops": flop / g_ms / 1e9})
         del hidden, weight
-    return {"what": "rlk_linear_logp_fwd / _bwd on fp32 inputs (v_mfma_f32_32x32x2_f32 tiles), "
-                    "TFLOP/s on 2NHV / 6NHV, peak 157.3 TFLOP/s", "rows": rows}
+    return {"what": "rlk_linear_logp_fwd / _bwd on fp32 inputs (six bf16 piece products a product, "
+                    f"v_mfma_f32_32x32x16_bf16), TFLOP/s on 2NHV / 6NHV, peak {peak:.0f} = a sixth of the "
+                    "16-bit peak", "rows": rows}
 
 
 def main() -> int:

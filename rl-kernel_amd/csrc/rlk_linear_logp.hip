@@ -171,10 +171,10 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
         return (head == 0 ? a.weight : a.weight2) + static_cast<int64_t>(tile_row(vt)) * a.H;
     };
     if constexpr (CHAIN) {
-        // every tile is full (or moved back) and every split has a tile (n_split <= vtiles): one pipeline runs through all tiles of the range (and then through
-        // the same range of the second head), the K loop of a tile already fetching the head of the
-        // next one while the softmax update runs (the pipeline looks two K steps ahead, which stays
-        // within the next tile from two steps up)
+        // every tile is full (or moved back) and every split has a tile (n_split <= vtiles): one pipeline
+        // runs through all tiles of the range (and then through the same range of the second head), the
+        // K loop of a tile already fetching the head of the next one while the softmax update runs (the
+        // pipeline looks two K steps ahead, which stays within the next tile from two steps up)
         typename Dtl::Stream st;
         Dtl::begin(st, Operand{tile_origin(0, t0), a.H, 256}, B, a.H, smem);
         for (int head = 0; head < n_heads; ++head) {
@@ -264,7 +264,8 @@ __device__ inline float combine_token(const CombineArgs& a, int64_t n)
 // side, then one thread per token adds the rescaled sums in split order, as combine_token would; the
 // merged state replaces the token's slot 0, which the combine kernels read as their only split.  One
 // thread walking all splits of a token through memory is a chain of dependent loads: 37 us for 160
-// tokens x 62 splits.  LDS: the terms [2][n_split][4] behind the group maxima. (16 x 16 took 14 us for 160 tokens x 251 splits.)
+// tokens x 62 splits.  LDS: the terms [2][n_split][4] behind the group maxima.  (16 tokens x 16 groups took
+// 14 us for 160 tokens x 251 splits.)
 constexpr int kMergeTokens = 4, kMergeGroups = 64;
 inline size_t merge_smem(int n_split) { return static_cast<size_t>(kMergeGroups + 2 * n_split) * kMergeTokens * 4; }
 __global__ __launch_bounds__(256) void linear_logp_merge_kernel(float* part_m, float* part_s, float* part_z, int N,
@@ -378,8 +379,8 @@ struct DzArgs {
     int tok_tiles;
     int v_tiles;        // vocab tiles of this launch
     int v_tile_lo;      // first vocab tile of this launch
-    int tok_shift;      // rows / vocab rows by which the last token / vocab tile is moved back (see
-    int v_shift;        // BwdShift; 0 in the unchained kernels)
+    int tok_shift;      // rows / vocab rows by which the last token / vocab tile is moved back so that it
+    int v_shift;        // ends at the last row there is (0 in the unchained kernels)
     int64_t v_global0;  // global id of the piece's first vocab row
     int64_t ignore_index;
     int use_ignore;
@@ -704,7 +705,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dh_kernel(DhArgs a)
             int ntt = tt, nht = ht;
             if (more) walk.coords(true, ntt, nht);
             zero_acc(acc);
-            // a full tile's epilogue issues TM * TN unconditional stores per wavefront
+            // a full tile's epilogue issues TM * TN unconditional stores per wavefront; half is enough
             Dtl::template tile<true, Acc16::TM * Acc16::TN / 2>(st, w_origin(nht), z_origin(ntt), acc, smem, counted);
             counted = dh_epilogue<T>(acc, a, tt, h_col(ht), ht * 256, a.acc, a.first != 0, a.last != 0);
             if (!more) break;
@@ -826,6 +827,14 @@ __device__ inline void gather_rows(u32x2_t (&p)[4])
     }
 }
 
+// Stores that the epilogue of a full dW tile issues per wavefront, all of them unconditional, the fewer of its
+// two forms: 16 bytes per quad of fp32 (TM * TN = 32), 16 bytes per pair of quads of 16-bit results (16).
+// The tile loop counts on them (TileGemmDtl::tile, YOUNGER): with one fewer it would take a load of the
+// next tile for a store and read a stage that has not landed, so there is no margin in the 16-bit form.
+constexpr int kDwPairsPerGroup = 2;  // 16-byte stores of 16-bit results per four quads, see the loop
+constexpr int kDwStores = Acc16::TM / 4 * kDwPairsPerGroup * Acc16::TN;
+static_assert(kDwStores <= Acc16::TM * Acc16::TN, "the fp32 form stores a quad at a time");
+
 // Epilogue of one dW tile.  Orientation: M (accumulator registers) = hidden column, N (lane) =
 // vocab row, so a lane holds 4 consecutive columns of one dW row and the read-modify-write of the
 // fp32 tile moves 16 bytes per lane (the four lane groups of a 16 x 16 tile make 64 contiguous
@@ -895,7 +904,7 @@ __device__ inline void dw_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
                         const int h16 = hgrp + (i - 3) * 16;  // 16 columns of this lane, in two chunks of 8
                         uint16_t* row = a.out + vrow[jj];
 #pragma unroll
-                        for (int q = 0; q < 2; ++q) {
+                        for (int q = 0; q < kDwPairsPerGroup; ++q) {
                             const int hq = h16 + 8 * q;  // H, h0 and h_min % 8 == 0: all-in or all-out
                             if (FULL || (v_ok[jj] && hq >= h_min && hq < a.H))
                                 *reinterpret_cast<u32x4_t*>(row + hq) =
@@ -952,8 +961,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dw_kernel(DwArgs a)
             int nvt = vt, nht = ht;
             if (more) walk.coords(true, nvt, nht);
             zero_acc(acc);
-            // a full tile's epilogue issues TM * TN unconditional stores per wavefront
-            Dtl::template tile<true, Acc16::TM * Acc16::TN / 2>(st, h_origin(nht), z_origin(nvt), acc, smem, counted);
+            Dtl::template tile<true, kDwStores>(st, h_origin(nht), z_origin(nvt), acc, smem, counted);
             counted = dw_epilogue<T>(acc, a, vt, h_col(ht), ht * 256);
             if (!more) break;
             walk.advance();
@@ -1215,7 +1223,8 @@ inline int dh_parts(int64_t ct, int64_t pt, int64_t ht)
     return parts;
 }
 
-// What a split dH launch really cuts its vocab range into: as many parts as give every CU a tile (at
+// What a split dH launch really cuts its vocab range into (the plan below prices and reports dh_parts, a
+// lower bound): as many parts as give every CU a tile (at
 // least 16 K steps each; their slots stay within 256 tiles of fp32).  The powers of two above left the
 // launch on 64 to 192 CUs: 64 x 2048 x 32000 318 -> 239, 64 x 4096 x 128256
 // 1306 -> 1168, 1000 x 1536 x 151936 1910 -> 1838 us a pass.
