@@ -8,7 +8,13 @@
 namespace rlk {
 
 constexpr int kNormThreads = 256;
-constexpr int kNormRowsPerGroup = 16;  // rows one workgroup of the backward takes (one d_gain partial)
+
+// Rows one workgroup of the backward takes (one d_gain partial [H] each).  The partials are an eighth of a
+// 16-bit x, a quarter of that with 64 rows; but the kernel that walks a row with a whole workgroup needs
+// the workgroups: 20000 x 4096 fp32 450 us with 16 rows, 1284 with 64 (65536 x 4096: 1114, 1634).  The
+// one-wavefront kernel would not mind from 16384 rows on (32768 x 4096 bf16 212 us, 187), but the workspace
+// query knows neither the type nor the alignment that choose between the two.
+constexpr int kNormRowsPerGroup = 16;
 
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4n;
 typedef __attribute__((ext_vector_type(4))) float f32x4n;
