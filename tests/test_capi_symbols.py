@@ -127,6 +127,41 @@ def test_backward_workspace_holds_the_dh_slots_of_every_block_kind(native):
         assert slots <= 67 << 20  # <= 256 tiles of fp32
 
 
+def _dh_cuts(ct, pt, ht):
+    """Parts that a split dH launch is really cut into (restated): as many as give every CU a tile, at
+    least 4 vocab tiles each, at most 32; never fewer than the plan query reports."""
+    parts = _dh_parts(ct, pt, ht)
+    return 1 if parts == 1 else max(parts, min(256 // (ct * ht), pt // 4, 32))
+
+
+def test_backward_workspace_holds_the_slots_of_the_dh_launches_that_run(native):
+    """The launch cuts finer than the plan query's lower bound; few tokens also need the padded token tile."""
+    import random
+
+    lib = native.load()
+    rng, finer = random.Random(11), 0
+    for _ in range(600):
+        n = rng.choice((rng.randrange(1, 256), rng.randrange(256, 4096), rng.randrange(1, 100) * 256))
+        h = rng.choice((64, 256, 896, 1024, 1536, 2048, 4096, 8192))
+        v = rng.randrange(300, 160000)
+        budget = rng.choice((0, 16 << 20, 64 << 20, 128 << 20))
+        tok_chunk, v_piece, n_chunks, n_pieces, _ = _plan(lib, n, h, v, 0, budget)
+        ct, pt, ht = tok_chunk // 256, v_piece // 256, (h + 255) // 256
+        ct_last = (n + 255) // 256 - (n_chunks - 1) * ct
+        pt_last = (v + 255) // 256 - (n_pieces - 1) * pt
+        kinds = [(c, p) for c in (ct, ct_last) for p in (pt, pt_last)]
+        slots = max([k * c * 256 * h * 4 for c, p in kinds for k in [_dh_cuts(c, p, ht)] if k > 1] or [0])
+        finer += any(_dh_cuts(c, p, ht) > _dh_parts(c, p, ht) for c, p in kinds)
+        need = ctypes.c_size_t(0)
+        assert lib.rlk_linear_logp_bwd_workspace_bytes(n, h, v, 0, budget, ctypes.byref(need)) == 0
+        acc = tok_chunk * h * 4 if n_pieces > 1 else 0
+        pad = 256 * h * 2 if n < 256 else 0
+        rest = 256 + tok_chunk * v_piece * 2 + acc + ct * v_piece * 4 + pad
+        assert need.value >= rest + slots, (n, h, v, budget)
+        assert slots <= 67 << 20  # <= 256 tiles of fp32
+    assert finer > 50
+
+
 def test_forward_workspace_is_small(native):
     lib = native.load()
     need = ctypes.c_size_t(0)
