@@ -983,36 +983,42 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dw_kernel(DwArgs a)
     }
 }
 
-// Fewer tokens than a tile: the rows of `hidden`, the last one repeated up to one 256-row tile, so that dZ
-// and dW run on the full-tile pipeline (at most 256 x H x 2 bytes, a few us against the register-staged
-// loop that a K tail of the whole dW contraction would need: 12 to 20 % of a backward at 160 tokens).
-// dZ evaluates a row past the end against the last token's log-sum-exp and a zero upstream gradient, so
-// that row has to hold that token's logits: a probability of at most 1 times 0.  (Rows of zeros have
-// logits of 0 or the bias; against a log-sum-exp below -88 their probability is inf and dZ NaN.)
+// Fewer tokens than a tile: the rows of `hidden`, the last one repeated up to row `used`, rows of zeros up to
+// one 256-row tile, so that dZ and dW run on the full-tile pipeline (at most 256 x H x 2 bytes, a few us
+// against the register-staged loop that a K tail of the whole dW contraction would need: 12 to 20 % of a
+// backward at 160 tokens).
+// dZ evaluates a row past the end against the last token's log-sum-exp and a zero upstream gradient.  The K
+// steps of dW read such rows up to `used`: they have to hold that token's logits, a probability of at
+// most 1 times 0.  (Rows of zeros have logits of 0 or the bias; against a log-sum-exp below -88 their
+// probability is inf and dZ NaN.)  From `used` on nobody reads dZ, and zeros draw the least power in the
+// products: backward of 64 x 4096 x 128256 890 us with copies up to the tile's end, 884 so, 882 with zeros alone.
 // One row per blockIdx.y, 16 bytes per thread.
-__global__ void linear_logp_pad_rows_kernel(const uint16_t* src, uint16_t* dst, int n_rows, int row8)
+__global__ void linear_logp_pad_rows_kernel(const uint16_t* src, uint16_t* dst, int n_rows, int used, int row8)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= row8) return;
     const int64_t row = blockIdx.y, from = row < n_rows ? row : n_rows - 1;
-    reinterpret_cast<u32x4_t*>(dst)[row * row8 + i] = reinterpret_cast<const u32x4_t*>(src)[from * row8 + i];
+    reinterpret_cast<u32x4_t*>(dst)[row * row8 + i] =
+        row < used ? reinterpret_cast<const u32x4_t*>(src)[from * row8 + i] : u32x4_t{0u, 0u, 0u, 0u};
 }
 
 // db[v] (+)= sum_tok dZ[tok][v] in two fixed-order levels.  Level 1: one workgroup per (256
 // columns) x (256-token tile); a thread owns 8 columns (one 16-byte load per row) of every eighth
 // row, the eight row groups are added in order through LDS: part[tile][v].  The dZ block is written
-// in whole tiles (padding rows and columns hold zeros), so no row or column check is needed here.
+// in whole tiles (rows and columns that nobody owns hold zeros), so no column check is needed here;
+// `rows` is 256 but for a padded tile, whose rows past the tokens are left out.
 template <class T>
-__global__ __launch_bounds__(256) void linear_logp_db_partial_kernel(const uint16_t* dz, int64_t ldz, float* part,
-                                                                     int64_t part_ld)
+__global__ __launch_bounds__(256) void linear_logp_db_partial_kernel(const uint16_t* dz, int64_t ldz, int rows,
+                                                                     float* part, int64_t part_ld)
 {
     __shared__ float red[8][256];
     const int cg = threadIdx.x & 31, rg = threadIdx.x >> 5;
     const int v0 = blockIdx.x * 256 + cg * 8;
     const uint16_t* p = dz + (static_cast<int64_t>(blockIdx.y) * 256 + rg) * ldz + v0;
     float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const int steps = (rows - rg + 7) >> 3;
 #pragma unroll 4
-    for (int k = 0; k < 32; ++k) {
+    for (int k = 0; k < steps; ++k) {
         const u32x4_t w = *reinterpret_cast<const u32x4_t*>(p + static_cast<int64_t>(k) * 8 * ldz);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -1478,9 +1484,10 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
     const bool padded = shifted && N < 256;
     if (padded) {
         uint16_t* pad = reinterpret_cast<uint16_t*>(ws + p.pad_off);
-        const int row8 = static_cast<int>(H / 8);
+        const int row8 = static_cast<int>(H / 8), n = static_cast<int>(N);
+        const int used = std::max(2, (n + kBK - 1) / kBK) * kBK;  // the rows of dW's K steps, see k_steps below
         hipLaunchKernelGGL(linear_logp_pad_rows_kernel, dim3((row8 + 255) / 256, 256), dim3(256), 0, stream, hid, pad,
-                           static_cast<int>(N), row8);
+                           n, used, row8);
         hid = pad;
     }
 
@@ -1651,7 +1658,8 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
             if (c.d_bias != nullptr) {
                 float* db_part = reinterpret_cast<float*>(ws + p.db_off);
                 hipLaunchKernelGGL(linear_logp_db_partial_kernel<T>, dim3(v_tiles, tok_tiles), dim3(256), 0,
-                                   stream, dz, p.ldz, db_part, static_cast<int64_t>(p.v_piece));
+                                   stream, dz, p.ldz, padded ? static_cast<int>(N) : 256, db_part,
+                                   static_cast<int64_t>(p.v_piece));
                 hipLaunchKernelGGL(linear_logp_db_finish_kernel, dim3((v_valid + 255) / 256), dim3(256), 0,
                                    stream, db_part, static_cast<int64_t>(p.v_piece), tok_tiles, v_valid,
                                    v_shift, scales, c.d_bias + v_lo, (ci > 0 || c.accumulate != 0) ? 1 : 0);

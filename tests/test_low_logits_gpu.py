@@ -84,3 +84,22 @@ def test_short_last_block_behind_the_norm(n):
         assert torch.isfinite(t).all()
     # (column 0 is a hundred times the others)
     assert rel(d_w[:, 1:], r_dw[:, 1:]) < GRAD_REL[torch.bfloat16] and rel(d_b, r_db) < GRAD_REL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("n", [1, 100, 255, 300])
+def test_a_logit_of_minus_infinity_gets_no_gradient(n):
+    """A weight row that is -inf in a column where every hidden value is positive: its logits are -inf, its
+    probability and its gradient 0, and no other row's gradient meets an infinity or NaN."""
+    from rl_kernel_amd.ops import linear_logp as LL
+
+    dev, h, v = torch.device("cuda"), 256, 577
+    hidden, weight, b, ids, grad = make(n, h, v, torch.bfloat16, True, n)
+    hidden[:, 3] = hidden[:, 3].abs() + 0.5
+    weight[7, 3] = weight[576, 3] = float("-inf")
+    ids = ids.clamp(8, 575)
+    hd, wd, td, bd = hidden.to(dev), weight.to(dev), ids.to(dev), b.to(dev)
+    _, lse, _ = LL.fused_linear_logp_forward(hd, wd, td, bd)
+    assert torch.isfinite(lse).all()
+    _, dw, db = LL.fused_linear_logp_backward(grad.to(dev), hd, wd, td, lse, bd, need_hidden=False)
+    assert torch.isfinite(dw).all() and torch.isfinite(db).all()
+    assert torch.all(dw[[7, 576]] == 0) and torch.all(db[[7, 576]] == 0)
