@@ -117,7 +117,7 @@ _wide_path_warned = False
 
 def _warn_if_wide_path(hidden_2d: torch.Tensor, weight: torch.Tensor) -> None:
     """The 16-bit MFMA tiles take bf16/f16 with H % 8 == 0 and 16-byte aligned matrices; 16-bit
-    inputs that miss that run on the fp32 kernels at roughly a sixth of the rate.  Say so
+    inputs that miss that run on the fp32 kernels at roughly a ninth of the rate.  Say so
     once when a large problem ends up there."""
     global _wide_path_warned
     if _wide_path_warned or hidden_2d.dtype == torch.float32:
@@ -129,7 +129,7 @@ def _warn_if_wide_path(hidden_2d: torch.Tensor, weight: torch.Tensor) -> None:
         logger.warning(
             "linear_logp: %s inputs with H=%d run on the fp32 matrix-core kernels (the 16-bit MFMA "
             "path takes H %% 8 == 0 and 16-byte aligned matrices); expect this %d x %d x %d problem "
-            "to run at about a sixth of the 16-bit rate", str(hidden_2d.dtype), h, n, h,
+            "to run at about a ninth of the 16-bit rate", str(hidden_2d.dtype), h, n, h,
             weight.size(0))
 
 
