@@ -559,7 +559,7 @@ def bench_registry_op(torch, hidden, weight, targets, grad, temp, ign, steps):
     res = {"class": type(op).__name__, "ms_per_step": ms, "tokens_per_s": n / (ms * 1e-3),
            "steps": steps, "peak_extra_hbm_bytes": int(peak_extra),
            "note": "declared outputs here are logp, dH and dW in the weight dtype; the extra bytes "
-                   "include the fp32 dW the kernels accumulate into before the cast (as the "
+                   "include the workspace with the running fp32 dW of the token chunks (as the "
                    "reference's backward keeps an fp32 grad_w) and the saved lse"}
     del out
     hid.grad = None
