@@ -441,6 +441,7 @@ struct DtlIO {
     int nk;                  // K steps per tile
     int wave;                // uniform wavefront index
     int tail_from;           // TAIL: first K step of the shifted last K tile
+    int next_tail_from;      // TAIL: the same of the tile that follows
     int64_t tail_adj;        // TAIL: uniform byte adjustment of those steps
 
     __device__ inline void init(const Operand& op, int K)
@@ -480,7 +481,7 @@ struct DtlIO {
         const bool over = kt >= nk;
         const int rel = over ? (kt - nk < nk ? kt - nk : nk - 1) : kt;
         const char* src = (over ? next : base) + static_cast<size_t>(rel) * step;
-        if constexpr (TAIL) src += rel >= tail_from ? tail_adj : 0;  // uniform
+        if constexpr (TAIL) src += rel >= (over ? next_tail_from : tail_from) ? tail_adj : 0;  // uniform
         const uint32_t dst = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
                                  (RLK_LDS char*)(lds))) + static_cast<uint32_t>((wave + kWaves * p) * 1024);
         asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
@@ -583,7 +584,7 @@ struct TileGemmDtl {
         IOB lb;
         u32x4_t fa[2][TM];
         u32x4_t fb[2][TN];
-        int wm, wn, nk, phase;
+        int wm, wn, nk, next_nk, phase;
     };
 
     __device__ static inline void first_frags(Stream& st, const char* stage)
@@ -605,10 +606,10 @@ struct TileGemmDtl {
         st.wn = wave % kWN;
         st.la.init(A, K);
         st.lb.init(B, K);
-        st.la.tail_from = st.lb.tail_from = tail.from;
+        st.la.tail_from = st.lb.tail_from = st.la.next_tail_from = st.lb.next_tail_from = tail.from;
         st.la.tail_adj = tail.a;
         st.lb.tail_adj = tail.b;
-        st.nk = K / BK;
+        st.nk = st.next_nk = K / BK;
         st.phase = 0;
         static_for<0, PA>([&](auto pc) { st.la.load_one(0, smem, decltype(pc)::value); });
         static_for<0, PB>(
@@ -622,6 +623,14 @@ struct TileGemmDtl {
         __builtin_amdgcn_s_waitcnt(wait_first);  // K step 0 has landed
         __syncthreads();
         first_frags(st, smem);
+    }
+
+    // K steps of the tile that follows and its `tail.from`, before tile() runs on the current one (tiles of
+    // one stream may be cut to different lengths of at least two steps).
+    __device__ static inline void next_steps(Stream& st, int nk, int tail_from)
+    {
+        st.next_nk = nk;
+        st.la.next_tail_from = st.lb.next_tail_from = tail_from;
     }
 
     // All K steps of the current tile into `acc`.  `next_a` / `next_b` are the operand origins of
@@ -664,6 +673,11 @@ struct TileGemmDtl {
         st.phase = (st.phase + nk) & 1;
         st.la.base = st.la.next;
         st.lb.base = st.lb.next;
+        st.nk = st.la.nk = st.lb.nk = st.next_nk;
+        if constexpr (TAIL) {
+            st.la.tail_from = st.la.next_tail_from;
+            st.lb.tail_from = st.lb.next_tail_from;
+        }
     }
 
     // Drain the fetches issued for a tile that will not be computed; LDS is free afterwards.

@@ -678,82 +678,46 @@ __device__ inline bool dh_epilogue(const f32x4_t (&acc)[Acc16::TM][Acc16::TN], c
     return full;
 }
 
-// CHAIN (needs ksplit == 1, H >= 256 and a.nk >= 2): the workgroup walks its tiles through one
-// pipeline.
-template <class T, int BK, bool CHAIN>
+// One tile (or one vocab part of a tile) per workgroup, for the sizes that the chained walk of
+// linear_logp_grads_kernel does not take (H < 256 or not a multiple of 64).
+template <class T, int BK>
 __global__ __launch_bounds__(kThreads) void linear_logp_dh_kernel(DhArgs a)
 {
     using Gemm = TileGemm<T, true, false, BK>;
-    using Dtl = TileGemmDtl<T, true, false, BK, kWinDh, true>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     f32x4_t acc[Acc16::TM][Acc16::TN];
-    if constexpr (CHAIN) {
-        TileWalk walk(a.tok_tiles * a.h_tiles, a.tok_tiles, a.h_tiles);
-        if (!walk.valid()) return;
-        int tt, ht;
-        walk.coords(false, tt, ht);
-        // first hidden column of h tile `h`: the last tile is shifted back so that it ends at H
-        auto h_col = [&](int h) { return min(h * 256, a.H - 256); };
-        auto w_origin = [&](int h) { return a.weight + h_col(h); };
-        auto z_origin = [&](int t) { return a.dz + static_cast<int64_t>(t) * 256 * a.ldz; };
-        typename Dtl::Stream st;
-        bool counted = false;
-        Dtl::begin(st, Operand{w_origin(ht), a.H, 256}, Operand{z_origin(tt), a.ldz, 256}, a.nk * BK, smem,
-                   a.tail);
-        for (;;) {
-            const bool more = walk.has_next();
-            int ntt = tt, nht = ht;
-            if (more) walk.coords(true, ntt, nht);
-            zero_acc(acc);
-            // a full tile's epilogue issues TM * TN unconditional stores per wavefront; half is enough
-            Dtl::template tile<true, Acc16::TM * Acc16::TN / 2>(st, w_origin(nht), z_origin(ntt), acc, smem, counted);
-            counted = dh_epilogue<T>(acc, a, tt, h_col(ht), ht * 256, a.acc, a.first != 0, a.last != 0);
-            if (!more) break;
-            walk.advance();
-            tt = ntt;
-            ht = nht;
+    int tt, ht, ks = 0;
+    xcd_tile(blockIdx.x, a.tok_tiles * a.h_tiles * a.ksplit, a.tok_tiles, a.h_tiles * a.ksplit, 8,
+             tt, ht);
+    // K range of this workgroup: whole BK-row steps, the first (steps % ksplit) parts take one more
+    int k0 = 0, kn = a.v_valid;
+    float* acc_dst = a.acc;
+    bool first = a.first != 0, last = a.last != 0, empty_part = false;
+    if (a.ksplit > 1) {  // uniform
+        ks = ht % a.ksplit;
+        ht /= a.ksplit;
+        const int steps = (a.v_valid + BK - 1) / BK;
+        const int base = steps / a.ksplit, extra = steps % a.ksplit;
+        const int s0 = ks * base + (ks < extra ? ks : extra);
+        const int s1 = s0 + base + (ks < extra ? 1 : 0);
+        k0 = s0 * BK;
+        kn = min(a.v_valid, s1 * BK) - k0;
+        if (kn <= 0) {  // a short last piece can leave a part without K steps: it computes one
+            empty_part = true;  // step of the piece's head and discards it
+            k0 = 0;
+            kn = min(a.v_valid, BK);
         }
-        Dtl::end(st);
-    } else {
-        int tt, ht, ks = 0;
-        xcd_tile(blockIdx.x, a.tok_tiles * a.h_tiles * a.ksplit, a.tok_tiles, a.h_tiles * a.ksplit, 8,
-                 tt, ht);
-        // K range of this workgroup: whole BK-row steps, the first (steps % ksplit) parts take one more
-        int k0 = 0, kn = a.v_valid;
-        float* acc_dst = a.acc;
-        bool first = a.first != 0, last = a.last != 0, empty_part = false;
-        if (a.ksplit > 1) {  // uniform
-            ks = ht % a.ksplit;
-            ht /= a.ksplit;
-            const int steps = a.nk > 0 ? a.nk : (a.v_valid + BK - 1) / BK;
-            const int base = steps / a.ksplit, extra = steps % a.ksplit;
-            const int s0 = ks * base + (ks < extra ? ks : extra);
-            const int s1 = s0 + base + (ks < extra ? 1 : 0);
-            k0 = s0 * BK;
-            kn = (a.nk > 0 ? s1 * BK : min(a.v_valid, s1 * BK)) - k0;
-            if (kn <= 0) {  // a short last piece can leave a part without K steps: it computes one
-                empty_part = true;  // step of the piece's head and discards it
-                k0 = 0;
-                kn = a.nk > 0 ? BK : min(a.v_valid, BK);
-            }
-            acc_dst = a.part + static_cast<int64_t>(ks) * a.part_stride;
-            first = true;
-            last = false;
-        }
-        const int tok0 = tt * 256, h0 = ht * 256;
-        Operand A{a.weight + static_cast<int64_t>(k0) * a.H + h0, a.H, min(256, a.H - h0)};
-        Operand B{a.dz + static_cast<int64_t>(tok0) * a.ldz + k0, a.ldz, 256};
-        zero_acc(acc);
-        if (a.nk > 0) {  // uniform
-            KTail tail = a.tail;
-            tail.from = max(0, tail.from - k0 / BK);
-            Dtl::run(A, B, a.ksplit > 1 ? kn : a.nk * BK, acc, smem, tail);
-        } else {
-            Gemm::run(A, B, kn, acc, smem);
-        }
-        if (empty_part) zero_acc(acc);  // uniform: this part's slot must hold zeros
-        dh_epilogue<T>(acc, a, tt, h0, h0, acc_dst, first, last);
+        acc_dst = a.part + static_cast<int64_t>(ks) * a.part_stride;
+        first = true;
+        last = false;
     }
+    const int tok0 = tt * 256, h0 = ht * 256;
+    Operand A{a.weight + static_cast<int64_t>(k0) * a.H + h0, a.H, min(256, a.H - h0)};
+    Operand B{a.dz + static_cast<int64_t>(tok0) * a.ldz + k0, a.ldz, 256};
+    zero_acc(acc);
+    Gemm::run(A, B, kn, acc, smem);
+    if (empty_part) zero_acc(acc);  // uniform: this part's slot must hold zeros
+    dh_epilogue<T>(acc, a, tt, h0, h0, acc_dst, first, last);
 }
 
 // Sum of the ksplit partial dH slots of one chunk in slot order (plus the running fp32 partial of
@@ -768,7 +732,15 @@ __global__ void linear_logp_dh_reduce_kernel(const float* part, int ksplit, int6
     if (i >= n4) return;
     f32x4_t v{0.f, 0.f, 0.f, 0.f};
     if (!first) v = reinterpret_cast<const f32x4_t*>(acc)[i];
-    for (int k = 0; k < ksplit; ++k) v += reinterpret_cast<const f32x4_t*>(part + k * part_stride)[i];
+    for (int k0 = 0; k0 < ksplit; k0 += 8) {  // eight loads in flight, added in slot order
+        f32x4_t p[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            p[k] = reinterpret_cast<const f32x4_t*>(part + (k0 + k < ksplit ? k0 + k : k0) * part_stride)[i];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (k0 + k < ksplit) v += p[k];
+    }
     if (last) {
         const float oscale = scales[1];
         u32x2_t pk{T::pack2(v.x * oscale, v.y * oscale), T::pack2(v.z * oscale, v.w * oscale)};
@@ -798,6 +770,8 @@ struct DwArgs {
     int nk;          // K steps (of 64 tokens) of the chunk, the shifted tile's among them; 0: the block
     KTail tail;      // has no shifted tiles, K runs over [0, tok_valid)
     int v_shift;     // vocab rows by which the last vocab tile is moved back
+    int busy, lead;  // joint launch: workgroups with one dH item more than the others, and the rounds of dW
+                     // tiles that those others have ahead of them (see LeadWalk)
 };
 
 // 16-bit results of four 16-row MFMA tiles of one column: lane group g (16 lanes) holds rows 4 g .. 4 g + 3
@@ -935,52 +909,113 @@ __device__ inline bool dw_epilogue(const f32x4_t (&acc)[Acc16::TM][Acc16::TN], c
     return full;
 }
 
-// CHAIN (needs H >= 256 and a.nk >= 2): the workgroup walks its tiles through one pipeline.
-template <class T, int BK, bool CHAIN>
+// The sizes that the chained walk of linear_logp_grads_kernel does not take.
+template <class T, int BK>
 __global__ __launch_bounds__(kThreads) void linear_logp_dw_kernel(DwArgs a)
 {
     using Gemm = TileGemm<T, true, true, BK>;
-    using Dtl = TileGemmDtl<T, true, true, BK, kWinDw, true>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     TileWalk walk(a.v_tiles * a.h_tiles, a.v_tiles, a.h_tiles);
     if (!walk.valid()) return;
     int vt, ht;
     walk.coords(false, vt, ht);
     f32x4_t acc[Acc16::TM][Acc16::TN];
-    auto z_origin = [&](int v) { return a.dz + static_cast<int64_t>(v) * 256; };      // N rows
-    if constexpr (CHAIN) {
-        // first hidden column of h tile `h`: the last tile is shifted back so that it ends at H
-        auto h_col = [&](int h) { return min(h * 256, a.H - 256); };
-        auto h_origin = [&](int h) { return a.hidden + h_col(h); };  // M rows
+    for (;;) {
+        Operand A{a.hidden + static_cast<int64_t>(ht) * 256, a.H, min(256, a.H - ht * 256)};
+        Operand B{a.dz + static_cast<int64_t>(vt) * 256, a.ldz, 256};
+        zero_acc(acc);
+        Gemm::run(A, B, a.tok_valid, acc, smem);
+        dw_epilogue<T>(acc, a, vt, ht * 256, ht * 256);
+        if (!walk.has_next()) break;
+        walk.advance();
+        walk.coords(false, vt, ht);
+    }
+}
+
+// dH and dW of one dZ block in one launch (needs H >= 256 and nk >= 2 of either): they read the same block
+// and do not depend on each other, so a workgroup walks its dH tiles through one pipeline and its dW
+// tiles through another right behind, and the CUs that the last round of dH tiles leaves idle are at dW
+// tiles meanwhile (grads_split).  Two launches each rounded their tile count up to whole rounds.
+// h.ksplit > 1: a dH item is one part of the vocab range of a tile and leaves for that part's fp32
+// slot.  The items of one range are neighbours in the list (they share dZ columns), so the part
+// is the slow index.
+template <class T, int BK>
+__global__ __launch_bounds__(kThreads) void linear_logp_grads_kernel(DhArgs h, DwArgs d)
+{
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    f32x4_t acc[Acc16::TM][Acc16::TN];
+    const int dh_items = h.tok_tiles * h.h_tiles * h.ksplit;
+    if (static_cast<int>(blockIdx.x) < dh_items) {
+        using Dtl = TileGemmDtl<T, true, false, BK, kWinDh, true>;
+        TileWalk walk(dh_items, h.tok_tiles, h.h_tiles * h.ksplit);
+        const int base = h.nk / h.ksplit, extra = h.nk % h.ksplit;
+        struct Item {
+            int tt, ht, ks, step0, nk;
+        };
+        auto item = [&](bool next) {
+            Item it;
+            walk.coords(next, it.tt, it.ht);
+            it.ks = 0;
+            if (h.ksplit > 1) {  // uniform
+                it.ks = it.ht / h.h_tiles;
+                it.ht -= it.ks * h.h_tiles;
+            }
+            // whole K steps, the first `extra` parts take one more
+            it.step0 = it.ks * base + min(it.ks, extra);
+            it.nk = base + (it.ks < extra ? 1 : 0);
+            return it;
+        };
+        // first hidden column of h tile `t`: the last tile is shifted back so that it ends at H
+        auto h_col = [&](int t) { return min(t * 256, h.H - 256); };
+        auto w_origin = [&](const Item& it) { return h.weight + static_cast<int64_t>(it.step0) * BK * h.H + h_col(it.ht); };
+        auto z_origin = [&](const Item& it) { return h.dz + static_cast<int64_t>(it.tt) * 256 * h.ldz + it.step0 * BK; };
+        auto tail_from = [&](const Item& it) { return h.tail.from - it.step0; };
+        Item cur = item(false);
         typename Dtl::Stream st;
         bool counted = false;
-        Dtl::begin(st, Operand{h_origin(ht), a.H, 256}, Operand{z_origin(vt), a.ldz, 256}, a.nk * BK, smem,
-                   a.tail);
+        Dtl::begin(st, Operand{w_origin(cur), h.H, 256}, Operand{z_origin(cur), h.ldz, 256}, cur.nk * BK, smem,
+                   KTail{tail_from(cur), h.tail.a, h.tail.b});
         for (;;) {
             const bool more = walk.has_next();
-            int nvt = vt, nht = ht;
-            if (more) walk.coords(true, nvt, nht);
+            const Item nxt = more ? item(true) : cur;
             zero_acc(acc);
-            Dtl::template tile<true, kDwStores>(st, h_origin(nht), z_origin(nvt), acc, smem, counted);
-            counted = dw_epilogue<T>(acc, a, vt, h_col(ht), ht * 256);
+            Dtl::next_steps(st, nxt.nk, tail_from(nxt));
+            // a full tile's epilogue issues TM * TN unconditional stores per wavefront; half is enough
+            Dtl::template tile<true, Acc16::TM * Acc16::TN / 2>(st, w_origin(nxt), z_origin(nxt), acc, smem, counted);
+            const bool part = h.ksplit > 1;
+            counted = dh_epilogue<T>(acc, h, cur.tt, h_col(cur.ht), cur.ht * 256,
+                                     part ? h.part + cur.ks * h.part_stride : h.acc, part || h.first != 0,
+                                     !part && h.last != 0);
             if (!more) break;
             walk.advance();
-            vt = nvt;
-            ht = nht;
+            cur = nxt;
         }
         Dtl::end(st);
-    } else {
-        for (;;) {
-            Operand A{a.hidden + static_cast<int64_t>(ht) * 256, a.H, min(256, a.H - ht * 256)};
-            Operand B{z_origin(vt), a.ldz, 256};
-            zero_acc(acc);
-            Gemm::run(A, B, a.tok_valid, acc, smem);
-            dw_epilogue<T>(acc, a, vt, ht * 256, ht * 256);
-            if (!walk.has_next()) break;
-            walk.advance();
-            walk.coords(false, vt, ht);
-        }
     }
+    LeadWalk walk(d.v_tiles * d.h_tiles, d.v_tiles, d.h_tiles, d.busy, d.lead);
+    if (!walk.valid()) return;
+    using Dtl = TileGemmDtl<T, true, true, BK, kWinDw, true>;
+    int vt, ht;
+    walk.coords(false, vt, ht);
+    auto h_col = [&](int t) { return min(t * 256, d.H - 256); };
+    auto h_origin = [&](int t) { return d.hidden + h_col(t); };                          // M rows
+    auto z_origin = [&](int v) { return d.dz + static_cast<int64_t>(v) * 256; };        // N rows
+    typename Dtl::Stream st;
+    bool counted = false;
+    Dtl::begin(st, Operand{h_origin(ht), d.H, 256}, Operand{z_origin(vt), d.ldz, 256}, d.nk * BK, smem, d.tail);
+    for (;;) {
+        const bool more = walk.has_next();
+        int nvt = vt, nht = ht;
+        if (more) walk.coords(true, nvt, nht);
+        zero_acc(acc);
+        Dtl::template tile<true, kDwStores>(st, h_origin(nht), z_origin(nvt), acc, smem, counted);
+        counted = dw_epilogue<T>(acc, d, vt, h_col(ht), ht * 256);
+        if (!more) break;
+        walk.advance();
+        vt = nvt;
+        ht = nht;
+    }
+    Dtl::end(st);
 }
 
 // Fewer tokens than a tile: the rows of `hidden`, the last one repeated up to row `used`, rows of zeros up to
@@ -1244,9 +1279,48 @@ inline int dh_cuts(int64_t ct, int64_t pt, int64_t ht)
     return cuts > parts ? static_cast<int>(cuts) : parts;
 }
 
-inline int64_t block_cost(int64_t ct, int64_t pt, int64_t ht, int64_t hk)
+// How linear_logp_grads_kernel hands out n1 dH items of cost c1 and n2 dW tiles of cost c2 (K steps) to `grid`
+// workgroups: dH items in rounds, so the first n1 % grid workgroups (`busy`, in whole groups of the eight
+// XCDs) have one more than the others; those others take `lead` rounds of dW tiles among themselves before
+// the common rounds, as many as make the longest walk (`cost`) shortest.
+struct GradsSplit {
+    int busy = 0, lead = 0;
+    int64_t cost = 0;
+};
+inline GradsSplit grads_split(int64_t n1, int64_t c1, int64_t n2, int64_t c2, int64_t grid)
+{
+    GradsSplit best;
+    const int64_t full = n1 / grid, over = n1 % grid;
+    int64_t busy = over;
+    if (grid % 8 == 0) busy = (over + 7) / 8 * 8;
+    const int64_t rest = grid - busy;  // 0: all but at most seven workgroups have the extra item
+    const int64_t most = rest > 0 && c1 > 0 ? std::min(c1 / c2 + 1, (n2 + rest - 1) / rest) : 0;
+    for (int64_t lead = 0; lead <= most; ++lead) {
+        const int64_t left = std::max<int64_t>(0, n2 - lead * rest), rounds = (left + grid - 1) / grid;
+        const int64_t last = left - (rounds - 1) * grid;  // tiles of the last common round: the others come first
+        const int64_t slow = (full + (over > 0)) * c1 + (last > rest ? rounds : std::max<int64_t>(0, rounds - 1)) * c2;
+        const int64_t fast = rest > 0 ? full * c1 + (lead + rounds) * c2 : 0;
+        const int64_t cost = busy > 0 ? std::max(slow, fast) : fast;
+        if (lead == 0 || cost < best.cost) best = GradsSplit{static_cast<int>(busy), static_cast<int>(lead), cost};
+    }
+    return best;
+}
+
+// The dH + dW launch of one block of ct x pt tiles, in K steps (the reduction of split dH tiles included).
+inline int64_t grads_cost(int64_t ct, int64_t pt, int64_t ht)
+{
+    const int cuts = dh_cuts(ct, pt, ht);
+    return grads_split(ct * ht * cuts, (4 * pt + cuts - 1) / cuts + 9, pt * ht, 4 * ct + 9, 256).cost +
+           (cuts > 1 ? 10 : 0);
+}
+
+// Sizes whose backward runs on the chained walks whatever the token count (ragged tiles are moved back).
+bool bwd_chained(int H, int64_t V) { return H % kBK == 0 && H >= 256 && V >= 256; }
+
+inline int64_t block_cost(bool chained, int64_t ct, int64_t pt, int64_t ht, int64_t hk)
 {
     const int64_t dz = (ct * pt + 255) / 256 * (hk + 3);
+    if (chained) return dz + grads_cost(ct, pt, ht) + 12;  // filling three pipelines, two launches
     const int parts = dh_parts(ct, pt, ht);
     // split launch: every part is a workgroup of its own; the slot reduction costs about 10 steps
     const int64_t dh = parts > 1 ? (ct * ht * parts + 255) / 256 * (4 * pt / parts + 9) + 10
@@ -1272,6 +1346,7 @@ BwdPlan bwd_plan(int64_t N, int H, int64_t V, size_t budget)
 
     const int64_t n_t = (N + 255) / 256, v_t = (V + 255) / 256;
     const int64_t ht = (H + 255) / 256, hk = (H + kBK - 1) / kBK;
+    const bool chained = bwd_chained(H, V);
     const int64_t tile_bytes = 131072;                          // 256 x 256 16-bit
     const int64_t max_tiles = static_cast<int64_t>(budget) / tile_bytes;
     const int64_t cap = static_cast<int64_t>(budget) + static_cast<int64_t>(budget) / 2;
@@ -1297,10 +1372,10 @@ BwdPlan bwd_plan(int64_t N, int H, int64_t V, size_t budget)
             const int64_t np = (v_t + pt - 1) / pt, pt_last = v_t - (np - 1) * pt;
             const int64_t bytes = ct * pt * tile_bytes + (np > 1 ? ct * 256 * H * 4 : 0);
             if (bytes > cap && ct * pt > 1) continue;
-            const int64_t cost = (nc - 1) * (np - 1) * block_cost(ct, pt, ht, hk) +
-                                 (np - 1) * block_cost(ct_last, pt, ht, hk) +
-                                 (nc - 1) * block_cost(ct, pt_last, ht, hk) +
-                                 block_cost(ct_last, pt_last, ht, hk);
+            const int64_t cost = (nc - 1) * (np - 1) * block_cost(chained, ct, pt, ht, hk) +
+                                 (np - 1) * block_cost(chained, ct_last, pt, ht, hk) +
+                                 (nc - 1) * block_cost(chained, ct, pt_last, ht, hk) +
+                                 block_cost(chained, ct_last, pt_last, ht, hk);
             if (best_cost < 0 || cost < best_cost || (cost == best_cost && bytes < best_bytes)) {
                 best_cost = cost;
                 best_ct = ct;
@@ -1480,7 +1555,7 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
     // unchained dZ / dW launches for ragged token counts (the dW figures with the typed gradient):
     // 1000 x 1536 x 151936 dZ 599 -> 498 us, dW and its cast 1197 -> 515 us; 4096 x 2048 x 50257 dZ
     // 789 -> 732 us, dH 732 -> 658 us.
-    const bool shifted = H % kBK == 0 && H >= 256 && V >= 256;
+    const bool shifted = bwd_chained(H, V);
     const bool padded = shifted && N < 256;
     if (padded) {
         uint16_t* pad = reinterpret_cast<uint16_t*>(ws + p.pad_off);
@@ -1498,10 +1573,9 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
     if (int rc = set_smem(linear_logp_dz_kernel<T, kBK, false, true>, kDzChainSmem)) return rc;
     if (int rc = set_smem(linear_logp_dz_kernel<T, kBK, false, false>, GZ::kSmemBytes)) return rc;
     if (int rc = set_smem(linear_logp_dz_kernel<T, kBK, true, false>, GZ::kSmemBytes)) return rc;
-    if (int rc = set_smem(linear_logp_dh_kernel<T, kBK, true>, kChainSmem)) return rc;
-    if (int rc = set_smem(linear_logp_dh_kernel<T, kBK, false>, GH::kSmemBytes)) return rc;
-    if (int rc = set_smem(linear_logp_dw_kernel<T, kBK, true>, kChainSmem)) return rc;
-    if (int rc = set_smem(linear_logp_dw_kernel<T, kBK, false>, GW::kSmemBytes)) return rc;
+    if (int rc = set_smem(linear_logp_grads_kernel<T, kBK>, kChainSmem)) return rc;
+    if (int rc = set_smem(linear_logp_dh_kernel<T, kBK>, GH::kSmemBytes)) return rc;
+    if (int rc = set_smem(linear_logp_dw_kernel<T, kBK>, GW::kSmemBytes)) return rc;
 
     for (int ci = 0; ci < p.n_chunks; ++ci) {
         const int64_t tok_lo = static_cast<int64_t>(ci) * p.tok_chunk;
@@ -1569,7 +1643,7 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
             h.ksplit = ksplit;
             h.part = ksplit > 1 ? reinterpret_cast<float*>(ws + p.part_off) : nullptr;
             h.part_stride = static_cast<int64_t>(tok_tiles) * 256 * H;
-            const bool dh_chain = ksplit == 1 && H >= 256 && (shifted || (v_valid % kBK == 0 && v_valid >= 2 * kBK));
+            const bool dh_chain = shifted || (ksplit == 1 && H >= 256 && v_valid % kBK == 0 && v_valid >= 2 * kBK);
             h.nk = shifted ? k_steps(v_valid, v_shift) : (dh_chain ? v_valid / kBK : 0);
             h.tok_shift = tok_shift;
             h.tail = KTail();
@@ -1627,34 +1701,35 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
                                    dim3(tok_tiles * gen_tiles), dim3(kThreads), GZ::kSmemBytes,
                                    stream, z);
             }
-            if (dh) {
-                const int tiles = tok_tiles * h_tiles;
-                if (dh_chain) {
-                    hipLaunchKernelGGL((linear_logp_dh_kernel<T, kBK, true>),
-                                       dim3(chain_grid(tiles, n_cu)), dim3(kThreads), kChainSmem,
-                                       stream, h);
-                } else {
-                    hipLaunchKernelGGL((linear_logp_dh_kernel<T, kBK, false>),
-                                       dim3(tiles * ksplit), dim3(kThreads), GH::kSmemBytes, stream, h);
-                    if (ksplit > 1) {
-                        const int64_t n4 = static_cast<int64_t>(tok_valid) * H / 4;
-                        hipLaunchKernelGGL((linear_logp_dh_reduce_kernel<T>),
-                                           dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0,
-                                           stream, h.part, ksplit, h.part_stride, h.acc, h.out,
-                                           scales, n4, h.first, h.last);
-                    }
-                }
+            const bool want_dw = c.d_weight || c.d_weight_cast;
+            // chained walks share a launch; a side that is not wanted or not chained has no tiles in it
+            const bool dh_in = dh && dh_chain, dw_in = want_dw && dw_chain;
+            if (dh && !dh_in)
+                hipLaunchKernelGGL((linear_logp_dh_kernel<T, kBK>), dim3(tok_tiles * h_tiles * ksplit),
+                                   dim3(kThreads), GH::kSmemBytes, stream, h);
+            if (dh_in || dw_in) {
+                DhArgs hj = h;
+                DwArgs dj = d;
+                if (!dh_in) hj.h_tiles = 0;
+                if (!dw_in) dj.h_tiles = 0;
+                const int items = tok_tiles * hj.h_tiles * ksplit + v_tiles * dj.h_tiles;
+                const int grid = chain_grid(items, n_cu);
+                const GradsSplit split = grads_split(tok_tiles * hj.h_tiles * ksplit, h.nk / ksplit + 9,
+                                                     v_tiles * dj.h_tiles, d.nk + 9, grid);
+                dj.busy = split.busy;
+                dj.lead = split.lead;
+                hipLaunchKernelGGL((linear_logp_grads_kernel<T, kBK>), dim3(grid), dim3(kThreads), kChainSmem,
+                                   stream, hj, dj);
             }
-            if (c.d_weight || c.d_weight_cast) {
-                const int tiles = v_tiles * h_tiles;
-                if (dw_chain)
-                    hipLaunchKernelGGL((linear_logp_dw_kernel<T, kBK, true>),
-                                       dim3(chain_grid(tiles, n_cu)), dim3(kThreads), kChainSmem,
-                                       stream, d);
-                else
-                    hipLaunchKernelGGL((linear_logp_dw_kernel<T, kBK, false>), dim3(tiles),
-                                       dim3(kThreads), GW::kSmemBytes, stream, d);
+            if (dh && ksplit > 1) {
+                const int64_t n4 = static_cast<int64_t>(tok_valid) * H / 4;
+                hipLaunchKernelGGL((linear_logp_dh_reduce_kernel<T>),
+                                   dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0, stream, h.part,
+                                   ksplit, h.part_stride, h.acc, h.out, scales, n4, h.first, h.last);
             }
+            if (want_dw && !dw_in)
+                hipLaunchKernelGGL((linear_logp_dw_kernel<T, kBK>), dim3(v_tiles * h_tiles), dim3(kThreads),
+                                   GW::kSmemBytes, stream, d);
             if (c.d_bias != nullptr) {
                 float* db_part = reinterpret_cast<float*>(ws + p.db_off);
                 hipLaunchKernelGGL(linear_logp_db_partial_kernel<T>, dim3(v_tiles, tok_tiles), dim3(256), 0,

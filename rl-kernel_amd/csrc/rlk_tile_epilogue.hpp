@@ -133,6 +133,31 @@ struct TileWalk {
     __device__ inline void advance() { lin += static_cast<int>(gridDim.x); }
 };
 
+// Walk of a tile list whose launch gives the first `busy` workgroups other work in front: the others start with
+// `lead` rounds among themselves, then all go through common rounds.  With a grid and a `busy` that are
+// multiples of 8 a workgroup keeps its XCD, as above.
+struct LeadWalk {
+    int k, at, total, gm, gn, lead, rest;
+    __device__ inline LeadWalk(int total_, int gm_, int gn_, int busy, int lead_)
+        : total(total_), gm(gm_), gn(gn_), lead(lead_), rest(static_cast<int>(gridDim.x) - busy)
+    {
+        const int b = static_cast<int>(blockIdx.x);
+        at = b < busy ? b + rest : b - busy;
+        k = b < busy ? lead : 0;
+    }
+    __device__ inline int lin(int round) const
+    {
+        return (round < lead ? round * rest : lead * rest + (round - lead) * static_cast<int>(gridDim.x)) + at;
+    }
+    __device__ inline bool valid() const { return lin(k) < total; }
+    __device__ inline bool has_next() const { return lin(k + 1) < total; }
+    __device__ inline void coords(bool next, int& tm, int& tn) const
+    {
+        xcd_tile(lin(next ? k + 1 : k), total, gm, gn, kWalkPatch, tm, tn);
+    }
+    __device__ inline void advance() { ++k; }
+};
+
 template <class V, int TM, int TN>
 __device__ inline void zero_acc(V (&acc)[TM][TN])
 {
