@@ -41,10 +41,10 @@ enum {
     RLK_ERR_LAUNCH = -3       /* HIP refused the launch */
 };
 
-/* ABI version of this header (major * 100 + minor): 103 (100 + rlk_device_info,
+/* ABI version of this header (major * 100 + minor): 104 (100 + rlk_device_info,
  * rlk_linear_logp_fwd_plan, the typed weight gradients rlk_linear_logp_bwd_typed and
- * rlk_linear_logp_rmsnorm_bwd_typed, rlk_check_targets, rlk_mark_targets and
- * rlk_logp_from_logits_pair_masked). */
+ * rlk_linear_logp_rmsnorm_bwd_typed, rlk_check_targets, rlk_mark_targets,
+ * rlk_logp_from_logits_pair_masked and the entry points with kept logits). */
 int rlk_version(void);
 
 /* Message of the last error returned on the calling thread ("" if none). Host pointer, valid
@@ -63,7 +63,7 @@ int rlk_device_info(int32_t device, int32_t* compute_units, int32_t* max_clock_k
  * (csrc/ops.cpp:84-85, csrc/cuda/fused_linear_logp_sm90.cu:305-381) and for the forward of
  * `NativeLinearLogpOp.apply` (rl_engine/kernels/ops/pytorch/loss/linear_logp.py:476-520):
  *   z = (hidden W^T + bias) / temperature ; lse = logsumexp_v z ; logp = z[target] - lse.
- * The [N, V] logits are never stored.
+ * The [N, V] logits are not stored (rlk_linear_logp_fwd_kept does, within a bound).
  *
  *   hidden   [N, H] bf16/f16          weight [V, H] same dtype (a vocab shard starting at
  *   bias     [V] f32 or NULL                  global id `vocab_start`)
@@ -217,6 +217,41 @@ int rlk_linear_logp_bwd_typed(const float* grad_logp, const void* hidden, const 
                               int64_t ignore_index, int32_t use_ignore, rlk_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------ *
+ * Training step of few logits: the forward keeps them for its backward (no counterpart in the
+ * reference, which recomputes them at any size).
+ *
+ * rlk_linear_logp_kept_bytes: size of the buffer, N x V fp32 in whole 256 x 256 tiles, or 0 where none
+ * is kept: more than 800 MiB (so that buffer and workspace stay below 1 GB whatever N is), fp32 inputs,
+ * H % 64 != 0, H < 256 or V < 256, and heads so narrow (H < 1024, less for fewer than 256 tokens)
+ * that the trip through memory costs what the products do.  Host only.
+ * rlk_linear_logp_fwd_kept is rlk_linear_logp_fwd (same bits, same workspace) that also fills `kept`
+ * (16-byte aligned); the layout is the library's own.  rlk_linear_logp_bwd_kept is the backward of
+ * the same arguments from that buffer, which it OVERWRITES: one forward serves one backward.
+ * d_weight (fp32, with `accumulate` as in rlk_linear_logp_bwd_accum) or d_weight_typed (the type
+ * of `weight`, as in rlk_linear_logp_bwd_typed), not both; any gradient may be NULL.  Values are those
+ * of rlk_linear_logp_bwd, whose fp32 sums are grouped by its dZ blocks.
+ * ------------------------------------------------------------------------------------------ */
+int rlk_linear_logp_kept_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes);
+
+int rlk_linear_logp_fwd_kept(const void* hidden, const void* weight, const float* bias,
+                             const int64_t* targets, float* logp, float* lse, void* workspace,
+                             size_t workspace_bytes, int64_t N, int32_t H, int64_t V,
+                             int64_t vocab_start, int32_t dtype, float temperature,
+                             int64_t ignore_index, int32_t use_ignore, int32_t strict_targets,
+                             int32_t* err_flag, void* kept, size_t kept_bytes, rlk_stream_t stream);
+
+int rlk_linear_logp_bwd_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype,
+                                             size_t* bytes);
+
+int rlk_linear_logp_bwd_kept(const float* grad_logp, const void* hidden, const void* weight,
+                             const float* bias, const int64_t* targets, const float* lse,
+                             void* d_hidden, float* d_weight, void* d_weight_typed, float* d_bias,
+                             void* kept, size_t kept_bytes, void* workspace, size_t workspace_bytes,
+                             int64_t N, int32_t H, int64_t V, int64_t vocab_start, int32_t dtype,
+                             float temperature, int64_t ignore_index, int32_t use_ignore,
+                             int32_t accumulate, rlk_stream_t stream);
+
+/* ------------------------------------------------------------------------------------------ *
  * Final RMSNorm in front of the head (the step before the path).
  *
  * rlk_rmsnorm_fwd stands in for NativeRMSNormOp.forward
@@ -273,6 +308,29 @@ int rlk_linear_logp_rmsnorm_bwd(const float* grad_logp, const void* x, const flo
                                 size_t dz_budget_bytes, int64_t N, int32_t H, int64_t V,
                                 int64_t vocab_start, int32_t dtype, float temperature,
                                 int64_t ignore_index, int32_t use_ignore, rlk_stream_t stream);
+
+/* Norm and head with kept logits, one block of tokens (N <= 8192, RLK_ERR_UNSUPPORTED above): see
+ * rlk_linear_logp_fwd_kept.  The workspace of the forward is rlk_linear_logp_rmsnorm_fwd's. */
+int rlk_linear_logp_rmsnorm_fwd_kept(const void* x, const float* gain, float eps, const void* weight,
+                                     const float* bias, const int64_t* targets, float* logp,
+                                     float* lse, void* workspace, size_t workspace_bytes, int64_t N,
+                                     int32_t H, int64_t V, int64_t vocab_start, int32_t dtype,
+                                     float temperature, int64_t ignore_index, int32_t use_ignore,
+                                     int32_t strict_targets, int32_t* err_flag, void* kept,
+                                     size_t kept_bytes, rlk_stream_t stream);
+
+int rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype,
+                                                     size_t* bytes);
+
+/* d_x and d_weight_typed as in rlk_linear_logp_rmsnorm_bwd_typed: both are written. */
+int rlk_linear_logp_rmsnorm_bwd_kept(const float* grad_logp, const void* x, const float* gain,
+                                     float eps, const void* weight, const float* bias,
+                                     const int64_t* targets, const float* lse, void* d_x,
+                                     float* d_gain, void* d_weight_typed, float* d_bias, void* kept,
+                                     size_t kept_bytes, void* workspace, size_t workspace_bytes,
+                                     int64_t N, int32_t H, int64_t V, int64_t vocab_start,
+                                     int32_t dtype, float temperature, int64_t ignore_index,
+                                     int32_t use_ignore, rlk_stream_t stream);
 
 /* rlk_linear_logp_rmsnorm_bwd with d_weight in the type of `weight`, as rlk_linear_logp_bwd_typed (same
  * restrictions; `weight` 16-byte aligned). */
@@ -390,6 +448,18 @@ int rlk_linear_logp_fwd_grpo(const void* hidden, const void* weight, const float
                              const float* advantages, int32_t adv_per_token, const uint8_t* mask,
                              int64_t seq_len, float clip_eps, float beta, float* out3, float* ratio,
                              float* kl_terms, float* d_cur, float* d_kl, rlk_stream_t stream);
+
+/* The same with kept logits (rlk_linear_logp_fwd_kept); kept == NULL keeps none. */
+int rlk_linear_logp_fwd_grpo_kept(const void* hidden, const void* weight, const float* bias,
+                                  const int64_t* targets, float* logp, float* lse, void* workspace,
+                                  size_t workspace_bytes, int64_t N, int32_t H, int64_t V,
+                                  int64_t vocab_start, int32_t dtype, float temperature,
+                                  int64_t ignore_index, int32_t use_ignore, int32_t strict_targets,
+                                  int32_t* err_flag, const float* old_logp, const float* ref_logp,
+                                  const float* advantages, int32_t adv_per_token,
+                                  const uint8_t* mask, int64_t seq_len, float clip_eps, float beta,
+                                  float* out3, float* ratio, float* kl_terms, float* d_cur,
+                                  float* d_kl, void* kept, size_t kept_bytes, rlk_stream_t stream);
 
 /* Per-token policy ratio exp(cur - old) and k3 KL exp(ref - cur) - (ref - cur) - 1 of the
  * logits-fed ratio/KL op, the mask applied to the differences BEFORE the exponentials, so an

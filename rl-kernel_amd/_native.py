@@ -41,6 +41,21 @@ SIGNATURES = {
                                                              _c.POINTER(_sz)]),
     "rlk_linear_logp_bwd_typed": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _sz,
                                              _i64, _i32, _i64, _i64, _i32, _f32, _i64, _i32, _vp]),
+    "rlk_linear_logp_kept_bytes": (_c.c_int, [_i64, _i32, _i64, _i32, _c.POINTER(_sz)]),
+    "rlk_linear_logp_fwd_kept": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i64, _i32, _i64,
+                                            _i64, _i32, _f32, _i64, _i32, _i32, _vp, _vp, _sz, _vp]),
+    "rlk_linear_logp_bwd_kept_workspace_bytes": (_c.c_int, [_i64, _i32, _i64, _i32, _c.POINTER(_sz)]),
+    "rlk_linear_logp_bwd_kept": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp,
+                                            _sz, _i64, _i32, _i64, _i64, _i32, _f32, _i64, _i32, _i32,
+                                            _vp]),
+    "rlk_linear_logp_rmsnorm_fwd_kept": (_c.c_int, [_vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _vp, _sz,
+                                                    _i64, _i32, _i64, _i64, _i32, _f32, _i64, _i32,
+                                                    _i32, _vp, _vp, _sz, _vp]),
+    "rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes": (_c.c_int, [_i64, _i32, _i64, _i32,
+                                                                    _c.POINTER(_sz)]),
+    "rlk_linear_logp_rmsnorm_bwd_kept": (_c.c_int, [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                                    _vp, _vp, _sz, _vp, _sz, _i64, _i32, _i64, _i64,
+                                                    _i32, _f32, _i64, _i32, _vp]),
     "rlk_rmsnorm_fwd": (_c.c_int, [_vp, _vp, _f32, _vp, _vp, _i64, _i32, _i32, _vp]),
     "rlk_rmsnorm_bwd_workspace_bytes": (_c.c_int, [_i64, _i32, _c.POINTER(_sz)]),
     "rlk_rmsnorm_bwd": (_c.c_int, [_vp, _vp, _f32, _vp, _vp, _vp, _vp, _sz, _i64, _i32, _i32, _vp]),
@@ -76,6 +91,10 @@ SIGNATURES = {
                                             _i64, _i32, _f32, _i64, _i32, _i32, _vp,
                                             _vp, _vp, _vp, _i32, _vp, _i64, _f32, _f32, _vp, _vp,
                                             _vp, _vp, _vp, _vp]),
+    "rlk_linear_logp_fwd_grpo_kept": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i64, _i32, _i64,
+                                                 _i64, _i32, _f32, _i64, _i32, _i32, _vp,
+                                                 _vp, _vp, _vp, _i32, _vp, _i64, _f32, _f32, _vp, _vp,
+                                                 _vp, _vp, _vp, _vp, _sz, _vp]),
     "rlk_ratio_kl_from_logp": (_c.c_int, [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp]),
     "rlk_ratio_kl_from_logp_bwd": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp]),
     "rlk_group_advantages": (_c.c_int, [_vp, _vp, _i64, _f32, _vp, _vp]),

@@ -18,6 +18,10 @@
 #define RLK_MAX_DZ_BUDGET (static_cast<size_t>(2) << 30)  // upper clamp of dz_budget_bytes
 #endif
 
+#ifndef RLK_KEPT_LOGITS_BYTES
+#define RLK_KEPT_LOGITS_BYTES (static_cast<size_t>(800) << 20)  // most that a training forward keeps of its logits
+#endif
+
 // Records `msg` as the calling thread's last error and returns `code` (always negative).
 int rlk_fail(int code, const char* msg);
 

@@ -129,6 +129,10 @@ struct Operand {
     const uint16_t* base;  // element (row 0, k 0) of the tile
     int64_t ld;            // elements between consecutive memory lines
     int rows;              // valid tile rows from the origin (>= 1)
+    // tiled operands only (see DtlIO): bytes between the end of 64 lines and the next 64, bytes per K step
+    // inside a group of four and per group
+    uint32_t gap = 0;
+    int64_t step = 0, step4 = 0;
 };
 
 // Compile-time loop: f(std::integral_constant<int, I>) for I in [B, E).
@@ -262,7 +266,7 @@ struct TileIO {
     }
 };
 
-template <class T, bool A_KMAJOR, bool B_KMAJOR, int BK, int WIN, bool TAIL = false>
+template <class T, bool A_KMAJOR, bool B_KMAJOR, int BK, int WIN, bool TAIL = false, bool B_TILED = false>
 struct TileGemmDtl;
 
 // Workgroup tile contraction for any K.  acc[i][j] (+)= A rows x B rows over k in [0, K).
@@ -425,7 +429,9 @@ struct KTail {
     int64_t a = 0, b = 0;
 };
 
-template <bool KMAJOR, int ROWS, int BK, bool TAIL = false>
+// TILED: the operand is not one matrix but blocks of 256 x 256 whose K steps advance by Operand::step four times
+// and by Operand::step4 per group of four; 64 lines of a K-contiguous tile lie Operand::gap bytes apart.
+template <bool KMAJOR, int ROWS, int BK, bool TAIL = false, bool TILED = false>
 struct DtlIO {
     static_assert(BK == 64 && ROWS == 256, "direct-to-LDS layout is written for 256 x 64 tiles");
     static constexpr int kBytes = ROWS * BK * 2;            // 32 KiB, dense
@@ -438,6 +444,7 @@ struct DtlIO {
     const char* next;        // uniform: origin of the tile whose first K steps follow this one's
     uint32_t off[kPasses];   // per-lane byte offset of this lane's chunk for load p at K step 0
     uint32_t step;           // uniform byte advance per K step
+    int64_t step4;           // TILED: uniform byte advance per four K steps
     int nk;                  // K steps per tile
     int wave;                // uniform wavefront index
     int tail_from;           // TAIL: first K step of the shifted last K tile
@@ -453,6 +460,10 @@ struct DtlIO {
         nk = K / BK;
         const uint32_t ld = static_cast<uint32_t>(op.ld);
         step = KMAJOR ? static_cast<uint32_t>(BK) * ld * 2u : static_cast<uint32_t>(BK) * 2u;
+        if constexpr (TILED) {
+            step = static_cast<uint32_t>(op.step);
+            step4 = op.step4;
+        }
 #pragma unroll
         for (int p = 0; p < kPasses; ++p) {
             const int q = wave + kWaves * p;  // which 1 KiB block of the tile
@@ -467,6 +478,7 @@ struct DtlIO {
                 const int c = (lane & 7) ^ ((r >> 1) & 7);
                 const int rc = r < op.rows ? r : op.rows - 1;
                 off[p] = (static_cast<uint32_t>(rc) * ld + static_cast<uint32_t>(c * 8)) * 2u;
+                if constexpr (TILED) off[p] += static_cast<uint32_t>(rc >> 6) * op.gap;
             }
         }
     }
@@ -480,7 +492,11 @@ struct DtlIO {
         // K steps past the end of this tile are the first steps of the next one (all uniform)
         const bool over = kt >= nk;
         const int rel = over ? (kt - nk < nk ? kt - nk : nk - 1) : kt;
-        const char* src = (over ? next : base) + static_cast<size_t>(rel) * step;
+        const char* src = over ? next : base;
+        if constexpr (TILED)
+            src += (rel >> 2) * step4 + static_cast<size_t>(rel & 3) * step;
+        else
+            src += static_cast<size_t>(rel) * step;
         if constexpr (TAIL) src += rel >= (over ? next_tail_from : tail_from) ? tail_adj : 0;  // uniform
         const uint32_t dst = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
                                  (RLK_LDS char*)(lds))) + static_cast<uint32_t>((wave + kWaves * p) * 1024);
@@ -519,7 +535,7 @@ struct DtlIO {
 // WIN: MFMA slots (of the 32 of the second slice) over which the 8 loads of a K step are spread.
 // 32 spaces them evenly over the slice; 16 sends them all out in its first half, which the
 // persistent dZ and dH kernels prefer (they stall more on operand loads than the forward).
-template <class T, bool A_KMAJOR, bool B_KMAJOR, int BK, int WIN, bool TAIL>
+template <class T, bool A_KMAJOR, bool B_KMAJOR, int BK, int WIN, bool TAIL, bool B_TILED>
 struct TileGemmDtl {
     using AT = Acc16;
     static constexpr int TM = AT::TM;
@@ -527,7 +543,7 @@ struct TileGemmDtl {
     static constexpr int KK = BK / 32;
     static_assert(KK == 2, "the loop is written for two 32-wide slices per K step");
     using IOA = DtlIO<A_KMAJOR, 256, BK, TAIL>;
-    using IOB = DtlIO<B_KMAJOR, 256, BK, TAIL>;
+    using IOB = DtlIO<B_KMAJOR, 256, BK, TAIL, B_TILED>;
     using Plan = FragPlan<TM, TN>;
     static constexpr int PA = IOA::kPasses;
     static constexpr int PB = IOB::kPasses;

@@ -1,5 +1,5 @@
 // Fused linear -> selected-token log-prob for gfx950: forward (online logsumexp over vocab
-// tiles, logits never stored), split combine, and the recompute-based backward (dZ block,
+// tiles, logits not stored but for a small training step), split combine, and the recompute-based backward (dZ block,
 // dH and dW contractions).  All reductions run in a fixed order: same input, same bits.
 //
 // Orientation used by every kernel here: the MFMA "M" index lives in accumulator registers (the
@@ -57,7 +57,17 @@ struct FwdArgs {
     int tile_lo;     // first vocab tile of this launch
     int vtiles;      // vocab tiles of this launch
     float scale2;    // log2(e) / temperature
+    float* kept;     // KEEP: logits of every tile, see "Kept logits"
 };
+
+// Kept logits: fp32 logits (bias added, masked vocab rows -inf) that a training forward leaves for its backward
+// when they are few (rlk_linear_logp_kept_bytes), so that dZ does not have to recompute them.  One block
+// of 256 KiB per (token tile, vocab tile), token tile the slow index, made of four slabs of 64 tokens;
+// a slab holds the accumulator quads as the wavefronts have them,
+// [2 wavefronts along vocab][TM][TN][64 lanes][4], so a wavefront stores a tile in 1 KiB pieces.  The last token tile
+// is moved back to end at N as in the backward; columns of 16 tokens past N (fewer than 256 tokens) are not stored.
+constexpr int kKeptSlab = 64 * 256;       // floats
+constexpr int kKeptTile = 4 * kKeptSlab;
 
 // One workgroup = one block of 256 tokens x one contiguous range of vocab tiles.
 // GENERAL = false covers vocab tiles [0, vtiles) split n_split ways, every one of 256 valid rows (a
@@ -68,10 +78,12 @@ struct FwdArgs {
 // row_blocks workgroups busy for a whole tile while the other CUs waited: 70 of 750 us at 4096 x
 // 2048 x 50257, 48 of 458 us at 1000 x 1536 x 151936.
 // CHAIN (!GENERAL, H a multiple of BK and >= 2 BK, V >= 256): all tiles run through one pipeline.
-template <class T, int BK, bool GENERAL, bool CHAIN>
+// KEEP (CHAIN, one head): the logits stay in a.kept.
+template <class T, int BK, bool GENERAL, bool CHAIN, bool KEEP = false>
 __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
 {
     static_assert(!(GENERAL && CHAIN), "the chained variant covers full tiles only");
+    static_assert(CHAIN || !KEEP, "logits are kept by the chained variant only");
     using AT = Acc16;
     constexpr int TM = AT::TM, TN = AT::TN;
     using Gemm = TileGemm<T, false, false, BK>;
@@ -88,8 +100,9 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int wm = wave / kWN, wn = wave % kWN;
-    const int tok0 = tb * 256;
+    const int tok0 = KEEP ? max(0, min(tb * 256, a.N - 256)) : tb * 256;
     const int tok_valid = min(256, a.N - tok0);
+    const int tok_own = KEEP ? tb * 256 - tok0 : 0;  // rows below belong to the token block in front
 
     float m[TN], s[TN], zt[TN];
     int tgt[TN];  // target id relative to the shard, -1 when not in [0, V)
@@ -143,7 +156,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
         }
         __syncthreads();
         const int t = threadIdx.x;
-        if (t < tok_valid) {
+        if (t >= tok_own && t < tok_valid) {
             float mm = -INFINITY;
 #pragma unroll
             for (int w = 0; w < kWM; ++w) mm = fmaxf(mm, red[(w * 256 + t) * 3]);
@@ -177,6 +190,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
         // pipeline looks two K steps ahead, which stays within the next tile from two steps up)
         typename Dtl::Stream st;
         Dtl::begin(st, Operand{tile_origin(0, t0), a.H, 256}, B, a.H, smem);
+        bool counted = false;
         for (int head = 0; head < n_heads; ++head) {
             reset_state();
             for (int vt = t0; vt < t1; ++vt) {
@@ -186,10 +200,22 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
                 const void* next = vt + 1 < t1 ? tile_origin(head, vt + 1)
                                                : (head + 1 < n_heads ? tile_origin(head + 1, t0)
                                                                      : tile_origin(head, vt));
-                Dtl::template tile<true>(st, next, B.base, acc, smem);
+                Dtl::template tile<true, KEEP ? TM * TN : 0>(st, next, B.base, acc, smem, counted);
                 const float* bias = head == 0 ? a.bias : a.bias2;
                 if (bias != nullptr) add_bias<AT>(acc, bias, row0 + wm * (TM * 16), lane);  // uniform
                 mask_rows<T>(acc, wm * (TM * 16), vt * 256 - row0, lane);
+                if constexpr (KEEP) {
+                    const int64_t tile = static_cast<int64_t>(tb) * a.vtiles + vt;
+                    float* dst = a.kept + tile * kKeptTile + wn * kKeptSlab + wm * (kKeptSlab / 2);
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        if (wn * (TN * 16) + j * 16 >= tok_valid) break;  // uniform
+#pragma unroll
+                        for (int i = 0; i < TM; ++i)
+                            *reinterpret_cast<f32x4_t*>(dst + (i * TN + j) * 256 + lane * 4) = acc[i][j];
+                    }
+                    counted = tok_valid == 256;
+                }
                 fwd_epilogue<GENERAL, AT>(acc, a, nullptr, row0 + wm * (TM * 16), vt * 256, lane, tgt, m, s, zt);
             }
             if (head == 0)
@@ -559,6 +585,128 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dz_kernel(DzArgs a)
     }
 }
 
+// dZ from kept logits, in place: the 64 KiB of a slab (64 tokens x 256 vocab rows, see "Kept logits") become the
+// 32 KiB of its dZ rows [64][256] of the 16-bit type at the slab's head.  One workgroup per slab reads all of it
+// before the first write.  A thread makes 8 consecutive vocab rows of a token from two quads, so eight
+// lanes store a full line; the reads are full lines too (8 tokens of one quad row).  Bound by memory: 6
+// bytes per logit against the 2 H / 1500e12 s that computing it again takes.
+// Tokens outside the tile's own rows get zeros (as far as dW's K steps read, row `used` of the tile), whatever
+// lies in the block there.  DB: column sums of the slab go to db_part[slab][v] for d_bias.
+struct KeptDzArgs {
+    float* kept;
+    const int64_t* targets;
+    const float* lse;
+    const float* grad;
+    const float* scales;
+    float* db_part;  // [4 * tok_tiles][v_tiles * 256]
+    int N;
+    int V;
+    int v_tiles;
+    int tok_tiles;
+    int tok_shift;  // rows / vocab rows by which the last token / vocab tile is moved back
+    int v_shift;
+    int used;       // rows of a padded tile that dW reads (256 otherwise)
+    int64_t vocab_start;
+    int64_t ignore_index;
+    int use_ignore;
+    float scale2;
+};
+
+template <class T, bool DB>
+__global__ __launch_bounds__(256) void linear_logp_dz_kept_kernel(KeptDzArgs a)
+{
+    const int tile = blockIdx.x >> 2, slab = blockIdx.x & 3;
+    const int tt = tile / a.v_tiles, vt = tile - tt * a.v_tiles;
+    const int tok_back = tt == a.tok_tiles - 1 ? a.tok_shift : 0;
+    const int v_back = vt == a.v_tiles - 1 ? a.v_shift : 0;
+    const int u = threadIdx.x & 7;  // 8 vocab rows of every group of 64
+    float* src = a.kept + static_cast<int64_t>(tile) * kKeptTile + slab * kKeptSlab;
+    const float gscale = a.scales[0];
+    f32x4_t z[2][4][2];
+    float gs[2], nlse2[2];
+    int hot[2];  // target's vocab row relative to this thread's first one, or out of reach
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int t = (threadIdx.x >> 3) + 32 * q, tl = slab * 64 + t;
+        const int n = tt * 256 - tok_back + tl;
+        gs[q] = 0.f;
+        nlse2[q] = -INFINITY;
+        hot[q] = -1;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) z[q][g][0] = z[q][g][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (tl >= tok_back && n < a.N) {
+            const int64_t tg = a.targets[n];
+            if (!(a.use_ignore && tg == a.ignore_index)) {
+                gs[q] = a.grad[n] * gscale;
+                nlse2[q] = -a.lse[n] * kLog2e;
+                const int64_t tv = tg - a.vocab_start;
+                if (tv >= static_cast<int64_t>(vt) * 256 && tv < a.V)
+                    hot[q] = static_cast<int>(min(tv - (vt * 256 - v_back), static_cast<int64_t>(256)));
+                const float* p = src + (t >> 4) * 256 + (t & 15) * 4;
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        // rows 64 g + 8 u + 4 e: wavefront g / 2, MFMA row tile 4 (g % 2) + u / 2, lane group 2 (u % 2) + e
+                        const int i = 4 * (g & 1) + (u >> 1), grp = 2 * (u & 1) + e;
+                        z[q][g][e] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(
+                            p + (g >> 1) * (kKeptSlab / 2) + i * (4 * 256) + grp * 64));
+                    }
+            }
+        }
+    }
+    u32x4_t out[2][4];
+    float sum[4][8];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            float d[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float pr = __builtin_amdgcn_exp2f(fmaf(z[q][g][e >> 2][e & 3], a.scale2, nlse2[q]));
+                d[e] = fmaf(-gs[q], pr, hot[q] == 64 * g + 8 * u + e ? gs[q] : 0.f);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                out[q][g][e] = T::pack2(d[2 * e], d[2 * e + 1]);
+                if (DB) {  // of the rounded values
+                    const float lo = T::to_float(static_cast<uint16_t>(out[q][g][e] & 0xffffu));
+                    const float hi = T::to_float(static_cast<uint16_t>(out[q][g][e] >> 16));
+                    sum[g][2 * e] = q == 0 ? lo : sum[g][2 * e] + lo;
+                    sum[g][2 * e + 1] = q == 0 ? hi : sum[g][2 * e + 1] + hi;
+                }
+            }
+        }
+    // every logit of the slab has been used before the first write (the arithmetic must not move behind it)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) asm volatile("" : "+v"(out[q][g]));
+    __syncthreads();
+    uint16_t* dst = reinterpret_cast<uint16_t*>(src);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int t = (threadIdx.x >> 3) + 32 * q;
+        if (slab * 64 + t < a.used)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *reinterpret_cast<u32x4_t*>(dst + t * 256 + g * 64 + u * 8) = out[q][g];
+    }
+    if constexpr (DB) {
+        __shared__ float red[32][257];
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) red[threadIdx.x >> 3][g * 64 + u * 8 + e] = sum[g][e];
+        __syncthreads();
+        float acc = red[0][threadIdx.x];
+#pragma unroll 8
+        for (int r = 1; r < 32; ++r) acc += red[r][threadIdx.x];
+        a.db_part[(static_cast<int64_t>(tt) * 4 + slab) * (a.v_tiles * 256) + vt * 256 + threadIdx.x] = acc;
+    }
+}
+
 // ------------------------------------------------------------------------------------------- //
 // Backward step 2: dH[tok][h] (+)= sum_v dZ[tok][v] W[v][h]      (M = h, N = token, K = vocab)
 // ------------------------------------------------------------------------------------------- //
@@ -581,6 +729,7 @@ struct DhArgs {
     int64_t part_stride;  //      (elements per slot); linear_logp_dh_reduce_kernel adds them up
     int nk;               // K steps (of 64 vocab rows) of the piece, the shifted tile's among them;
     KTail tail;           //      0: the block has no shifted tiles, K runs over [0, v_valid)
+    int v_tiles;          // KEPT: vocab tiles of the block
     int tok_shift;        // rows by which the last token tile is moved back
 };
 
@@ -939,16 +1088,21 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dw_kernel(DwArgs a)
 // h.ksplit > 1: a dH item is one part of the vocab range of a tile and leaves for that part's fp32
 // slot.  The items of one range are neighbours in the list (they share dZ columns), so the part
 // is the slow index.
-template <class T, int BK>
+// KEPT: dz is the block of kept logits that linear_logp_dz_kept_kernel has turned into dZ in place.
+template <class T, int BK, bool KEPT>
 __global__ __launch_bounds__(kThreads) void linear_logp_grads_kernel(DhArgs h, DwArgs d)
 {
+    constexpr int kTileEls = kKeptTile * 2, kSlabEls = kKeptSlab * 2;  // 16-bit elements
     extern __shared__ __attribute__((aligned(16))) char smem[];
     f32x4_t acc[Acc16::TM][Acc16::TN];
     const int dh_items = h.tok_tiles * h.h_tiles * h.ksplit;
     if (static_cast<int>(blockIdx.x) < dh_items) {
-        using Dtl = TileGemmDtl<T, true, false, BK, kWinDh, true>;
+        using Dtl = TileGemmDtl<T, true, false, BK, kWinDh, true, KEPT>;
         TileWalk walk(dh_items, h.tok_tiles, h.h_tiles * h.ksplit);
-        const int base = h.nk / h.ksplit, extra = h.nk % h.ksplit;
+        // parts are whole K steps, of kept logits whole vocab tiles (the last one is cut off at nk)
+        constexpr int kUnit = KEPT ? 4 : 1;
+        const int units = (h.nk + kUnit - 1) / kUnit;
+        const int base = units / h.ksplit, extra = units % h.ksplit;
         struct Item {
             int tt, ht, ks, step0, nk;
         };
@@ -960,20 +1114,29 @@ __global__ __launch_bounds__(kThreads) void linear_logp_grads_kernel(DhArgs h, D
                 it.ks = it.ht / h.h_tiles;
                 it.ht -= it.ks * h.h_tiles;
             }
-            // whole K steps, the first `extra` parts take one more
-            it.step0 = it.ks * base + min(it.ks, extra);
-            it.nk = base + (it.ks < extra ? 1 : 0);
+            // the first `extra` parts take one unit more
+            it.step0 = (it.ks * base + min(it.ks, extra)) * kUnit;
+            it.nk = (base + (it.ks < extra ? 1 : 0)) * kUnit;
+            if (KEPT) it.nk = min(it.nk, h.nk - it.step0);
             return it;
         };
         // first hidden column of h tile `t`: the last tile is shifted back so that it ends at H
         auto h_col = [&](int t) { return min(t * 256, h.H - 256); };
         auto w_origin = [&](const Item& it) { return h.weight + static_cast<int64_t>(it.step0) * BK * h.H + h_col(it.ht); };
-        auto z_origin = [&](const Item& it) { return h.dz + static_cast<int64_t>(it.tt) * 256 * h.ldz + it.step0 * BK; };
+        auto z_origin = [&](const Item& it) {
+            return KEPT ? h.dz + (static_cast<int64_t>(it.tt) * h.v_tiles + it.step0 / 4) * kTileEls
+                        : h.dz + static_cast<int64_t>(it.tt) * 256 * h.ldz + it.step0 * BK;
+        };
+        // kept: rows of 256 elements, 64 of them at the head of a slab
+        auto z_operand = [&](const Item& it) {
+            return KEPT ? Operand{z_origin(it), 256, 256, (kSlabEls - 64 * 256) * 2, BK * 2, kTileEls * 2}
+                        : Operand{z_origin(it), h.ldz, 256};
+        };
         auto tail_from = [&](const Item& it) { return h.tail.from - it.step0; };
         Item cur = item(false);
         typename Dtl::Stream st;
         bool counted = false;
-        Dtl::begin(st, Operand{w_origin(cur), h.H, 256}, Operand{z_origin(cur), h.ldz, 256}, cur.nk * BK, smem,
+        Dtl::begin(st, Operand{w_origin(cur), h.H, 256}, z_operand(cur), cur.nk * BK, smem,
                    KTail{tail_from(cur), h.tail.a, h.tail.b});
         for (;;) {
             const bool more = walk.has_next();
@@ -994,15 +1157,19 @@ __global__ __launch_bounds__(kThreads) void linear_logp_grads_kernel(DhArgs h, D
     }
     LeadWalk walk(d.v_tiles * d.h_tiles, d.v_tiles, d.h_tiles, d.busy, d.lead);
     if (!walk.valid()) return;
-    using Dtl = TileGemmDtl<T, true, true, BK, kWinDw, true>;
+    using Dtl = TileGemmDtl<T, true, true, BK, kWinDw, true, KEPT>;
     int vt, ht;
     walk.coords(false, vt, ht);
     auto h_col = [&](int t) { return min(t * 256, d.H - 256); };
-    auto h_origin = [&](int t) { return d.hidden + h_col(t); };                          // M rows
-    auto z_origin = [&](int v) { return d.dz + static_cast<int64_t>(v) * 256; };        // N rows
+    auto h_origin = [&](int t) { return d.hidden + h_col(t); };                                         // M rows
+    auto z_origin = [&](int v) { return d.dz + static_cast<int64_t>(v) * (KEPT ? kTileEls : 256); };  // N rows
+    // kept: a K step is the head of one slab of 64 tokens
+    const Operand z = KEPT ? Operand{z_origin(vt), 256, 256, 0, kSlabEls * 2,
+                                     static_cast<int64_t>(d.v_tiles) * kTileEls * 2}
+                           : Operand{z_origin(vt), d.ldz, 256};
     typename Dtl::Stream st;
     bool counted = false;
-    Dtl::begin(st, Operand{h_origin(ht), d.H, 256}, Operand{z_origin(vt), d.ldz, 256}, d.nk * BK, smem, d.tail);
+    Dtl::begin(st, Operand{h_origin(ht), d.H, 256}, z, d.nk * BK, smem, d.tail);
     for (;;) {
         const bool more = walk.has_next();
         int nvt = vt, nht = ht;
@@ -1070,7 +1237,7 @@ __global__ __launch_bounds__(256) void linear_logp_db_partial_kernel(const uint1
     part[static_cast<int64_t>(blockIdx.y) * part_ld + blockIdx.x * 256 + threadIdx.x] = acc;
 }
 
-// Level 2: the token tiles of the block in ascending order, times 1 / loss_scale.
+// Level 2: the token tiles (slabs) of the block in ascending order, times 1 / loss_scale.
 // v_shift: the last vocab tile's columns start that many vocab rows earlier than its place says.
 __global__ void linear_logp_db_finish_kernel(const float* part, int64_t part_ld, int tok_tiles, int v_valid,
                                              int v_shift, const float* scales, float* db, int accumulate)
@@ -1079,6 +1246,7 @@ __global__ void linear_logp_db_finish_kernel(const float* part, int64_t part_ld,
     if (v >= v_valid) return;
     const int c = v < v_valid / 256 * 256 ? v : v + v_shift;
     float sum = part[c];
+#pragma unroll 8
     for (int t = 1; t < tok_tiles; ++t) sum += part[static_cast<int64_t>(t) * part_ld + c];
     sum *= scales[1];
     db[v] = accumulate ? db[v] + sum : sum;
@@ -1279,6 +1447,11 @@ inline int dh_cuts(int64_t ct, int64_t pt, int64_t ht)
     return cuts > parts ? static_cast<int>(cuts) : parts;
 }
 
+// Epilogues of linear_logp_grads_kernel in K steps, from launches whose tiles fill whole rounds (256 vocab tiles
+// x 4096 x 8192 tokens: dH 400 us for 256 steps, dW with the fp32 read-modify-write 212 us for 128; 1024
+// tokens x 4096: dW written once in 16 bits 34.5 us for 16; a step is 1.45 - 1.5 us).
+constexpr int kDhSteps = 10, kDwSteps = 8, kDwAddSteps = 14;
+
 // How linear_logp_grads_kernel hands out n1 dH items of cost c1 and n2 dW tiles of cost c2 (K steps) to `grid`
 // workgroups: dH items in rounds, so the first n1 % grid workgroups (`busy`, in whole groups of the eight
 // XCDs) have one more than the others; those others take `lead` rounds of dW tiles among themselves before
@@ -1306,21 +1479,22 @@ inline GradsSplit grads_split(int64_t n1, int64_t c1, int64_t n2, int64_t c2, in
     return best;
 }
 
-// The dH + dW launch of one block of ct x pt tiles, in K steps (the reduction of split dH tiles included).
-inline int64_t grads_cost(int64_t ct, int64_t pt, int64_t ht)
+// The dH + dW launch of one block of ct x pt tiles, in K steps (the reduction of split dH tiles included);
+// several: dW is read, added to and written by every token chunk.
+inline int64_t grads_cost(int64_t ct, int64_t pt, int64_t ht, bool several)
 {
     const int cuts = dh_cuts(ct, pt, ht);
-    return grads_split(ct * ht * cuts, (4 * pt + cuts - 1) / cuts + 9, pt * ht, 4 * ct + 9, 256).cost +
-           (cuts > 1 ? 10 : 0);
+    return grads_split(ct * ht * cuts, (4 * pt + cuts - 1) / cuts + kDhSteps, pt * ht,
+                       4 * ct + (several ? kDwAddSteps : kDwSteps), 256).cost + (cuts > 1 ? 10 : 0);
 }
 
 // Sizes whose backward runs on the chained walks whatever the token count (ragged tiles are moved back).
 bool bwd_chained(int H, int64_t V) { return H % kBK == 0 && H >= 256 && V >= 256; }
 
-inline int64_t block_cost(bool chained, int64_t ct, int64_t pt, int64_t ht, int64_t hk)
+inline int64_t block_cost(bool chained, int64_t ct, int64_t pt, int64_t ht, int64_t hk, bool several)
 {
     const int64_t dz = (ct * pt + 255) / 256 * (hk + 3);
-    if (chained) return dz + grads_cost(ct, pt, ht) + 12;  // filling three pipelines, two launches
+    if (chained) return dz + grads_cost(ct, pt, ht, several) + 12;  // filling three pipelines, two launches
     const int parts = dh_parts(ct, pt, ht);
     // split launch: every part is a workgroup of its own; the slot reduction costs about 10 steps
     const int64_t dh = parts > 1 ? (ct * ht * parts + 255) / 256 * (4 * pt / parts + 9) + 10
@@ -1372,10 +1546,10 @@ BwdPlan bwd_plan(int64_t N, int H, int64_t V, size_t budget)
             const int64_t np = (v_t + pt - 1) / pt, pt_last = v_t - (np - 1) * pt;
             const int64_t bytes = ct * pt * tile_bytes + (np > 1 ? ct * 256 * H * 4 : 0);
             if (bytes > cap && ct * pt > 1) continue;
-            const int64_t cost = (nc - 1) * (np - 1) * block_cost(chained, ct, pt, ht, hk) +
-                                 (np - 1) * block_cost(chained, ct_last, pt, ht, hk) +
-                                 (nc - 1) * block_cost(chained, ct, pt_last, ht, hk) +
-                                 block_cost(chained, ct_last, pt_last, ht, hk);
+            const int64_t cost = (nc - 1) * (np - 1) * block_cost(chained, ct, pt, ht, hk, nc > 1) +
+                                 (np - 1) * block_cost(chained, ct_last, pt, ht, hk, nc > 1) +
+                                 (nc - 1) * block_cost(chained, ct, pt_last, ht, hk, nc > 1) +
+                                 block_cost(chained, ct_last, pt_last, ht, hk, nc > 1);
             if (best_cost < 0 || cost < best_cost || (cost == best_cost && bytes < best_bytes)) {
                 best_cost = cost;
                 best_ct = ct;
@@ -1417,6 +1591,40 @@ BwdPlan bwd_plan(int64_t N, int H, int64_t V, size_t budget)
     p.pad_off = p.db_off + align_up(p.db_bytes, 256);
     p.total = p.pad_off + align_up(p.pad_bytes, 256);
     memo = Key{N, V, H, budget, p};
+    return p;
+}
+
+// Bytes of the kept logits, or 0 where a training forward keeps none: sizes off the chained 16-bit kernels, and
+// more than RLK_KEPT_LOGITS_BYTES, the bound that keeps the extra memory of a step below 1 GB whatever N is.
+// Narrow heads keep none either: a tile of logits costs 12 us of stores in the forward and 17 us of dZ pass
+// (proportionally less with fewer than 256 tokens, whose columns past N stay out), computing it again
+// about 1.7 us per 64 of H plus 4 (forward and dZ, kept against computed again: 1000 x 1536 x 151936 715 against
+// 957 us, 1000 x 896 x 50257 192 against 211, 1000 x 512 x 50257 154 against 138).
+size_t kept_bytes(int64_t N, int H, int64_t V, int dtype)
+{
+    if (dtype == RLK_DTYPE_F32 || !bwd_chained(H, V) || H < std::min<int64_t>(1024, 4 * N)) return 0;
+    const int64_t tiles = ((N + 255) / 256) * ((V + 255) / 256);
+    if (tiles > static_cast<int64_t>(RLK_KEPT_LOGITS_BYTES / (kKeptTile * 4))) return 0;
+    return static_cast<size_t>(tiles) * kKeptTile * 4;
+}
+
+// Backward from kept logits: one block of the whole problem, dZ in the place of the logits.
+BwdPlan kept_plan(int64_t N, int H, int64_t V)
+{
+    const int64_t n_t = (N + 255) / 256, v_t = (V + 255) / 256, ht = (H + 255) / 256;
+    BwdPlan p{};
+    p.tok_chunk = static_cast<int>(n_t) * 256;
+    p.v_piece = static_cast<int>(v_t) * 256;
+    p.n_chunks = p.n_pieces = 1;
+    p.ldz = p.v_piece;
+    p.ksplit = dh_cuts(n_t, v_t, ht);
+    p.part_off = 256;
+    p.part_bytes = p.ksplit > 1 ? static_cast<size_t>(p.ksplit) * n_t * 256 * H * 4 : 0;
+    p.db_off = p.part_off + align_up(p.part_bytes, 256);
+    p.db_bytes = static_cast<size_t>(4) * n_t * p.v_piece * 4;  // column sums per slab of 64 tokens
+    p.pad_off = p.db_off + align_up(p.db_bytes, 256);
+    p.pad_bytes = N < 256 ? static_cast<size_t>(256) * H * 2 : 0;
+    p.total = p.pad_off + align_up(p.pad_bytes, 256);
     return p;
 }
 
@@ -1471,6 +1679,17 @@ bool use_mfma(const void* hidden, const void* weight, int32_t H, int dtype)
            (reinterpret_cast<uintptr_t>(hidden) & 15) == 0 && (reinterpret_cast<uintptr_t>(weight) & 15) == 0;
 }
 
+// A buffer for kept logits as the forward or the backward is given it.
+int check_kept(const void* kept, size_t bytes, bool mfma, int64_t N, int32_t H, int64_t V, int dtype)
+{
+    const size_t need = kept_bytes(N, H, V, dtype);
+    if (!mfma || need == 0)
+        return rlk_fail(RLK_ERR_UNSUPPORTED, "no logits are kept for these sizes (rlk_linear_logp_kept_bytes)");
+    if (bytes < need || (reinterpret_cast<uintptr_t>(kept) & 15) != 0)
+        return rlk_fail(RLK_ERR_ARG, "kept logits: buffer too small or not 16-byte aligned");
+    return 0;
+}
+
 // Compute units of the current device (looked up once per device): the chained kernels launch
 // one workgroup per compute unit.  Which workgroup computes a tile never changes the tile's bits.
 int compute_units(int* out)
@@ -1516,6 +1735,7 @@ struct BwdCall {
     int accumulate;  // 1: d_weight / d_bias already hold the sums of earlier tokens, add to them
     void* d_weight_cast;  // [V][H] of the weight's type or null: the finished d_weight sum goes here and
                           // d_weight only holds the running sums of earlier chunks
+    float* kept;          // logits that the forward left (the plan is then kept_plan), or null
 };
 
 // Grid of a chained launch: one workgroup per compute unit, rounded down to a multiple of 8 so
@@ -1542,7 +1762,7 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
 
     char* ws = static_cast<char*>(c.workspace);
     float* scales = reinterpret_cast<float*>(ws + p.scales_off);
-    uint16_t* dz = reinterpret_cast<uint16_t*>(ws + p.dz_off);
+    uint16_t* dz = reinterpret_cast<uint16_t*>(c.kept ? reinterpret_cast<char*>(c.kept) : ws + p.dz_off);
     float* hacc = p.acc_bytes ? reinterpret_cast<float*>(ws + p.acc_off) : nullptr;
     const uint16_t* hid = static_cast<const uint16_t*>(c.hidden);
     const uint16_t* w = static_cast<const uint16_t*>(c.weight);
@@ -1573,7 +1793,8 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
     if (int rc = set_smem(linear_logp_dz_kernel<T, kBK, false, true>, kDzChainSmem)) return rc;
     if (int rc = set_smem(linear_logp_dz_kernel<T, kBK, false, false>, GZ::kSmemBytes)) return rc;
     if (int rc = set_smem(linear_logp_dz_kernel<T, kBK, true, false>, GZ::kSmemBytes)) return rc;
-    if (int rc = set_smem(linear_logp_grads_kernel<T, kBK>, kChainSmem)) return rc;
+    if (int rc = set_smem(linear_logp_grads_kernel<T, kBK, false>, kChainSmem)) return rc;
+    if (int rc = set_smem(linear_logp_grads_kernel<T, kBK, true>, kChainSmem)) return rc;
     if (int rc = set_smem(linear_logp_dh_kernel<T, kBK>, GH::kSmemBytes)) return rc;
     if (int rc = set_smem(linear_logp_dw_kernel<T, kBK>, GW::kSmemBytes)) return rc;
 
@@ -1646,6 +1867,7 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
             const bool dh_chain = shifted || (ksplit == 1 && H >= 256 && v_valid % kBK == 0 && v_valid >= 2 * kBK);
             h.nk = shifted ? k_steps(v_valid, v_shift) : (dh_chain ? v_valid / kBK : 0);
             h.tok_shift = tok_shift;
+            h.v_tiles = v_tiles;
             h.tail = KTail();
             if (v_shift != 0) {
                 const int64_t skip = static_cast<int64_t>(k_skip(v_valid, v_shift)) * kBK;
@@ -1672,15 +1894,42 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
             d.tail = KTail();
             if (tok_shift != 0) {
                 const int64_t skip = static_cast<int64_t>(k_skip(tok_valid, tok_shift)) * kBK;
-                d.tail = KTail{tok_valid / 256 * 4, (skip - tok_shift) * H * 2, skip * p.ldz * 2};
+                d.tail = KTail{tok_valid / 256 * 4, (skip - tok_shift) * H * 2,
+                               c.kept ? skip / kBK * kKeptSlab * 4 : skip * p.ldz * 2};
             }
+            float* db_part = c.d_bias ? reinterpret_cast<float*>(ws + p.db_off) : nullptr;
 
             // dZ block: chained through one pipeline when every tile can read 256 rows; otherwise the
             // full vocab tiles through the fast variant and the ragged last one through the general one
             // (all through the general one when the launch is tiny)
             const bool tiny = v_rag != 0 && tok_tiles * v_tiles <= 32;
-            const int fast_tiles = shifted ? v_tiles : (tiny ? 0 : v_valid / 256);
-            const int gen_tiles = v_tiles - fast_tiles;
+            if (c.kept) {
+                KeptDzArgs k;
+                k.kept = c.kept;
+                k.targets = z.targets;
+                k.lse = z.lse;
+                k.grad = z.grad;
+                k.scales = scales;
+                k.db_part = db_part;
+                k.N = tok_valid;
+                k.V = v_valid;
+                k.v_tiles = v_tiles;
+                k.tok_tiles = tok_tiles;
+                k.tok_shift = tok_shift;
+                k.v_shift = v_shift;
+                k.used = padded ? d.nk * kBK : 256;
+                k.vocab_start = z.v_global0;
+                k.ignore_index = z.ignore_index;
+                k.use_ignore = z.use_ignore;
+                k.scale2 = z.scale2;
+                const dim3 slabs(tok_tiles * v_tiles * 4);
+                if (db_part)
+                    hipLaunchKernelGGL((linear_logp_dz_kept_kernel<T, true>), slabs, dim3(256), 0, stream, k);
+                else
+                    hipLaunchKernelGGL((linear_logp_dz_kept_kernel<T, false>), slabs, dim3(256), 0, stream, k);
+            }
+            const int fast_tiles = c.kept ? 0 : shifted ? v_tiles : (tiny ? 0 : v_valid / 256);
+            const int gen_tiles = c.kept ? 0 : v_tiles - fast_tiles;
             const bool k_ok = H % kBK == 0 && H >= 2 * kBK;
             if (fast_tiles > 0) {
                 z.v_tiles = fast_tiles;
@@ -1714,12 +1963,17 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
                 if (!dw_in) dj.h_tiles = 0;
                 const int items = tok_tiles * hj.h_tiles * ksplit + v_tiles * dj.h_tiles;
                 const int grid = chain_grid(items, n_cu);
-                const GradsSplit split = grads_split(tok_tiles * hj.h_tiles * ksplit, h.nk / ksplit + 9,
-                                                     v_tiles * dj.h_tiles, d.nk + 9, grid);
+                const GradsSplit split = grads_split(tok_tiles * hj.h_tiles * ksplit, h.nk / ksplit + kDhSteps,
+                                                     v_tiles * dj.h_tiles, d.nk + (d.accumulate ? kDwAddSteps : kDwSteps),
+                                                     grid);
                 dj.busy = split.busy;
                 dj.lead = split.lead;
-                hipLaunchKernelGGL((linear_logp_grads_kernel<T, kBK>), dim3(grid), dim3(kThreads), kChainSmem,
-                                   stream, hj, dj);
+                if (c.kept)
+                    hipLaunchKernelGGL((linear_logp_grads_kernel<T, kBK, true>), dim3(grid), dim3(kThreads),
+                                       kChainSmem, stream, hj, dj);
+                else
+                    hipLaunchKernelGGL((linear_logp_grads_kernel<T, kBK, false>), dim3(grid), dim3(kThreads),
+                                       kChainSmem, stream, hj, dj);
             }
             if (dh && ksplit > 1) {
                 const int64_t n4 = static_cast<int64_t>(tok_valid) * H / 4;
@@ -1731,13 +1985,13 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
                 hipLaunchKernelGGL((linear_logp_dw_kernel<T, kBK>), dim3(v_tiles * h_tiles), dim3(kThreads),
                                    GW::kSmemBytes, stream, d);
             if (c.d_bias != nullptr) {
-                float* db_part = reinterpret_cast<float*>(ws + p.db_off);
-                hipLaunchKernelGGL(linear_logp_db_partial_kernel<T>, dim3(v_tiles, tok_tiles), dim3(256), 0,
-                                   stream, dz, p.ldz, padded ? static_cast<int>(N) : 256, db_part,
-                                   static_cast<int64_t>(p.v_piece));
+                if (!c.kept)
+                    hipLaunchKernelGGL(linear_logp_db_partial_kernel<T>, dim3(v_tiles, tok_tiles), dim3(256), 0,
+                                       stream, dz, p.ldz, padded ? static_cast<int>(N) : 256, db_part,
+                                       static_cast<int64_t>(p.v_piece));
                 hipLaunchKernelGGL(linear_logp_db_finish_kernel, dim3((v_valid + 255) / 256), dim3(256), 0,
-                                   stream, db_part, static_cast<int64_t>(p.v_piece), tok_tiles, v_valid,
-                                   v_shift, scales, c.d_bias + v_lo, (ci > 0 || c.accumulate != 0) ? 1 : 0);
+                                   stream, db_part, static_cast<int64_t>(p.v_piece),
+                                   c.kept ? 4 * tok_tiles : tok_tiles, v_valid, v_shift, scales, c.d_bias + v_lo, (ci > 0 || c.accumulate != 0) ? 1 : 0);
             }
             if (int rc = check_launch("linear_logp backward launch failed")) return rc;
         }
@@ -1752,6 +2006,16 @@ int launch_fwd_as(const FwdArgs& a, hipStream_t stream)
     using G = TileGemm<T, false, false, kBK>;
     if (int rc = set_smem(linear_logp_fwd_kernel<T, kBK, GENERAL, CHAIN>, G::kSmemBytes)) return rc;
     hipLaunchKernelGGL((linear_logp_fwd_kernel<T, kBK, GENERAL, CHAIN>), dim3(a.row_blocks * a.n_split),
+                       dim3(kThreads), G::kSmemBytes, stream, a);
+    return 0;
+}
+
+template <class T>
+int launch_fwd_kept(const FwdArgs& a, hipStream_t stream)
+{
+    using G = TileGemm<T, false, false, kBK>;
+    if (int rc = set_smem(linear_logp_fwd_kernel<T, kBK, false, true, true>, G::kSmemBytes)) return rc;
+    hipLaunchKernelGGL((linear_logp_fwd_kernel<T, kBK, false, true, true>), dim3(a.row_blocks * a.n_split),
                        dim3(kThreads), G::kSmemBytes, stream, a);
     return 0;
 }
@@ -1776,7 +2040,7 @@ int fwd_enqueue(const void* hidden, const void* weight, const float* bias, const
                 int32_t H, int64_t V, int64_t vocab_start, int32_t dtype, float temperature,
                 int64_t ignore_index, int32_t use_ignore, int32_t strict_targets,
                 int32_t* err_flag, hipStream_t stream, const GrpoArgs* epilogue = nullptr,
-                const SecondHead* second = nullptr);
+                const SecondHead* second = nullptr, float* kept = nullptr, size_t kept_size = 0);
 
 }  // namespace
 
@@ -1906,6 +2170,42 @@ int rlk_linear_logp_fwd_grpo(const void* hidden, const void* weight, const float
                              int64_t seq_len, float clip_eps, float beta, float* out3, float* ratio,
                              float* kl_terms, float* d_cur, float* d_kl, hipStream_t stream)
 {
+    return rlk_linear_logp_fwd_grpo_kept(hidden, weight, bias, targets, logp, lse, workspace, workspace_bytes, N, H, V,
+                                         vocab_start, dtype, temperature, ignore_index, use_ignore, strict_targets,
+                                         err_flag, old_logp, ref_logp, advantages, adv_per_token, mask, seq_len,
+                                         clip_eps, beta, out3, ratio, kl_terms, d_cur, d_kl, nullptr, 0, stream);
+}
+
+int rlk_linear_logp_kept_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes)
+{
+    if (!bytes || N <= 0 || V <= 0 || H <= 0) return rlk_fail(RLK_ERR_ARG, "bad kept-logits query");
+    *bytes = kept_bytes(N, H, V, dtype);
+    return 0;
+}
+
+int rlk_linear_logp_fwd_kept(const void* hidden, const void* weight, const float* bias,
+                             const int64_t* targets, float* logp, float* lse, void* workspace,
+                             size_t workspace_bytes, int64_t N, int32_t H, int64_t V,
+                             int64_t vocab_start, int32_t dtype, float temperature,
+                             int64_t ignore_index, int32_t use_ignore, int32_t strict_targets,
+                             int32_t* err_flag, void* kept, size_t kept_bytes, hipStream_t stream)
+{
+    return fwd_enqueue(hidden, weight, bias, targets, logp, lse, workspace, workspace_bytes, N, H, V, vocab_start, dtype,
+                       temperature, ignore_index, use_ignore, strict_targets, err_flag, stream, nullptr, nullptr,
+                       static_cast<float*>(kept), kept_bytes);
+}
+
+int rlk_linear_logp_fwd_grpo_kept(const void* hidden, const void* weight, const float* bias,
+                             const int64_t* targets, float* logp, float* lse, void* workspace,
+                             size_t workspace_bytes, int64_t N, int32_t H, int64_t V,
+                             int64_t vocab_start, int32_t dtype, float temperature,
+                             int64_t ignore_index, int32_t use_ignore, int32_t strict_targets,
+                             int32_t* err_flag, const float* old_logp, const float* ref_logp,
+                             const float* advantages, int32_t adv_per_token, const uint8_t* mask,
+                             int64_t seq_len, float clip_eps, float beta, float* out3, float* ratio,
+                             float* kl_terms, float* d_cur, float* d_kl, void* kept, size_t kept_bytes,
+                             hipStream_t stream)
+{
     if (int rc = check_common(N, H, V, dtype)) return rc;
     if (!old_logp || !advantages || !out3 || !logp) return rlk_fail(RLK_ERR_ARG, "null pointer");
     if (seq_len <= 0) return rlk_fail(RLK_ERR_ARG, "bad sizes");
@@ -1941,7 +2241,7 @@ int rlk_linear_logp_fwd_grpo(const void* hidden, const void* weight, const float
     g.blocks = grpo_blocks(N);
     return fwd_enqueue(hidden, weight, bias, targets, logp, lse, workspace, fwd, N, H, V, vocab_start,
                        dtype, temperature, ignore_index, use_ignore, strict_targets, err_flag, stream,
-                       &g);
+                       &g, nullptr, static_cast<float*>(kept), kept_bytes);
 }
 
 }  // extern "C"
@@ -1955,7 +2255,7 @@ int fwd_enqueue(const void* hidden, const void* weight, const float* bias, const
                 int32_t H, int64_t V, int64_t vocab_start, int32_t dtype, float temperature,
                 int64_t ignore_index, int32_t use_ignore, int32_t strict_targets,
                 int32_t* err_flag, hipStream_t stream, const GrpoArgs* epilogue,
-                const SecondHead* second)
+                const SecondHead* second, float* kept, size_t kept_size)
 {
     if (int rc = check_common(N, H, V, dtype)) return rc;
     if (!(temperature > 0.f)) return rlk_fail(RLK_ERR_ARG, "temperature must be greater than zero");
@@ -1963,6 +2263,8 @@ int fwd_enqueue(const void* hidden, const void* weight, const float* bias, const
     if (strict_targets && !err_flag)
         return rlk_fail(RLK_ERR_ARG, "strict_targets needs an err_flag to report through");
     const bool mfma = use_mfma(hidden, weight, H, dtype);
+    if (kept != nullptr)
+        if (int rc = check_kept(kept, kept_size, mfma, N, H, V, dtype)) return rc;
     // Both heads of a pair run through one launch, so they must take the same kind of kernel:
     // otherwise the policy head's results would depend on the reference head's alignment and no
     // longer equal the single-head call bit for bit.
@@ -2021,8 +2323,11 @@ int fwd_enqueue(const void* hidden, const void* weight, const float* bias, const
         a.split_lo = 0;
         a.tile_lo = 0;
         a.vtiles = plan.fast_tiles;
-        if (int rc = fwd_chained(H, V) ? launch_fwd<false, true>(a, dtype, stream)
-                                       : launch_fwd<false, false>(a, dtype, stream))
+        a.kept = kept;
+        if (int rc = kept != nullptr ? (dtype == RLK_DTYPE_BF16 ? launch_fwd_kept<Bf16>(a, stream)
+                                                                : launch_fwd_kept<F16>(a, stream))
+                     : fwd_chained(H, V) ? launch_fwd<false, true>(a, dtype, stream)
+                                         : launch_fwd<false, false>(a, dtype, stream))
             return rc;
     }
     if (mfma && plan.n_gen > 0) {
@@ -2149,6 +2454,44 @@ int rlk_linear_logp_bwd_accum(const float* grad_logp, const void* hidden, const 
                                              ignore_index, use_ignore, accumulate != 0 ? 1 : 0, stream);
 }
 
+int rlk_linear_logp_bwd_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes)
+{
+    if (!bytes || N <= 0 || V <= 0 || H <= 0) return rlk_fail(RLK_ERR_ARG, "bad workspace query");
+    if (kept_bytes(N, H, V, dtype) == 0)
+        return rlk_fail(RLK_ERR_UNSUPPORTED, "no logits are kept for these sizes (rlk_linear_logp_kept_bytes)");
+    *bytes = kept_plan(N, H, V).total;
+    return 0;
+}
+
+int rlk_linear_logp_bwd_kept(const float* grad_logp, const void* hidden, const void* weight,
+                             const float* bias, const int64_t* targets, const float* lse,
+                             void* d_hidden, float* d_weight, void* d_weight_typed, float* d_bias, void* kept,
+                             size_t kept_size, void* workspace, size_t workspace_bytes, int64_t N, int32_t H,
+                             int64_t V, int64_t vocab_start, int32_t dtype, float temperature,
+                             int64_t ignore_index, int32_t use_ignore, int32_t accumulate, hipStream_t stream)
+{
+    if (int rc = check_common(N, H, V, dtype)) return rc;
+    if (!(temperature > 0.f)) return rlk_fail(RLK_ERR_ARG, "temperature must be greater than zero");
+    if (!grad_logp || !hidden || !weight || !targets || !lse || !kept) return rlk_fail(RLK_ERR_ARG, "null pointer");
+    if (!d_hidden && !d_weight && !d_bias && !d_weight_typed)
+        return rlk_fail(RLK_ERR_ARG, "no gradient requested");
+    if (bias == nullptr && d_bias != nullptr) return rlk_fail(RLK_ERR_ARG, "d_bias given without bias");
+    if (d_weight_typed != nullptr &&
+        (d_weight != nullptr || accumulate != 0 || (reinterpret_cast<uintptr_t>(d_weight_typed) & 15) != 0))
+        return rlk_fail(RLK_ERR_ARG, "d_weight_typed takes no fp32 d_weight beside it and starts on a 16-byte boundary");
+    if (int rc = check_kept(kept, kept_size, use_mfma(hidden, weight, H, dtype), N, H, V, dtype)) return rc;
+    const BwdPlan p = kept_plan(N, H, V);
+    if (!workspace || workspace_bytes < p.total) return rlk_fail(RLK_ERR_ARG, "workspace too small");
+    if (reinterpret_cast<uintptr_t>(workspace) & 255)
+        return rlk_fail(RLK_ERR_ARG, "workspace must be 256-byte aligned");
+    int n_cu = 0;
+    if (int rc = compute_units(&n_cu)) return rc;
+    BwdCall c{grad_logp, hidden, weight, bias, targets, lse, d_hidden, d_weight, d_bias, workspace, N, H, V, vocab_start,
+              dtype, temperature, ignore_index, use_ignore, stream, accumulate != 0 ? 1 : 0, d_weight_typed,
+              static_cast<float*>(kept)};
+    return dtype == RLK_DTYPE_BF16 ? bwd_enqueue<Bf16>(c, p, n_cu) : bwd_enqueue<F16>(c, p, n_cu);
+}
+
 int rlk_linear_logp_bwd_typed_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype,
                                               size_t dz_budget_bytes, size_t* bytes)
 {
@@ -2219,6 +2562,7 @@ int rlk::linear_logp_bwd_accumulating(const float* grad_logp, const void* hidden
     int n_cu = 0;
     if (int rc = compute_units(&n_cu)) return rc;
     BwdCall c{grad_logp, hidden, weight, bias, targets, lse, d_hidden, d_weight, d_bias, workspace,
-              N, H, V, vocab_start, dtype, temperature, ignore_index, use_ignore, stream, accumulate, d_weight_cast};
+              N, H, V, vocab_start, dtype, temperature, ignore_index, use_ignore, stream, accumulate, d_weight_cast,
+              nullptr};
     return dtype == RLK_DTYPE_BF16 ? bwd_enqueue<Bf16>(c, p, n_cu) : bwd_enqueue<F16>(c, p, n_cu);
 }

@@ -616,4 +616,63 @@ int rlk_linear_logp_rmsnorm_bwd_typed(const float* grad_logp, const void* x, con
                     use_ignore, stream);
 }
 
+int rlk_linear_logp_rmsnorm_fwd_kept(const void* x, const float* gain, float eps, const void* weight,
+                                     const float* bias, const int64_t* targets, float* logp, float* lse,
+                                     void* workspace, size_t workspace_bytes, int64_t N, int32_t H,
+                                     int64_t V, int64_t vocab_start, int32_t dtype, float temperature,
+                                     int64_t ignore_index, int32_t use_ignore, int32_t strict_targets,
+                                     int32_t* err_flag, void* kept, size_t kept_bytes, hipStream_t stream)
+{
+    if (int rc = check_norm(x, gain, N, H, dtype)) return rc;
+    if (!weight || !targets || !logp || !lse || !kept) return rlk_fail(RLK_ERR_ARG, "null pointer");
+    if (N > kNormBlockTokens) return rlk_fail(RLK_ERR_UNSUPPORTED, "kept logits behind the norm: one block of tokens");
+    size_t need = 0;
+    if (int rc = rlk_linear_logp_rmsnorm_fwd_workspace_bytes(N, H, V, dtype, &need)) return rc;
+    if (!workspace || workspace_bytes < need) return rlk_fail(RLK_ERR_ARG, "workspace too small");
+    if (reinterpret_cast<uintptr_t>(workspace) & 255)
+        return rlk_fail(RLK_ERR_ARG, "workspace must be 256-byte aligned");
+    const size_t rows = up256(static_cast<size_t>(N) * H * elt_bytes(dtype));
+    char* ws = static_cast<char*>(workspace);
+    if (int rc = rmsnorm_fwd_enqueue(x, gain, eps, ws, nullptr, N, H, dtype, stream)) return rc;
+    return rlk_linear_logp_fwd_kept(ws, weight, bias, targets, logp, lse, ws + rows, need - rows, N, H, V, vocab_start,
+                                    dtype, temperature, ignore_index, use_ignore, strict_targets, err_flag, kept,
+                                    kept_bytes, stream);
+}
+
+int rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes)
+{
+    if (!bytes || N <= 0 || H <= 0 || V <= 0) return rlk_fail(RLK_ERR_ARG, "bad workspace query");
+    if (N > kNormBlockTokens) return rlk_fail(RLK_ERR_UNSUPPORTED, "kept logits behind the norm: one block of tokens");
+    size_t bwd = 0;
+    if (int rc = rlk_linear_logp_bwd_kept_workspace_bytes(N, H, V, dtype, &bwd)) return rc;
+    *bytes = up256(static_cast<size_t>(N) * H * elt_bytes(dtype)) + up256(rmsnorm_bwd_workspace(N, H)) + bwd;
+    return 0;
+}
+
+int rlk_linear_logp_rmsnorm_bwd_kept(const float* grad_logp, const void* x, const float* gain, float eps,
+                                     const void* weight, const float* bias, const int64_t* targets,
+                                     const float* lse, void* d_x, float* d_gain, void* d_weight_typed,
+                                     float* d_bias, void* kept, size_t kept_bytes, void* workspace,
+                                     size_t workspace_bytes, int64_t N, int32_t H, int64_t V,
+                                     int64_t vocab_start, int32_t dtype, float temperature,
+                                     int64_t ignore_index, int32_t use_ignore, hipStream_t stream)
+{
+    if (int rc = check_norm(x, gain, N, H, dtype)) return rc;
+    if (!d_x || !d_weight_typed) return rlk_fail(RLK_ERR_ARG, "d_x and d_weight are both written");
+    size_t need = 0;
+    if (int rc = rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(N, H, V, dtype, &need)) return rc;
+    if (!workspace || workspace_bytes < need) return rlk_fail(RLK_ERR_ARG, "workspace too small");
+    if (reinterpret_cast<uintptr_t>(workspace) & 255)
+        return rlk_fail(RLK_ERR_ARG, "workspace must be 256-byte aligned");
+    const size_t rows = up256(static_cast<size_t>(N) * H * elt_bytes(dtype)), norm = up256(rmsnorm_bwd_workspace(N, H));
+    char* ws = static_cast<char*>(workspace);
+    if (int rc = rmsnorm_fwd_enqueue(x, gain, eps, ws, nullptr, N, H, dtype, stream)) return rc;
+    // the gradient w.r.t. the normalised rows goes through d_x, as in norm_bwd
+    if (int rc = rlk_linear_logp_bwd_kept(grad_logp, ws, weight, bias, targets, lse, d_x, nullptr, d_weight_typed, d_bias,
+                                          kept, kept_bytes, ws + rows + norm, need - rows - norm, N, H, V, vocab_start,
+                                          dtype, temperature, ignore_index, use_ignore, 0, stream))
+        return rc;
+    return rmsnorm_bwd_enqueue(x, gain, eps, d_x, d_x, d_gain, 0, ws + rows, N, H, dtype, stream);
+}
+
 }  // extern "C"

@@ -75,11 +75,12 @@ std::vector<at::Tensor> fused_linear_logp(at::Tensor hidden, at::Tensor weight, 
 
 // Forward with the keyword extensions of the op classes (temperature, ignore-index, strictness):
 // [logp, lse, err_flag]; err_flag (int32[1], device) is non-zero when strict_targets and a
-// non-ignored target lies outside the shard.  Does not synchronise.
+// non-ignored target lies outside the shard.  Does not synchronise.  keep: a fourth tensor, the kept logits for
+// fused_linear_logp_backward (rlk_linear_logp_kept_bytes has to be non-zero for these sizes).
 std::vector<at::Tensor> fused_linear_logp_forward_ex(at::Tensor hidden, at::Tensor weight, at::Tensor target,
                                                      c10::optional<at::Tensor> bias, double temperature,
                                                      c10::optional<int64_t> ignore_index, int64_t vocab_start,
-                                                     bool strict_targets)
+                                                     bool strict_targets, bool keep)
 {
     TORCH_CHECK(hidden.dim() == 2 && weight.dim() == 2, "hidden and weight must be 2D tensors");
     TORCH_CHECK(hidden.is_cuda() && weight.is_cuda(), "hidden and weight must be CUDA tensors");
@@ -109,6 +110,19 @@ std::vector<at::Tensor> fused_linear_logp_forward_ex(at::Tensor hidden, at::Tens
         bias_f = bias->detach().to(hidden.device(), at::kFloat).contiguous();
         bias_p = bias_f.data_ptr<float>();
     }
+    if (keep) {
+        size_t bytes = 0;
+        TORCH_CHECK(rlk_linear_logp_kept_bytes(n, hd, v, dt, &bytes) == 0, rlk_last_error());
+        auto kept = at::empty({static_cast<int64_t>(bytes)}, hidden.options().dtype(at::kByte));
+        const int rc = rlk_linear_logp_fwd_kept(hidden.data_ptr(), weight.data_ptr(), bias_p, target.data_ptr<int64_t>(),
+                                                logp.data_ptr<float>(), lse.data_ptr<float>(), ws.data_ptr(),
+                                                static_cast<size_t>(ws.numel()), n, hd, v, vocab_start, dt,
+                                                static_cast<float>(temperature), ignore_index.value_or(0),
+                                                ignore_index.has_value() ? 1 : 0, strict_targets ? 1 : 0,
+                                                err.data_ptr<int32_t>(), kept.data_ptr(), bytes, current_stream(hidden));
+        TORCH_CHECK(rc == 0, "rlk_linear_logp_fwd_kept: ", rlk_last_error());
+        return {logp, lse, err, kept};
+    }
     const int rc = rlk_linear_logp_fwd(hidden.data_ptr(), weight.data_ptr(), bias_p, target.data_ptr<int64_t>(),
                                        logp.data_ptr<float>(), lse.data_ptr<float>(), ws.data_ptr(),
                                        static_cast<size_t>(ws.numel()), n, hd, v, vocab_start, dt,
@@ -124,6 +138,8 @@ std::vector<at::Tensor> fused_linear_logp_forward_ex(at::Tensor hidden, at::Tens
 // gradient that is not wanted.  weight_grad_out / bias_grad_out: caller-owned fp32 buffers that
 // receive (accumulate: are added) the gradients and are what the call returns in their place.
 // typed_weight: d_weight is a fresh tensor of the weight's type (rlk_linear_logp_bwd_typed).
+// kept: logits that the forward kept for this call, overwritten (rlk_linear_logp_bwd_kept; dz_budget_bytes has
+// no part in it).
 std::vector<at::Tensor> fused_linear_logp_backward(at::Tensor grad_logp, at::Tensor hidden, at::Tensor weight,
                                                    at::Tensor target, at::Tensor lse,
                                                    c10::optional<at::Tensor> bias, double temperature,
@@ -132,7 +148,7 @@ std::vector<at::Tensor> fused_linear_logp_backward(at::Tensor grad_logp, at::Ten
                                                    int64_t dz_budget_bytes,
                                                    c10::optional<at::Tensor> weight_grad_out,
                                                    c10::optional<at::Tensor> bias_grad_out, bool accumulate,
-                                                   bool typed_weight)
+                                                   bool typed_weight, c10::optional<at::Tensor> kept)
 {
     TORCH_CHECK(hidden.dim() == 2 && weight.dim() == 2, "hidden and weight must be 2D tensors");
     TORCH_CHECK(hidden.is_cuda() && weight.is_cuda(), "hidden and weight must be CUDA tensors");
@@ -173,6 +189,20 @@ std::vector<at::Tensor> fused_linear_logp_backward(at::Tensor grad_logp, at::Ten
         bias_p = bias_f.data_ptr<float>();
     }
     size_t ws_bytes = 0;
+    if (kept.has_value() && kept->defined()) {
+        TORCH_CHECK(rlk_linear_logp_bwd_kept_workspace_bytes(n, hd, v, dt, &ws_bytes) == 0, rlk_last_error());
+        auto ws = at::empty({static_cast<int64_t>(ws_bytes)}, hidden.options().dtype(at::kByte));
+        const int rc = rlk_linear_logp_bwd_kept(
+            g.data_ptr<float>(), hidden.data_ptr(), weight.data_ptr(), bias_p, target.data_ptr<int64_t>(),
+            lse.data_ptr<float>(), d_hidden.defined() ? d_hidden.data_ptr() : nullptr,
+            d_weight.defined() && !typed_weight ? d_weight.data_ptr<float>() : nullptr,
+            typed_weight ? d_weight.data_ptr() : nullptr, d_bias.defined() ? d_bias.data_ptr<float>() : nullptr,
+            kept->data_ptr(), static_cast<size_t>(kept->numel()), ws.data_ptr(), static_cast<size_t>(ws.numel()), n, hd,
+            v, vocab_start, dt, static_cast<float>(temperature), ignore_index.value_or(0),
+            ignore_index.has_value() ? 1 : 0, accumulate ? 1 : 0, current_stream(hidden));
+        TORCH_CHECK(rc == 0, "rlk_linear_logp_bwd_kept: ", rlk_last_error());
+        return {d_hidden, d_weight, d_bias};
+    }
     const auto query = typed_weight ? rlk_linear_logp_bwd_typed_workspace_bytes : rlk_linear_logp_bwd_workspace_bytes;
     TORCH_CHECK(query(n, hd, v, dt, static_cast<size_t>(dz_budget_bytes), &ws_bytes) == 0, rlk_last_error());
     auto ws = at::empty({static_cast<int64_t>(ws_bytes)}, hidden.options().dtype(at::kByte));
@@ -283,7 +313,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
           pybind11::arg("hidden"), pybind11::arg("weight"), pybind11::arg("target"),
           pybind11::arg("bias") = pybind11::none(), pybind11::arg("temperature") = 1.0,
           pybind11::arg("ignore_index") = pybind11::none(), pybind11::arg("vocab_start") = 0,
-          pybind11::arg("strict_targets") = true);
+          pybind11::arg("strict_targets") = true, pybind11::arg("keep") = false);
     m.def("fused_linear_logp_backward", &fused_linear_logp_backward,
           "Backward of the fused linear log-prob -> [d_hidden, d_weight (f32), d_bias (f32)]",
           pybind11::arg("grad_logp"), pybind11::arg("hidden"), pybind11::arg("weight"),
@@ -293,7 +323,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
           pybind11::arg("need_weight") = true, pybind11::arg("need_bias") = true,
           pybind11::arg("dz_budget_bytes") = 0, pybind11::arg("weight_grad_out") = pybind11::none(),
           pybind11::arg("bias_grad_out") = pybind11::none(), pybind11::arg("accumulate") = false,
-          pybind11::arg("typed_weight") = false);
+          pybind11::arg("typed_weight") = false, pybind11::arg("kept") = pybind11::none());
     m.def("fused_logp_forward_out", &fused_logp_forward_out, "Fused logp out");
     m.def("fused_logp_forward_fp32", &fused_logp_forward_fp32, "Fused logp fp32");
     m.def("fused_logp_forward_indexed_out", &fused_logp_forward_indexed_out, "Fused logp indexed out");

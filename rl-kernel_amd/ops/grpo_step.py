@@ -26,10 +26,11 @@ IGNORE_INDEX = -100
 def fused_linear_logp_grpo_forward(hidden_2d, weight, target_1d, bias, old, ref, adv, mask, *,
                                    seq_len: int, clip_eps: float, beta: float,
                                    temperature: float = 1.0, ignore_index: Optional[int] = None,
-                                   want_grad: bool = True, want_terms: bool = False):
+                                   want_grad: bool = True, want_terms: bool = False, keep: bool = False):
     """Raw launch set of ``rlk_linear_logp_fwd_grpo``; all per-token tensors are flat ``[N]``
     fp32 (``mask`` bool / uint8, ``adv`` per token ``[N]`` or per sequence ``[N / seq_len]``).
-    Returns ``(logp, lse, err, out3, ratio, kl_terms, d_cur, d_kl)``."""
+    Returns ``(logp, lse, err, out3, ratio, kl_terms, d_cur, d_kl)``, and with ``keep`` the kept logits
+    (see ``fused_linear_logp_forward``)."""
     lib = _native.load()
     n, h = hidden_2d.shape
     v = weight.size(0)
@@ -63,28 +64,33 @@ def fused_linear_logp_grpo_forward(hidden_2d, weight, target_1d, bias, old, ref,
     ws = torch.empty(need.value, device=dev, dtype=torch.uint8)
     bias_f = None if bias is None else bias.detach().to(torch.float32).contiguous()
     p = LL._ptr
-    rc = lib.rlk_linear_logp_fwd_grpo(
+    kept = torch.empty(LL._kept_bytes(hidden_2d, weight), device=dev, dtype=torch.uint8) if keep else None
+    rc = lib.rlk_linear_logp_fwd_grpo_kept(
         p(hidden_2d), p(weight), p(bias_f), p(target_1d), p(logp), p(lse), p(ws), ws.numel(), n, h, v,
         0, dt, float(temperature), 0 if ignore_index is None else int(ignore_index),
         int(ignore_index is not None), 1, p(err), p(old_f), p(ref_f), p(adv_f), per_token,
         p(mask_u8), max(int(seq_len), 1), float(clip_eps), float(beta), p(out3), p(ratio), p(klt),
-        p(dcur), p(dkl), LL._stream(dev))
+        p(dcur), p(dkl), p(kept), kept.numel() if keep else 0, LL._stream(dev))
     _native.check(rc, "rlk_linear_logp_fwd_grpo")
-    return logp, lse, err, out3, ratio, klt, dcur, dkl
+    out = (logp, lse, err, out3, ratio, klt, dcur, dkl)
+    return (*out, kept) if keep else out
 
 
 class _FusedGRPOStepFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, weight, bias, marked_ids, old, ref, adv, mask, clip_eps, beta,
-                temperature, check_targets):
+                temperature, check_targets, train=False):
         hidden_2d = LL._aligned_contiguous(hidden.reshape(-1, hidden.size(-1)))
         w = LL._aligned_contiguous(weight)
         target_1d = marked_ids.reshape(-1).to(device=hidden_2d.device, dtype=torch.long).contiguous()
         seq_len = hidden.shape[-2] if hidden.dim() >= 2 else 1
+        ctx.keeps = train and LL._kept_bytes(hidden_2d, w) > 0
+        keep = ctx.keeps and LL._may_keep()
         with LL._checked_targets(target_1d, w.size(0), IGNORE_INDEX, check_targets):
-            logp, lse, _, out3, _, _, dcur, dkl = fused_linear_logp_grpo_forward(
+            logp, lse, _, out3, _, _, dcur, dkl, *kept = fused_linear_logp_grpo_forward(
                 hidden_2d, w, target_1d, bias, old, ref, adv, mask, seq_len=seq_len, clip_eps=clip_eps,
-                beta=beta, temperature=temperature, ignore_index=IGNORE_INDEX)
+                beta=beta, temperature=temperature, ignore_index=IGNORE_INDEX, keep=keep)
+        ctx.kept = kept[0] if keep else None
         ctx.save_for_backward(hidden_2d, w, bias if bias is not None else hidden_2d, target_1d, lse,
                               dcur, dkl)
         ctx.has_bias = bias is not None
@@ -104,14 +110,17 @@ class _FusedGRPOStepFunction(torch.autograd.Function):
         need_b = ctx.has_bias and ctx.needs_input_grad[2]
         # d loss / d logp and d kl / d logp were left by the forward; policy = loss - beta * kl
         upstream = dcur * (g_loss + g_pol) + dkl * (g_kl - ctx.beta * g_pol)
+        bias = bias_t if ctx.has_bias else None
+        keys = dict(temperature=ctx.temperature, ignore_index=IGNORE_INDEX)
+        kept = LL._take_kept(ctx, lambda: LL.fused_linear_logp_forward(
+            hidden_2d, w, target_1d, bias, keep=True, **keys)[3])
         d_h, d_w, d_b = LL.fused_linear_logp_backward(
-            upstream, hidden_2d, w, target_1d, lse, bias_t if ctx.has_bias else None,
-            temperature=ctx.temperature, ignore_index=IGNORE_INDEX, need_hidden=need_h,
-            need_weight=need_w, need_bias=need_b, typed_weight=True)
+            upstream, hidden_2d, w, target_1d, lse, bias, need_hidden=need_h, need_weight=need_w,
+            need_bias=need_b, typed_weight=True, kept=kept, **keys)
         grad_hidden = d_h.reshape(tuple(ctx.lead_shape) + (hidden_2d.size(1),)) if need_h else None
         grad_weight = d_w.to(ctx.weight_dtype) if need_w else None
         grad_bias = d_b.to(ctx.bias_dtype) if need_b else None
-        return (grad_hidden, grad_weight, grad_bias) + (None,) * 9
+        return (grad_hidden, grad_weight, grad_bias) + (None,) * 10
 
 
 class RocmFusedGRPOStepOp:
@@ -158,4 +167,5 @@ class RocmFusedGRPOStepOp:
             ids = ids.masked_fill(~mask, IGNORE_INDEX)
         return _FusedGRPOStepFunction.apply(hidden, lm_head_weight, bias, ids, old_logps, ref_logps,
                                             advantages, mask, float(clip_eps), float(beta),
-                                            float(temperature), check_targets)
+                                            float(temperature), check_targets,
+                                            LL._trains(hidden, lm_head_weight, bias))

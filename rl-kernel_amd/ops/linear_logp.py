@@ -133,6 +133,27 @@ def _warn_if_wide_path(hidden_2d: torch.Tensor, weight: torch.Tensor) -> None:
             weight.size(0))
 
 
+def _kept_bytes(hidden_2d: torch.Tensor, weight: torch.Tensor) -> int:
+    """Size of the logits that a training forward keeps for its backward, 0 where it keeps none."""
+    n, h = hidden_2d.shape
+    if n == 0 or hidden_2d.data_ptr() % 16 or weight.data_ptr() % 16:
+        return 0
+    need = _native.ctypes.c_size_t(0)
+    _native.check(_native.load().rlk_linear_logp_kept_bytes(
+        n, h, weight.size(0), _DTYPES[hidden_2d.dtype], _native.ctypes.byref(need)), "kept logits query")
+    return need.value
+
+
+def _trains(*tensors: Optional[torch.Tensor]) -> bool:
+    """Whether autograd records a call with these differentiable inputs."""
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+
+def _may_keep() -> bool:
+    """Not under saved-tensor hooks: who offloads or recomputes what a forward saves wants its memory."""
+    return torch._C._autograd._top_saved_tensors_default_hooks(True) is None
+
+
 @_native.on_tensor_device
 def fused_linear_logp_forward(
     hidden_2d: torch.Tensor,
@@ -144,8 +165,10 @@ def fused_linear_logp_forward(
     ignore_index: Optional[int] = None,
     vocab_start: int = 0,
     strict_targets: bool = True,
+    keep: bool = False,
 ):
     """Raw forward: returns ``(logp, lse, err_flag)`` fp32 / fp32 / int32[1] device tensors.
+    ``keep`` (sizes with ``_kept_bytes`` only): a fourth tensor, the logits for ``kept`` of the backward.
 
     Stand-in for ``_C.fused_linear_logp_sm90`` (csrc/cuda/fused_linear_logp_sm90.cu:305-381 of the
     reference) with int64 global targets.  Does not synchronise; ``err_flag`` is non-zero when
@@ -160,10 +183,9 @@ def fused_linear_logp_forward(
             and target_1d.dtype == torch.long and target_1d.is_contiguous():
         # same C ABI through the compiled binding: no per-argument ctypes marshalling
         _warn_if_wide_path(hidden_2d, weight)
-        logp, lse, err = compiled.fused_linear_logp_forward_ex(
+        return tuple(compiled.fused_linear_logp_forward_ex(
             hidden_2d, weight, target_1d, bias, float(temperature), ignore_index, int(vocab_start),
-            bool(strict_targets))
-        return logp, lse, err
+            bool(strict_targets), bool(keep)))
     logp = torch.empty(n, device=dev, dtype=torch.float32)
     lse = torch.empty(n, device=dev, dtype=torch.float32)
     err = torch.zeros(1, device=dev, dtype=torch.int32)
@@ -176,6 +198,15 @@ def fused_linear_logp_forward(
                   "linear_logp workspace query")
     ws = torch.empty(max(need.value, 16), device=dev, dtype=torch.uint8)
     bias_f = None if bias is None else bias.detach().to(torch.float32).contiguous()
+    if keep:
+        kept = torch.empty(_kept_bytes(hidden_2d, weight), device=dev, dtype=torch.uint8)
+        rc = lib.rlk_linear_logp_fwd_kept(
+            _ptr(hidden_2d), _ptr(weight), _ptr(bias_f), _ptr(target_1d), _ptr(logp), _ptr(lse),
+            _ptr(ws), ws.numel(), n, h, v, int(vocab_start), dt, float(temperature),
+            0 if ignore_index is None else int(ignore_index), int(ignore_index is not None),
+            int(strict_targets), _ptr(err), _ptr(kept), kept.numel(), _stream(dev))
+        _native.check(rc, "rlk_linear_logp_fwd_kept")
+        return logp, lse, err, kept
     rc = lib.rlk_linear_logp_fwd(
         _ptr(hidden_2d), _ptr(weight), _ptr(bias_f), _ptr(target_1d), _ptr(logp), _ptr(lse),
         _ptr(ws), ws.numel(), n, h, v, int(vocab_start), dt, float(temperature),
@@ -241,10 +272,11 @@ def fused_norm_linear_logp_forward(
     eps: float = 1e-6,
     temperature: float = 1.0,
     ignore_index: Optional[int] = None,
+    keep: bool = False,
 ):
     """Raw forward from UN-normalised hidden states: ``(logp, lse, err_flag)`` of
     ``linear_logp(rmsnorm(x, gain, eps), weight, bias)``; the normalised rows live only in the
-    call's workspace."""
+    call's workspace.  ``keep``: see ``fused_linear_logp_forward`` (at most ``_NORM_BLOCK`` rows)."""
     lib = _native.load()
     n, h = x_2d.shape
     v = weight.size(0)
@@ -262,6 +294,15 @@ def fused_norm_linear_logp_forward(
                   "norm + linear_logp workspace query")
     ws = torch.empty(max(need.value, 256), device=dev, dtype=torch.uint8)
     bias_f = None if bias is None else bias.detach().to(torch.float32).contiguous()
+    if keep:
+        kept = torch.empty(_kept_bytes(x_2d, weight), device=dev, dtype=torch.uint8)
+        rc = lib.rlk_linear_logp_rmsnorm_fwd_kept(
+            _ptr(x_2d), _ptr(gain), float(eps), _ptr(weight), _ptr(bias_f), _ptr(target_1d), _ptr(logp),
+            _ptr(lse), _ptr(ws), ws.numel(), n, h, v, 0, dt, float(temperature),
+            0 if ignore_index is None else int(ignore_index), int(ignore_index is not None), 1,
+            _ptr(err), _ptr(kept), kept.numel(), _stream(dev))
+        _native.check(rc, "rlk_linear_logp_rmsnorm_fwd_kept")
+        return logp, lse, err, kept
     rc = lib.rlk_linear_logp_rmsnorm_fwd(
         _ptr(x_2d), _ptr(gain), float(eps), _ptr(weight), _ptr(bias_f), _ptr(target_1d), _ptr(logp),
         _ptr(lse), _ptr(ws), ws.numel(), n, h, v, 0, dt, float(temperature),
@@ -297,10 +338,12 @@ def fused_norm_linear_logp_backward(
     need_bias: bool = True,
     dz_budget_bytes: int = 0,
     typed_weight: bool = False,
+    kept: Optional[torch.Tensor] = None,
 ):
     """Raw backward: ``(d_x [N,H] input dtype, d_gain [H] fp32, d_weight [V,H] fp32, d_bias [V]
     fp32)``; ``d_x`` is the gradient w.r.t. the UN-normalised hidden states.  ``typed_weight``:
-    ``d_weight`` in the weight's type where the library can write it (see ``_typed_weight_ok``)."""
+    ``d_weight`` in the weight's type where the library can write it (see ``_typed_weight_ok``).
+    ``kept``: the forward's kept logits, overwritten (needs ``need_x`` and a typed ``d_weight``)."""
     lib = _native.load()
     n, h = x_2d.shape
     v = weight.size(0)
@@ -317,6 +360,17 @@ def fused_norm_linear_logp_backward(
     d_bias = torch.empty(v, device=dev, dtype=torch.float32) if want_bias else None
     bias_f = None if bias is None else bias.detach().to(torch.float32).contiguous()
     need = _native.ctypes.c_size_t(0)
+    if kept is not None:
+        _native.check(lib.rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(
+            n, h, v, dt, _native.ctypes.byref(need)), "norm + linear_logp backward workspace query")
+        ws = torch.empty(need.value, device=dev, dtype=torch.uint8)
+        rc = lib.rlk_linear_logp_rmsnorm_bwd_kept(
+            _ptr(g), _ptr(x_2d), _ptr(gain), float(eps), _ptr(weight), _ptr(bias_f), _ptr(target_1d),
+            _ptr(lse), _ptr(d_x), _ptr(d_gain), _ptr(d_weight), _ptr(d_bias), _ptr(kept), kept.numel(),
+            _ptr(ws), ws.numel(), n, h, v, 0, dt, float(temperature),
+            0 if ignore_index is None else int(ignore_index), int(ignore_index is not None), _stream(dev))
+        _native.check(rc, "rlk_linear_logp_rmsnorm_bwd_kept")
+        return d_x, d_gain, d_weight, d_bias
     query = lib.rlk_linear_logp_rmsnorm_bwd_typed_workspace_bytes if typed else \
         lib.rlk_linear_logp_rmsnorm_bwd_workspace_bytes
     _native.check(query(n, h, v, dt, int(dz_budget_bytes), _native.ctypes.byref(need)),
@@ -352,6 +406,7 @@ def fused_linear_logp_backward(
     bias_grad_out: Optional[torch.Tensor] = None,
     accumulate: bool = False,
     typed_weight: bool = False,
+    kept: Optional[torch.Tensor] = None,
 ):
     """Raw backward: ``(d_hidden [N,H] input dtype, d_weight [V,H] fp32, d_bias [V] fp32)``.
 
@@ -366,6 +421,9 @@ def fused_linear_logp_backward(
 
     ``typed_weight``: ``d_weight`` in the weight's type, rounded once from the fp32 sum by the kernel
     that finishes it, where the library can write it (see ``_typed_weight_ok``; fp32 otherwise).
+
+    ``kept``: the logits that the forward of these arguments kept; they are overwritten, and
+    ``dz_budget_bytes`` has no part in the call.
     """
     lib = _native.load()
     n, h = hidden_2d.shape
@@ -388,7 +446,7 @@ def fused_linear_logp_backward(
         d_hidden, d_weight, d_bias = compiled.fused_linear_logp_backward(
             grad_logp, hidden_2d, weight, target_1d, lse, bias, float(temperature), ignore_index,
             int(vocab_start), bool(need_hidden), bool(need_weight), bool(want_bias),
-            int(dz_budget_bytes), weight_grad_out, bias_grad_out, bool(accumulate), typed)
+            int(dz_budget_bytes), weight_grad_out, bias_grad_out, bool(accumulate), typed, kept)
         return d_hidden, d_weight, d_bias
     g = grad_logp.reshape(-1).to(torch.float32).contiguous()
     d_hidden = torch.empty_like(hidden_2d) if need_hidden else None
@@ -402,6 +460,18 @@ def fused_linear_logp_backward(
             torch.empty(v, device=dev, dtype=torch.float32)
     bias_f = None if bias is None else bias.detach().to(torch.float32).contiguous()
     need = _native.ctypes.c_size_t(0)
+    if kept is not None:
+        _native.check(lib.rlk_linear_logp_bwd_kept_workspace_bytes(n, h, v, dt, _native.ctypes.byref(need)),
+                      "linear_logp backward workspace query")
+        ws = torch.empty(need.value, device=dev, dtype=torch.uint8)
+        rc = lib.rlk_linear_logp_bwd_kept(
+            _ptr(g), _ptr(hidden_2d), _ptr(weight), _ptr(bias_f), _ptr(target_1d), _ptr(lse),
+            _ptr(d_hidden), None if typed else _ptr(d_weight), _ptr(d_weight) if typed else None,
+            _ptr(d_bias), _ptr(kept), kept.numel(), _ptr(ws), ws.numel(), n, h, v, int(vocab_start), dt,
+            float(temperature), 0 if ignore_index is None else int(ignore_index),
+            int(ignore_index is not None), int(bool(accumulate)), _stream(dev))
+        _native.check(rc, "rlk_linear_logp_bwd_kept")
+        return d_hidden, d_weight, d_bias
     query = lib.rlk_linear_logp_bwd_typed_workspace_bytes if typed else lib.rlk_linear_logp_bwd_workspace_bytes
     _native.check(query(n, h, v, dt, int(dz_budget_bytes), _native.ctypes.byref(need)),
                   "linear_logp backward workspace query")
@@ -424,10 +494,18 @@ def fused_linear_logp_backward(
     return d_hidden, d_weight, d_bias
 
 
+def _take_kept(ctx, again):
+    """The kept logits for one backward, or ``None`` for sizes that keep none.  The backward overwrites them, so
+    the context gives them up; a second backward, or one behind a forward that was not allowed to keep
+    them, makes them again (``again()``) so that its sums are grouped alike and its bits the same."""
+    kept, ctx.kept = ctx.kept, None
+    return again() if kept is None and ctx.keeps else kept
+
+
 class _FusedLinearLogpFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, weight, bias, target_ids, temperature, ignore_index, check_targets,
-                weight_grad_out=None, bias_grad_out=None, accumulate=True):
+                weight_grad_out=None, bias_grad_out=None, accumulate=True, train=False):
         hidden_2d = _aligned_contiguous(hidden.reshape(-1, hidden.size(-1)))
         w = _aligned_contiguous(weight)
         target_1d = target_ids.reshape(-1).to(device=hidden_2d.device, dtype=torch.long).contiguous()
@@ -441,9 +519,12 @@ class _FusedLinearLogpFunction(torch.autograd.Function):
             ctx.weight_dtype = weight.dtype
             ctx.bias_dtype = bias.dtype if bias is not None else None
             return hidden_2d.new_zeros(hidden.shape[:-1], dtype=torch.float32)
+        ctx.keeps = train and _kept_bytes(hidden_2d, w) > 0
+        keep = ctx.keeps and _may_keep()
         with _checked_targets(target_1d, w.size(0), ignore_index, check_targets):
-            logp, lse, _ = fused_linear_logp_forward(
-                hidden_2d, w, target_1d, bias, temperature=temperature, ignore_index=ignore_index)
+            logp, lse, _, *kept = fused_linear_logp_forward(
+                hidden_2d, w, target_1d, bias, temperature=temperature, ignore_index=ignore_index, keep=keep)
+        ctx.kept = kept[0] if keep else None
         ctx.save_for_backward(hidden_2d, w, bias if bias is not None else hidden_2d, target_1d, lse)
         ctx.has_bias = bias is not None
         ctx.lead_shape = hidden.shape[:-1]
@@ -461,7 +542,7 @@ class _FusedLinearLogpFunction(torch.autograd.Function):
         w_out = getattr(ctx, "weight_grad_out", None)
         b_out = getattr(ctx, "bias_grad_out", None)
         accumulate = getattr(ctx, "accumulate", True)
-        nones = (None,) * 7
+        nones = (None,) * 8
         if ctx.empty:
             # no tokens: the gradients are zeros; buffers that accumulate stay as they are
             if w_out is not None and not accumulate:
@@ -485,15 +566,19 @@ class _FusedLinearLogpFunction(torch.autograd.Function):
                 w_buf = torch.zeros(w.shape, device=w.device, dtype=torch.float32)
             if want_b and b_buf is None:
                 b_buf = torch.zeros(w.size(0), device=w.device, dtype=torch.float32)
+        bias = bias_t if ctx.has_bias else None
+        keys = dict(temperature=ctx.temperature, ignore_index=ctx.ignore_index)
+        kept = _take_kept(ctx, lambda: fused_linear_logp_forward(hidden_2d, w, target_1d, bias, keep=True, **keys)[3])
         d_h, d_w, d_b = fused_linear_logp_backward(
-            grad_logp, hidden_2d, w, target_1d, lse, bias_t if ctx.has_bias else None,
-            temperature=ctx.temperature, ignore_index=ctx.ignore_index,
-            need_hidden=need_h, need_weight=want_w, need_bias=want_b,
-            weight_grad_out=w_buf, bias_grad_out=b_buf, accumulate=adding, typed_weight=w_out is None)
+            grad_logp, hidden_2d, w, target_1d, lse, bias, need_hidden=need_h, need_weight=want_w, need_bias=want_b,
+            weight_grad_out=w_buf, bias_grad_out=b_buf, accumulate=adding, typed_weight=w_out is None, kept=kept, **keys)
         grad_hidden = d_h.reshape(tuple(ctx.lead_shape) + (hidden_2d.size(1),)) if need_h else None
         grad_weight = d_w.to(ctx.weight_dtype) if need_w and w_out is None else None
         grad_bias = d_b.to(ctx.bias_dtype) if need_b and b_out is None else None
         return (grad_hidden, grad_weight, grad_bias, *nones)
+
+
+_NORM_BLOCK = 8192  # rows of a norm + head call that the library runs as one block
 
 
 class _FusedNormLinearLogpFunction(torch.autograd.Function):
@@ -501,15 +586,22 @@ class _FusedNormLinearLogpFunction(torch.autograd.Function):
     normalised rows."""
 
     @staticmethod
-    def forward(ctx, x, gain, weight, bias, target_ids, eps, temperature, ignore_index, check_targets):
+    def forward(ctx, x, gain, weight, bias, target_ids, eps, temperature, ignore_index, check_targets,
+                train=False):
         x_2d = _aligned_contiguous(x.reshape(-1, x.size(-1)))
         g = _aligned_contiguous(gain.detach().to(torch.float32))  # the reference multiplies by weight.float()
         w = _aligned_contiguous(weight)
         target_1d = target_ids.reshape(-1).to(device=x_2d.device, dtype=torch.long).contiguous()
         ctx.empty = x_2d.size(0) == 0
+        # the gradients that rlk_linear_logp_rmsnorm_bwd_kept always writes have to be wanted
+        ctx.keeps = train and ctx.needs_input_grad[0] and ctx.needs_input_grad[2] \
+            and x_2d.size(0) <= _NORM_BLOCK and _kept_bytes(x_2d, w) > 0
+        keep = ctx.keeps and _may_keep()
         with _checked_targets(target_1d, w.size(0), ignore_index, check_targets):
-            logp, lse, _ = fused_norm_linear_logp_forward(
-                x_2d, g, w, target_1d, bias, eps=eps, temperature=temperature, ignore_index=ignore_index)
+            logp, lse, _, *kept = fused_norm_linear_logp_forward(
+                x_2d, g, w, target_1d, bias, eps=eps, temperature=temperature, ignore_index=ignore_index,
+                keep=keep)
+        ctx.kept = kept[0] if keep else None
         ctx.save_for_backward(x_2d, g, w, bias if bias is not None else x_2d, target_1d, lse)
         ctx.has_bias = bias is not None
         ctx.lead_shape = x.shape[:-1]
@@ -529,15 +621,22 @@ class _FusedNormLinearLogpFunction(torch.autograd.Function):
                     torch.zeros_like(g, dtype=ctx.gain_dtype) if need_g else None,
                     torch.zeros_like(w, dtype=ctx.weight_dtype) if need_w else None,
                     torch.zeros_like(bias_t, dtype=ctx.bias_dtype) if need_b else None,
-                    None, None, None, None, None)
+                    None, None, None, None, None, None)
+        bias = bias_t if ctx.has_bias else None
+        keys = dict(eps=ctx.eps, temperature=ctx.temperature, ignore_index=ctx.ignore_index)
+        kept = None
+        if not (need_x and need_w):  # fewer gradients wanted than when the forward ran
+            ctx.kept = None
+        else:
+            kept = _take_kept(ctx, lambda: fused_norm_linear_logp_forward(
+                x_2d, g, w, target_1d, bias, keep=True, **keys)[3])
         d_x, d_g, d_w, d_b = fused_norm_linear_logp_backward(
-            grad_logp, x_2d, g, w, target_1d, lse, bias_t if ctx.has_bias else None, eps=ctx.eps,
-            temperature=ctx.temperature, ignore_index=ctx.ignore_index, need_x=need_x,
-            need_gain=need_g, need_weight=need_w, need_bias=need_b, typed_weight=True)
+            grad_logp, x_2d, g, w, target_1d, lse, bias, need_x=need_x,
+            need_gain=need_g, need_weight=need_w, need_bias=need_b, typed_weight=True, kept=kept, **keys)
         return (d_x.reshape(tuple(ctx.lead_shape) + (x_2d.size(1),)) if need_x else None,
                 d_g.to(ctx.gain_dtype) if need_g else None,
                 d_w.to(ctx.weight_dtype) if need_w else None,
-                d_b.to(ctx.bias_dtype) if need_b else None, None, None, None, None, None)
+                d_b.to(ctx.bias_dtype) if need_b else None, None, None, None, None, None, None)
 
 
 class _FusedLinearLogpPairFunction(torch.autograd.Function):
@@ -555,6 +654,7 @@ class _FusedLinearLogpPairFunction(torch.autograd.Function):
                 hidden_2d, w, w_ref, target_1d, bias, ref_bias, temperature=temperature,
                 ignore_index=ignore_index)
         ctx.empty = hidden_2d.size(0) == 0
+        ctx.keeps, ctx.kept = False, None
         ctx.save_for_backward(hidden_2d, w, bias if bias is not None else hidden_2d, target_1d, lse)
         ctx.has_bias = bias is not None
         ctx.lead_shape = hidden.shape[:-1]
@@ -574,7 +674,8 @@ class _FusedLinearLogpPairFunction(torch.autograd.Function):
 
 class RocmFusedLinearLogpOp:
     """gfx950 MFMA fused linear log-prob: ``log_softmax((hidden W^T + b)/T)[target]`` without the
-    ``[N, V]`` logits.  Constructor raises ``RuntimeError`` when the HIP library or a ROCm GPU is
+    ``[N, V]`` logits (a training call of at most 800 MiB of fp32 logits holds them from its forward to its
+    backward, not under saved-tensor hooks; more are computed again).  Constructor raises ``RuntimeError`` when the HIP library or a ROCm GPU is
     missing so that a registry can fall through to its next backend
     (rl_engine/kernels/registry.py:219-229 of the reference)."""
 
@@ -702,10 +803,12 @@ class RocmFusedLinearLogpOp:
                                  f"{hidden.device}")
             return _FusedNormLinearLogpFunction.apply(hidden, norm_weight, lm_head_weight, bias,
                                                       target_ids, float(norm_eps), float(temperature),
-                                                      ignore_index, check_targets)
+                                                      ignore_index, check_targets,
+                                                      _trains(hidden, norm_weight, lm_head_weight, bias))
         return _FusedLinearLogpFunction.apply(hidden, lm_head_weight, bias, target_ids,
                                               float(temperature), ignore_index, check_targets,
-                                              weight_grad_out, bias_grad_out, bool(accumulate))
+                                              weight_grad_out, bias_grad_out, bool(accumulate),
+                                              _trains(hidden, lm_head_weight, bias))
 
     def with_reference(self, hidden, lm_head_weight, ref_lm_head_weight, target_ids, bias=None,
                        ref_bias=None, *, temperature: float = 1.0,
