@@ -32,7 +32,16 @@ namespace rlk {
 // whole vocabulary cut into n_split <= ceil(V / 256) ranges, in the layout the split combine reads.
 int wide_fwd_partials(const void* hidden, const void* weight, const float* bias, const int64_t* targets,
                       float* part_m, float* part_s, float* part_z, int n_split, int64_t N, int32_t H,
-                      int64_t V, int64_t vocab_start, int32_t dtype, float temperature, hipStream_t stream);
+                      int64_t V, int64_t vocab_start, int32_t dtype, float temperature, hipStream_t stream,
+                      float* kept = nullptr);
+// Kept logits of fp32 inputs: [N][V rounded up to 4], see rlk_linear_logp_fwd_kept.
+size_t wide_kept_bytes(int64_t N, int32_t H, int64_t V);
+size_t wide_bwd_kept_workspace(int64_t N, int32_t H, int64_t V);
+int wide_bwd_kept(const float* grad_logp, const void* hidden, const void* weight, const float* bias,
+                  const int64_t* targets, const float* lse, void* d_hidden, float* d_weight, float* d_bias,
+                  float* kept, void* workspace, int64_t N, int32_t H, int64_t V, int64_t vocab_start,
+                  float temperature, int64_t ignore_index, int32_t use_ignore, int32_t accumulate,
+                  hipStream_t stream);
 size_t wide_bwd_workspace(int64_t N, int32_t H, int64_t V, size_t dz_budget_bytes);
 int wide_bwd(const float* grad_logp, const void* hidden, const void* weight, const float* bias,
              const int64_t* targets, const float* lse, void* d_hidden, float* d_weight, float* d_bias,

@@ -1602,7 +1602,8 @@ BwdPlan bwd_plan(int64_t N, int H, int64_t V, size_t budget)
 // 957 us, 1000 x 896 x 50257 192 against 211, 1000 x 512 x 50257 154 against 138).
 size_t kept_bytes(int64_t N, int H, int64_t V, int dtype)
 {
-    if (dtype == RLK_DTYPE_F32 || !bwd_chained(H, V) || H < std::min<int64_t>(1024, 4 * N)) return 0;
+    if (dtype == RLK_DTYPE_F32) return wide_kept_bytes(N, H, V);
+    if (!bwd_chained(H, V) || H < std::min<int64_t>(1024, 4 * N)) return 0;
     const int64_t tiles = ((N + 255) / 256) * ((V + 255) / 256);
     if (tiles > static_cast<int64_t>(RLK_KEPT_LOGITS_BYTES / (kKeptTile * 4))) return 0;
     return static_cast<size_t>(tiles) * kKeptTile * 4;
@@ -1683,7 +1684,7 @@ bool use_mfma(const void* hidden, const void* weight, int32_t H, int dtype)
 int check_kept(const void* kept, size_t bytes, bool mfma, int64_t N, int32_t H, int64_t V, int dtype)
 {
     const size_t need = kept_bytes(N, H, V, dtype);
-    if (!mfma || need == 0)
+    if ((!mfma && dtype != RLK_DTYPE_F32) || need == 0)
         return rlk_fail(RLK_ERR_UNSUPPORTED, "no logits are kept for these sizes (rlk_linear_logp_kept_bytes)");
     if (bytes < need || (reinterpret_cast<uintptr_t>(kept) & 15) != 0)
         return rlk_fail(RLK_ERR_ARG, "kept logits: buffer too small or not 16-byte aligned");
@@ -2310,7 +2311,7 @@ int fwd_enqueue(const void* hidden, const void* weight, const float* bias, const
 
     if (!mfma) {
         if (int rc = wide_fwd_partials(hidden, weight, bias, targets, a.part_m, a.part_s, a.part_z,
-                                       plan.total_splits, N, H, V, vocab_start, dtype, temperature, stream))
+                                       plan.total_splits, N, H, V, vocab_start, dtype, temperature, stream, kept))
             return rc;
         if (second != nullptr)
             if (int rc = wide_fwd_partials(hidden, second->weight, second->bias, targets, a.part2_m,
@@ -2459,7 +2460,7 @@ int rlk_linear_logp_bwd_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, in
     if (!bytes || N <= 0 || V <= 0 || H <= 0) return rlk_fail(RLK_ERR_ARG, "bad workspace query");
     if (kept_bytes(N, H, V, dtype) == 0)
         return rlk_fail(RLK_ERR_UNSUPPORTED, "no logits are kept for these sizes (rlk_linear_logp_kept_bytes)");
-    *bytes = kept_plan(N, H, V).total;
+    *bytes = dtype == RLK_DTYPE_F32 ? wide_bwd_kept_workspace(N, H, V) : kept_plan(N, H, V).total;
     return 0;
 }
 
@@ -2480,10 +2481,17 @@ int rlk_linear_logp_bwd_kept(const float* grad_logp, const void* hidden, const v
         (d_weight != nullptr || accumulate != 0 || (reinterpret_cast<uintptr_t>(d_weight_typed) & 15) != 0))
         return rlk_fail(RLK_ERR_ARG, "d_weight_typed takes no fp32 d_weight beside it and starts on a 16-byte boundary");
     if (int rc = check_kept(kept, kept_size, use_mfma(hidden, weight, H, dtype), N, H, V, dtype)) return rc;
-    const BwdPlan p = kept_plan(N, H, V);
-    if (!workspace || workspace_bytes < p.total) return rlk_fail(RLK_ERR_ARG, "workspace too small");
+    size_t need = 0;
+    if (int rc = rlk_linear_logp_bwd_kept_workspace_bytes(N, H, V, dtype, &need)) return rc;
+    if (!workspace || workspace_bytes < need) return rlk_fail(RLK_ERR_ARG, "workspace too small");
     if (reinterpret_cast<uintptr_t>(workspace) & 255)
         return rlk_fail(RLK_ERR_ARG, "workspace must be 256-byte aligned");
+    if (dtype == RLK_DTYPE_F32)  // the weight's type is fp32
+        return wide_bwd_kept(grad_logp, hidden, weight, bias, targets, lse, d_hidden,
+                             d_weight_typed ? static_cast<float*>(d_weight_typed) : d_weight, d_bias,
+                             static_cast<float*>(kept), workspace, N, H, V, vocab_start, temperature, ignore_index,
+                             use_ignore, accumulate != 0 ? 1 : 0, stream);
+    const BwdPlan p = kept_plan(N, H, V);
     int n_cu = 0;
     if (int rc = compute_units(&n_cu)) return rc;
     BwdCall c{grad_logp, hidden, weight, bias, targets, lse, d_hidden, d_weight, d_bias, workspace, N, H, V, vocab_start,

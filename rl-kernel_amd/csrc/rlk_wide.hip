@@ -577,9 +577,11 @@ struct WideFwdArgs {
     int vtiles;
     float scale2;  // log2(e) / temperature
     bool vec_h, vec_w;
+    float* kept;  // KEEP: logits (bias added) for the backward, [N][ldz]
+    int64_t ldz;
 };
 
-template <int DT>
+template <int DT, bool KEEP>
 __global__ __launch_bounds__(kThreads) void wide_fwd_kernel(WideFwdArgs a)
 {
     using Gemm = SplitGemm<DT, DT, false, false>;
@@ -618,6 +620,27 @@ __global__ __launch_bounds__(kThreads) void wide_fwd_kernel(WideFwdArgs a)
         f32x16_t acc[kTM][kTN];
         zero_acc(acc);
         Gemm::run(A, B, a.H, acc, smem);
+        if constexpr (KEEP) {
+#pragma unroll
+            for (int j = 0; j < kTN; ++j) {
+                const int tl = wn * (kTN * 32) + j * 32 + (lane & 31);
+                float* row = a.kept + static_cast<int64_t>(tok0 + min(tl, tok_valid - 1)) * a.ldz;
+#pragma unroll
+                for (int i = 0; i < kTM; ++i)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int v = v0 + wm * (kTM * 32) + Acc32::quad_row(i, q, lane);
+                        f32x4_t z;
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            z[c] = acc[i][j][q * 4 + c];
+                            if (a.bias != nullptr) z[c] += a.bias[v + c < a.V ? v + c : a.V - 1];
+                        }
+                        // ldz is a multiple of 4 >= V: a quad that starts below V ends below ldz
+                        if (tl < tok_valid && v < a.V) *reinterpret_cast<f32x4_t*>(row + v) = z;
+                    }
+            }
+        }
         fwd_epilogue<true, Acc32>(acc, a, a.bias, v0 + wm * (kTM * 32), v0, lane, tgt, m, s, zt);
     }
 
@@ -741,6 +764,73 @@ __global__ __launch_bounds__(kThreads) void wide_dz_kernel(WideDzArgs a)
                 }
         }
     }
+}
+
+// dZ from the logits that the forward kept, in place: the same expressions as above on one pass over memory
+// (8 bytes per logit against six products of H terms).  A workgroup takes 256 columns of 64 tokens, a thread
+// four of them of every fourth token.  db_part (or null): column sums of the 64 tokens for d_bias,
+// [slab][ldz].
+struct WideKeptArgs {
+    float* kept;  // [N][ldz]
+    const int64_t* targets;
+    const float* lse;
+    const float* grad;
+    float* db_part;
+    int64_t ldz;
+    int N;
+    int V;
+    int64_t vocab_start;
+    int64_t ignore_index;
+    int use_ignore;
+    float scale2;
+    float inv_t;
+};
+
+constexpr int kWideSlab = 64;  // tokens
+__global__ __launch_bounds__(256) void wide_dz_kept_kernel(WideKeptArgs a)
+{
+    const int v = blockIdx.x * 256 + (threadIdx.x & 63) * 4;
+    const int wave = threadIdx.x >> 6, lo = blockIdx.y * kWideSlab;
+    f32x4_t sum{0.f, 0.f, 0.f, 0.f};
+    if (v < a.V) {
+#pragma unroll 4
+        for (int t = lo + wave; t < min(lo + kWideSlab, a.N); t += 4) {
+            const int64_t tg = a.targets[t];
+            const bool live = !(a.use_ignore && tg == a.ignore_index);
+            const float gs = live ? a.grad[t] * a.inv_t : 0.f;
+            const float nlse2 = -a.lse[t] * kLog2e;
+            const int64_t trel = tg - a.vocab_start;
+            f32x4_t* p = reinterpret_cast<f32x4_t*>(a.kept + static_cast<int64_t>(t) * a.ldz + v);
+            const f32x4_t z = *p;
+            f32x4_t d;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float pr = v + c < a.V ? __builtin_amdgcn_exp2f(fmaf(z[c], a.scale2, nlse2)) : 0.f;
+                d[c] = gs * ((trel == v + c ? 1.f : 0.f) - pr);
+                sum[c] += d[c];
+            }
+            *p = d;
+        }
+    }
+    if (a.db_part == nullptr) return;  // uniform
+    __shared__ f32x4_t red[4][64];
+    red[wave][threadIdx.x & 63] = sum;
+    __syncthreads();
+    if (wave == 0 && v < a.V) {
+        for (int w = 1; w < 4; ++w) sum += red[w][threadIdx.x];
+        *reinterpret_cast<f32x4_t*>(a.db_part + blockIdx.y * a.ldz + v) = sum;
+    }
+}
+
+// Slabs in ascending order.
+__global__ void wide_db_finish_kernel(const float* part, int64_t ld, int slabs, int V, float* db, int accumulate)
+{
+    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= V) return;
+    float sum = part[v];
+#pragma unroll 8
+    for (int s = 1; s < slabs; ++s) sum += part[s * ld + v];
+    db[v] = accumulate ? db[v] + sum : sum;
 }
 
 // ------------------------------------------------------------------------------------------- //
@@ -929,7 +1019,7 @@ struct WidePlan {
     int64_t ldz;
     int ksplit;
     int k_per;
-    size_t dz_bytes, part_bytes, total;
+    size_t dz_bytes, part_bytes, db_bytes, total;
 };
 
 WidePlan wide_plan(int64_t N, int32_t H, int64_t V, size_t budget)
@@ -957,16 +1047,28 @@ WidePlan wide_plan(int64_t N, int32_t H, int64_t V, size_t budget)
     p.k_per = static_cast<int>(k_per);
     p.dz_bytes = align256(static_cast<size_t>(chunk) * p.ldz * 4);
     p.part_bytes = align256(static_cast<size_t>(p.ksplit) * chunk * H * 4);
+    p.db_bytes = 0;
     p.total = p.dz_bytes + p.part_bytes;
     return p;
 }
 
-template <int DT>
+// Backward from kept logits: the chunks of the default budget, so that the sums are grouped as without; dZ lies in
+// the place of the logits.
+WidePlan wide_kept_plan(int64_t N, int32_t H, int64_t V)
+{
+    WidePlan p = wide_plan(N, H, V, RLK_DEFAULT_DZ_BUDGET);
+    p.dz_bytes = 0;
+    p.db_bytes = align256(static_cast<size_t>(p.chunk + kWideSlab - 1) / kWideSlab * p.ldz * 4);
+    p.total = p.part_bytes + p.db_bytes;
+    return p;
+}
+
+template <int DT, bool KEEP = false>
 int wide_fwd_launch(const WideFwdArgs& a, hipStream_t stream)
 {
     using G = SplitGemm<DT, DT, false, false>;
-    if (int rc = wide_smem(wide_fwd_kernel<DT>, G::kSmemBytes)) return rc;
-    hipLaunchKernelGGL(wide_fwd_kernel<DT>, dim3(a.row_blocks * a.n_split), dim3(kThreads), G::kSmemBytes,
+    if (int rc = wide_smem(wide_fwd_kernel<DT, KEEP>, G::kSmemBytes)) return rc;
+    hipLaunchKernelGGL((wide_fwd_kernel<DT, KEEP>), dim3(a.row_blocks * a.n_split), dim3(kThreads), G::kSmemBytes,
                        stream, a);
     return wide_check("wide_fwd_kernel launch failed");
 }
@@ -974,7 +1076,7 @@ int wide_fwd_launch(const WideFwdArgs& a, hipStream_t stream)
 template <int DT>
 int wide_bwd_launch(const float* grad_logp, const void* hidden, const void* weight, const float* bias,
                     const int64_t* targets, const float* lse, void* d_hidden, float* d_weight,
-                    float* d_bias, void* workspace, const WidePlan& p, int64_t N, int32_t H, int64_t V,
+                    float* d_bias, float* kept, void* workspace, const WidePlan& p, int64_t N, int32_t H, int64_t V,
                     int64_t vocab_start, float temperature, int64_t ignore_index, int32_t use_ignore,
                     int32_t accumulate, hipStream_t stream)
 {
@@ -987,6 +1089,7 @@ int wide_bwd_launch(const float* grad_logp, const void* hidden, const void* weig
     constexpr int esz = WideElem<DT>::kBytes;
     float* dz = static_cast<float*>(workspace);
     float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + p.dz_bytes);
+    float* db_part = kept && d_bias ? reinterpret_cast<float*>(static_cast<char*>(workspace) + p.part_bytes) : nullptr;
     const int v_tiles = static_cast<int>((V + 255) / 256);
     const int h_tiles = (H + 255) / 256;
     const bool vec_h = quad_aligned(hidden, H, DT), vec_w = quad_aligned(weight, H, DT);
@@ -994,6 +1097,8 @@ int wide_bwd_launch(const float* grad_logp, const void* hidden, const void* weig
         const int nt = static_cast<int>(N - t0 < p.chunk ? N - t0 : p.chunk);
         const int tok_tiles = (nt + 255) / 256;
         const void* hid = static_cast<const char*>(hidden) + t0 * H * esz;
+        if (kept) dz = kept + t0 * p.ldz;
+        const int slabs = (nt + kWideSlab - 1) / kWideSlab;
         WideDzArgs z;
         z.hidden = hid;
         z.weight = weight;
@@ -1015,7 +1120,13 @@ int wide_bwd_launch(const float* grad_logp, const void* hidden, const void* weig
         z.inv_t = 1.f / temperature;
         z.vec_h = vec_h;
         z.vec_w = vec_w;
-        hipLaunchKernelGGL(wide_dz_kernel<DT>, dim3(tok_tiles * v_tiles), dim3(kThreads), GZ::kSmemBytes, stream, z);
+        if (kept) {
+            const WideKeptArgs k{dz, z.targets, z.lse, z.grad, db_part, p.ldz, nt, z.V, vocab_start,
+                                 ignore_index, use_ignore, z.scale2, z.inv_t};
+            hipLaunchKernelGGL(wide_dz_kept_kernel, dim3(v_tiles, slabs), dim3(256), 0, stream, k);
+        } else {
+            hipLaunchKernelGGL(wide_dz_kernel<DT>, dim3(tok_tiles * v_tiles), dim3(kThreads), GZ::kSmemBytes, stream, z);
+        }
         if (d_hidden) {
             WideDhArgs h;
             h.dz = dz;
@@ -1054,7 +1165,10 @@ int wide_bwd_launch(const float* grad_logp, const void* hidden, const void* weig
             w.vec_h = vec_h;
             hipLaunchKernelGGL(wide_dw_kernel<DT>, dim3(v_tiles * h_tiles), dim3(kThreads), GW::kSmemBytes, stream, w);
         }
-        if (d_bias)
+        if (db_part)
+            hipLaunchKernelGGL(wide_db_finish_kernel, dim3(static_cast<unsigned>((V + 255) / 256)), dim3(256), 0, stream,
+                               db_part, p.ldz, slabs, static_cast<int>(V), d_bias, acc);
+        else if (d_bias)
             hipLaunchKernelGGL(wide_db_kernel, dim3(static_cast<unsigned>((V + 255) / 256)), dim3(256), 0, stream,
                                dz, p.ldz, nt, static_cast<int>(V), d_bias, acc);
         if (int rc = wide_check("wide backward launch failed")) return rc;
@@ -1066,9 +1180,12 @@ int wide_bwd_launch(const float* grad_logp, const void* hidden, const void* weig
 
 int wide_fwd_partials(const void* hidden, const void* weight, const float* bias, const int64_t* targets,
                       float* part_m, float* part_s, float* part_z, int n_split, int64_t N, int32_t H,
-                      int64_t V, int64_t vocab_start, int32_t dtype, float temperature, hipStream_t stream)
+                      int64_t V, int64_t vocab_start, int32_t dtype, float temperature, hipStream_t stream,
+                      float* kept)
 {
     WideFwdArgs a;
+    a.kept = kept;
+    a.ldz = (V + 3) / 4 * 4;
     a.hidden = hidden;
     a.weight = weight;
     a.bias = bias;
@@ -1087,6 +1204,9 @@ int wide_fwd_partials(const void* hidden, const void* weight, const float* bias,
     a.scale2 = kLog2e / temperature;
     a.vec_h = quad_aligned(hidden, H, dtype);
     a.vec_w = quad_aligned(weight, H, dtype);
+    if (kept != nullptr)
+        return dtype == RLK_DTYPE_F32 ? wide_fwd_launch<RLK_DTYPE_F32, true>(a, stream)
+                                      : rlk_fail(RLK_ERR_UNSUPPORTED, "the fp32 kernels keep logits of fp32 inputs only");
     if (dtype == RLK_DTYPE_F32) return wide_fwd_launch<RLK_DTYPE_F32>(a, stream);
     if (dtype == RLK_DTYPE_BF16) return wide_fwd_launch<RLK_DTYPE_BF16>(a, stream);
     return wide_fwd_launch<RLK_DTYPE_F16>(a, stream);
@@ -1106,14 +1226,34 @@ int wide_bwd(const float* grad_logp, const void* hidden, const void* weight, con
     const WidePlan p = wide_plan(N, H, V, dz_budget_bytes);
     if (dtype == RLK_DTYPE_F32)
         return wide_bwd_launch<RLK_DTYPE_F32>(grad_logp, hidden, weight, bias, targets, lse, d_hidden, d_weight,
-                                              d_bias, workspace, p, N, H, V, vocab_start, temperature,
+                                              d_bias, nullptr, workspace, p, N, H, V, vocab_start, temperature,
                                               ignore_index, use_ignore, accumulate, stream);
     if (dtype == RLK_DTYPE_BF16)
         return wide_bwd_launch<RLK_DTYPE_BF16>(grad_logp, hidden, weight, bias, targets, lse, d_hidden, d_weight,
-                                               d_bias, workspace, p, N, H, V, vocab_start, temperature,
+                                               d_bias, nullptr, workspace, p, N, H, V, vocab_start, temperature,
                                                ignore_index, use_ignore, accumulate, stream);
     return wide_bwd_launch<RLK_DTYPE_F16>(grad_logp, hidden, weight, bias, targets, lse, d_hidden, d_weight,
-                                          d_bias, workspace, p, N, H, V, vocab_start, temperature,
+                                          d_bias, nullptr, workspace, p, N, H, V, vocab_start, temperature,
+                                          ignore_index, use_ignore, accumulate, stream);
+}
+
+// Size of the kept logits of an fp32 head, 0 where none are kept: more than the bound, or a head so narrow that the
+// products cost what the trip through memory does.
+size_t wide_kept_bytes(int64_t N, int32_t H, int64_t V)
+{
+    const size_t bytes = static_cast<size_t>(N) * ((V + 3) / 4 * 4) * 4;
+    return bytes > RLK_KEPT_LOGITS_BYTES || H < 128 ? 0 : bytes;
+}
+
+size_t wide_bwd_kept_workspace(int64_t N, int32_t H, int64_t V) { return wide_kept_plan(N, H, V).total; }
+
+int wide_bwd_kept(const float* grad_logp, const void* hidden, const void* weight, const float* bias,
+                  const int64_t* targets, const float* lse, void* d_hidden, float* d_weight, float* d_bias,
+                  float* kept, void* workspace, int64_t N, int32_t H, int64_t V, int64_t vocab_start,
+                  float temperature, int64_t ignore_index, int32_t use_ignore, int32_t accumulate, hipStream_t stream)
+{
+    return wide_bwd_launch<RLK_DTYPE_F32>(grad_logp, hidden, weight, bias, targets, lse, d_hidden, d_weight, d_bias, kept,
+                                          workspace, wide_kept_plan(N, H, V), N, H, V, vocab_start, temperature,
                                           ignore_index, use_ignore, accumulate, stream);
 }
 

@@ -9,7 +9,8 @@ from oracle import oracle as O
 pytestmark = pytest.mark.gpu
 
 # one rounding of dZ to the input type (2^-9 bf16, 2^-12 f16 at most, random signs) and one of the result
-GRAD_REL = {torch.bfloat16: 5e-3, torch.float16: 1e-3}
+# (fp32: sums of at most 2050 fp32 products against another order of them)
+GRAD_REL = {torch.bfloat16: 5e-3, torch.float16: 1e-3, torch.float32: 1e-5}
 
 
 def make(n, h, v, dtype, bias, seed, low=0.0):
@@ -39,6 +40,10 @@ def rel(a, b):
     (256, 1024, 512, torch.bfloat16, False, 0.0),
     (300, 1088, 1281, torch.bfloat16, True, 0.0),
     (1000, 1024, 9000, torch.bfloat16, True, 0.0),
+    (1, 128, 3, torch.float32, True, 0.0),
+    (63, 130, 1001, torch.float32, True, -200.0),
+    (300, 257, 2050, torch.float32, True, 0.0),
+    (513, 256, 1024, torch.float32, False, 0.0),
 ])
 def test_kept_logits_give_the_gradients(n, h, v, dtype, bias, low):
     from rl_kernel_amd.ops import linear_logp as LL
@@ -49,7 +54,8 @@ def test_kept_logits_give_the_gradients(n, h, v, dtype, bias, low):
     r_dh, r_dw, r_db = O.linear_logp_backward(grad, hidden, weight, ids, b, **keys)
     hd, wd, td, gd = hidden.to(dev), weight.to(dev), ids.to(dev), grad.to(dev)
     bd = b.to(dev) if bias else None
-    assert LL._kept_bytes(hd, wd) == -(-n // 256) * -(-v // 256) * (256 << 10)
+    assert LL._kept_bytes(hd, wd) == (n * -(-v // 4) * 16 if dtype == torch.float32
+                                      else -(-n // 256) * -(-v // 256) * (256 << 10))
     plain = LL.fused_linear_logp_forward(hd, wd, td, bd, **keys)
 
     def backward(**more):

@@ -12,15 +12,16 @@ def test_kept_logits_and_workspace_stay_below_one_gigabyte():
         n = int(2 ** rng.uniform(0, 18))
         h = rng.choice((256, 512, 896, 1024, 1536, 2048, 4096, 4160, 8192))
         v = int(2 ** rng.uniform(8, 18))
+        dtype = rng.choice((0, 1, 2))
         kept, ws = ctypes.c_size_t(0), ctypes.c_size_t(0)
-        assert lib.rlk_linear_logp_kept_bytes(n, h, v, 0, ctypes.byref(kept)) == 0
-        rc = lib.rlk_linear_logp_bwd_kept_workspace_bytes(n, h, v, 0, ctypes.byref(ws))
+        assert lib.rlk_linear_logp_kept_bytes(n, h, v, dtype, ctypes.byref(kept)) == 0
+        rc = lib.rlk_linear_logp_bwd_kept_workspace_bytes(n, h, v, dtype, ctypes.byref(ws))
         if kept.value == 0:
             assert rc == -2
             continue
         kept_some += 1
         tiles = -(-n // 256) * -(-v // 256)
-        assert rc == 0 and kept.value == tiles * (256 << 10) <= 800 << 20
+        assert rc == 0 and kept.value == (n * -(-v // 4) * 16 if dtype == 2 else tiles * (256 << 10)) <= 800 << 20
         assert kept.value + ws.value <= 10 ** 9, (n, h, v)
     assert kept_some > 500
 
@@ -29,7 +30,7 @@ def test_sizes_that_keep_none():
     from rl_kernel_amd import _native
 
     lib, kept = _native.load(), ctypes.c_size_t(1)
-    for n, h, v, dtype in ((32768, 4096, 128256, 0), (100, 1024, 5000, 2), (100, 1000, 5000, 0), (100, 192, 5000, 0),
+    for n, h, v, dtype in ((32768, 4096, 128256, 0), (100, 64, 5000, 2), (32768, 2048, 32000, 2), (100, 1000, 5000, 0), (100, 192, 5000, 0),
                            (100, 1024, 255, 0), (1000, 896, 5000, 0), (1638 * 2, 4096, 128256, 1)):
         assert lib.rlk_linear_logp_kept_bytes(n, h, v, dtype, ctypes.byref(kept)) == 0 and kept.value == 0
     assert lib.rlk_linear_logp_kept_bytes(0, 1024, 5000, 0, ctypes.byref(kept)) == -1
