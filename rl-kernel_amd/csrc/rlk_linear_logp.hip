@@ -66,6 +66,8 @@ struct FwdArgs {
 // a slab holds the accumulator quads as the wavefronts have them,
 // [2 wavefronts along vocab][TM][TN][64 lanes][4], so a wavefront stores a tile in 1 KiB pieces.  The last token tile
 // is moved back to end at N as in the backward; columns of 16 tokens past N (fewer than 256 tokens) are not stored.
+// They are stored past the L2 (stream_store): left in it as dirty lines they cost their whole trip to memory
+// on top of the products (4096 x 2048 x 50257: 585 us without them, 774 with plain or `nt` stores, 652 so).
 constexpr int kKeptSlab = 64 * 256;       // floats
 constexpr int kKeptTile = 4 * kKeptSlab;
 
@@ -212,7 +214,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
                         if (wn * (TN * 16) + j * 16 >= tok_valid) break;  // uniform
 #pragma unroll
                         for (int i = 0; i < TM; ++i)
-                            *reinterpret_cast<f32x4_t*>(dst + (i * TN + j) * 256 + lane * 4) = acc[i][j];
+                            stream_store(dst + (i * TN + j) * 256, lane * 16, acc[i][j]);
                     }
                     counted = tok_valid == 256;
                 }
@@ -924,11 +926,11 @@ struct DwArgs {
 };
 
 // 16-bit results of four 16-row MFMA tiles of one column: lane group g (16 lanes) holds rows 4 g .. 4 g + 3
-// of every tile, p[i] = its quad of tile i.  Afterwards it holds rows 16 g .. 16 g + 15 of the 64, p[k] =
-// rows 16 g + 4 k .. + 3: a 4 x 4 transpose over lane groups and registers in two rounds of half-swaps.
-// A lane then stores 32 consecutive bytes and the four groups one full 128-byte line, where quads leave
-// in pieces of 32 bytes a row: 64 x 4096 x 128256 forward + backward 1166 -> 1121 us, 500 x 2048 x 151936
-// 1316 -> 1285, same bits.
+// of every tile, p[i] = its quad of tile i.  Afterwards p[0], p[1] are rows 8 g .. 8 g + 7 of the first 32 and
+// p[2], p[3] those of the other 32: two rounds of half-swaps over lane groups and registers.  The four groups
+// then store 64 consecutive bytes of a row at a time, where quads leave in pieces of 8 bytes, 32 apart
+// (64 x 4096 x 128256 forward + backward 1166 -> 1121 us with 16-byte pieces; backward from kept logits 617 ->
+// 590 with 64-byte ones), same bits.
 __device__ inline void gather_rows(u32x2_t (&p)[4])
 {
 #pragma unroll
@@ -943,12 +945,17 @@ __device__ inline void gather_rows(u32x2_t (&p)[4])
             p[a][c] = r[0];
             p[b][c] = r[1];
         };
-        swap32(0, 2);
-        swap32(1, 3);
+        swap32(0, 1);
+        swap32(2, 3);
         swap16(0, 1);
         swap16(2, 3);
     }
 }
+
+// K steps up to which the tiles of a dW launch are written past the L2: with few tokens the launch is bound by its
+// stores (backward from kept logits of 64 x 4096 x 128256 590 -> 558 us, 300 x 2048 x 50257 into fp32 291 ->
+// 254), from 1000 tokens on the two are the same.
+constexpr int kDwStreamSteps = 8;
 
 // Stores that the epilogue of a full dW tile issues per wavefront, all of them unconditional, the fewer of its
 // two forms: 16 bytes per quad of fp32 (TM * TN = 32), 16 bytes per pair of quads of 16-bit results (16).
@@ -982,7 +989,8 @@ __device__ inline void dw_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
     const uint32_t ldw = static_cast<uint32_t>(a.H);
     // FULL: byte offsets inside the tile stay below 256 * H * 4 (32 bits)
     char* tile = reinterpret_cast<char*>(a.dw + static_cast<int64_t>(v0) * a.H + h0);
-    const int hgrp = h0 + wm * (TM * 16) + 16 * (lane >> 4);  // see gather_rows
+    const bool stream = a.nk <= kDwStreamSteps;                // uniform
+    const int hgrp = h0 + wm * (TM * 16) + 8 * (lane >> 4);  // see gather_rows
     const uint32_t lane_el = static_cast<uint32_t>(wn * (TN * 16) + (lane & 15)) * ldw +
                              static_cast<uint32_t>(wm * (TM * 16) + 4 * (lane >> 4));
 #pragma unroll
@@ -1024,18 +1032,21 @@ __device__ inline void dw_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
                     pk[i & 3] = u32x2_t{T::pack2(val.x, val.y), T::pack2(val.z, val.w)};
                     if ((i & 3) == 3) {
                         gather_rows(pk);
-                        const int h16 = hgrp + (i - 3) * 16;  // 16 columns of this lane, in two chunks of 8
                         uint16_t* row = a.out + vrow[jj];
 #pragma unroll
                         for (int q = 0; q < kDwPairsPerGroup; ++q) {
-                            const int hq = h16 + 8 * q;  // H, h0 and h_min % 8 == 0: all-in or all-out
-                            if (FULL || (v_ok[jj] && hq >= h_min && hq < a.H))
-                                *reinterpret_cast<u32x4_t*>(row + hq) =
-                                    u32x4_t{pk[2 * q].x, pk[2 * q].y, pk[2 * q + 1].x, pk[2 * q + 1].y};
+                            const int hq = hgrp + (i - 3) * 16 + 32 * q;  // H, h0, h_min % 8 == 0: all-in or all-out
+                            const u32x4_t out{pk[2 * q].x, pk[2 * q].y, pk[2 * q + 1].x, pk[2 * q + 1].y};
+                            if (FULL && stream)
+                                stream_store(row + hq, 0, out);
+                            else if (FULL || (v_ok[jj] && hq >= h_min && hq < a.H))
+                                *reinterpret_cast<u32x4_t*>(row + hq) = out;
                         }
                     }
                 } else {
-                    if (FULL)
+                    if (FULL && stream)
+                        stream_store(tile + uni * 4u, lane_el * 4u, val);
+                    else if (FULL)
                         *reinterpret_cast<f32x4_t*>(tile + uni * 4u + lane_el * 4u) = val;
                     else if (mine)
                         *reinterpret_cast<f32x4_t*>(a.dw + vrow[jj] + h) = val;

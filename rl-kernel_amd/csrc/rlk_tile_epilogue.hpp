@@ -115,6 +115,21 @@ __device__ inline void mask_rows(f32x4_t (&acc)[Acc16::TM][Acc16::TN], int slab_
     }
 }
 
+// 16-byte store of results that no kernel reads soon, past the L2 (system scope and non-temporal cache policy;
+// either alone leaves the lines dirty in the L2).  Inline assembly because no builtin gives a global store both
+// bits.  The value stays of the type it has: accumulators bit-cast to integers for the operand (or for the buffer
+// store builtins) cost the forward 100 spilled registers.  The s_nop keeps the data registers one cycle beyond
+// a store of more than 8 bytes, as the compiler does for its own.
+template <class V>
+__device__ inline void stream_store(void* p, uint32_t lane_offset, V v)
+{
+    static_assert(sizeof(V) == 16, "16 bytes a lane");
+    asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 0"
+                 :
+                 : "v"(static_cast<char*>(p) + lane_offset), "v"(v)
+                 : "memory");
+}
+
 // Tiles of a launch are handed out round by round: workgroup b computes the tiles with linear ids
 // b, b + gridDim.x, b + 2 gridDim.x, ...  With a grid that is a multiple of 8, a workgroup keeps
 // its XCD from round to round, so every round forms the same L2-sharing patches as a launch with
