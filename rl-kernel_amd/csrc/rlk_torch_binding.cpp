@@ -80,7 +80,7 @@ std::vector<at::Tensor> fused_linear_logp(at::Tensor hidden, at::Tensor weight, 
 std::vector<at::Tensor> fused_linear_logp_forward_ex(at::Tensor hidden, at::Tensor weight, at::Tensor target,
                                                      c10::optional<at::Tensor> bias, double temperature,
                                                      c10::optional<int64_t> ignore_index, int64_t vocab_start,
-                                                     bool strict_targets, bool keep)
+                                                     c10::optional<bool> strict_targets, bool keep)
 {
     TORCH_CHECK(hidden.dim() == 2 && weight.dim() == 2, "hidden and weight must be 2D tensors");
     TORCH_CHECK(hidden.is_cuda() && weight.is_cuda(), "hidden and weight must be CUDA tensors");
@@ -98,7 +98,11 @@ std::vector<at::Tensor> fused_linear_logp_forward_ex(at::Tensor hidden, at::Tens
     const int32_t hd = static_cast<int32_t>(hidden.size(1));
     auto f32 = hidden.options().dtype(at::kFloat);
     auto logp = at::empty({n}, f32), lse = at::empty({n}, f32);
-    auto err = at::zeros({1}, hidden.options().dtype(at::kInt));
+    // no flag is made for a caller that does not ask for one
+    const int strict = strict_targets.value_or(false) ? 1 : 0;
+    at::Tensor err;
+    if (strict_targets.has_value()) err = at::zeros({1}, hidden.options().dtype(at::kInt));
+    int32_t* err_p = err.defined() ? err.data_ptr<int32_t>() : nullptr;
     if (n == 0) return {logp, lse, err};
     size_t ws_bytes = 0;
     TORCH_CHECK(rlk_linear_logp_fwd_workspace_bytes(n, hd, v, dt, &ws_bytes) == 0, rlk_last_error());
@@ -118,8 +122,7 @@ std::vector<at::Tensor> fused_linear_logp_forward_ex(at::Tensor hidden, at::Tens
                                                 logp.data_ptr<float>(), lse.data_ptr<float>(), ws.data_ptr(),
                                                 static_cast<size_t>(ws.numel()), n, hd, v, vocab_start, dt,
                                                 static_cast<float>(temperature), ignore_index.value_or(0),
-                                                ignore_index.has_value() ? 1 : 0, strict_targets ? 1 : 0,
-                                                err.data_ptr<int32_t>(), kept.data_ptr(), bytes, current_stream(hidden));
+                                                ignore_index.has_value() ? 1 : 0, strict, err_p, kept.data_ptr(), bytes, current_stream(hidden));
         TORCH_CHECK(rc == 0, "rlk_linear_logp_fwd_kept: ", rlk_last_error());
         return {logp, lse, err, kept};
     }
@@ -127,8 +130,7 @@ std::vector<at::Tensor> fused_linear_logp_forward_ex(at::Tensor hidden, at::Tens
                                        logp.data_ptr<float>(), lse.data_ptr<float>(), ws.data_ptr(),
                                        static_cast<size_t>(ws.numel()), n, hd, v, vocab_start, dt,
                                        static_cast<float>(temperature), ignore_index.value_or(0),
-                                       ignore_index.has_value() ? 1 : 0, strict_targets ? 1 : 0,
-                                       err.data_ptr<int32_t>(), current_stream(hidden));
+                                       ignore_index.has_value() ? 1 : 0, strict, err_p, current_stream(hidden));
     TORCH_CHECK(rc != RLK_ERR_ARG, "rlk_linear_logp_fwd: ", rlk_last_error());
     TORCH_CHECK(rc == 0, "rlk_linear_logp_fwd: ", rlk_last_error());
     return {logp, lse, err};

@@ -81,9 +81,22 @@ def grpo_from_logp_raw(cur, old, ref, adv, mask, *, clip_eps, beta, want_grad, w
             None if dkl is None else dkl.view(shape))
 
 
+def loss_upstream(dcur, dkl, beta, g_loss, g_pol, g_kl):
+    """d (what is differentiated) / d logp from ``dcur`` = d loss / d logp, ``dkl`` = d kl / d logp and
+    the gradients of ``(loss, policy, kl)``, policy = loss - beta * kl; ``None`` is zero.  A plain
+    ``loss.backward()`` is one product: the zeros for the other two outputs and their terms were eight
+    launches of the forty microseconds in which a small step has nothing else to do."""
+    if g_pol is None and g_kl is None:
+        return torch.zeros_like(dcur) if g_loss is None else dcur * g_loss
+    zero = dcur.new_zeros(())
+    g_loss, g_pol, g_kl = (zero if g is None else g for g in (g_loss, g_pol, g_kl))
+    return dcur * (g_loss + g_pol) + dkl * (g_kl - beta * g_pol)
+
+
 class _GRPOFromLogpFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, cur, old, ref, adv, mask, clip_eps, beta):
+        ctx.set_materialize_grads(False)
         out3, _, _, dcur, dkl = grpo_from_logp_raw(cur, old, ref, adv, mask, clip_eps=clip_eps,
                                                    beta=beta, want_grad=True)
         ctx.save_for_backward(dcur, dkl)
@@ -93,8 +106,8 @@ class _GRPOFromLogpFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g_loss, g_pol, g_kl):
-        dcur, dkl = ctx.saved_tensors  # d loss / d cur and d kl / d cur
-        grad = dcur * (g_loss + g_pol) + dkl * (g_kl - ctx.beta * g_pol)
+        dcur, dkl = ctx.saved_tensors
+        grad = loss_upstream(dcur, dkl, ctx.beta, g_loss, g_pol, g_kl)
         return grad.to(ctx.cur_dtype), None, None, None, None, None, None
 
 

@@ -18,6 +18,7 @@ import torch
 from .. import _native
 from ..platform import logger
 from . import linear_logp as LL
+from .grpo import loss_upstream
 
 IGNORE_INDEX = -100
 
@@ -26,7 +27,8 @@ IGNORE_INDEX = -100
 def fused_linear_logp_grpo_forward(hidden_2d, weight, target_1d, bias, old, ref, adv, mask, *,
                                    seq_len: int, clip_eps: float, beta: float,
                                    temperature: float = 1.0, ignore_index: Optional[int] = None,
-                                   want_grad: bool = True, want_terms: bool = False, keep: bool = False):
+                                   want_grad: bool = True, want_terms: bool = False, keep: bool = False,
+                                   strict_targets: Optional[bool] = True):
     """Raw launch set of ``rlk_linear_logp_fwd_grpo``; all per-token tensors are flat ``[N]``
     fp32 (``mask`` bool / uint8, ``adv`` per token ``[N]`` or per sequence ``[N / seq_len]``).
     Returns ``(logp, lse, err, out3, ratio, kl_terms, d_cur, d_kl)``, and with ``keep`` the kept logits
@@ -54,7 +56,7 @@ def fused_linear_logp_grpo_forward(hidden_2d, weight, target_1d, bias, old, ref,
         mask_u8 = mask.to(device=dev, dtype=torch.bool).contiguous().view(torch.uint8).reshape(-1)
     logp = torch.empty(n, device=dev, dtype=torch.float32)
     lse = torch.empty(n, device=dev, dtype=torch.float32)
-    err = torch.zeros(1, device=dev, dtype=torch.int32)
+    err = None if strict_targets is None else torch.zeros(1, device=dev, dtype=torch.int32)
     out3 = torch.empty(3, device=dev, dtype=torch.float32)
     new = lambda want: torch.empty(n, device=dev, dtype=torch.float32) if want else None
     ratio, klt, dcur, dkl = new(want_terms), new(want_terms), new(want_grad), new(want_grad)
@@ -68,7 +70,7 @@ def fused_linear_logp_grpo_forward(hidden_2d, weight, target_1d, bias, old, ref,
     rc = lib.rlk_linear_logp_fwd_grpo_kept(
         p(hidden_2d), p(weight), p(bias_f), p(target_1d), p(logp), p(lse), p(ws), ws.numel(), n, h, v,
         0, dt, float(temperature), 0 if ignore_index is None else int(ignore_index),
-        int(ignore_index is not None), 1, p(err), p(old_f), p(ref_f), p(adv_f), per_token,
+        int(ignore_index is not None), int(bool(strict_targets)), p(err), p(old_f), p(ref_f), p(adv_f), per_token,
         p(mask_u8), max(int(seq_len), 1), float(clip_eps), float(beta), p(out3), p(ratio), p(klt),
         p(dcur), p(dkl), p(kept), kept.numel() if keep else 0, LL._stream(dev))
     _native.check(rc, "rlk_linear_logp_fwd_grpo")
@@ -80,6 +82,7 @@ class _FusedGRPOStepFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, weight, bias, marked_ids, old, ref, adv, mask, clip_eps, beta,
                 temperature, check_targets, train=False):
+        ctx.set_materialize_grads(False)
         hidden_2d = LL._aligned_contiguous(hidden.reshape(-1, hidden.size(-1)))
         w = LL._aligned_contiguous(weight)
         target_1d = marked_ids.reshape(-1).to(device=hidden_2d.device, dtype=torch.long).contiguous()
@@ -89,7 +92,7 @@ class _FusedGRPOStepFunction(torch.autograd.Function):
         with LL._checked_targets(target_1d, w.size(0), IGNORE_INDEX, check_targets):
             logp, lse, _, out3, _, _, dcur, dkl, *kept = fused_linear_logp_grpo_forward(
                 hidden_2d, w, target_1d, bias, old, ref, adv, mask, seq_len=seq_len, clip_eps=clip_eps,
-                beta=beta, temperature=temperature, ignore_index=IGNORE_INDEX, keep=keep)
+                beta=beta, temperature=temperature, ignore_index=IGNORE_INDEX, keep=keep, strict_targets=None)
         ctx.kept = kept[0] if keep else None
         ctx.save_for_backward(hidden_2d, w, bias if bias is not None else hidden_2d, target_1d, lse,
                               dcur, dkl)
@@ -108,8 +111,7 @@ class _FusedGRPOStepFunction(torch.autograd.Function):
         hidden_2d, w, bias_t, target_1d, lse, dcur, dkl = ctx.saved_tensors
         need_h, need_w = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         need_b = ctx.has_bias and ctx.needs_input_grad[2]
-        # d loss / d logp and d kl / d logp were left by the forward; policy = loss - beta * kl
-        upstream = dcur * (g_loss + g_pol) + dkl * (g_kl - ctx.beta * g_pol)
+        upstream = loss_upstream(dcur, dkl, ctx.beta, g_loss, g_pol, g_kl)
         bias = bias_t if ctx.has_bias else None
         keys = dict(temperature=ctx.temperature, ignore_index=IGNORE_INDEX)
         kept = LL._take_kept(ctx, lambda: LL.fused_linear_logp_forward(

@@ -164,7 +164,7 @@ def fused_linear_logp_forward(
     temperature: float = 1.0,
     ignore_index: Optional[int] = None,
     vocab_start: int = 0,
-    strict_targets: bool = True,
+    strict_targets: Optional[bool] = True,
     keep: bool = False,
 ):
     """Raw forward: returns ``(logp, lse, err_flag)`` fp32 / fp32 / int32[1] device tensors.
@@ -172,7 +172,8 @@ def fused_linear_logp_forward(
 
     Stand-in for ``_C.fused_linear_logp_sm90`` (csrc/cuda/fused_linear_logp_sm90.cu:305-381 of the
     reference) with int64 global targets.  Does not synchronise; ``err_flag`` is non-zero when
-    ``strict_targets`` and some non-ignored target lies outside the weight shard.
+    ``strict_targets`` and some non-ignored target lies outside the weight shard; ``strict_targets=None``
+    (the ops, which check the ids themselves) makes no flag and returns ``None`` for it.
     """
     lib = _native.load()
     n, h = hidden_2d.shape
@@ -185,10 +186,10 @@ def fused_linear_logp_forward(
         _warn_if_wide_path(hidden_2d, weight)
         return tuple(compiled.fused_linear_logp_forward_ex(
             hidden_2d, weight, target_1d, bias, float(temperature), ignore_index, int(vocab_start),
-            bool(strict_targets), bool(keep)))
+            strict_targets, bool(keep)))
     logp = torch.empty(n, device=dev, dtype=torch.float32)
     lse = torch.empty(n, device=dev, dtype=torch.float32)
-    err = torch.zeros(1, device=dev, dtype=torch.int32)
+    err = None if strict_targets is None else torch.zeros(1, device=dev, dtype=torch.int32)
     if n == 0:  # nothing to launch
         return logp, lse, err
     _warn_if_wide_path(hidden_2d, weight)
@@ -204,14 +205,14 @@ def fused_linear_logp_forward(
             _ptr(hidden_2d), _ptr(weight), _ptr(bias_f), _ptr(target_1d), _ptr(logp), _ptr(lse),
             _ptr(ws), ws.numel(), n, h, v, int(vocab_start), dt, float(temperature),
             0 if ignore_index is None else int(ignore_index), int(ignore_index is not None),
-            int(strict_targets), _ptr(err), _ptr(kept), kept.numel(), _stream(dev))
+            int(bool(strict_targets)), _ptr(err), _ptr(kept), kept.numel(), _stream(dev))
         _native.check(rc, "rlk_linear_logp_fwd_kept")
         return logp, lse, err, kept
     rc = lib.rlk_linear_logp_fwd(
         _ptr(hidden_2d), _ptr(weight), _ptr(bias_f), _ptr(target_1d), _ptr(logp), _ptr(lse),
         _ptr(ws), ws.numel(), n, h, v, int(vocab_start), dt, float(temperature),
         0 if ignore_index is None else int(ignore_index), int(ignore_index is not None),
-        int(strict_targets), _ptr(err), _stream(dev))
+        int(bool(strict_targets)), _ptr(err), _stream(dev))
     _native.check(rc, "rlk_linear_logp_fwd")
     return logp, lse, err
 
@@ -523,7 +524,8 @@ class _FusedLinearLogpFunction(torch.autograd.Function):
         keep = ctx.keeps and _may_keep()
         with _checked_targets(target_1d, w.size(0), ignore_index, check_targets):
             logp, lse, _, *kept = fused_linear_logp_forward(
-                hidden_2d, w, target_1d, bias, temperature=temperature, ignore_index=ignore_index, keep=keep)
+                hidden_2d, w, target_1d, bias, temperature=temperature, ignore_index=ignore_index, keep=keep,
+                strict_targets=None)
         ctx.kept = kept[0] if keep else None
         ctx.save_for_backward(hidden_2d, w, bias if bias is not None else hidden_2d, target_1d, lse)
         ctx.has_bias = bias is not None
