@@ -71,6 +71,11 @@ struct AccTile {
 };
 
 using Acc16 = AccTile<16>;  // 16-bit kernels
+// 16-bit kernels of a token tile of 64 * TN_ < 256 columns: the same slab rows, fewer columns.
+template <int TN_>
+struct Acc16Few : AccTile<16> {
+    static constexpr int TN = TN_;
+};
 using Acc32 = AccTile<32>;  // fp32 matrix-core kernels
 constexpr int kTM = Acc32::TM;  // slab of the fp32 kernels in 32 x 32 tiles
 constexpr int kTN = Acc32::TN;
@@ -266,7 +271,8 @@ struct TileIO {
     }
 };
 
-template <class T, bool A_KMAJOR, bool B_KMAJOR, int BK, int WIN, bool TAIL = false, bool B_TILED = false>
+template <class T, bool A_KMAJOR, bool B_KMAJOR, int BK, int WIN, bool TAIL = false, bool B_TILED = false,
+          class AT_ = Acc16>
 struct TileGemmDtl;
 
 // Workgroup tile contraction for any K.  acc[i][j] (+)= A rows x B rows over k in [0, K).
@@ -433,7 +439,7 @@ struct KTail {
 // and by Operand::step4 per group of four; 64 lines of a K-contiguous tile lie Operand::gap bytes apart.
 template <bool KMAJOR, int ROWS, int BK, bool TAIL = false, bool TILED = false>
 struct DtlIO {
-    static_assert(BK == 64 && ROWS == 256, "direct-to-LDS layout is written for 256 x 64 tiles");
+    static_assert(BK == 64 && (ROWS == 256 || (!KMAJOR && ROWS % 64 == 0)), "direct-to-LDS layout of 256 x 64 tiles");
     static constexpr int kBytes = ROWS * BK * 2;            // 32 KiB, dense
     static constexpr int kInstr = kBytes / 1024;            // wavefront loads per tile (32)
     static constexpr int kWaves = kThreads / 64;
@@ -535,15 +541,15 @@ struct DtlIO {
 // WIN: MFMA slots (of the 32 of the second slice) over which the 8 loads of a K step are spread.
 // 32 spaces them evenly over the slice; 16 sends them all out in its first half, which the
 // persistent dZ and dH kernels prefer (they stall more on operand loads than the forward).
-template <class T, bool A_KMAJOR, bool B_KMAJOR, int BK, int WIN, bool TAIL, bool B_TILED>
+template <class T, bool A_KMAJOR, bool B_KMAJOR, int BK, int WIN, bool TAIL, bool B_TILED, class AT_>
 struct TileGemmDtl {
-    using AT = Acc16;
+    using AT = AT_;
     static constexpr int TM = AT::TM;
     static constexpr int TN = AT::TN;
     static constexpr int KK = BK / 32;
     static_assert(KK == 2, "the loop is written for two 32-wide slices per K step");
     using IOA = DtlIO<A_KMAJOR, 256, BK, TAIL>;
-    using IOB = DtlIO<B_KMAJOR, 256, BK, TAIL, B_TILED>;
+    using IOB = DtlIO<B_KMAJOR, kWN * TN * 16, BK, TAIL, B_TILED>;
     using Plan = FragPlan<TM, TN>;
     static constexpr int PA = IOA::kPasses;
     static constexpr int PB = IOB::kPasses;

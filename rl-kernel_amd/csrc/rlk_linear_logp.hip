@@ -81,15 +81,18 @@ constexpr int kKeptTile = 4 * kKeptSlab;
 // 2048 x 50257, 48 of 458 us at 1000 x 1536 x 151936.
 // CHAIN (!GENERAL, H a multiple of BK and >= 2 BK, V >= 256): all tiles run through one pipeline.
 // KEEP (CHAIN, one head): the logits stay in a.kept.
-template <class T, int BK, bool GENERAL, bool CHAIN, bool KEEP = false>
+// AT: Acc16, or with at most 192 tokens the narrower token tile of Acc16Few (CHAIN): the launch is bound by reading
+// the weight then and the products of a 256-token tile were the larger part of it.  A token's sums are taken over
+// the same rows in the same order, so its bits are those of the full tile.
+template <class T, int BK, bool GENERAL, bool CHAIN, bool KEEP = false, class AT = Acc16>
 __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
 {
     static_assert(!(GENERAL && CHAIN), "the chained variant covers full tiles only");
     static_assert(CHAIN || !KEEP, "logits are kept by the chained variant only");
-    using AT = Acc16;
+    static_assert(CHAIN || std::is_same<AT, Acc16>::value, "narrow token tiles are for the chained variant");
     constexpr int TM = AT::TM, TN = AT::TN;
     using Gemm = TileGemm<T, false, false, BK>;
-    using Dtl = TileGemmDtl<T, false, false, BK, kWinFwd>;
+    using Dtl = TileGemmDtl<T, false, false, BK, kWinFwd * TN / 4, false, false, AT>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     int tb, sp;
@@ -208,13 +211,15 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
                 mask_rows<T>(acc, wm * (TM * 16), vt * 256 - row0, lane);
                 if constexpr (KEEP) {
                     const int64_t tile = static_cast<int64_t>(tb) * a.vtiles + vt;
-                    float* dst = a.kept + tile * kKeptTile + wn * kKeptSlab + wm * (kKeptSlab / 2);
+                    float* dst = a.kept + tile * kKeptTile + wm * (kKeptSlab / 2);
 #pragma unroll
                     for (int j = 0; j < TN; ++j) {
-                        if (wn * (TN * 16) + j * 16 >= tok_valid) break;  // uniform
+                        const int cols = wn * TN + j;  // 16 tokens; four of them make a slab
+                        if (cols * 16 >= tok_valid) break;  // uniform
+                        float* quads = dst + (cols >> 2) * kKeptSlab + (cols & 3) * 256;
 #pragma unroll
                         for (int i = 0; i < TM; ++i)
-                            stream_store(dst + (i * TN + j) * 256, lane * 16, acc[i][j]);
+                            stream_store(quads + i * (Acc16::TN * 256), lane * 16, acc[i][j]);
                     }
                     counted = tok_valid == 256;
                 }
@@ -2012,31 +2017,41 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
 }
 
 // One forward contraction launch: a.row_blocks x a.n_split workgroups of the given variant.
-template <class T, bool GENERAL, bool CHAIN>
+template <class T, bool GENERAL>
 int launch_fwd_as(const FwdArgs& a, hipStream_t stream)
 {
     using G = TileGemm<T, false, false, kBK>;
-    if (int rc = set_smem(linear_logp_fwd_kernel<T, kBK, GENERAL, CHAIN>, G::kSmemBytes)) return rc;
-    hipLaunchKernelGGL((linear_logp_fwd_kernel<T, kBK, GENERAL, CHAIN>), dim3(a.row_blocks * a.n_split),
+    if (int rc = set_smem(linear_logp_fwd_kernel<T, kBK, GENERAL, false>, G::kSmemBytes)) return rc;
+    hipLaunchKernelGGL((linear_logp_fwd_kernel<T, kBK, GENERAL, false>), dim3(a.row_blocks * a.n_split),
                        dim3(kThreads), G::kSmemBytes, stream, a);
     return 0;
 }
 
-template <class T>
-int launch_fwd_kept(const FwdArgs& a, hipStream_t stream)
+// The chained variants: by the width of the token tile (tokens below a full tile only) and whether logits are kept.
+template <class T, bool KEEP, class AT>
+int launch_fwd_chained_as(const FwdArgs& a, hipStream_t stream)
 {
     using G = TileGemm<T, false, false, kBK>;
-    if (int rc = set_smem(linear_logp_fwd_kernel<T, kBK, false, true, true>, G::kSmemBytes)) return rc;
-    hipLaunchKernelGGL((linear_logp_fwd_kernel<T, kBK, false, true, true>), dim3(a.row_blocks * a.n_split),
+    if (int rc = set_smem(linear_logp_fwd_kernel<T, kBK, false, true, KEEP, AT>, G::kSmemBytes)) return rc;
+    hipLaunchKernelGGL((linear_logp_fwd_kernel<T, kBK, false, true, KEEP, AT>), dim3(a.row_blocks * a.n_split),
                        dim3(kThreads), G::kSmemBytes, stream, a);
     return 0;
 }
 
-template <bool GENERAL, bool CHAIN>
+template <class T, bool KEEP>
+int launch_fwd_chained(const FwdArgs& a, hipStream_t stream)
+{
+    if (a.N <= 64) return launch_fwd_chained_as<T, KEEP, Acc16Few<1>>(a, stream);
+    if (a.N <= 128) return launch_fwd_chained_as<T, KEEP, Acc16Few<2>>(a, stream);
+    if (a.N <= 192) return launch_fwd_chained_as<T, KEEP, Acc16Few<3>>(a, stream);
+    return launch_fwd_chained_as<T, KEEP, Acc16>(a, stream);
+}
+
+template <bool GENERAL>
 int launch_fwd(const FwdArgs& a, int32_t dtype, hipStream_t stream)
 {
-    return dtype == RLK_DTYPE_BF16 ? launch_fwd_as<Bf16, GENERAL, CHAIN>(a, stream)
-                                   : launch_fwd_as<F16, GENERAL, CHAIN>(a, stream);
+    return dtype == RLK_DTYPE_BF16 ? launch_fwd_as<Bf16, GENERAL>(a, stream)
+                                   : launch_fwd_as<F16, GENERAL>(a, stream);
 }
 
 // A second head over the same hidden states and targets (a frozen reference model).
@@ -2336,10 +2351,12 @@ int fwd_enqueue(const void* hidden, const void* weight, const float* bias, const
         a.tile_lo = 0;
         a.vtiles = plan.fast_tiles;
         a.kept = kept;
-        if (int rc = kept != nullptr ? (dtype == RLK_DTYPE_BF16 ? launch_fwd_kept<Bf16>(a, stream)
-                                                                : launch_fwd_kept<F16>(a, stream))
-                     : fwd_chained(H, V) ? launch_fwd<false, true>(a, dtype, stream)
-                                         : launch_fwd<false, false>(a, dtype, stream))
+        const bool bf16 = dtype == RLK_DTYPE_BF16;
+        if (int rc = kept != nullptr ? (bf16 ? launch_fwd_chained<Bf16, true>(a, stream)
+                                             : launch_fwd_chained<F16, true>(a, stream))
+                     : fwd_chained(H, V) ? (bf16 ? launch_fwd_chained<Bf16, false>(a, stream)
+                                                 : launch_fwd_chained<F16, false>(a, stream))
+                                         : launch_fwd<false>(a, dtype, stream))
             return rc;
     }
     if (mfma && plan.n_gen > 0) {
@@ -2347,7 +2364,7 @@ int fwd_enqueue(const void* hidden, const void* weight, const float* bias, const
         a.split_lo = plan.n_fast;
         a.tile_lo = plan.fast_tiles;
         a.vtiles = plan.gen_tiles;
-        if (int rc = launch_fwd<true, false>(a, dtype, stream)) return rc;
+        if (int rc = launch_fwd<true>(a, dtype, stream)) return rc;
     }
     if (int rc = check_launch("linear_logp_fwd_kernel launch failed")) return rc;
 

@@ -100,18 +100,18 @@ __device__ inline void add_bias(typename AT::vec (&acc)[AT::TM][AT::TN], const f
 // the softmax sum and in dZ alike.  One more product does it: A holds -inf in k = 0 of those rows, B
 // holds 1 there, everything else is zero.  (Selecting in the accumulators, on a branch or before the
 // first product, cost the forward 28 to 497 spilled registers and 2 % of its time.)
-template <class T>
-__device__ inline void mask_rows(f32x4_t (&acc)[Acc16::TM][Acc16::TN], int slab_row0, int skip, int lane)
+template <class T, int TM, int TN>
+__device__ inline void mask_rows(f32x4_t (&acc)[TM][TN], int slab_row0, int skip, int lane)
 {
     if (skip <= __builtin_amdgcn_readfirstlane(slab_row0)) return;  // uniform
     const bool k0 = lane < 16;  // lanes 0 .. 15 hold k = 0 .. 7 of an operand fragment, k = 0 in the low half
     const u32x4_t one{k0 ? static_cast<uint32_t>(T::from_float(1.f)) : 0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int i = 0; i < Acc16::TM; ++i) {
+    for (int i = 0; i < TM; ++i) {
         const bool out = k0 && slab_row0 + i * 16 + lane < skip;
         const u32x4_t low{out ? static_cast<uint32_t>(T::from_float(-INFINITY)) : 0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int j = 0; j < Acc16::TN; ++j) acc[i][j] = T::mfma(low, one, acc[i][j]);
+        for (int j = 0; j < TN; ++j) acc[i][j] = T::mfma(low, one, acc[i][j]);
     }
 }
 
