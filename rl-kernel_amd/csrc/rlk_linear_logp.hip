@@ -748,11 +748,10 @@ struct DhArgs {
 // The tile covers hidden columns [h0, h0 + 256) and owns those from h_min on (h_min > h0 for the
 // last tile of a persistent walk when H is not a multiple of 256: it is shifted back to end at H
 // and must leave the columns of its left neighbour alone).
-template <class T, bool FULL>
-__device__ inline void dh_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::TN], const DhArgs& a, int tt,
+template <class T, bool FULL, class AT = Acc16>
+__device__ inline void dh_epilogue_impl(const f32x4_t (&acc)[AT::TM][AT::TN], const DhArgs& a, int tt,
                                         int h0, int h_min, float* acc_dst, bool first, bool last)
 {
-    using AT = Acc16;
     constexpr int TM = AT::TM, TN = AT::TN;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -768,13 +767,14 @@ __device__ inline void dh_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
     char* out_tile = reinterpret_cast<char*>(a.out + origin);
     const uint32_t lane_el = static_cast<uint32_t>(wn * (TN * 16) + (lane & 15)) * ldh +
                              static_cast<uint32_t>(wm * (TM * 16) + 4 * (lane >> 4));
+    constexpr int JB = TN % 2 == 0 ? 2 : 1;
 #pragma unroll
-    for (int jb = 0; jb < TN; jb += 2) {
-        f32x4_t old[2][TM];
-        bool tok_ok[2];
-        int64_t trow[2];
+    for (int jb = 0; jb < TN; jb += JB) {
+        f32x4_t old[JB][TM];
+        bool tok_ok[JB];
+        int64_t trow[JB];
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
+        for (int jj = 0; jj < JB; ++jj) {
             const int j = jb + jj;
             const int tl = tok0 + wn * (TN * 16) + AT::col(j, lane);
             tok_ok[jj] = FULL || (tl >= tok_min && tl < a.tok_valid);
@@ -794,7 +794,7 @@ __device__ inline void dh_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
             }
         }
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
+        for (int jj = 0; jj < JB; ++jj) {
             const int j = jb + jj;
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
@@ -1105,15 +1105,18 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dw_kernel(DwArgs a)
 // slot.  The items of one range are neighbours in the list (they share dZ columns), so the part
 // is the slow index.
 // KEPT: dz is the block of kept logits that linear_logp_dz_kept_kernel has turned into dZ in place.
-template <class T, int BK, bool KEPT>
+// HT (KEPT): Acc16, or for at most 192 tokens the narrower token tile of dH (bound by reading the weight, as in
+// the forward; the bits stay).
+template <class T, int BK, bool KEPT, class HT = Acc16>
 __global__ __launch_bounds__(kThreads) void linear_logp_grads_kernel(DhArgs h, DwArgs d)
 {
+    static_assert(KEPT || std::is_same<HT, Acc16>::value, "narrow token tiles are for kept logits");
     constexpr int kTileEls = kKeptTile * 2, kSlabEls = kKeptSlab * 2;  // 16-bit elements
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    f32x4_t acc[Acc16::TM][Acc16::TN];
     const int dh_items = h.tok_tiles * h.h_tiles * h.ksplit;
     if (static_cast<int>(blockIdx.x) < dh_items) {
-        using Dtl = TileGemmDtl<T, true, false, BK, kWinDh, true, KEPT>;
+        using Dtl = TileGemmDtl<T, true, false, BK, kWinDh * HT::TN / 4, true, KEPT, HT>;
+        f32x4_t acc[HT::TM][HT::TN];
         TileWalk walk(dh_items, h.tok_tiles, h.h_tiles * h.ksplit);
         // parts are whole K steps, of kept logits whole vocab tiles (the last one is cut off at nk)
         constexpr int kUnit = KEPT ? 4 : 1;
@@ -1160,11 +1163,15 @@ __global__ __launch_bounds__(kThreads) void linear_logp_grads_kernel(DhArgs h, D
             zero_acc(acc);
             Dtl::next_steps(st, nxt.nk, tail_from(nxt));
             // a full tile's epilogue issues TM * TN unconditional stores per wavefront; half is enough
-            Dtl::template tile<true, Acc16::TM * Acc16::TN / 2>(st, w_origin(nxt), z_origin(nxt), acc, smem, counted);
+            Dtl::template tile<true, HT::TM * HT::TN / 2>(st, w_origin(nxt), z_origin(nxt), acc, smem, counted);
             const bool part = h.ksplit > 1;
-            counted = dh_epilogue<T>(acc, h, cur.tt, h_col(cur.ht), cur.ht * 256,
-                                     part ? h.part + cur.ks * h.part_stride : h.acc, part || h.first != 0,
-                                     !part && h.last != 0);
+            float* to = part ? h.part + cur.ks * h.part_stride : h.acc;
+            if constexpr (HT::TN == Acc16::TN)
+                counted = dh_epilogue<T>(acc, h, cur.tt, h_col(cur.ht), cur.ht * 256, to, part || h.first != 0,
+                                         !part && h.last != 0);
+            else
+                dh_epilogue_impl<T, false, HT>(acc, h, cur.tt, h_col(cur.ht), cur.ht * 256, to, part || h.first != 0,
+                                               !part && h.last != 0);
             if (!more) break;
             walk.advance();
             cur = nxt;
@@ -1174,6 +1181,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_grads_kernel(DhArgs h, D
     LeadWalk walk(d.v_tiles * d.h_tiles, d.v_tiles, d.h_tiles, d.busy, d.lead);
     if (!walk.valid()) return;
     using Dtl = TileGemmDtl<T, true, true, BK, kWinDw, true, KEPT>;
+    f32x4_t acc[Acc16::TM][Acc16::TN];
     int vt, ht;
     walk.coords(false, vt, ht);
     auto h_col = [&](int t) { return min(t * 256, d.H - 256); };
@@ -1647,8 +1655,8 @@ BwdPlan kept_plan(int64_t N, int H, int64_t V)
 
 // Raises the dynamic-LDS limit of `kernel` to `bytes` on the current device.  The attribute is
 // per device and sticks, so each (kernel instance, device) pair pays the runtime call once.
-template <class K>
-int set_smem(K kernel, int bytes)
+template <auto kernel>
+int set_smem(int bytes)
 {
     constexpr int kMaxDev = 64;
     static std::mutex mu;
@@ -1807,13 +1815,12 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
                        static_cast<int>(N), 1.f / c.temperature, c.dtype, scales);
     if (int rc = check_launch("scales kernel launch failed")) return rc;
 
-    if (int rc = set_smem(linear_logp_dz_kernel<T, kBK, false, true>, kDzChainSmem)) return rc;
-    if (int rc = set_smem(linear_logp_dz_kernel<T, kBK, false, false>, GZ::kSmemBytes)) return rc;
-    if (int rc = set_smem(linear_logp_dz_kernel<T, kBK, true, false>, GZ::kSmemBytes)) return rc;
-    if (int rc = set_smem(linear_logp_grads_kernel<T, kBK, false>, kChainSmem)) return rc;
-    if (int rc = set_smem(linear_logp_grads_kernel<T, kBK, true>, kChainSmem)) return rc;
-    if (int rc = set_smem(linear_logp_dh_kernel<T, kBK>, GH::kSmemBytes)) return rc;
-    if (int rc = set_smem(linear_logp_dw_kernel<T, kBK>, GW::kSmemBytes)) return rc;
+    if (int rc = set_smem<linear_logp_dz_kernel<T, kBK, false, true>>(kDzChainSmem)) return rc;
+    if (int rc = set_smem<linear_logp_dz_kernel<T, kBK, false, false>>(GZ::kSmemBytes)) return rc;
+    if (int rc = set_smem<linear_logp_dz_kernel<T, kBK, true, false>>(GZ::kSmemBytes)) return rc;
+    if (int rc = set_smem<linear_logp_grads_kernel<T, kBK, false>>(kChainSmem)) return rc;
+    if (int rc = set_smem<linear_logp_dh_kernel<T, kBK>>(GH::kSmemBytes)) return rc;
+    if (int rc = set_smem<linear_logp_dw_kernel<T, kBK>>(GW::kSmemBytes)) return rc;
 
     for (int ci = 0; ci < p.n_chunks; ++ci) {
         const int64_t tok_lo = static_cast<int64_t>(ci) * p.tok_chunk;
@@ -1985,10 +1992,17 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
                                                      grid);
                 dj.busy = split.busy;
                 dj.lead = split.lead;
-                if (c.kept)
-                    hipLaunchKernelGGL((linear_logp_grads_kernel<T, kBK, true>), dim3(grid), dim3(kThreads),
-                                       kChainSmem, stream, hj, dj);
-                else
+                auto launch_kept = [&](auto ht) -> int {
+                    constexpr auto kernel = linear_logp_grads_kernel<T, kBK, true, decltype(ht)>;
+                    if (int rc = set_smem<kernel>(kChainSmem)) return rc;
+                    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), kChainSmem, stream, hj, dj);
+                    return 0;
+                };
+                if (c.kept) {
+                    if (int rc = N <= 64 ? launch_kept(Acc16Few<1>{}) : N <= 128 ? launch_kept(Acc16Few<2>{})
+                                 : N <= 192 ? launch_kept(Acc16Few<3>{}) : launch_kept(Acc16{}))
+                        return rc;
+                } else
                     hipLaunchKernelGGL((linear_logp_grads_kernel<T, kBK, false>), dim3(grid), dim3(kThreads),
                                        kChainSmem, stream, hj, dj);
             }
@@ -2021,7 +2035,7 @@ template <class T, bool GENERAL>
 int launch_fwd_as(const FwdArgs& a, hipStream_t stream)
 {
     using G = TileGemm<T, false, false, kBK>;
-    if (int rc = set_smem(linear_logp_fwd_kernel<T, kBK, GENERAL, false>, G::kSmemBytes)) return rc;
+    if (int rc = set_smem<linear_logp_fwd_kernel<T, kBK, GENERAL, false>>(G::kSmemBytes)) return rc;
     hipLaunchKernelGGL((linear_logp_fwd_kernel<T, kBK, GENERAL, false>), dim3(a.row_blocks * a.n_split),
                        dim3(kThreads), G::kSmemBytes, stream, a);
     return 0;
@@ -2032,7 +2046,7 @@ template <class T, bool KEEP, class AT>
 int launch_fwd_chained_as(const FwdArgs& a, hipStream_t stream)
 {
     using G = TileGemm<T, false, false, kBK>;
-    if (int rc = set_smem(linear_logp_fwd_kernel<T, kBK, false, true, KEEP, AT>, G::kSmemBytes)) return rc;
+    if (int rc = set_smem<linear_logp_fwd_kernel<T, kBK, false, true, KEEP, AT>>(G::kSmemBytes)) return rc;
     hipLaunchKernelGGL((linear_logp_fwd_kernel<T, kBK, false, true, KEEP, AT>), dim3(a.row_blocks * a.n_split),
                        dim3(kThreads), G::kSmemBytes, stream, a);
     return 0;
