@@ -440,14 +440,13 @@ def bench_linear(torch, name, cfg, steps, warmup, mode="fwd+bwd", detailed=False
         elt = 2
         c, p = min(plan["tok_chunk"], n), min(plan["v_piece"], v)
         alg = {"linear_logp_dz_kernel": (c * h + p * h + c * p) * elt,
-               "linear_logp_dh_kernel": (c * p + p * h) * elt + c * h * 4,
-               "linear_logp_dw_kernel": (c * p + c * h) * elt + p * h * 4}
-        for kname, total in (("linear_logp_dz_kernel", t_h + t_w - t_all),
-                             ("linear_logp_dh_kernel", t_all - t_w),
-                             ("linear_logp_dw_kernel", t_all - t_h)):
+               # dH and dW tiles of a block in one launch
+               "linear_logp_grads_kernel": (c * p + p * h + c * h) * elt + (c * h + p * h) * 4}
+        for kname, total, products in (("linear_logp_dz_kernel", t_h + t_w - t_all, 1),
+                                       ("linear_logp_grads_kernel", 2 * t_all - t_h - t_w, 2)):
             kernels.append({"kernel": kname, "launches_per_step": blocks,
-                            "launch_ms": total / blocks, "flops_per_launch": blk_flops,
-                            "achieved": blk_flops / (total / blocks * 1e-3) / 1e12,
+                            "launch_ms": total / blocks, "flops_per_launch": products * blk_flops,
+                            "achieved": products * blk_flops / (total / blocks * 1e-3) / 1e12,
                             "algorithmic_bytes": float(alg[kname])})
         res["backward_plan"] = plan
         res["forward_plan"] = fwd_plan(n, h, v, 0 if cfg["dtype"] == "bf16" else 1)
@@ -474,7 +473,7 @@ def bench_linear(torch, name, cfg, steps, warmup, mode="fwd+bwd", detailed=False
     res["kernel_source_sha16"] = sha
     dominant = max(kernels, key=lambda k: k["launch_ms"] * k["launches_per_step"])
     res["roofline"] = dict(dominant)
-    res["roofline"]["note"] = "the kernel with the largest share of the step; see `kernels` for all four"
+    res["roofline"]["note"] = "the kernel with the largest share of the step; see `kernels` for all"
 
     if registry_op and do_bwd and not grpo:
         res["through_registry_op"] = bench_registry_op(torch, hidden, weight, targets, grad, temp, ign,

@@ -223,7 +223,7 @@ int rlk_linear_logp_bwd_typed(const float* grad_logp, const void* hidden, const 
  * rlk_linear_logp_kept_bytes: size of the buffer, N x V fp32 (of 16-bit inputs in whole 256 x 256
  * tiles), or 0 where none is kept: more than 800 MiB (so that buffer and workspace stay below 1 GB
  * whatever N is), 16-bit inputs with H % 64 != 0, H < 256 or V < 256, and heads so narrow (16 bit: H <
- * 1024, less for fewer than 256 tokens; fp32: H < 128) that the trip through memory costs what
+ * 896, less for fewer than 224 tokens; fp32: H < 128) that the trip through memory costs what
  * the products do.  Host only.
  * rlk_linear_logp_fwd_kept is rlk_linear_logp_fwd (same bits, same workspace) that also fills `kept`
  * (16-byte aligned); the layout is the library's own.  rlk_linear_logp_bwd_kept is the backward of

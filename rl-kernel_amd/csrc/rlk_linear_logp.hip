@@ -1620,14 +1620,14 @@ BwdPlan bwd_plan(int64_t N, int H, int64_t V, size_t budget)
 
 // Bytes of the kept logits, or 0 where a training forward keeps none: sizes off the chained 16-bit kernels, and
 // more than RLK_KEPT_LOGITS_BYTES, the bound that keeps the extra memory of a step below 1 GB whatever N is.
-// Narrow heads keep none either: a tile of logits costs 12 us of stores in the forward and 17 us of dZ pass
+// Narrow heads keep none either: a tile of logits costs 4 - 10 us of stores in the forward and 17 us of dZ pass
 // (proportionally less with fewer than 256 tokens, whose columns past N stay out), computing it again
-// about 1.7 us per 64 of H plus 4 (forward and dZ, kept against computed again: 1000 x 1536 x 151936 715 against
-// 957 us, 1000 x 896 x 50257 192 against 211, 1000 x 512 x 50257 154 against 138).
+// about 1.7 us per 64 of H plus 4 (forward + backward, kept against computed again: 1305 x 896 x 32768 400 against
+// 457 us, 325 x 896 x 50257 264 against 323, 2856 x 768 x 32768 636 against 625).
 size_t kept_bytes(int64_t N, int H, int64_t V, int dtype)
 {
     if (dtype == RLK_DTYPE_F32) return wide_kept_bytes(N, H, V);
-    if (!bwd_chained(H, V) || H < std::min<int64_t>(1024, 4 * N)) return 0;
+    if (!bwd_chained(H, V) || H < std::min<int64_t>(896, 4 * N)) return 0;
     const int64_t tiles = ((N + 255) / 256) * ((V + 255) / 256);
     if (tiles > static_cast<int64_t>(RLK_KEPT_LOGITS_BYTES / (kKeptTile * 4))) return 0;
     return static_cast<size_t>(tiles) * kKeptTile * 4;
