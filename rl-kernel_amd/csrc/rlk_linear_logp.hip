@@ -66,8 +66,10 @@ struct FwdArgs {
 // a slab holds the accumulator quads as the wavefronts have them,
 // [2 wavefronts along vocab][TM][TN][64 lanes][4], so a wavefront stores a tile in 1 KiB pieces.  The last token tile
 // is moved back to end at N as in the backward; columns of 16 tokens past N (fewer than 256 tokens) are not stored.
-// They are stored past the L2 (stream_store): left in it as dirty lines they cost their whole trip to memory
-// on top of the products (4096 x 2048 x 50257: 585 us without them, 774 with plain or `nt` stores, 652 so).
+// They are stored past the L2 (stream_store): forward + backward of 1500 x 4096 x 128256 4067 -> 4020 us, of 64 x
+// 4096 x 128256 730 -> 719, of 300 x 2048 x 50257 359 -> 349, of 4096 x 2048 x 50257 2252 -> 2238, of 2000 x 2560 x
+// 32000 934 -> 940.  (A forward repeated alone, whose weight stays in the memory-side cache when they bypass it,
+// goes from 774 to 655 us at 4096 x 2048 x 50257, 585 without keeping; inside a step keeping costs it 140 us.)
 constexpr int kKeptSlab = 64 * 256;       // floats
 constexpr int kKeptTile = 4 * kKeptSlab;
 
