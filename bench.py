@@ -42,14 +42,13 @@ PEAK_HBM_GBS = 8000.0
 # the kernel sources whose digest is recorded with them; with other sources `traffic` is null.
 MEASURED_TRAFFIC = {
     "workload": "llama3-8b-head",
-    "kernel_source_sha16": "91e8514c96c325e3",
-    "measured_at_commit": "e115510",
+    "kernel_source_sha16": "aea22cae80384ab4",
+    "measured_at_commit": "82a5928",
     "counter_scale": {"FETCH_SIZE": 2.000, "WRITE_SIZE": 1.000},
     "bytes_per_launch": {
-        "linear_logp_fwd_kernel": 53563219968,
-        "linear_logp_dz_kernel": 1949225984,
-        "linear_logp_dh_kernel": 1832643584,
-        "linear_logp_dw_kernel": 2112219136,
+        "linear_logp_fwd_kernel": 51297517568,
+        "linear_logp_dz_kernel": 1953206272,
+        "linear_logp_grads_kernel": 3955787776,
     },
 }
 
