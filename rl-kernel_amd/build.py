@@ -44,6 +44,45 @@ def _check_no_packed_fp32(asm_path: str, src: str) -> None:
                            f"({len(hits)}, first: {hits[0]}); the -packed-fp32-ops switch did not take effect")
 
 
+# Wait states that the hardware wants around a 16-byte store and that the compiler only provides for its own:
+# before a matrix instruction's result is stored, and before the stored registers are overwritten.
+STREAM_STORE = re.compile(r"global_store_dwordx4 v\[\d+:\d+\], ([av])\[(\d+):(\d+)\], off sc1 nt$")
+MFMA_TO_STORE = 12
+STORE_TO_WRITE = 2
+
+
+def _check_stream_stores(asm_path: str, src: str) -> int:
+    """The inline-assembly stores (stream_store) are opaque to the compiler's hazard pass: each has to be
+    followed by ``s_nop 1`` (or more) at once, and no matrix instruction may write its data within the
+    twelve wait states in front of it.  Returns how many there are."""
+    with open(asm_path) as fh:
+        lines = [line.split(";")[0].strip() for line in fh]
+    code = [line for line in lines if line and not line.startswith((".", "//"))]
+
+    def states(line):
+        return int(line.split()[1]) + 1 if line.startswith("s_nop") else 1
+
+    found = 0
+    for at, line in enumerate(code):
+        hit = STREAM_STORE.match(line)
+        if hit is None:
+            continue
+        found += 1
+        after = code[at + 1] if at + 1 < len(code) else ""
+        if not after.startswith("s_nop") or states(after) < STORE_TO_WRITE:
+            raise RuntimeError(f"{src}: '{line}' is followed by '{after}', not by s_nop 1")
+        kind, lo, hi = hit.group(1), int(hit.group(2)), int(hit.group(3))
+        passed = 0
+        for back in range(at - 1, -1, -1):
+            if passed >= MFMA_TO_STORE or code[back].endswith(":"):
+                break
+            wrote = re.match(r"v_mfma\S+ ([av])\[(\d+):(\d+)\]", code[back])
+            if wrote and wrote.group(1) == kind and int(wrote.group(2)) <= hi and int(wrote.group(3)) >= lo:
+                raise RuntimeError(f"{src}: '{line}' stores the result of '{code[back]}' after {passed} wait states")
+            passed += states(code[back])
+    return found
+
+
 BINDING_SRC = "rlk_torch_binding.cpp"
 BINDING_NAME = "_rlk_C"
 BINDING_PATH = os.path.join(LIB_DIR, BINDING_NAME + ".so")
@@ -107,6 +146,7 @@ def build(verbose: bool = False, extra_flags=()) -> str:
             print(out)
         if asm is not None:
             _check_no_packed_fp32(asm, src)
+            _check_stream_stores(asm, src)
             os.remove(asm)
     tmp = LIB_PATH + ".tmp"
     link = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs]

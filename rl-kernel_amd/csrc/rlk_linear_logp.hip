@@ -218,6 +218,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
                     for (int j = 0; j < TN; ++j) {
                         const int cols = wn * TN + j;  // 16 tokens; four of them make a slab
                         if (cols * 16 >= tok_valid) break;  // uniform
+                        settle_column(acc, j);
                         float* quads = dst + (cols >> 2) * kKeptSlab + (cols & 3) * 256;
 #pragma unroll
                         for (int i = 0; i < TM; ++i)

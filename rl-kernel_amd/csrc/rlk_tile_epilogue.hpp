@@ -115,19 +115,34 @@ __device__ inline void mask_rows(f32x4_t (&acc)[TM][TN], int slab_row0, int skip
     }
 }
 
-// 16-byte store of results that no kernel reads soon, past the L2 (system scope and non-temporal cache policy;
+// 16-byte store of results that no kernel reads soon, past the L2 (agent scope, sc1, and non-temporal cache policy;
 // either alone leaves the lines dirty in the L2).  Inline assembly because no builtin gives a global store both
 // bits.  The value stays of the type it has: accumulators bit-cast to integers for the operand (or for the buffer
-// store builtins) cost the forward 100 spilled registers.  The s_nop keeps the data registers one cycle beyond
-// a store of more than 8 bytes, as the compiler does for its own.
+// store builtins) cost the forward 100 spilled registers.
+// The compiler sees no hazards of an inline store, so both sides of it are kept here (build.py checks the device
+// code for them):
+// - behind it two wait states (s_nop 1) before a vector instruction may overwrite its data registers, as the
+//   compiler puts them behind its own stores of more than 8 bytes on this target;
+// - in front of it twelve between a matrix instruction and the store of its result: a value that no vector
+//   instruction has touched since goes through settle_column first.
 template <class V>
 __device__ inline void stream_store(void* p, uint32_t lane_offset, V v)
 {
     static_assert(sizeof(V) == 16, "16 bytes a lane");
-    asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 0"
+    asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1"
                  :
                  : "v"(static_cast<char*>(p) + lane_offset), "v"(v)
                  : "memory");
+}
+
+// The matrix instructions that write column j of the accumulators are done: sixteen wait states, tied to the
+// registers so that none of them moves behind.
+template <int TN>
+__device__ inline void settle_column(f32x4_t (&acc)[8][TN], int j)
+{
+    asm volatile("s_nop 15"
+                 : "+v"(acc[0][j]), "+v"(acc[1][j]), "+v"(acc[2][j]), "+v"(acc[3][j]), "+v"(acc[4][j]),
+                   "+v"(acc[5][j]), "+v"(acc[6][j]), "+v"(acc[7][j]));
 }
 
 // Tiles of a launch are handed out round by round: workgroup b computes the tiles with linear ids
