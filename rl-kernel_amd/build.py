@@ -83,6 +83,21 @@ def _check_stream_stores(asm_path: str, src: str) -> int:
     return found
 
 
+def _check_m0_loads(asm_path: str, src: str) -> int:
+    """A load to LDS takes its destination from M0, and one wait state has to lie between a scalar write of M0
+    and the load; in inline assembly nothing provides it.  Returns how many such loads there are."""
+    with open(asm_path) as fh:
+        lines = [line.split(";")[0].strip() for line in fh]
+    code = [line for line in lines if line and not line.startswith((".", "//"))]
+    found = 0
+    for before, line in zip([""] + code, code):
+        if re.match(r"(global|buffer|scratch)_load_(lds_|\S+.*\blds\b)", line):
+            found += 1
+            if re.match(r"s_\S+ m0,", before):
+                raise RuntimeError(f"{src}: '{line}' follows '{before}' without a wait state")
+    return found
+
+
 BINDING_SRC = "rlk_torch_binding.cpp"
 BINDING_NAME = "_rlk_C"
 BINDING_PATH = os.path.join(LIB_DIR, BINDING_NAME + ".so")
@@ -147,6 +162,7 @@ def build(verbose: bool = False, extra_flags=()) -> str:
         if asm is not None:
             _check_no_packed_fp32(asm, src)
             _check_stream_stores(asm, src)
+            _check_m0_loads(asm, src)
             os.remove(asm)
     tmp = LIB_PATH + ".tmp"
     link = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs]

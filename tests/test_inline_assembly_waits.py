@@ -1,4 +1,4 @@
-"""Wait states around the inline-assembly stores, which the compiler's hazard pass does not see."""
+"""Wait states around inline assembly, which the compiler's hazard pass does not see."""
 
 import importlib
 import os
@@ -29,15 +29,42 @@ def builder():
     return importlib.import_module("rl_kernel_amd.build")
 
 
-def test_stores_of_accumulators_keep_their_distances(builder, tmp_path):
+def device_code(builder, tmp_path, text):
     src, asm = tmp_path / "probe.hip", tmp_path / "probe.s"
-    text = PROBE.format(csrc=builder.CSRC)
-    src.write_text(text)
+    src.write_text(text.format(csrc=builder.CSRC))
     res = subprocess.run([builder.hipcc(), *builder.HIPCC_FLAGS, "--cuda-device-only", "-S", str(src), "-o", str(asm),
                           f"-I{builder.CSRC}", f"-I{os.path.dirname(builder.HERE)}/include"],
                          capture_output=True, text=True)
     assert res.returncode == 0, res.stderr[-2000:]
-    assert builder._check_stream_stores(str(asm), "probe") == 8
+    return str(asm)
+
+
+def test_stores_of_accumulators_keep_their_distances(builder, tmp_path):
+    assert builder._check_stream_stores(device_code(builder, tmp_path, PROBE), "probe") == 8
+
+
+LOAD_PROBE = """
+#include "{csrc}/rlk_gemm.hpp"
+
+__global__ __launch_bounds__(512) void probe(const uint16_t* a, float* out)
+{{
+    __shared__ __attribute__((aligned(16))) char tile[32768];
+    rlk::DtlIO<false, 256, 64> io;
+    io.init(rlk::Operand{{a, 64, 256}}, 64);
+    for (int p = 0; p < decltype(io)::kPasses; ++p) io.load_one(0, tile, p);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    out[threadIdx.x] = reinterpret_cast<float*>(tile)[threadIdx.x];
+}}
+"""
+
+
+def test_loads_to_lds_wait_for_their_destination(builder, tmp_path):
+    assert builder._check_m0_loads(device_code(builder, tmp_path, LOAD_PROBE), "probe") == 4
+    short = tmp_path / "short.s"
+    short.write_text("\ts_mov_b32 m0, s4\n\tglobal_load_lds_dwordx4 v2, s[0:1]\n")
+    with pytest.raises(RuntimeError):
+        builder._check_m0_loads(str(short), "short")
 
 
 STORE = "\tglobal_store_dwordx4 v[0:1], v[8:11], off sc1 nt\n"
