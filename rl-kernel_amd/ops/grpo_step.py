@@ -114,7 +114,7 @@ class _FusedGRPOStepFunction(torch.autograd.Function):
         upstream = loss_upstream(dcur, dkl, ctx.beta, g_loss, g_pol, g_kl)
         bias = bias_t if ctx.has_bias else None
         keys = dict(temperature=ctx.temperature, ignore_index=IGNORE_INDEX)
-        kept = LL._take_kept(ctx, lambda: LL.fused_linear_logp_forward(
+        kept = LL._take_kept(ctx, hidden_2d, w, lambda: LL.fused_linear_logp_forward(
             hidden_2d, w, target_1d, bias, keep=True, **keys)[3])
         d_h, d_w, d_b = LL.fused_linear_logp_backward(
             upstream, hidden_2d, w, target_1d, lse, bias, need_hidden=need_h, need_weight=need_w,

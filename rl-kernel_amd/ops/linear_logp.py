@@ -495,12 +495,16 @@ def fused_linear_logp_backward(
     return d_hidden, d_weight, d_bias
 
 
-def _take_kept(ctx, again):
+def _take_kept(ctx, hidden_2d, weight, again):
     """The kept logits for one backward, or ``None`` for sizes that keep none.  The backward overwrites them, so
     the context gives them up; a second backward, or one behind a forward that was not allowed to keep
-    them, makes them again (``again()``) so that its sums are grouped alike and its bits the same."""
+    them, makes them again (``again()``) so that its sums are grouped alike and its bits the same.  An unpack
+    hook may return the saved matrices off the 16-byte boundary that the forward had: no logits are kept
+    for such, and the backward runs on the kernels that take them."""
     kept, ctx.kept = ctx.kept, None
-    return again() if kept is None and ctx.keeps else kept
+    if not ctx.keeps or _kept_bytes(hidden_2d, weight) == 0:
+        return None
+    return again() if kept is None else kept
 
 
 class _FusedLinearLogpFunction(torch.autograd.Function):
@@ -570,7 +574,8 @@ class _FusedLinearLogpFunction(torch.autograd.Function):
                 b_buf = torch.zeros(w.size(0), device=w.device, dtype=torch.float32)
         bias = bias_t if ctx.has_bias else None
         keys = dict(temperature=ctx.temperature, ignore_index=ctx.ignore_index)
-        kept = _take_kept(ctx, lambda: fused_linear_logp_forward(hidden_2d, w, target_1d, bias, keep=True, **keys)[3])
+        kept = _take_kept(ctx, hidden_2d, w, lambda: fused_linear_logp_forward(
+            hidden_2d, w, target_1d, bias, keep=True, **keys)[3])
         d_h, d_w, d_b = fused_linear_logp_backward(
             grad_logp, hidden_2d, w, target_1d, lse, bias, need_hidden=need_h, need_weight=want_w, need_bias=want_b,
             weight_grad_out=w_buf, bias_grad_out=b_buf, accumulate=adding, typed_weight=w_out is None, kept=kept, **keys)
@@ -630,7 +635,7 @@ class _FusedNormLinearLogpFunction(torch.autograd.Function):
         if not (need_x and need_w):  # fewer gradients wanted than when the forward ran
             ctx.kept = None
         else:
-            kept = _take_kept(ctx, lambda: fused_norm_linear_logp_forward(
+            kept = _take_kept(ctx, x_2d, w, lambda: fused_norm_linear_logp_forward(
                 x_2d, g, w, target_1d, bias, keep=True, **keys)[3])
         d_x, d_g, d_w, d_b = fused_norm_linear_logp_backward(
             grad_logp, x_2d, g, w, target_1d, lse, bias, need_x=need_x,
