@@ -231,6 +231,9 @@ int rlk_linear_logp_bwd_typed(const float* grad_logp, const void* hidden, const 
  * d_weight (fp32, with `accumulate` as in rlk_linear_logp_bwd_accum) or d_weight_typed (the type
  * of `weight`, as in rlk_linear_logp_bwd_typed), not both; any gradient may be NULL.  Values are those
  * of rlk_linear_logp_bwd, whose fp32 sums are grouped by its dZ blocks.
+ * kept == NULL (kept_bytes 0): the logits are computed again and the gradients have the same bits, for a second
+ * backward or behind a forward that kept none; the workspace then holds dZ (16-bit inputs: 2 bytes a logit) and
+ * its size comes from rlk_linear_logp_bwd_as_kept_workspace_bytes.
  * ------------------------------------------------------------------------------------------ */
 int rlk_linear_logp_kept_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes);
 
@@ -243,6 +246,9 @@ int rlk_linear_logp_fwd_kept(const void* hidden, const void* weight, const float
 
 int rlk_linear_logp_bwd_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype,
                                              size_t* bytes);
+
+int rlk_linear_logp_bwd_as_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype,
+                                                size_t* bytes);
 
 int rlk_linear_logp_bwd_kept(const float* grad_logp, const void* hidden, const void* weight,
                              const float* bias, const int64_t* targets, const float* lse,
@@ -323,7 +329,11 @@ int rlk_linear_logp_rmsnorm_fwd_kept(const void* x, const float* gain, float eps
 int rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype,
                                                      size_t* bytes);
 
-/* d_x and d_weight_typed as in rlk_linear_logp_rmsnorm_bwd_typed: both are written. */
+int rlk_linear_logp_rmsnorm_bwd_as_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype,
+                                                        size_t* bytes);
+
+/* d_x and d_weight_typed as in rlk_linear_logp_rmsnorm_bwd_typed: both are written.  kept == NULL as in
+ * rlk_linear_logp_bwd_kept. */
 int rlk_linear_logp_rmsnorm_bwd_kept(const float* grad_logp, const void* x, const float* gain,
                                      float eps, const void* weight, const float* bias,
                                      const int64_t* targets, const float* lse, void* d_x,

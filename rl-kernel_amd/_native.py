@@ -45,6 +45,7 @@ SIGNATURES = {
     "rlk_linear_logp_fwd_kept": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i64, _i32, _i64,
                                             _i64, _i32, _f32, _i64, _i32, _i32, _vp, _vp, _sz, _vp]),
     "rlk_linear_logp_bwd_kept_workspace_bytes": (_c.c_int, [_i64, _i32, _i64, _i32, _c.POINTER(_sz)]),
+    "rlk_linear_logp_bwd_as_kept_workspace_bytes": (_c.c_int, [_i64, _i32, _i64, _i32, _c.POINTER(_sz)]),
     "rlk_linear_logp_bwd_kept": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp,
                                             _sz, _i64, _i32, _i64, _i64, _i32, _f32, _i64, _i32, _i32,
                                             _vp]),
@@ -53,6 +54,8 @@ SIGNATURES = {
                                                     _i32, _vp, _vp, _sz, _vp]),
     "rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes": (_c.c_int, [_i64, _i32, _i64, _i32,
                                                                     _c.POINTER(_sz)]),
+    "rlk_linear_logp_rmsnorm_bwd_as_kept_workspace_bytes": (_c.c_int, [_i64, _i32, _i64, _i32,
+                                                                       _c.POINTER(_sz)]),
     "rlk_linear_logp_rmsnorm_bwd_kept": (_c.c_int, [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                                     _vp, _vp, _sz, _vp, _sz, _i64, _i32, _i64, _i64,
                                                     _i32, _f32, _i64, _i32, _vp]),

@@ -36,7 +36,7 @@ int wide_fwd_partials(const void* hidden, const void* weight, const float* bias,
                       float* kept = nullptr);
 // Kept logits of fp32 inputs: [N][V rounded up to 4], see rlk_linear_logp_fwd_kept.
 size_t wide_kept_bytes(int64_t N, int32_t H, int64_t V);
-size_t wide_bwd_kept_workspace(int64_t N, int32_t H, int64_t V);
+size_t wide_bwd_kept_workspace(int64_t N, int32_t H, int64_t V, bool again);
 int wide_bwd_kept(const float* grad_logp, const void* hidden, const void* weight, const float* bias,
                   const int64_t* targets, const float* lse, void* d_hidden, float* d_weight, float* d_bias,
                   float* kept, void* workspace, int64_t N, int32_t H, int64_t V, int64_t vocab_start,

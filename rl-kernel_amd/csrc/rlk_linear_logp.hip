@@ -740,6 +740,7 @@ struct DhArgs {
     int nk;               // K steps (of 64 vocab rows) of the piece, the shifted tile's among them;
     KTail tail;           //      0: the block has no shifted tiles, K runs over [0, v_valid)
     int v_tiles;          // KEPT: vocab tiles of the block
+    int unit;             // !KEPT: K steps that a part is a multiple of
     int tok_shift;        // rows by which the last token tile is moved back
 };
 
@@ -1121,9 +1122,10 @@ __global__ __launch_bounds__(kThreads) void linear_logp_grads_kernel(DhArgs h, D
         using Dtl = TileGemmDtl<T, true, false, BK, kWinDh * HT::TN / 4, true, KEPT, HT>;
         f32x4_t acc[HT::TM][HT::TN];
         TileWalk walk(dh_items, h.tok_tiles, h.h_tiles * h.ksplit);
-        // parts are whole K steps, of kept logits whole vocab tiles (the last one is cut off at nk)
-        constexpr int kUnit = KEPT ? 4 : 1;
-        const int units = (h.nk + kUnit - 1) / kUnit;
+        // parts are whole K steps, of a block of kept logits (or of one that takes its place) whole vocab tiles
+        // (the last one is cut off at nk)
+        const int unit = KEPT ? 4 : h.unit;
+        const int units = (h.nk + unit - 1) / unit;
         const int base = units / h.ksplit, extra = units % h.ksplit;
         struct Item {
             int tt, ht, ks, step0, nk;
@@ -1137,9 +1139,8 @@ __global__ __launch_bounds__(kThreads) void linear_logp_grads_kernel(DhArgs h, D
                 it.ht -= it.ks * h.h_tiles;
             }
             // the first `extra` parts take one unit more
-            it.step0 = (it.ks * base + min(it.ks, extra)) * kUnit;
-            it.nk = (base + (it.ks < extra ? 1 : 0)) * kUnit;
-            if (KEPT) it.nk = min(it.nk, h.nk - it.step0);
+            it.step0 = (it.ks * base + min(it.ks, extra)) * unit;
+            it.nk = min((base + (it.ks < extra ? 1 : 0)) * unit, h.nk - it.step0);
             return it;
         };
         // first hidden column of h tile `t`: the last tile is shifted back so that it ends at H
@@ -1262,6 +1263,24 @@ __global__ __launch_bounds__(256) void linear_logp_db_partial_kernel(const uint1
 #pragma unroll
     for (int r = 1; r < 8; ++r) acc += red[r][threadIdx.x];
     part[static_cast<int64_t>(blockIdx.y) * part_ld + blockIdx.x * 256 + threadIdx.x] = acc;
+}
+
+// Level 1 of a block that takes the place of kept logits: sums per slab of 64 tokens in the order of
+// linear_logp_dz_kept_kernel (rows r and r + 32, then r ascending).  One column per thread.
+template <class T>
+__global__ __launch_bounds__(256) void linear_logp_db_slab_kernel(const uint16_t* dz, int64_t ldz, int rows, float* part,
+                                                                  int64_t part_ld)
+{
+    const int col = blockIdx.x * 256 + threadIdx.x, first = (blockIdx.y & 3) * 64;
+    const uint16_t* p = dz + static_cast<int64_t>(blockIdx.y) * 64 * ldz + col;
+    float acc = 0.f;
+#pragma unroll 8
+    for (int r = 0; r < 32; ++r) {
+        const float lo = first + r < rows ? T::to_float(p[r * ldz]) : 0.f;
+        const float hi = first + r + 32 < rows ? T::to_float(p[(r + 32) * ldz]) : 0.f;
+        acc = r == 0 ? lo + hi : acc + (lo + hi);
+    }
+    part[blockIdx.y * part_ld + col] = acc;
 }
 
 // Level 2: the token tiles (slabs) of the block in ascending order, times 1 / loss_scale.
@@ -1436,6 +1455,7 @@ struct BwdPlan {
     size_t part_bytes;
     size_t db_bytes;
     size_t pad_bytes;  // rows of one token tile when there are fewer tokens than that
+    bool whole;        // kept_plan: dH parts in whole vocab tiles, d_bias by slabs of 64 tokens
     size_t scales_off, dz_off, acc_off, part_off, db_off, pad_off, total;
 };
 
@@ -1604,7 +1624,7 @@ BwdPlan bwd_plan(int64_t N, int H, int64_t V, size_t budget)
     const Best& best = chained && joint.cost * 1025 < sep.joint * 1000 ? joint : sep;
     const int64_t best_ct = best.ct, best_pt = best.pt;
 
-    BwdPlan p;
+    BwdPlan p{};
     p.tok_chunk = static_cast<int>(best_ct) * 256;
     p.v_piece = static_cast<int>(best_pt) * 256;
     p.n_chunks = static_cast<int>((n_t + best_ct - 1) / best_ct);
@@ -1654,17 +1674,21 @@ size_t kept_bytes(int64_t N, int H, int64_t V, int dtype)
     return static_cast<size_t>(tiles) * kKeptTile * 4;
 }
 
-// Backward from kept logits: one block of the whole problem, dZ in the place of the logits.
-BwdPlan kept_plan(int64_t N, int H, int64_t V)
+// Backward from kept logits: one block of the whole problem, dZ in the place of the logits.  again: none were kept
+// (or they are used up); dZ is computed into the workspace, 2 bytes a logit, and every sum is grouped as with them.
+BwdPlan kept_plan(int64_t N, int H, int64_t V, bool again)
 {
     const int64_t n_t = (N + 255) / 256, v_t = (V + 255) / 256, ht = (H + 255) / 256;
     BwdPlan p{};
     p.tok_chunk = static_cast<int>(n_t) * 256;
     p.v_piece = static_cast<int>(v_t) * 256;
     p.n_chunks = p.n_pieces = 1;
+    p.whole = true;
     p.ldz = p.v_piece;
     p.ksplit = dh_cuts(n_t, v_t, ht);
-    p.part_off = 256;
+    p.dz_off = 256;
+    p.dz_bytes = again ? static_cast<size_t>(n_t) * v_t * 131072 : 0;
+    p.part_off = p.dz_off + p.dz_bytes;
     p.part_bytes = p.ksplit > 1 ? static_cast<size_t>(p.ksplit) * n_t * 256 * H * 4 : 0;
     p.db_off = p.part_off + align_up(p.part_bytes, 256);
     p.db_bytes = static_cast<size_t>(4) * n_t * p.v_piece * 4;  // column sums per slab of 64 tokens
@@ -1725,13 +1749,13 @@ bool use_mfma(const void* hidden, const void* weight, int32_t H, int dtype)
            (reinterpret_cast<uintptr_t>(hidden) & 15) == 0 && (reinterpret_cast<uintptr_t>(weight) & 15) == 0;
 }
 
-// A buffer for kept logits as the forward or the backward is given it.
+// A buffer for kept logits as the forward or the backward is given it (null: the backward computes them again).
 int check_kept(const void* kept, size_t bytes, bool mfma, int64_t N, int32_t H, int64_t V, int dtype)
 {
     const size_t need = kept_bytes(N, H, V, dtype);
     if ((!mfma && dtype != RLK_DTYPE_F32) || need == 0)
         return rlk_fail(RLK_ERR_UNSUPPORTED, "no logits are kept for these sizes (rlk_linear_logp_kept_bytes)");
-    if (bytes < need || (reinterpret_cast<uintptr_t>(kept) & 15) != 0)
+    if (kept != nullptr && (bytes < need || (reinterpret_cast<uintptr_t>(kept) & 15) != 0))
         return rlk_fail(RLK_ERR_ARG, "kept logits: buffer too small or not 16-byte aligned");
     return 0;
 }
@@ -1781,7 +1805,7 @@ struct BwdCall {
     int accumulate;  // 1: d_weight / d_bias already hold the sums of earlier tokens, add to them
     void* d_weight_cast;  // [V][H] of the weight's type or null: the finished d_weight sum goes here and
                           // d_weight only holds the running sums of earlier chunks
-    float* kept;          // logits that the forward left (the plan is then kept_plan), or null
+    float* kept;          // logits that the forward left (the plan is then kept_plan), or null: computed again
 };
 
 // Grid of a chained launch: one workgroup per compute unit, rounded down to a multiple of 8 so
@@ -1911,6 +1935,7 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
             h.part_stride = static_cast<int64_t>(tok_tiles) * 256 * H;
             const bool dh_chain = shifted || (ksplit == 1 && H >= 256 && v_valid % kBK == 0 && v_valid >= 2 * kBK);
             h.nk = shifted ? k_steps(v_valid, v_shift) : (dh_chain ? v_valid / kBK : 0);
+            h.unit = p.whole ? 4 : 1;
             h.tok_shift = tok_shift;
             h.v_tiles = v_tiles;
             h.tail = KTail();
@@ -2037,13 +2062,17 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
                 hipLaunchKernelGGL((linear_logp_dw_kernel<T, kBK>), dim3(v_tiles * h_tiles), dim3(kThreads),
                                    GW::kSmemBytes, stream, d);
             if (c.d_bias != nullptr) {
-                if (!c.kept)
+                const int rows = padded ? static_cast<int>(N) : 256;
+                if (p.whole && !c.kept)
+                    hipLaunchKernelGGL(linear_logp_db_slab_kernel<T>, dim3(v_tiles, 4 * tok_tiles), dim3(256), 0,
+                                       stream, dz, p.ldz, rows, db_part, static_cast<int64_t>(p.v_piece));
+                else if (!c.kept)
                     hipLaunchKernelGGL(linear_logp_db_partial_kernel<T>, dim3(v_tiles, tok_tiles), dim3(256), 0,
-                                       stream, dz, p.ldz, padded ? static_cast<int>(N) : 256, db_part,
-                                       static_cast<int64_t>(p.v_piece));
+                                       stream, dz, p.ldz, rows, db_part, static_cast<int64_t>(p.v_piece));
                 hipLaunchKernelGGL(linear_logp_db_finish_kernel, dim3((v_valid + 255) / 256), dim3(256), 0,
                                    stream, db_part, static_cast<int64_t>(p.v_piece),
-                                   c.kept ? 4 * tok_tiles : tok_tiles, v_valid, v_shift, scales, c.d_bias + v_lo, (ci > 0 || c.accumulate != 0) ? 1 : 0);
+                                   p.whole ? 4 * tok_tiles : tok_tiles, v_valid, v_shift, scales, c.d_bias + v_lo,
+                                   (ci > 0 || c.accumulate != 0) ? 1 : 0);
             }
             if (int rc = check_launch("linear_logp backward launch failed")) return rc;
         }
@@ -2523,7 +2552,14 @@ int rlk_linear_logp_bwd_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, in
     if (!bytes || N <= 0 || V <= 0 || H <= 0) return rlk_fail(RLK_ERR_ARG, "bad workspace query");
     if (kept_bytes(N, H, V, dtype) == 0)
         return rlk_fail(RLK_ERR_UNSUPPORTED, "no logits are kept for these sizes (rlk_linear_logp_kept_bytes)");
-    *bytes = dtype == RLK_DTYPE_F32 ? wide_bwd_kept_workspace(N, H, V) : kept_plan(N, H, V).total;
+    *bytes = dtype == RLK_DTYPE_F32 ? wide_bwd_kept_workspace(N, H, V, false) : kept_plan(N, H, V, false).total;
+    return 0;
+}
+
+int rlk_linear_logp_bwd_as_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes)
+{
+    if (int rc = rlk_linear_logp_bwd_kept_workspace_bytes(N, H, V, dtype, bytes)) return rc;
+    *bytes = dtype == RLK_DTYPE_F32 ? wide_bwd_kept_workspace(N, H, V, true) : kept_plan(N, H, V, true).total;
     return 0;
 }
 
@@ -2536,7 +2572,8 @@ int rlk_linear_logp_bwd_kept(const float* grad_logp, const void* hidden, const v
 {
     if (int rc = check_common(N, H, V, dtype)) return rc;
     if (!(temperature > 0.f)) return rlk_fail(RLK_ERR_ARG, "temperature must be greater than zero");
-    if (!grad_logp || !hidden || !weight || !targets || !lse || !kept) return rlk_fail(RLK_ERR_ARG, "null pointer");
+    if (!grad_logp || !hidden || !weight || !targets || !lse) return rlk_fail(RLK_ERR_ARG, "null pointer");
+    if (kept == nullptr && kept_size != 0) return rlk_fail(RLK_ERR_ARG, "no kept logits and a size of them");
     if (!d_hidden && !d_weight && !d_bias && !d_weight_typed)
         return rlk_fail(RLK_ERR_ARG, "no gradient requested");
     if (bias == nullptr && d_bias != nullptr) return rlk_fail(RLK_ERR_ARG, "d_bias given without bias");
@@ -2545,7 +2582,9 @@ int rlk_linear_logp_bwd_kept(const float* grad_logp, const void* hidden, const v
         return rlk_fail(RLK_ERR_ARG, "d_weight_typed takes no fp32 d_weight beside it and starts on a 16-byte boundary");
     if (int rc = check_kept(kept, kept_size, use_mfma(hidden, weight, H, dtype), N, H, V, dtype)) return rc;
     size_t need = 0;
-    if (int rc = rlk_linear_logp_bwd_kept_workspace_bytes(N, H, V, dtype, &need)) return rc;
+    if (int rc = kept ? rlk_linear_logp_bwd_kept_workspace_bytes(N, H, V, dtype, &need)
+                      : rlk_linear_logp_bwd_as_kept_workspace_bytes(N, H, V, dtype, &need))
+        return rc;
     if (!workspace || workspace_bytes < need) return rlk_fail(RLK_ERR_ARG, "workspace too small");
     if (reinterpret_cast<uintptr_t>(workspace) & 255)
         return rlk_fail(RLK_ERR_ARG, "workspace must be 256-byte aligned");
@@ -2554,7 +2593,7 @@ int rlk_linear_logp_bwd_kept(const float* grad_logp, const void* hidden, const v
                              d_weight_typed ? static_cast<float*>(d_weight_typed) : d_weight, d_bias,
                              static_cast<float*>(kept), workspace, N, H, V, vocab_start, temperature, ignore_index,
                              use_ignore, accumulate != 0 ? 1 : 0, stream);
-    const BwdPlan p = kept_plan(N, H, V);
+    const BwdPlan p = kept_plan(N, H, V, kept == nullptr);
     int n_cu = 0;
     if (int rc = compute_units(&n_cu)) return rc;
     BwdCall c{grad_logp, hidden, weight, bias, targets, lse, d_hidden, d_weight, d_bias, workspace, N, H, V, vocab_start,

@@ -649,6 +649,16 @@ int rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(int64_t N, int32_t H, int64
     return 0;
 }
 
+int rlk_linear_logp_rmsnorm_bwd_as_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes)
+{
+    size_t kept = 0, again = 0;
+    if (int rc = rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(N, H, V, dtype, bytes)) return rc;
+    if (int rc = rlk_linear_logp_bwd_kept_workspace_bytes(N, H, V, dtype, &kept)) return rc;
+    if (int rc = rlk_linear_logp_bwd_as_kept_workspace_bytes(N, H, V, dtype, &again)) return rc;
+    *bytes += again - kept;
+    return 0;
+}
+
 int rlk_linear_logp_rmsnorm_bwd_kept(const float* grad_logp, const void* x, const float* gain, float eps,
                                      const void* weight, const float* bias, const int64_t* targets,
                                      const float* lse, void* d_x, float* d_gain, void* d_weight_typed,
@@ -660,7 +670,9 @@ int rlk_linear_logp_rmsnorm_bwd_kept(const float* grad_logp, const void* x, cons
     if (int rc = check_norm(x, gain, N, H, dtype)) return rc;
     if (!d_x || !d_weight_typed) return rlk_fail(RLK_ERR_ARG, "d_x and d_weight are both written");
     size_t need = 0;
-    if (int rc = rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(N, H, V, dtype, &need)) return rc;
+    if (int rc = kept ? rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(N, H, V, dtype, &need)
+                      : rlk_linear_logp_rmsnorm_bwd_as_kept_workspace_bytes(N, H, V, dtype, &need))
+        return rc;
     if (!workspace || workspace_bytes < need) return rlk_fail(RLK_ERR_ARG, "workspace too small");
     if (reinterpret_cast<uintptr_t>(workspace) & 255)
         return rlk_fail(RLK_ERR_ARG, "workspace must be 256-byte aligned");

@@ -141,7 +141,7 @@ std::vector<at::Tensor> fused_linear_logp_forward_ex(at::Tensor hidden, at::Tens
 // receive (accumulate: are added) the gradients and are what the call returns in their place.
 // typed_weight: d_weight is a fresh tensor of the weight's type (rlk_linear_logp_bwd_typed).
 // kept: logits that the forward kept for this call, overwritten (rlk_linear_logp_bwd_kept; dz_budget_bytes has
-// no part in it).
+// no part in it).  as_kept: none were kept, the same bits from logits computed again.
 std::vector<at::Tensor> fused_linear_logp_backward(at::Tensor grad_logp, at::Tensor hidden, at::Tensor weight,
                                                    at::Tensor target, at::Tensor lse,
                                                    c10::optional<at::Tensor> bias, double temperature,
@@ -150,7 +150,7 @@ std::vector<at::Tensor> fused_linear_logp_backward(at::Tensor grad_logp, at::Ten
                                                    int64_t dz_budget_bytes,
                                                    c10::optional<at::Tensor> weight_grad_out,
                                                    c10::optional<at::Tensor> bias_grad_out, bool accumulate,
-                                                   bool typed_weight, c10::optional<at::Tensor> kept)
+                                                   bool typed_weight, c10::optional<at::Tensor> kept, bool as_kept)
 {
     TORCH_CHECK(hidden.dim() == 2 && weight.dim() == 2, "hidden and weight must be 2D tensors");
     TORCH_CHECK(hidden.is_cuda() && weight.is_cuda(), "hidden and weight must be CUDA tensors");
@@ -191,15 +191,18 @@ std::vector<at::Tensor> fused_linear_logp_backward(at::Tensor grad_logp, at::Ten
         bias_p = bias_f.data_ptr<float>();
     }
     size_t ws_bytes = 0;
-    if (kept.has_value() && kept->defined()) {
-        TORCH_CHECK(rlk_linear_logp_bwd_kept_workspace_bytes(n, hd, v, dt, &ws_bytes) == 0, rlk_last_error());
+    const bool from_kept = kept.has_value() && kept->defined();
+    if (from_kept || as_kept) {
+        const auto kept_query = from_kept ? rlk_linear_logp_bwd_kept_workspace_bytes
+                                          : rlk_linear_logp_bwd_as_kept_workspace_bytes;
+        TORCH_CHECK(kept_query(n, hd, v, dt, &ws_bytes) == 0, rlk_last_error());
         auto ws = at::empty({static_cast<int64_t>(ws_bytes)}, hidden.options().dtype(at::kByte));
         const int rc = rlk_linear_logp_bwd_kept(
             g.data_ptr<float>(), hidden.data_ptr(), weight.data_ptr(), bias_p, target.data_ptr<int64_t>(),
             lse.data_ptr<float>(), d_hidden.defined() ? d_hidden.data_ptr() : nullptr,
             d_weight.defined() && !typed_weight ? d_weight.data_ptr<float>() : nullptr,
             typed_weight ? d_weight.data_ptr() : nullptr, d_bias.defined() ? d_bias.data_ptr<float>() : nullptr,
-            kept->data_ptr(), static_cast<size_t>(kept->numel()), ws.data_ptr(), static_cast<size_t>(ws.numel()), n, hd,
+            from_kept ? kept->data_ptr() : nullptr, from_kept ? static_cast<size_t>(kept->numel()) : 0, ws.data_ptr(), static_cast<size_t>(ws.numel()), n, hd,
             v, vocab_start, dt, static_cast<float>(temperature), ignore_index.value_or(0),
             ignore_index.has_value() ? 1 : 0, accumulate ? 1 : 0, current_stream(hidden));
         TORCH_CHECK(rc == 0, "rlk_linear_logp_bwd_kept: ", rlk_last_error());
@@ -325,7 +328,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
           pybind11::arg("need_weight") = true, pybind11::arg("need_bias") = true,
           pybind11::arg("dz_budget_bytes") = 0, pybind11::arg("weight_grad_out") = pybind11::none(),
           pybind11::arg("bias_grad_out") = pybind11::none(), pybind11::arg("accumulate") = false,
-          pybind11::arg("typed_weight") = false, pybind11::arg("kept") = pybind11::none());
+          pybind11::arg("typed_weight") = false, pybind11::arg("kept") = pybind11::none(),
+          pybind11::arg("as_kept") = false);
     m.def("fused_logp_forward_out", &fused_logp_forward_out, "Fused logp out");
     m.def("fused_logp_forward_fp32", &fused_logp_forward_fp32, "Fused logp fp32");
     m.def("fused_logp_forward_indexed_out", &fused_logp_forward_indexed_out, "Fused logp indexed out");

@@ -769,7 +769,8 @@ __global__ __launch_bounds__(kThreads) void wide_dz_kernel(WideDzArgs a)
 // dZ from the logits that the forward kept, in place: the same expressions as above on one pass over memory
 // (8 bytes per logit against six products of H terms).  A workgroup takes 256 columns of 64 tokens, a thread
 // four of them of every fourth token.  db_part (or null): column sums of the 64 tokens for d_bias,
-// [slab][ldz].
+// [slab][ldz].  MAKE = false: `kept` is dZ already (computed again, nothing was kept) and only its column sums are
+// taken, in the same order.
 struct WideKeptArgs {
     float* kept;  // [N][ldz]
     const int64_t* targets;
@@ -787,6 +788,7 @@ struct WideKeptArgs {
 };
 
 constexpr int kWideSlab = 64;  // tokens
+template <bool MAKE>
 __global__ __launch_bounds__(256) void wide_dz_kept_kernel(WideKeptArgs a)
 {
     const int v = blockIdx.x * 256 + (threadIdx.x & 63) * 4;
@@ -795,21 +797,29 @@ __global__ __launch_bounds__(256) void wide_dz_kept_kernel(WideKeptArgs a)
     if (v < a.V) {
 #pragma unroll 4
         for (int t = lo + wave; t < min(lo + kWideSlab, a.N); t += 4) {
+            f32x4_t* p = reinterpret_cast<f32x4_t*>(a.kept + static_cast<int64_t>(t) * a.ldz + v);
+            if constexpr (!MAKE) {
+                const f32x4_t made = *p;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) sum[c] += v + c < a.V ? made[c] : 0.f;
+                continue;
+            }
             const int64_t tg = a.targets[t];
             const bool live = !(a.use_ignore && tg == a.ignore_index);
             const float gs = live ? a.grad[t] * a.inv_t : 0.f;
             const float nlse2 = -a.lse[t] * kLog2e;
             const int64_t trel = tg - a.vocab_start;
-            f32x4_t* p = reinterpret_cast<f32x4_t*>(a.kept + static_cast<int64_t>(t) * a.ldz + v);
             const f32x4_t z = *p;
             f32x4_t d;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const float pr = v + c < a.V ? __builtin_amdgcn_exp2f(fmaf(z[c], a.scale2, nlse2)) : 0.f;
                 d[c] = gs * ((trel == v + c ? 1.f : 0.f) - pr);
-                sum[c] += d[c];
             }
             *p = d;
+            // the sums take the rounded values that dW takes: no product may be contracted into them
+            asm volatile("" : "+v"(d));
+            sum += d;
         }
     }
     if (a.db_part == nullptr) return;  // uniform
@@ -1053,13 +1063,13 @@ WidePlan wide_plan(int64_t N, int32_t H, int64_t V, size_t budget)
 }
 
 // Backward from kept logits: the chunks of the default budget, so that the sums are grouped as without; dZ lies in
-// the place of the logits.
-WidePlan wide_kept_plan(int64_t N, int32_t H, int64_t V)
+// the place of the logits.  again: none were kept, dZ is computed into the workspace.
+WidePlan wide_kept_plan(int64_t N, int32_t H, int64_t V, bool again)
 {
     WidePlan p = wide_plan(N, H, V, RLK_DEFAULT_DZ_BUDGET);
-    p.dz_bytes = 0;
+    if (!again) p.dz_bytes = 0;
     p.db_bytes = align256(static_cast<size_t>(p.chunk + kWideSlab - 1) / kWideSlab * p.ldz * 4);
-    p.total = p.part_bytes + p.db_bytes;
+    p.total = p.dz_bytes + p.part_bytes + p.db_bytes;
     return p;
 }
 
@@ -1089,7 +1099,8 @@ int wide_bwd_launch(const float* grad_logp, const void* hidden, const void* weig
     constexpr int esz = WideElem<DT>::kBytes;
     float* dz = static_cast<float*>(workspace);
     float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + p.dz_bytes);
-    float* db_part = kept && d_bias ? reinterpret_cast<float*>(static_cast<char*>(workspace) + p.part_bytes) : nullptr;
+    float* db_part = p.db_bytes && d_bias
+                         ? reinterpret_cast<float*>(static_cast<char*>(workspace) + p.dz_bytes + p.part_bytes) : nullptr;
     const int v_tiles = static_cast<int>((V + 255) / 256);
     const int h_tiles = (H + 255) / 256;
     const bool vec_h = quad_aligned(hidden, H, DT), vec_w = quad_aligned(weight, H, DT);
@@ -1120,12 +1131,14 @@ int wide_bwd_launch(const float* grad_logp, const void* hidden, const void* weig
         z.inv_t = 1.f / temperature;
         z.vec_h = vec_h;
         z.vec_w = vec_w;
+        const WideKeptArgs k{dz, z.targets, z.lse, z.grad, db_part, p.ldz, nt, z.V, vocab_start,
+                             ignore_index, use_ignore, z.scale2, z.inv_t};
         if (kept) {
-            const WideKeptArgs k{dz, z.targets, z.lse, z.grad, db_part, p.ldz, nt, z.V, vocab_start,
-                                 ignore_index, use_ignore, z.scale2, z.inv_t};
-            hipLaunchKernelGGL(wide_dz_kept_kernel, dim3(v_tiles, slabs), dim3(256), 0, stream, k);
+            hipLaunchKernelGGL(wide_dz_kept_kernel<true>, dim3(v_tiles, slabs), dim3(256), 0, stream, k);
         } else {
             hipLaunchKernelGGL(wide_dz_kernel<DT>, dim3(tok_tiles * v_tiles), dim3(kThreads), GZ::kSmemBytes, stream, z);
+            if (db_part)
+                hipLaunchKernelGGL(wide_dz_kept_kernel<false>, dim3(v_tiles, slabs), dim3(256), 0, stream, k);
         }
         if (d_hidden) {
             WideDhArgs h;
@@ -1245,7 +1258,7 @@ size_t wide_kept_bytes(int64_t N, int32_t H, int64_t V)
     return bytes > RLK_KEPT_LOGITS_BYTES || H < 128 ? 0 : bytes;
 }
 
-size_t wide_bwd_kept_workspace(int64_t N, int32_t H, int64_t V) { return wide_kept_plan(N, H, V).total; }
+size_t wide_bwd_kept_workspace(int64_t N, int32_t H, int64_t V, bool again) { return wide_kept_plan(N, H, V, again).total; }
 
 int wide_bwd_kept(const float* grad_logp, const void* hidden, const void* weight, const float* bias,
                   const int64_t* targets, const float* lse, void* d_hidden, float* d_weight, float* d_bias,
@@ -1253,7 +1266,7 @@ int wide_bwd_kept(const float* grad_logp, const void* hidden, const void* weight
                   float temperature, int64_t ignore_index, int32_t use_ignore, int32_t accumulate, hipStream_t stream)
 {
     return wide_bwd_launch<RLK_DTYPE_F32>(grad_logp, hidden, weight, bias, targets, lse, d_hidden, d_weight, d_bias, kept,
-                                          workspace, wide_kept_plan(N, H, V), N, H, V, vocab_start, temperature,
+                                          workspace, wide_kept_plan(N, H, V, kept == nullptr), N, H, V, vocab_start, temperature,
                                           ignore_index, use_ignore, accumulate, stream);
 }
 

@@ -114,11 +114,9 @@ class _FusedGRPOStepFunction(torch.autograd.Function):
         upstream = loss_upstream(dcur, dkl, ctx.beta, g_loss, g_pol, g_kl)
         bias = bias_t if ctx.has_bias else None
         keys = dict(temperature=ctx.temperature, ignore_index=IGNORE_INDEX)
-        kept = LL._take_kept(ctx, hidden_2d, w, lambda: LL.fused_linear_logp_forward(
-            hidden_2d, w, target_1d, bias, keep=True, **keys)[3])
         d_h, d_w, d_b = LL.fused_linear_logp_backward(
             upstream, hidden_2d, w, target_1d, lse, bias, need_hidden=need_h, need_weight=need_w,
-            need_bias=need_b, typed_weight=True, kept=kept, **keys)
+            need_bias=need_b, typed_weight=True, **LL._take_kept(ctx, hidden_2d, w), **keys)
         grad_hidden = d_h.reshape(tuple(ctx.lead_shape) + (hidden_2d.size(1),)) if need_h else None
         grad_weight = d_w.to(ctx.weight_dtype) if need_w else None
         grad_bias = d_b.to(ctx.bias_dtype) if need_b else None

@@ -340,11 +340,13 @@ def fused_norm_linear_logp_backward(
     dz_budget_bytes: int = 0,
     typed_weight: bool = False,
     kept: Optional[torch.Tensor] = None,
+    as_kept: bool = False,
 ):
     """Raw backward: ``(d_x [N,H] input dtype, d_gain [H] fp32, d_weight [V,H] fp32, d_bias [V]
     fp32)``; ``d_x`` is the gradient w.r.t. the UN-normalised hidden states.  ``typed_weight``:
     ``d_weight`` in the weight's type where the library can write it (see ``_typed_weight_ok``).
-    ``kept``: the forward's kept logits, overwritten (needs ``need_x`` and a typed ``d_weight``)."""
+    ``kept``: the forward's kept logits, overwritten; ``as_kept``: see ``fused_linear_logp_backward`` (both need
+    ``need_x`` and a typed ``d_weight``)."""
     lib = _native.load()
     n, h = x_2d.shape
     v = weight.size(0)
@@ -361,13 +363,16 @@ def fused_norm_linear_logp_backward(
     d_bias = torch.empty(v, device=dev, dtype=torch.float32) if want_bias else None
     bias_f = None if bias is None else bias.detach().to(torch.float32).contiguous()
     need = _native.ctypes.c_size_t(0)
-    if kept is not None:
-        _native.check(lib.rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(
-            n, h, v, dt, _native.ctypes.byref(need)), "norm + linear_logp backward workspace query")
+    if kept is not None or as_kept:
+        query = lib.rlk_linear_logp_rmsnorm_bwd_as_kept_workspace_bytes if kept is None else \
+            lib.rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes
+        _native.check(query(n, h, v, dt, _native.ctypes.byref(need)),
+                      "norm + linear_logp backward workspace query")
         ws = torch.empty(need.value, device=dev, dtype=torch.uint8)
         rc = lib.rlk_linear_logp_rmsnorm_bwd_kept(
             _ptr(g), _ptr(x_2d), _ptr(gain), float(eps), _ptr(weight), _ptr(bias_f), _ptr(target_1d),
-            _ptr(lse), _ptr(d_x), _ptr(d_gain), _ptr(d_weight), _ptr(d_bias), _ptr(kept), kept.numel(),
+            _ptr(lse), _ptr(d_x), _ptr(d_gain), _ptr(d_weight), _ptr(d_bias), _ptr(kept),
+            0 if kept is None else kept.numel(),
             _ptr(ws), ws.numel(), n, h, v, 0, dt, float(temperature),
             0 if ignore_index is None else int(ignore_index), int(ignore_index is not None), _stream(dev))
         _native.check(rc, "rlk_linear_logp_rmsnorm_bwd_kept")
@@ -408,6 +413,7 @@ def fused_linear_logp_backward(
     accumulate: bool = False,
     typed_weight: bool = False,
     kept: Optional[torch.Tensor] = None,
+    as_kept: bool = False,
 ):
     """Raw backward: ``(d_hidden [N,H] input dtype, d_weight [V,H] fp32, d_bias [V] fp32)``.
 
@@ -425,6 +431,8 @@ def fused_linear_logp_backward(
 
     ``kept``: the logits that the forward of these arguments kept; they are overwritten, and
     ``dz_budget_bytes`` has no part in the call.
+    ``as_kept`` (sizes with ``_kept_bytes``, ``kept`` gone or never made): the same bits from logits that
+    are computed again, 2 bytes of workspace for each.
     """
     lib = _native.load()
     n, h = hidden_2d.shape
@@ -447,7 +455,7 @@ def fused_linear_logp_backward(
         d_hidden, d_weight, d_bias = compiled.fused_linear_logp_backward(
             grad_logp, hidden_2d, weight, target_1d, lse, bias, float(temperature), ignore_index,
             int(vocab_start), bool(need_hidden), bool(need_weight), bool(want_bias),
-            int(dz_budget_bytes), weight_grad_out, bias_grad_out, bool(accumulate), typed, kept)
+            int(dz_budget_bytes), weight_grad_out, bias_grad_out, bool(accumulate), typed, kept, bool(as_kept))
         return d_hidden, d_weight, d_bias
     g = grad_logp.reshape(-1).to(torch.float32).contiguous()
     d_hidden = torch.empty_like(hidden_2d) if need_hidden else None
@@ -461,14 +469,16 @@ def fused_linear_logp_backward(
             torch.empty(v, device=dev, dtype=torch.float32)
     bias_f = None if bias is None else bias.detach().to(torch.float32).contiguous()
     need = _native.ctypes.c_size_t(0)
-    if kept is not None:
-        _native.check(lib.rlk_linear_logp_bwd_kept_workspace_bytes(n, h, v, dt, _native.ctypes.byref(need)),
-                      "linear_logp backward workspace query")
+    if kept is not None or as_kept:
+        query = lib.rlk_linear_logp_bwd_as_kept_workspace_bytes if kept is None else \
+            lib.rlk_linear_logp_bwd_kept_workspace_bytes
+        _native.check(query(n, h, v, dt, _native.ctypes.byref(need)), "linear_logp backward workspace query")
         ws = torch.empty(need.value, device=dev, dtype=torch.uint8)
         rc = lib.rlk_linear_logp_bwd_kept(
             _ptr(g), _ptr(hidden_2d), _ptr(weight), _ptr(bias_f), _ptr(target_1d), _ptr(lse),
             _ptr(d_hidden), None if typed else _ptr(d_weight), _ptr(d_weight) if typed else None,
-            _ptr(d_bias), _ptr(kept), kept.numel(), _ptr(ws), ws.numel(), n, h, v, int(vocab_start), dt,
+            _ptr(d_bias), _ptr(kept), 0 if kept is None else kept.numel(), _ptr(ws), ws.numel(), n, h, v,
+            int(vocab_start), dt,
             float(temperature), 0 if ignore_index is None else int(ignore_index),
             int(ignore_index is not None), int(bool(accumulate)), _stream(dev))
         _native.check(rc, "rlk_linear_logp_bwd_kept")
@@ -495,16 +505,16 @@ def fused_linear_logp_backward(
     return d_hidden, d_weight, d_bias
 
 
-def _take_kept(ctx, hidden_2d, weight, again):
-    """The kept logits for one backward, or ``None`` for sizes that keep none.  The backward overwrites them, so
-    the context gives them up; a second backward, or one behind a forward that was not allowed to keep
-    them, makes them again (``again()``) so that its sums are grouped alike and its bits the same.  An unpack
-    hook may return the saved matrices off the 16-byte boundary that the forward had: no logits are kept
-    for such, and the backward runs on the kernels that take them."""
+def _take_kept(ctx, hidden_2d, weight) -> dict:
+    """``kept`` / ``as_kept`` of one backward.  It overwrites the kept logits, so the context gives them up; a second
+    backward, or one behind a forward that was not allowed to keep them, computes them again with its sums
+    grouped alike and its bits the same.  An unpack hook may return the saved matrices off the 16-byte
+    boundary that the forward had: no logits are kept for such, and the backward runs on the kernels that
+    take them."""
     kept, ctx.kept = ctx.kept, None
     if not ctx.keeps or _kept_bytes(hidden_2d, weight) == 0:
-        return None
-    return again() if kept is None else kept
+        return {}
+    return dict(kept=kept, as_kept=kept is None)
 
 
 class _FusedLinearLogpFunction(torch.autograd.Function):
@@ -574,11 +584,10 @@ class _FusedLinearLogpFunction(torch.autograd.Function):
                 b_buf = torch.zeros(w.size(0), device=w.device, dtype=torch.float32)
         bias = bias_t if ctx.has_bias else None
         keys = dict(temperature=ctx.temperature, ignore_index=ctx.ignore_index)
-        kept = _take_kept(ctx, hidden_2d, w, lambda: fused_linear_logp_forward(
-            hidden_2d, w, target_1d, bias, keep=True, **keys)[3])
         d_h, d_w, d_b = fused_linear_logp_backward(
             grad_logp, hidden_2d, w, target_1d, lse, bias, need_hidden=need_h, need_weight=want_w, need_bias=want_b,
-            weight_grad_out=w_buf, bias_grad_out=b_buf, accumulate=adding, typed_weight=w_out is None, kept=kept, **keys)
+            weight_grad_out=w_buf, bias_grad_out=b_buf, accumulate=adding, typed_weight=w_out is None,
+            **_take_kept(ctx, hidden_2d, w), **keys)
         grad_hidden = d_h.reshape(tuple(ctx.lead_shape) + (hidden_2d.size(1),)) if need_h else None
         grad_weight = d_w.to(ctx.weight_dtype) if need_w and w_out is None else None
         grad_bias = d_b.to(ctx.bias_dtype) if need_b and b_out is None else None
@@ -631,15 +640,12 @@ class _FusedNormLinearLogpFunction(torch.autograd.Function):
                     None, None, None, None, None, None)
         bias = bias_t if ctx.has_bias else None
         keys = dict(eps=ctx.eps, temperature=ctx.temperature, ignore_index=ctx.ignore_index)
-        kept = None
+        kept = _take_kept(ctx, x_2d, w)
         if not (need_x and need_w):  # fewer gradients wanted than when the forward ran
-            ctx.kept = None
-        else:
-            kept = _take_kept(ctx, x_2d, w, lambda: fused_norm_linear_logp_forward(
-                x_2d, g, w, target_1d, bias, keep=True, **keys)[3])
+            kept = {}
         d_x, d_g, d_w, d_b = fused_norm_linear_logp_backward(
             grad_logp, x_2d, g, w, target_1d, lse, bias, need_x=need_x,
-            need_gain=need_g, need_weight=need_w, need_bias=need_b, typed_weight=True, kept=kept, **keys)
+            need_gain=need_g, need_weight=need_w, need_bias=need_b, typed_weight=True, **kept, **keys)
         return (d_x.reshape(tuple(ctx.lead_shape) + (x_2d.size(1),)) if need_x else None,
                 d_g.to(ctx.gain_dtype) if need_g else None,
                 d_w.to(ctx.weight_dtype) if need_w else None,

@@ -48,3 +48,74 @@ def test_unpacked_tensors_may_lie_off_the_16_byte_boundary(dtype, tol, norm):
         logp = op(hidden, weight, ids, **keys)
     for got, want in zip(torch.autograd.grad(logp, [hidden, weight], grad), plain):
         assert ((got.float() - want.float()).norm() / want.float().norm()).item() < tol
+
+
+# padded, moved and split tiles of the 16-bit kernels, chunks of the fp32 ones
+@pytest.mark.parametrize("n,h,v,dtype", [
+    (1, 256, 256, torch.bfloat16),
+    (17, 320, 257, torch.bfloat16),
+    (100, 448, 2300, torch.float16),
+    (255, 1024, 511, torch.bfloat16),
+    (256, 1024, 512, torch.float16),
+    (300, 1088, 1281, torch.bfloat16),
+    (1000, 1024, 9000, torch.bfloat16),
+    (64, 512, 33000, torch.bfloat16),
+    (1, 128, 3, torch.float32),
+    (63, 130, 1001, torch.float32),
+    (513, 256, 1026, torch.float32),
+    (2900, 128, 50001, torch.float32),
+])
+def test_logits_computed_again_give_the_bits_of_kept_ones(n, h, v, dtype):
+    from rl_kernel_amd.ops import linear_logp as LL
+
+    hidden, weight, bias, ids, grad = (t.detach() for t in inputs(dtype, n, h, v))
+    keys = dict(temperature=0.8, ignore_index=-100)
+    _, lse, _, kept = LL.fused_linear_logp_forward(hidden, weight, ids, bias, keep=True, **keys)
+    want = LL.fused_linear_logp_backward(grad, hidden, weight, ids, lse, bias, kept=kept, **keys)
+    got = LL.fused_linear_logp_backward(grad, hidden, weight, ids, lse, bias, as_kept=True, **keys)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    dh, _, db = LL.fused_linear_logp_backward(grad, hidden, weight, ids, lse, bias, as_kept=True, need_weight=False,
+                                              **keys)
+    assert torch.equal(dh, want[0]) and torch.equal(db, want[2])
+
+
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("dtype,h", [(torch.bfloat16, 1024), (torch.float32, 256)])
+def test_a_backward_that_was_left_no_logits_does_not_make_them(dtype, h, norm):
+    """Behind saved-tensor hooks and in a second backward the fp32 logits are not stored again: beyond the
+    gradients there is the workspace, with dZ in the 16-bit type where the inputs have one."""
+    import ctypes
+
+    from rl_kernel_amd import _native
+    from rl_kernel_amd.ops import linear_logp as LL
+
+    hidden, weight, _, ids, grad = inputs(dtype, 1000, h, 9000)
+    keys = dict(ignore_index=-100)
+    if norm:
+        keys["norm_weight"] = torch.ones(h, device="cuda", dtype=dtype)
+    op, need = get_op(), ctypes.c_size_t(0)
+    query = _native.load().rlk_linear_logp_rmsnorm_bwd_as_kept_workspace_bytes if norm else \
+        _native.load().rlk_linear_logp_bwd_as_kept_workspace_bytes
+    assert query(1000, h, 9000, LL._DTYPES[dtype], ctypes.byref(need)) == 0
+
+    def backward(logp, **more):
+        base = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        grads = torch.autograd.grad(logp, [hidden, weight], grad, **more)
+        extra = torch.cuda.max_memory_allocated() - base - sum(g.nbytes for g in grads)
+        return grads, extra
+
+    plain = op(hidden, weight, ids, **keys)
+    first, with_kept = backward(plain, retain_graph=True)
+    second, extra = backward(plain)
+    assert extra <= need.value + (1 << 20)
+    # the logits themselves are no part of `with_kept`: dZ adds no more than it needs
+    dz = 1024 * 36 * 256 * 2 if dtype == torch.bfloat16 else LL._kept_bytes(hidden, weight)
+    assert extra <= with_kept + dz + (1 << 20)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t):
+        logp = op(hidden, weight, ids, **keys)
+    third, extra = backward(logp)
+    assert extra <= need.value + (1 << 20)
+    for a, b, c in zip(first, second, third):
+        assert torch.equal(a, b) and torch.equal(a, c)
