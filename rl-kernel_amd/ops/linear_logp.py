@@ -150,8 +150,10 @@ def _trains(*tensors: Optional[torch.Tensor]) -> bool:
 
 
 def _may_keep() -> bool:
-    """Not under saved-tensor hooks: who offloads or recomputes what a forward saves wants its memory."""
-    return torch._C._autograd._top_saved_tensors_default_hooks(True) is None
+    """Not under saved-tensor hooks: who offloads or recomputes what a forward saves wants its memory.  No public
+    name tells; a torch without this one keeps nothing."""
+    top_hooks = getattr(torch._C._autograd, "_top_saved_tensors_default_hooks", None)
+    return top_hooks is not None and top_hooks(True) is None
 
 
 @_native.on_tensor_device

@@ -3,6 +3,8 @@
 import ctypes
 import random
 
+import torch
+
 
 def test_kept_logits_and_workspace_stay_below_one_gigabyte():
     from rl_kernel_amd import _native
@@ -34,3 +36,13 @@ def test_sizes_that_keep_none():
                            (100, 1024, 255, 0), (1000, 704, 5000, 0), (1638 * 2, 4096, 128256, 1)):
         assert lib.rlk_linear_logp_kept_bytes(n, h, v, dtype, ctypes.byref(kept)) == 0 and kept.value == 0
     assert lib.rlk_linear_logp_kept_bytes(0, 1024, 5000, 0, ctypes.byref(kept)) == -1
+
+
+def test_a_torch_that_does_not_tell_its_hooks_keeps_none(monkeypatch):
+    from rl_kernel_amd.ops import linear_logp as LL
+
+    assert LL._may_keep()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t):
+        assert not LL._may_keep()
+    monkeypatch.delattr(torch._C._autograd, "_top_saved_tensors_default_hooks")
+    assert not LL._may_keep()
