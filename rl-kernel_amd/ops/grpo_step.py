@@ -81,19 +81,19 @@ def fused_linear_logp_grpo_forward(hidden_2d, weight, target_1d, bias, old, ref,
 class _FusedGRPOStepFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, weight, bias, marked_ids, old, ref, adv, mask, clip_eps, beta,
-                temperature, check_targets, train=False):
+                temperature, check_targets, keep_limit=None):
         ctx.set_materialize_grads(False)
         hidden_2d = LL._aligned_contiguous(hidden.reshape(-1, hidden.size(-1)))
         w = LL._aligned_contiguous(weight)
         target_1d = marked_ids.reshape(-1).to(device=hidden_2d.device, dtype=torch.long).contiguous()
         seq_len = hidden.shape[-2] if hidden.dim() >= 2 else 1
-        ctx.keeps = train and LL._kept_bytes(hidden_2d, w) > 0
-        keep = ctx.keeps and LL._may_keep()
+        share = LL._share(ctx, w.device, 0 if keep_limit is None else LL._kept_bytes(hidden_2d, w), keep_limit)
         with LL._checked_targets(target_1d, w.size(0), IGNORE_INDEX, check_targets):
             logp, lse, _, out3, _, _, dcur, dkl, *kept = fused_linear_logp_grpo_forward(
                 hidden_2d, w, target_1d, bias, old, ref, adv, mask, seq_len=seq_len, clip_eps=clip_eps,
-                beta=beta, temperature=temperature, ignore_index=IGNORE_INDEX, keep=keep, strict_targets=None)
-        ctx.kept = kept[0] if keep else None
+                beta=beta, temperature=temperature, ignore_index=IGNORE_INDEX, keep=share is not None,
+                strict_targets=None)
+        LL._hold(ctx, share, kept)
         ctx.save_for_backward(hidden_2d, w, bias if bias is not None else hidden_2d, target_1d, lse,
                               dcur, dkl)
         ctx.has_bias = bias is not None
@@ -128,7 +128,7 @@ class RocmFusedGRPOStepOp:
     weight, token ids / completion mask ``[B, T]``, old / reference log-probs ``[B, T]`` and
     advantages (``[B]`` per sequence or ``[B, T]`` per token).  The three scalars are
     differentiable w.r.t. hidden, weight and bias; masked positions have log-prob exactly 0 and
-    no gradient."""
+    no gradient.  ``kept_logits_bytes``: as in ``RocmFusedLinearLogpOp``."""
 
     def __init__(self) -> None:
         if not torch.cuda.is_available() or getattr(torch.version, "hip", None) is None:
@@ -138,14 +138,16 @@ class RocmFusedGRPOStepOp:
 
     def __call__(self, hidden, lm_head_weight, token_ids, completion_mask, old_logps, ref_logps,
                  advantages, bias=None, *, clip_eps: float = 0.2, beta: float = 0.0,
-                 temperature: float = 1.0, check_targets: bool = True):
+                 temperature: float = 1.0, check_targets: bool = True,
+                 kept_logits_bytes: Optional[int] = None):
         return self.apply(hidden, lm_head_weight, token_ids, completion_mask, old_logps, ref_logps,
                           advantages, bias, clip_eps=clip_eps, beta=beta, temperature=temperature,
-                          check_targets=check_targets)
+                          check_targets=check_targets, kept_logits_bytes=kept_logits_bytes)
 
     def apply(self, hidden, lm_head_weight, token_ids, completion_mask, old_logps, ref_logps,
               advantages, bias=None, *, clip_eps: float = 0.2, beta: float = 0.0,
-              temperature: float = 1.0, check_targets: bool = True):
+              temperature: float = 1.0, check_targets: bool = True,
+              kept_logits_bytes: Optional[int] = None):
         if temperature <= 0.0:
             raise ValueError("temperature must be greater than zero")
         if hidden.dim() < 2 or hidden.shape[:-1] != token_ids.shape:
@@ -168,4 +170,4 @@ class RocmFusedGRPOStepOp:
         return _FusedGRPOStepFunction.apply(hidden, lm_head_weight, bias, ids, old_logps, ref_logps,
                                             advantages, mask, float(clip_eps), float(beta),
                                             float(temperature), check_targets,
-                                            LL._trains(hidden, lm_head_weight, bias))
+                                            LL._keep_limit(kept_logits_bytes, hidden, lm_head_weight, bias))

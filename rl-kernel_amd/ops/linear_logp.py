@@ -11,6 +11,7 @@ conventions of rl_engine/testing/reference_ops.py:15-47 into the kernel: ``tempe
 from __future__ import annotations
 
 import contextlib
+import threading
 from typing import Any, Optional
 
 import torch
@@ -144,9 +145,57 @@ def _kept_bytes(hidden_2d: torch.Tensor, weight: torch.Tensor) -> int:
     return need.value
 
 
-def _trains(*tensors: Optional[torch.Tensor]) -> bool:
-    """Whether autograd records a call with these differentiable inputs."""
-    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+_KEPT_BOUND = 800 << 20  # what the library keeps for one call at most
+
+
+class _KeptShare:
+    """One call's part of the kept logits that are alive on a device: together they stay within ``_KEPT_BOUND``, so
+    that the losses of many micro-batches behind one backward hold no more than one large call.  A call
+    that finds no room computes its logits again (same bits).  Given back when the buffer dies, in
+    ``__del__``, which may run anywhere and therefore takes no lock."""
+
+    _alive: dict = {}
+    _taking = threading.Lock()
+
+    @classmethod
+    def take(cls, device: torch.device, size: int):
+        share = cls()
+        with cls._taking:
+            # one call each on the dict: safe against a __del__ in another thread or in the garbage collector
+            if size + sum(b for d, b in list(cls._alive.values()) if d == device) > _KEPT_BOUND:
+                return None
+            cls._alive[id(share)] = (device, size)
+        return share
+
+    def __del__(self):
+        self._alive.pop(id(self), None)
+
+
+def _share(ctx, device: torch.device, size: int, keep_limit: Optional[int]) -> Optional[_KeptShare]:
+    """Whether this forward keeps its logits, ``size`` bytes of them (0: a size that keeps none).  The sums of the
+    backward are grouped by ``ctx.keeps``, the size's rule alone: what else is alive, ``keep_limit`` and hooks
+    never change a bit."""
+    ctx.keeps, ctx.kept = size > 0, None
+    if size == 0 or size > keep_limit or not _may_keep():
+        return None
+    return _KeptShare.take(device, size)
+
+
+def _hold(ctx, share: Optional[_KeptShare], kept) -> None:
+    """The kept logits go to the context; their share lives as long as the tensor."""
+    if share is not None:
+        ctx.kept = kept[0]
+        ctx.kept.share = share
+
+
+def _keep_limit(limit: Optional[int], *tensors: Optional[torch.Tensor]) -> Optional[int]:
+    """Bytes of logits that a call with these differentiable inputs may keep, ``None`` when autograd does not
+    record it."""
+    if limit is not None and limit < 0:
+        raise ValueError(f"kept_logits_bytes must not be negative, got {limit}")
+    if not torch.is_grad_enabled() or not any(t is not None and t.requires_grad for t in tensors):
+        return None
+    return _KEPT_BOUND if limit is None else int(limit)
 
 
 def _may_keep() -> bool:
@@ -522,7 +571,7 @@ def _take_kept(ctx, hidden_2d, weight) -> dict:
 class _FusedLinearLogpFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, weight, bias, target_ids, temperature, ignore_index, check_targets,
-                weight_grad_out=None, bias_grad_out=None, accumulate=True, train=False):
+                weight_grad_out=None, bias_grad_out=None, accumulate=True, keep_limit=None):
         hidden_2d = _aligned_contiguous(hidden.reshape(-1, hidden.size(-1)))
         w = _aligned_contiguous(weight)
         target_1d = target_ids.reshape(-1).to(device=hidden_2d.device, dtype=torch.long).contiguous()
@@ -536,13 +585,12 @@ class _FusedLinearLogpFunction(torch.autograd.Function):
             ctx.weight_dtype = weight.dtype
             ctx.bias_dtype = bias.dtype if bias is not None else None
             return hidden_2d.new_zeros(hidden.shape[:-1], dtype=torch.float32)
-        ctx.keeps = train and _kept_bytes(hidden_2d, w) > 0
-        keep = ctx.keeps and _may_keep()
+        share = _share(ctx, w.device, 0 if keep_limit is None else _kept_bytes(hidden_2d, w), keep_limit)
         with _checked_targets(target_1d, w.size(0), ignore_index, check_targets):
             logp, lse, _, *kept = fused_linear_logp_forward(
-                hidden_2d, w, target_1d, bias, temperature=temperature, ignore_index=ignore_index, keep=keep,
-                strict_targets=None)
-        ctx.kept = kept[0] if keep else None
+                hidden_2d, w, target_1d, bias, temperature=temperature, ignore_index=ignore_index,
+                keep=share is not None, strict_targets=None)
+        _hold(ctx, share, kept)
         ctx.save_for_backward(hidden_2d, w, bias if bias is not None else hidden_2d, target_1d, lse)
         ctx.has_bias = bias is not None
         ctx.lead_shape = hidden.shape[:-1]
@@ -605,21 +653,21 @@ class _FusedNormLinearLogpFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, gain, weight, bias, target_ids, eps, temperature, ignore_index, check_targets,
-                train=False):
+                keep_limit=None):
         x_2d = _aligned_contiguous(x.reshape(-1, x.size(-1)))
         g = _aligned_contiguous(gain.detach().to(torch.float32))  # the reference multiplies by weight.float()
         w = _aligned_contiguous(weight)
         target_1d = target_ids.reshape(-1).to(device=x_2d.device, dtype=torch.long).contiguous()
         ctx.empty = x_2d.size(0) == 0
         # the gradients that rlk_linear_logp_rmsnorm_bwd_kept always writes have to be wanted
-        ctx.keeps = train and ctx.needs_input_grad[0] and ctx.needs_input_grad[2] \
-            and x_2d.size(0) <= _NORM_BLOCK and _kept_bytes(x_2d, w) > 0
-        keep = ctx.keeps and _may_keep()
+        keeps = keep_limit is not None and ctx.needs_input_grad[0] and ctx.needs_input_grad[2] \
+            and x_2d.size(0) <= _NORM_BLOCK
+        share = _share(ctx, w.device, _kept_bytes(x_2d, w) if keeps else 0, keep_limit)
         with _checked_targets(target_1d, w.size(0), ignore_index, check_targets):
             logp, lse, _, *kept = fused_norm_linear_logp_forward(
                 x_2d, g, w, target_1d, bias, eps=eps, temperature=temperature, ignore_index=ignore_index,
-                keep=keep)
-        ctx.kept = kept[0] if keep else None
+                keep=share is not None)
+        _hold(ctx, share, kept)
         ctx.save_for_backward(x_2d, g, w, bias if bias is not None else x_2d, target_1d, lse)
         ctx.has_bias = bias is not None
         ctx.lead_shape = x.shape[:-1]
@@ -689,9 +737,9 @@ class _FusedLinearLogpPairFunction(torch.autograd.Function):
 
 class RocmFusedLinearLogpOp:
     """gfx950 MFMA fused linear log-prob: ``log_softmax((hidden W^T + b)/T)[target]`` without the
-    ``[N, V]`` logits (a training call of at most 800 MiB of fp32 logits holds them from its forward to its
-    backward, not under saved-tensor hooks; more are computed again).  Constructor raises ``RuntimeError`` when the HIP library or a ROCm GPU is
-    missing so that a registry can fall through to its next backend
+    ``[N, V]`` logits (a training call of few holds them from its forward to its backward, see
+    ``kept_logits_bytes``; not under saved-tensor hooks).  Constructor raises ``RuntimeError`` when the
+    HIP library or a ROCm GPU is missing so that a registry can fall through to its next backend
     (rl_engine/kernels/registry.py:219-229 of the reference)."""
 
     def __init__(self) -> None:
@@ -706,13 +754,15 @@ class RocmFusedLinearLogpOp:
                  check_targets: bool = True, norm_weight: Optional[torch.Tensor] = None,
                  norm_eps: float = 1e-6, weight_grad_out: Optional[torch.Tensor] = None,
                  bias_grad_out: Optional[torch.Tensor] = None,
-                 accumulate: bool = True, compact_ignored: bool = False) -> torch.Tensor:
+                 accumulate: bool = True, compact_ignored: bool = False,
+                 kept_logits_bytes: Optional[int] = None) -> torch.Tensor:
         return self.apply(hidden, lm_head_weight, target_ids, bias, tp_group=tp_group,
                           vocab_start_index=vocab_start_index, global_vocab_size=global_vocab_size,
                           temperature=temperature, ignore_index=ignore_index,
                           check_targets=check_targets, norm_weight=norm_weight, norm_eps=norm_eps,
                           weight_grad_out=weight_grad_out, bias_grad_out=bias_grad_out,
-                          accumulate=accumulate, compact_ignored=compact_ignored)
+                          accumulate=accumulate, compact_ignored=compact_ignored,
+                          kept_logits_bytes=kept_logits_bytes)
 
     def apply(self, hidden, lm_head_weight, target_ids, bias=None, *, tp_group: Any = None,
               vocab_start_index: int = 0, global_vocab_size: Optional[int] = None,
@@ -720,7 +770,7 @@ class RocmFusedLinearLogpOp:
               check_targets: bool = True, norm_weight: Optional[torch.Tensor] = None,
               norm_eps: float = 1e-6, weight_grad_out: Optional[torch.Tensor] = None,
               bias_grad_out: Optional[torch.Tensor] = None, accumulate: bool = True,
-              compact_ignored: bool = False) -> torch.Tensor:
+              compact_ignored: bool = False, kept_logits_bytes: Optional[int] = None) -> torch.Tensor:
         """Selected-token log-prob in float32 with the leading shape of ``hidden``.
 
         ``compact_ignored`` (keyword-only, default off; needs ``ignore_index``): the rows whose
@@ -747,7 +797,12 @@ class RocmFusedLinearLogpOp:
         of the last layer and the model's final RMSNorm
         (rl_engine/kernels/ops/pytorch/norm/rms_norm.py:54-70 of the reference, gain
         ``norm_weight``, ``norm_eps``) runs inside the op; the gradient flows to the un-normalised
-        hidden states and to the gain, and the normalised activations are never kept."""
+        hidden states and to the gain, and the normalised activations are never kept.
+
+        ``kept_logits_bytes`` (keyword-only): the most fp32 logits that this call, when autograd records
+        it, may hold from its forward to its backward, which otherwise computes them again; the results
+        are the same bits.  0: none, for a step short of memory or a recorded forward without a
+        backward.  Default: 800 MiB, which is also what all calls alive on a device hold together."""
         if temperature <= 0.0:
             raise ValueError("temperature must be greater than zero")
         if lm_head_weight.size(-1) != hidden.size(-1):
@@ -803,7 +858,7 @@ class RocmFusedLinearLogpOp:
                                     ignore_index=ignore_index, check_targets=check_targets,
                                     norm_weight=norm_weight, norm_eps=norm_eps,
                                     weight_grad_out=weight_grad_out, bias_grad_out=bias_grad_out,
-                                    accumulate=accumulate)
+                                    accumulate=accumulate, kept_logits_bytes=kept_logits_bytes)
                 full = logp_c.new_zeros(target_ids.numel()).index_copy(0, rows, logp_c)
                 return full.reshape(target_ids.shape)
         if norm_weight is not None:
@@ -819,11 +874,12 @@ class RocmFusedLinearLogpOp:
             return _FusedNormLinearLogpFunction.apply(hidden, norm_weight, lm_head_weight, bias,
                                                       target_ids, float(norm_eps), float(temperature),
                                                       ignore_index, check_targets,
-                                                      _trains(hidden, norm_weight, lm_head_weight, bias))
+                                                      _keep_limit(kept_logits_bytes, hidden, norm_weight,
+                                                                  lm_head_weight, bias))
         return _FusedLinearLogpFunction.apply(hidden, lm_head_weight, bias, target_ids,
                                               float(temperature), ignore_index, check_targets,
                                               weight_grad_out, bias_grad_out, bool(accumulate),
-                                              _trains(hidden, lm_head_weight, bias))
+                                              _keep_limit(kept_logits_bytes, hidden, lm_head_weight, bias))
 
     def with_reference(self, hidden, lm_head_weight, ref_lm_head_weight, target_ids, bias=None,
                        ref_bias=None, *, temperature: float = 1.0,

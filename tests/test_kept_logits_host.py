@@ -2,6 +2,7 @@
 
 import ctypes
 import random
+import threading
 
 import torch
 
@@ -46,3 +47,35 @@ def test_a_torch_that_does_not_tell_its_hooks_keeps_none(monkeypatch):
         assert not LL._may_keep()
     monkeypatch.delattr(torch._C._autograd, "_top_saved_tensors_default_hooks")
     assert not LL._may_keep()
+
+
+def test_shares_of_all_threads_stay_within_the_bound():
+    from rl_kernel_amd.ops.linear_logp import _KEPT_BOUND, _KeptShare
+
+    here, there = torch.device("cuda", 0), torch.device("cuda", 1)
+    size, held, most = _KEPT_BOUND // 5 - 1, [], []
+
+    def work(seed):
+        rng, mine = random.Random(seed), []
+        for _ in range(400):
+            if mine and rng.random() < 0.5:
+                mine.pop()
+            else:
+                share = _KeptShare.take(here, size)
+                if share is not None:
+                    mine.append(share)
+            most.append(sum(b for _, b in list(_KeptShare._alive.values())))
+        held.append(mine)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert max(most) == 5 * size <= _KEPT_BOUND
+    others = [_KeptShare.take(there, size) for _ in range(6)]  # another device has its own
+    assert others[4] is not None and others[5] is None
+    held.clear()
+    others.clear()
+    del t, threads
+    assert not _KeptShare._alive and _KeptShare.take(here, _KEPT_BOUND) and _KeptShare.take(here, _KEPT_BOUND + 1) is None

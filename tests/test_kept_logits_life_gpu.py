@@ -1,6 +1,8 @@
 """What becomes of the logits that a training forward keeps: hooks that hand saved tensors back elsewhere, further
 backwards, several forwards before one backward, captured passes."""
 
+import gc
+
 import pytest
 import torch
 
@@ -119,3 +121,68 @@ def test_a_backward_that_was_left_no_logits_does_not_make_them(dtype, h, norm):
     assert extra <= need.value + (1 << 20)
     for a, b, c in zip(first, second, third):
         assert torch.equal(a, b) and torch.equal(a, c)
+
+
+def grpo_inputs(n):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rand = lambda: torch.randn(1, n, device="cuda", generator=g)
+    return (torch.ones(1, n, device="cuda", dtype=torch.bool), rand() - 11, rand() - 11,
+            torch.randn(1, device="cuda", generator=g))
+
+
+@pytest.mark.parametrize("form", ["plain", "norm", "grpo"])
+def test_many_forwards_before_one_backward_share_one_bound(form):
+    """Six micro-batches whose losses are summed would hold six buffers of 206 MB; together they stay within the
+    bound, the rest is computed again, and every gradient is the one it is alone."""
+    from rl_kernel_amd.ops import linear_logp as LL
+    from rl_kernel_amd.registry import kernel_registry
+
+    n, h, v, calls = 1024, 1024, 50257, 6
+    hidden, weight, _, ids, grad = inputs(torch.bfloat16, n, h, v)
+    ids = ids.clamp_min(0)
+    op, step = get_op(), kernel_registry.get_op("grpo_step_from_hidden") if form == "grpo" else None
+    norm = dict(norm_weight=torch.ones(h, device="cuda", dtype=torch.bfloat16)) if form == "norm" else {}
+    rest = grpo_inputs(n)
+
+    def call(x):
+        if form == "grpo":
+            return step(x[None], weight, ids[None], *rest)[0]
+        return (op(x, weight, ids, **norm) * grad).sum()
+
+    xs = [(hidden.detach() * (1 + k / 8)).requires_grad_(True) for k in range(calls)]
+    alone = [torch.autograd.grad(call(x), [x, weight]) for x in xs[-2:]]
+    size = LL._kept_bytes(hidden, weight)
+    assert calls * size > LL._KEPT_BOUND > 3 * size
+    base = torch.cuda.memory_allocated()
+    losses = [call(x) for x in xs]
+    held = torch.cuda.memory_allocated() - base
+    assert 3 * size < held < LL._KEPT_BOUND + calls * (64 * n + 4096)  # beside the logits O(n) a call
+    got = torch.autograd.grad(sum(losses), xs)
+    for a, b in zip(alone, got[-2:]):
+        assert torch.equal(a[0], b)
+    del losses, got
+    assert not LL._KeptShare._alive
+    # a call whose backward never comes gives its share back when it dies, and so does one that raises
+    call(xs[0])
+    with pytest.raises(ValueError):
+        op(hidden, weight, ids + v)
+    gc.collect()  # the traceback's frames
+    assert not LL._KeptShare._alive
+
+
+@pytest.mark.parametrize("norm", [False, True])
+def test_a_call_can_be_told_to_keep_none(norm):
+    hidden, weight, _, ids, grad = inputs()
+    keys = dict(ignore_index=-100)
+    if norm:
+        keys["norm_weight"] = torch.ones(H, device="cuda", dtype=torch.bfloat16)
+    op = get_op()
+    want = torch.autograd.grad(op(hidden, weight, ids, **keys), [hidden, weight], grad)
+    for limit in (0, KEPT - 1, KEPT):
+        base = torch.cuda.memory_allocated()
+        logp = op(hidden, weight, ids, kept_logits_bytes=limit, **keys)
+        assert (torch.cuda.memory_allocated() - base >= KEPT) == (limit == KEPT)
+        got = torch.autograd.grad(logp, [hidden, weight], grad)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    with pytest.raises(ValueError):
+        op(hidden, weight, ids, kept_logits_bytes=-1, **keys)
