@@ -317,7 +317,11 @@ int rlk_linear_logp_rmsnorm_bwd(const float* grad_logp, const void* x, const flo
                                 int64_t ignore_index, int32_t use_ignore, rlk_stream_t stream);
 
 /* Norm and head with kept logits, one block of tokens (N <= 8192, RLK_ERR_UNSUPPORTED above): see
- * rlk_linear_logp_fwd_kept.  The workspace of the forward is rlk_linear_logp_rmsnorm_fwd's. */
+ * rlk_linear_logp_fwd_kept.  The workspace of the forward is rlk_linear_logp_rmsnorm_fwd's.
+ * rlk_linear_logp_rmsnorm_kept_bytes is 0 also where the buffer and the workspace of the backward, which holds
+ * the normalised rows, come to more than 1 GB together.  Host only. */
+int rlk_linear_logp_rmsnorm_kept_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes);
+
 int rlk_linear_logp_rmsnorm_fwd_kept(const void* x, const float* gain, float eps, const void* weight,
                                      const float* bias, const int64_t* targets, float* logp,
                                      float* lse, void* workspace, size_t workspace_bytes, int64_t N,

@@ -54,6 +54,7 @@ SIGNATURES = {
                                                     _i32, _vp, _vp, _sz, _vp]),
     "rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes": (_c.c_int, [_i64, _i32, _i64, _i32,
                                                                     _c.POINTER(_sz)]),
+    "rlk_linear_logp_rmsnorm_kept_bytes": (_c.c_int, [_i64, _i32, _i64, _i32, _c.POINTER(_sz)]),
     "rlk_linear_logp_rmsnorm_bwd_as_kept_workspace_bytes": (_c.c_int, [_i64, _i32, _i64, _i32,
                                                                        _c.POINTER(_sz)]),
     "rlk_linear_logp_rmsnorm_bwd_kept": (_c.c_int, [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _vp, _vp,

@@ -18,6 +18,8 @@
 #define RLK_MAX_DZ_BUDGET (static_cast<size_t>(2) << 30)  // upper clamp of dz_budget_bytes
 #endif
 
+#define RLK_KEPT_STEP_BYTES static_cast<size_t>(1000000000)  // kept logits and workspace of a call
+
 #ifndef RLK_KEPT_LOGITS_BYTES
 #define RLK_KEPT_LOGITS_BYTES (static_cast<size_t>(800) << 20)  // most that a training forward keeps of its logits
 #endif

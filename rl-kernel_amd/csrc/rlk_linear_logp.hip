@@ -1661,7 +1661,7 @@ BwdPlan bwd_plan(int64_t N, int H, int64_t V, size_t budget)
 
 // Bytes of the kept logits, or 0 where a training forward keeps none: sizes off the chained 16-bit kernels, and
 // more than RLK_KEPT_LOGITS_BYTES, the bound that keeps the extra memory of a call below 1 GB whatever N is (a choice,
-// three of the dZ blocks that a larger call has in its backward; the ops hold all live calls of a device to it).
+// about three of the dZ blocks that a larger call has in its backward; the ops hold all live calls of a device to it).
 // Whole tiles: fewer than 256 tokens take what 256 take, 131 MB at V = 128256.
 // Narrow heads keep none either: a tile of logits costs 4 - 10 us of stores in the forward and 17 us of dZ pass
 // (proportionally less with fewer than 256 tokens, whose columns past N stay out), computing it again

@@ -649,6 +649,20 @@ int rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(int64_t N, int32_t H, int64
     return 0;
 }
 
+int rlk_linear_logp_rmsnorm_kept_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes)
+{
+    if (int rc = rlk_linear_logp_kept_bytes(N, H, V, dtype, bytes)) return rc;
+    size_t ws = 0;
+    if (*bytes == 0 || N > kNormBlockTokens) {
+        *bytes = 0;
+        return 0;
+    }
+    if (int rc = rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(N, H, V, dtype, &ws)) return rc;
+    // the normalised rows and the norm's scratch lie in the workspace too: 315 MB at 8192 x 16384
+    if (*bytes + ws > RLK_KEPT_STEP_BYTES) *bytes = 0;
+    return 0;
+}
+
 int rlk_linear_logp_rmsnorm_bwd_as_kept_workspace_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes)
 {
     size_t kept = 0, again = 0;

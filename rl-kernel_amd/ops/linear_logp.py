@@ -134,14 +134,17 @@ def _warn_if_wide_path(hidden_2d: torch.Tensor, weight: torch.Tensor) -> None:
             weight.size(0))
 
 
-def _kept_bytes(hidden_2d: torch.Tensor, weight: torch.Tensor) -> int:
-    """Size of the logits that a training forward keeps for its backward, 0 where it keeps none."""
+def _kept_bytes(hidden_2d: torch.Tensor, weight: torch.Tensor, norm: bool = False) -> int:
+    """Size of the logits that a training forward (``norm``: with the norm in front) keeps for its backward, 0 where
+    it keeps none."""
     n, h = hidden_2d.shape
     if n == 0 or hidden_2d.data_ptr() % 16 or weight.data_ptr() % 16:
         return 0
     need = _native.ctypes.c_size_t(0)
-    _native.check(_native.load().rlk_linear_logp_kept_bytes(
-        n, h, weight.size(0), _DTYPES[hidden_2d.dtype], _native.ctypes.byref(need)), "kept logits query")
+    lib = _native.load()
+    query = lib.rlk_linear_logp_rmsnorm_kept_bytes if norm else lib.rlk_linear_logp_kept_bytes
+    _native.check(query(n, h, weight.size(0), _DTYPES[hidden_2d.dtype], _native.ctypes.byref(need)),
+                  "kept logits query")
     return need.value
 
 
@@ -328,7 +331,7 @@ def fused_norm_linear_logp_forward(
 ):
     """Raw forward from UN-normalised hidden states: ``(logp, lse, err_flag)`` of
     ``linear_logp(rmsnorm(x, gain, eps), weight, bias)``; the normalised rows live only in the
-    call's workspace.  ``keep``: see ``fused_linear_logp_forward`` (at most ``_NORM_BLOCK`` rows)."""
+    call's workspace.  ``keep``: see ``fused_linear_logp_forward`` (sizes with ``_kept_bytes(norm=True)`` only)."""
     lib = _native.load()
     n, h = x_2d.shape
     v = weight.size(0)
@@ -644,9 +647,6 @@ class _FusedLinearLogpFunction(torch.autograd.Function):
         return (grad_hidden, grad_weight, grad_bias, *nones)
 
 
-_NORM_BLOCK = 8192  # rows of a norm + head call that the library runs as one block
-
-
 class _FusedNormLinearLogpFunction(torch.autograd.Function):
     """linear_logp(rmsnorm(x, gain)) from the un-normalised hidden states; saves x, not the
     normalised rows."""
@@ -660,9 +660,8 @@ class _FusedNormLinearLogpFunction(torch.autograd.Function):
         target_1d = target_ids.reshape(-1).to(device=x_2d.device, dtype=torch.long).contiguous()
         ctx.empty = x_2d.size(0) == 0
         # the gradients that rlk_linear_logp_rmsnorm_bwd_kept always writes have to be wanted
-        keeps = keep_limit is not None and ctx.needs_input_grad[0] and ctx.needs_input_grad[2] \
-            and x_2d.size(0) <= _NORM_BLOCK
-        share = _share(ctx, w.device, _kept_bytes(x_2d, w) if keeps else 0, keep_limit)
+        keeps = keep_limit is not None and ctx.needs_input_grad[0] and ctx.needs_input_grad[2]
+        share = _share(ctx, w.device, _kept_bytes(x_2d, w, norm=True) if keeps else 0, keep_limit)
         with _checked_targets(target_1d, w.size(0), ignore_index, check_targets):
             logp, lse, _, *kept = fused_norm_linear_logp_forward(
                 x_2d, g, w, target_1d, bias, eps=eps, temperature=temperature, ignore_index=ignore_index,

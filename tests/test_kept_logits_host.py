@@ -29,6 +29,33 @@ def test_kept_logits_and_workspace_stay_below_one_gigabyte():
     assert kept_some > 500
 
 
+def test_behind_the_norm_kept_logits_and_workspace_stay_below_one_gigabyte():
+    from rl_kernel_amd import _native
+
+    lib, rng, kept_some, refused = _native.load(), random.Random(4), 0, 0
+    sizes = [(8192, 8192, 25600, 0), (8192, 12288, 25600, 0), (8192, 16384, 25600, 0), (8193, 1024, 25600, 0)]
+    for _ in range(3000):
+        sizes.append((int(2 ** rng.uniform(0, 14)), rng.choice((896, 1024, 2048, 4096, 8192, 12288, 16384)),
+                      int(2 ** rng.uniform(8, 18)), rng.choice((0, 1, 2))))
+    for n, h, v, dtype in sizes:
+        kept, head, ws, again = (ctypes.c_size_t(0) for _ in range(4))
+        assert lib.rlk_linear_logp_rmsnorm_kept_bytes(n, h, v, dtype, ctypes.byref(kept)) == 0
+        assert lib.rlk_linear_logp_kept_bytes(n, h, v, dtype, ctypes.byref(head)) == 0
+        if n > 8192 or head.value == 0:
+            assert kept.value == 0
+            continue
+        assert lib.rlk_linear_logp_rmsnorm_bwd_kept_workspace_bytes(n, h, v, dtype, ctypes.byref(ws)) == 0
+        assert lib.rlk_linear_logp_rmsnorm_bwd_as_kept_workspace_bytes(n, h, v, dtype, ctypes.byref(again)) == 0
+        fits = head.value + ws.value <= 10 ** 9
+        assert kept.value == (head.value if fits else 0), (n, h, v)
+        # fp32 chunks are whole 256-row tiles
+        dz = -(-n // 256) * 256 * -(-v // 4) * 16 if dtype == 2 else head.value // 2
+        assert again.value <= dz + ws.value + 256, (n, h, v, dtype)
+        kept_some += fits
+        refused += not fits
+    assert kept_some > 500 and refused >= 3
+
+
 def test_sizes_that_keep_none():
     from rl_kernel_amd import _native
 

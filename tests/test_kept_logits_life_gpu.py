@@ -186,3 +186,17 @@ def test_a_call_can_be_told_to_keep_none(norm):
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
     with pytest.raises(ValueError):
         op(hidden, weight, ids, kept_logits_bytes=-1, **keys)
+
+
+def test_behind_the_norm_the_workspace_counts():
+    """8192 rows of 12288 beside 839 MB of logits: more than the bound on the two together, so none are kept."""
+    dev = torch.device("cuda")
+    x = torch.randn(8192, 12288, device=dev, dtype=torch.bfloat16).requires_grad_(True)
+    weight = (torch.randn(25600, 12288, device=dev) * 0.01).to(torch.bfloat16).requires_grad_(True)
+    ids = torch.randint(0, 25600, (8192,), device=dev)
+    gain = torch.ones(12288, device=dev, dtype=torch.bfloat16)
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    logp = get_op()(x, weight, ids, norm_weight=gain)
+    assert torch.cuda.memory_allocated() - base < 100 << 20
+    assert all(torch.isfinite(g).all() for g in torch.autograd.grad(logp.sum(), [x, weight]))
