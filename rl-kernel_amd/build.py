@@ -98,6 +98,22 @@ def _check_m0_loads(asm_path: str, src: str) -> int:
     return found
 
 
+def _check_cached_stores(asm_path: str, src: str) -> int:
+    """The unchained dW kernel is up to half as slow again with stores past the L2: none of its stores may be one.
+    Returns how many such kernels there are."""
+    found, inside = 0, None
+    with open(asm_path) as fh:
+        for line in fh:
+            code = line.split(";")[0].strip()
+            if re.match(r"\w*linear_logp_dw_kernel\w*:$", code):
+                found, inside = found + 1, code
+            elif code.startswith("s_endpgm"):
+                inside = None
+            elif inside and STREAM_STORE.match(code):
+                raise RuntimeError(f"{src}: '{code}' in {inside}")
+    return found
+
+
 BINDING_SRC = "rlk_torch_binding.cpp"
 BINDING_NAME = "_rlk_C"
 BINDING_PATH = os.path.join(LIB_DIR, BINDING_NAME + ".so")
@@ -163,6 +179,7 @@ def build(verbose: bool = False, extra_flags=()) -> str:
             _check_no_packed_fp32(asm, src)
             _check_stream_stores(asm, src)
             _check_m0_loads(asm, src)
+            _check_cached_stores(asm, src)
             os.remove(asm)
     tmp = LIB_PATH + ".tmp"
     link = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs]

@@ -963,7 +963,10 @@ __device__ inline void gather_rows(u32x2_t (&p)[4])
 
 // K steps up to which the tiles of a dW launch are written past the L2: with few tokens the launch is bound by its
 // stores (backward from kept logits of 64 x 4096 x 128256 590 -> 558 us, 300 x 2048 x 50257 into fp32 291 ->
-// 254), from 1000 tokens on the two are the same.
+// 254), from 1000 tokens on the two are the same.  Also for sums that a later chunk of the call adds to: dW of 9000 x
+// 2048 x 32768 in blocks of 8 MiB 7.08 ms from the L2, 6.27 past it.  The unchained kernel never streams (CHAIN =
+// false; its `nk` of 0 counts nothing): dW of 300 x 2056 x 50257 678 us past the L2, 437 without, 1000 x 1032 x 50257
+// 514 and 477, from 4000 tokens on the same.
 constexpr int kDwStreamSteps = 8;
 
 // Stores that the epilogue of a full dW tile issues per wavefront, all of them unconditional, the fewer of its
@@ -982,7 +985,7 @@ static_assert(kDwStores <= Acc16::TM * Acc16::TN, "the fp32 form stores a quad a
 // piece and inside H): a uniform tile origin plus a 32-bit lane offset, no predicates; otherwise
 // clamped reads and predicated stores.
 // The tile covers hidden columns [h0, h0 + 256) and owns those from h_min on (see dh_epilogue_impl).
-template <class T, bool FULL>
+template <class T, bool FULL, bool CHAIN>
 __device__ inline void dw_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::TN], const DwArgs& a, int vt,
                                         int h0, int h_min)
 {
@@ -998,7 +1001,7 @@ __device__ inline void dw_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
     const uint32_t ldw = static_cast<uint32_t>(a.H);
     // FULL: byte offsets inside the tile stay below 256 * H * 4 (32 bits)
     char* tile = reinterpret_cast<char*>(a.dw + static_cast<int64_t>(v0) * a.H + h0);
-    const bool stream = a.nk <= kDwStreamSteps;                // uniform
+    const bool stream = CHAIN && a.nk <= kDwStreamSteps;       // uniform
     const int hgrp = h0 + wm * (TM * 16) + 8 * (lane >> 4);  // see gather_rows
     const uint32_t lane_el = static_cast<uint32_t>(wn * (TN * 16) + (lane & 15)) * ldw +
                              static_cast<uint32_t>(wm * (TM * 16) + 4 * (lane >> 4));
@@ -1066,15 +1069,15 @@ __device__ inline void dw_epilogue_impl(const f32x4_t (&acc)[Acc16::TM][Acc16::T
 }
 
 // Returns whether the tile was full (then every wavefront issued all its stores unconditionally).
-template <class T>
+template <class T, bool CHAIN>
 __device__ inline bool dw_epilogue(const f32x4_t (&acc)[Acc16::TM][Acc16::TN], const DwArgs& a, int vt, int h0,
                                    int h_min)
 {
     const bool full = vt * 256 + 256 <= a.v_valid && h0 + 256 <= a.H && h_min == h0;  // uniform
     if (full)
-        dw_epilogue_impl<T, true>(acc, a, vt, h0, h_min);
+        dw_epilogue_impl<T, true, CHAIN>(acc, a, vt, h0, h_min);
     else
-        dw_epilogue_impl<T, false>(acc, a, vt, h0, h_min);
+        dw_epilogue_impl<T, false, CHAIN>(acc, a, vt, h0, h_min);
     return full;
 }
 
@@ -1094,7 +1097,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dw_kernel(DwArgs a)
         Operand B{a.dz + static_cast<int64_t>(vt) * 256, a.ldz, 256};
         zero_acc(acc);
         Gemm::run(A, B, a.tok_valid, acc, smem);
-        dw_epilogue<T>(acc, a, vt, ht * 256, ht * 256);
+        dw_epilogue<T, false>(acc, a, vt, ht * 256, ht * 256);
         if (!walk.has_next()) break;
         walk.advance();
         walk.coords(false, vt, ht);
@@ -1204,7 +1207,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_grads_kernel(DhArgs h, D
         if (more) walk.coords(true, nvt, nht);
         zero_acc(acc);
         Dtl::template tile<true, kDwStores>(st, h_origin(nht), z_origin(nvt), acc, smem, counted);
-        counted = dw_epilogue<T>(acc, d, vt, h_col(ht), ht * 256);
+        counted = dw_epilogue<T, true>(acc, d, vt, h_col(ht), ht * 256);
         if (!more) break;
         walk.advance();
         vt = nvt;

@@ -87,3 +87,15 @@ def test_the_build_refuses_short_distances(builder, tmp_path, asm, ok):
     else:
         with pytest.raises(RuntimeError):
             builder._check_stream_stores(str(path), "x")
+
+
+@pytest.mark.parametrize("name,ok", [("_ZN3rlk21linear_logp_dw_kernelI4Bf16Li64EEvT_", False),
+                                     ("_ZN3rlk24linear_logp_grads_kernelI4Bf16Li64ELb1EEvT_", True)])
+def test_the_build_refuses_streaming_stores_in_the_unchained_kernel(builder, tmp_path, name, ok):
+    path = tmp_path / "x.s"
+    path.write_text(f"{name}:  ; @{name}\n" + STORE + "\ts_nop 1\n\ts_endpgm\n")
+    if ok:
+        assert builder._check_cached_stores(str(path), "x") == 0
+    else:
+        with pytest.raises(RuntimeError):
+            builder._check_cached_stores(str(path), "x")
