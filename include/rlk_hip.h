@@ -41,10 +41,11 @@ enum {
     RLK_ERR_LAUNCH = -3       /* HIP refused the launch */
 };
 
-/* ABI version of this header (major * 100 + minor): 104 (100 + rlk_device_info,
+/* ABI version of this header (major * 100 + minor): 105 (100 + rlk_device_info,
  * rlk_linear_logp_fwd_plan, the typed weight gradients rlk_linear_logp_bwd_typed and
  * rlk_linear_logp_rmsnorm_bwd_typed, rlk_check_targets, rlk_mark_targets,
- * rlk_logp_from_logits_pair_masked and the entry points with kept logits). */
+ * rlk_logp_from_logits_pair_masked, the entry points with kept logits and
+ * their three `as_kept` / norm queries). */
 int rlk_version(void);
 
 /* Message of the last error returned on the calling thread ("" if none). Host pointer, valid

@@ -1108,6 +1108,9 @@ __global__ __launch_bounds__(kThreads) void linear_logp_dw_kernel(DwArgs a)
 // and do not depend on each other, so a workgroup walks its dH tiles through one pipeline and its dW
 // tiles through another right behind, and the CUs that the last round of dH tiles leaves idle are at dW
 // tiles meanwhile (grads_split).  Two launches each rounded their tile count up to whole rounds.
+// Both argument sets are live over the first walk: 22 - 25 spilled vector registers (5 with the narrowest token
+// tile; the separate launches had 0 and 5), about 19 scratch accesses a tile outside the K loop, which only
+// tiles of few K steps feel.
 // h.ksplit > 1: a dH item is one part of the vocab range of a tile and leaves for that part's fp32
 // slot.  The items of one range are neighbours in the list (they share dZ columns), so the part
 // is the slow index.

@@ -84,8 +84,8 @@ def grpo_from_logp_raw(cur, old, ref, adv, mask, *, clip_eps, beta, want_grad, w
 def loss_upstream(dcur, dkl, beta, g_loss, g_pol, g_kl):
     """d (what is differentiated) / d logp from ``dcur`` = d loss / d logp, ``dkl`` = d kl / d logp and
     the gradients of ``(loss, policy, kl)``, policy = loss - beta * kl; ``None`` is zero.  A plain
-    ``loss.backward()`` is one product: the zeros for the other two outputs and their terms were eight
-    launches of the forty microseconds in which a small step has nothing else to do."""
+    ``loss.backward()`` is one product; with zeros made for the other two outputs it was eight launches
+    (two fills, six element-wise)."""
     if g_pol is None and g_kl is None:
         return torch.zeros_like(dcur) if g_loss is None else dcur * g_loss
     zero = dcur.new_zeros(())

@@ -200,3 +200,40 @@ def test_behind_the_norm_the_workspace_counts():
     logp = get_op()(x, weight, ids, norm_weight=gain)
     assert torch.cuda.memory_allocated() - base < 100 << 20
     assert all(torch.isfinite(g).all() for g in torch.autograd.grad(logp.sum(), [x, weight]))
+
+
+@pytest.mark.parametrize("dtype,h,as_kept", [(torch.bfloat16, 1024, False), (torch.bfloat16, 1024, True),
+                                             (torch.float32, 250, False), (torch.float32, 250, True)])
+def test_a_captured_pass_replays_with_kept_logits(dtype, h, as_kept):
+    """Forward and backward in one HIP graph: every replay fills the logits again before the backward uses them
+    up, and equals the eager pass on the same inputs."""
+    from rl_kernel_amd.ops import linear_logp as LL
+
+    n, v = 700, 3000
+    hidden, weight, bias, ids, grad = (t.detach() for t in inputs(dtype, n, h, v))
+    keys = dict(temperature=0.9, ignore_index=-100)
+
+    def step():
+        logp, lse, _, *kept = LL.fused_linear_logp_forward(hidden, weight, ids, bias, keep=not as_kept,
+                                                           strict_targets=None, **keys)
+        return logp, *LL.fused_linear_logp_backward(grad, hidden, weight, ids, lse, bias, as_kept=as_kept,
+                                                    kept=None if as_kept else kept[0], **keys)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = step()
+    for k in range(3):
+        hidden.copy_(torch.randn(n, h, device="cuda").to(dtype))
+        grad.copy_(torch.randn(n, device="cuda"))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in out]
+        assert torch.isfinite(torch.randn(1 << 20, device="cuda").sum())  # eager work and a synchronisation between
+        for a, b in zip(got, step()):
+            assert torch.equal(a, b), f"replay {k} differs"
