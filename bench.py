@@ -42,13 +42,13 @@ PEAK_HBM_GBS = 8000.0
 # the kernel sources whose digest is recorded with them; with other sources `traffic` is null.
 MEASURED_TRAFFIC = {
     "workload": "llama3-8b-head",
-    "kernel_source_sha16": "aea22cae80384ab4",
-    "measured_at_commit": "82a5928",
+    "kernel_source_sha16": "51dedae046fdce3b",
+    "measured_at_commit": "19900cc",
     "counter_scale": {"FETCH_SIZE": 2.000, "WRITE_SIZE": 1.000},
     "bytes_per_launch": {
-        "linear_logp_fwd_kernel": 51297517568,
-        "linear_logp_dz_kernel": 1953206272,
-        "linear_logp_grads_kernel": 3955787776,
+        "linear_logp_fwd_kernel": 57884435200,
+        "linear_logp_dz_kernel": 1942712636,
+        "linear_logp_grads_kernel": 3992529031,
     },
 }
 
