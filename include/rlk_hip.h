@@ -45,7 +45,7 @@ enum {
  * rlk_linear_logp_fwd_plan, the typed weight gradients rlk_linear_logp_bwd_typed and
  * rlk_linear_logp_rmsnorm_bwd_typed, rlk_check_targets, rlk_mark_targets,
  * rlk_logp_from_logits_pair_masked, the entry points with kept logits and
- * their three `as_kept` / norm queries). */
+ * their `as_kept`, `least` and norm queries). */
 int rlk_version(void);
 
 /* Message of the last error returned on the calling thread ("" if none). Host pointer, valid
@@ -226,6 +226,8 @@ int rlk_linear_logp_bwd_typed(const float* grad_logp, const void* hidden, const 
  * whatever N is), 16-bit inputs with H % 64 != 0, H < 256 or V < 256, and heads so narrow (16 bit: H <
  * 896, less for fewer than 224 tokens; fp32: H < 128) that the trip through memory costs what
  * the products do.  Host only.
+ * rlk_linear_logp_kept_least_bytes: what of it a buffer has to have, less for at most 192 tokens of 16-bit
+ * inputs.  Host only.
  * rlk_linear_logp_fwd_kept is rlk_linear_logp_fwd (same bits, same workspace) that also fills `kept`
  * (16-byte aligned); the layout is the library's own.  rlk_linear_logp_bwd_kept is the backward of
  * the same arguments from that buffer, which it OVERWRITES: one forward serves one backward.
@@ -237,6 +239,8 @@ int rlk_linear_logp_bwd_typed(const float* grad_logp, const void* hidden, const 
  * its size comes from rlk_linear_logp_bwd_as_kept_workspace_bytes.
  * ------------------------------------------------------------------------------------------ */
 int rlk_linear_logp_kept_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes);
+
+int rlk_linear_logp_kept_least_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes);
 
 int rlk_linear_logp_fwd_kept(const void* hidden, const void* weight, const float* bias,
                              const int64_t* targets, float* logp, float* lse, void* workspace,

@@ -42,6 +42,7 @@ SIGNATURES = {
     "rlk_linear_logp_bwd_typed": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _sz,
                                              _i64, _i32, _i64, _i64, _i32, _f32, _i64, _i32, _vp]),
     "rlk_linear_logp_kept_bytes": (_c.c_int, [_i64, _i32, _i64, _i32, _c.POINTER(_sz)]),
+    "rlk_linear_logp_kept_least_bytes": (_c.c_int, [_i64, _i32, _i64, _i32, _c.POINTER(_sz)]),
     "rlk_linear_logp_fwd_kept": (_c.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i64, _i32, _i64,
                                             _i64, _i32, _f32, _i64, _i32, _i32, _vp, _vp, _sz, _vp]),
     "rlk_linear_logp_bwd_kept_workspace_bytes": (_c.c_int, [_i64, _i32, _i64, _i32, _c.POINTER(_sz)]),

@@ -65,13 +65,17 @@ struct FwdArgs {
 // of 256 KiB per (token tile, vocab tile), token tile the slow index, made of four slabs of 64 tokens;
 // a slab holds the accumulator quads as the wavefronts have them,
 // [2 wavefronts along vocab][TM][TN][64 lanes][4], so a wavefront stores a tile in 1 KiB pieces.  The last token tile
-// is moved back to end at N as in the backward; columns of 16 tokens past N (fewer than 256 tokens) are not stored.
+// is moved back to end at N as in the backward; columns of 16 tokens past N (fewer than 256 tokens) are not stored,
+// and a tile has only the slabs that hold tokens, two at least (dW takes two K steps): kept_slabs.
 // They are stored past the L2 (stream_store): forward + backward of 1500 x 4096 x 128256 4067 -> 4020 us, of 64 x
 // 4096 x 128256 730 -> 719, of 300 x 2048 x 50257 359 -> 349, of 4096 x 2048 x 50257 2252 -> 2238, of 2000 x 2560 x
 // 32000 934 -> 940.  (A forward repeated alone, whose weight stays in the memory-side cache when they bypass it,
 // goes from 774 to 655 us at 4096 x 2048 x 50257, 585 without keeping; inside a step keeping costs it 140 us.)
 constexpr int kKeptSlab = 64 * 256;       // floats
 constexpr int kKeptTile = 4 * kKeptSlab;
+// By the width of the token tile in 64 tokens, which follows N up to 192 (launch_fwd_chained, launch_kept).
+constexpr int kept_tile_slabs(int tn) { return tn < 2 ? 2 : tn; }
+constexpr int kept_slabs(int64_t N) { return kept_tile_slabs(N <= 64 ? 1 : N <= 128 ? 2 : N <= 192 ? 3 : 4); }
 
 // One workgroup = one block of 256 tokens x one contiguous range of vocab tiles.
 // GENERAL = false covers vocab tiles [0, vtiles) split n_split ways, every one of 256 valid rows (a
@@ -213,7 +217,7 @@ __global__ __launch_bounds__(kThreads) void linear_logp_fwd_kernel(FwdArgs a)
                 mask_rows<T>(acc, wm * (TM * 16), vt * 256 - row0, lane);
                 if constexpr (KEEP) {
                     const int64_t tile = static_cast<int64_t>(tb) * a.vtiles + vt;
-                    float* dst = a.kept + tile * kKeptTile + wm * (kKeptSlab / 2);
+                    float* dst = a.kept + tile * (kept_tile_slabs(TN) * kKeptSlab) + wm * (kKeptSlab / 2);
 #pragma unroll
                     for (int j = 0; j < TN; ++j) {
                         const int cols = wn * TN + j;  // 16 tokens; four of them make a slab
@@ -608,7 +612,8 @@ struct KeptDzArgs {
     const float* lse;
     const float* grad;
     const float* scales;
-    float* db_part;  // [4 * tok_tiles][v_tiles * 256]
+    float* db_part;  // [slabs * tok_tiles][v_tiles * 256]
+    int slabs;       // of a tile: kept_slabs
     int N;
     int V;
     int v_tiles;
@@ -625,12 +630,11 @@ struct KeptDzArgs {
 template <class T, bool DB>
 __global__ __launch_bounds__(256) void linear_logp_dz_kept_kernel(KeptDzArgs a)
 {
-    const int tile = blockIdx.x >> 2, slab = blockIdx.x & 3;
-    const int tt = tile / a.v_tiles, vt = tile - tt * a.v_tiles;
+    const int slab = blockIdx.x, vt = blockIdx.y, tt = blockIdx.z;
     const int tok_back = tt == a.tok_tiles - 1 ? a.tok_shift : 0;
     const int v_back = vt == a.v_tiles - 1 ? a.v_shift : 0;
     const int u = threadIdx.x & 7;  // 8 vocab rows of every group of 64
-    float* src = a.kept + static_cast<int64_t>(tile) * kKeptTile + slab * kKeptSlab;
+    float* src = a.kept + ((static_cast<int64_t>(tt) * a.v_tiles + vt) * a.slabs + slab) * kKeptSlab;
     const float gscale = a.scales[0];
     f32x4_t z[2][4][2];
     float gs[2], nlse2[2];
@@ -713,7 +717,7 @@ __global__ __launch_bounds__(256) void linear_logp_dz_kept_kernel(KeptDzArgs a)
         float acc = red[0][threadIdx.x];
 #pragma unroll 8
         for (int r = 1; r < 32; ++r) acc += red[r][threadIdx.x];
-        a.db_part[(static_cast<int64_t>(tt) * 4 + slab) * (a.v_tiles * 256) + vt * 256 + threadIdx.x] = acc;
+        a.db_part[(static_cast<int64_t>(tt) * a.slabs + slab) * (a.v_tiles * 256) + vt * 256 + threadIdx.x] = acc;
     }
 }
 
@@ -1121,7 +1125,7 @@ template <class T, int BK, bool KEPT, class HT = Acc16>
 __global__ __launch_bounds__(kThreads) void linear_logp_grads_kernel(DhArgs h, DwArgs d)
 {
     static_assert(KEPT || std::is_same<HT, Acc16>::value, "narrow token tiles are for kept logits");
-    constexpr int kTileEls = kKeptTile * 2, kSlabEls = kKeptSlab * 2;  // 16-bit elements
+    constexpr int kSlabEls = kKeptSlab * 2, kTileEls = kept_tile_slabs(HT::TN) * kSlabEls;  // 16-bit elements
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int dh_items = h.tok_tiles * h.h_tiles * h.ksplit;
     if (static_cast<int>(blockIdx.x) < dh_items) {
@@ -1668,7 +1672,7 @@ BwdPlan bwd_plan(int64_t N, int H, int64_t V, size_t budget)
 // Bytes of the kept logits, or 0 where a training forward keeps none: sizes off the chained 16-bit kernels, and
 // more than RLK_KEPT_LOGITS_BYTES, the bound that keeps the extra memory of a call below 1 GB whatever N is (a choice,
 // about three of the dZ blocks that a larger call has in its backward; the ops hold all live calls of a device to it).
-// Whole tiles: fewer than 256 tokens take what 256 take, 131 MB at V = 128256.
+// In whole tiles; fewer than 192 tokens need less of it (kept_least).
 // Narrow heads keep none either: a tile of logits costs 4 - 10 us of stores in the forward and 17 us of dZ pass
 // (proportionally less with fewer than 256 tokens, whose columns past N stay out), computing it again
 // about 1.7 us per 64 of H plus 4 (forward + backward, kept against computed again: 1305 x 896 x 32768 400 against
@@ -1680,6 +1684,13 @@ size_t kept_bytes(int64_t N, int H, int64_t V, int dtype)
     const int64_t tiles = ((N + 255) / 256) * ((V + 255) / 256);
     if (tiles > static_cast<int64_t>(RLK_KEPT_LOGITS_BYTES / (kKeptTile * 4))) return 0;
     return static_cast<size_t>(tiles) * kKeptTile * 4;
+}
+
+// What a buffer has to have of kept_bytes: 66 of 131 MB at 128 x 128256.
+size_t kept_least(int64_t N, int H, int64_t V, int dtype)
+{
+    const size_t whole = kept_bytes(N, H, V, dtype);
+    return dtype == RLK_DTYPE_F32 ? whole : whole / 4 * kept_slabs(N);
 }
 
 // Backward from kept logits: one block of the whole problem, dZ in the place of the logits.  again: none were kept
@@ -1760,7 +1771,7 @@ bool use_mfma(const void* hidden, const void* weight, int32_t H, int dtype)
 // A buffer for kept logits as the forward or the backward is given it (null: the backward computes them again).
 int check_kept(const void* kept, size_t bytes, bool mfma, int64_t N, int32_t H, int64_t V, int dtype)
 {
-    const size_t need = kept_bytes(N, H, V, dtype);
+    const size_t need = kept_least(N, H, V, dtype);
     if ((!mfma && dtype != RLK_DTYPE_F32) || need == 0)
         return rlk_fail(RLK_ERR_UNSUPPORTED, "no logits are kept for these sizes (rlk_linear_logp_kept_bytes)");
     if (kept != nullptr && (bytes < need || (reinterpret_cast<uintptr_t>(kept) & 15) != 0))
@@ -2000,7 +2011,8 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
                 k.ignore_index = z.ignore_index;
                 k.use_ignore = z.use_ignore;
                 k.scale2 = z.scale2;
-                const dim3 slabs(tok_tiles * v_tiles * 4);
+                k.slabs = kept_slabs(N);
+                const dim3 slabs(k.slabs, v_tiles, tok_tiles);  // at most 3200 tiles in all
                 if (db_part)
                     hipLaunchKernelGGL((linear_logp_dz_kept_kernel<T, true>), slabs, dim3(256), 0, stream, k);
                 else
@@ -2079,7 +2091,7 @@ int bwd_enqueue(const BwdCall& c, const BwdPlan& p, int n_cu)
                                        stream, dz, p.ldz, rows, db_part, static_cast<int64_t>(p.v_piece));
                 hipLaunchKernelGGL(linear_logp_db_finish_kernel, dim3((v_valid + 255) / 256), dim3(256), 0,
                                    stream, db_part, static_cast<int64_t>(p.v_piece),
-                                   p.whole ? 4 * tok_tiles : tok_tiles, v_valid, v_shift, scales, c.d_bias + v_lo,
+                                   c.kept ? kept_slabs(N) * tok_tiles : p.whole ? 4 * tok_tiles : tok_tiles, v_valid, v_shift, scales, c.d_bias + v_lo,
                                    (ci > 0 || c.accumulate != 0) ? 1 : 0);
             }
             if (int rc = check_launch("linear_logp backward launch failed")) return rc;
@@ -2279,6 +2291,13 @@ int rlk_linear_logp_kept_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, s
 {
     if (!bytes || N <= 0 || V <= 0 || H <= 0) return rlk_fail(RLK_ERR_ARG, "bad kept-logits query");
     *bytes = kept_bytes(N, H, V, dtype);
+    return 0;
+}
+
+int rlk_linear_logp_kept_least_bytes(int64_t N, int32_t H, int64_t V, int32_t dtype, size_t* bytes)
+{
+    if (!bytes || N <= 0 || V <= 0 || H <= 0) return rlk_fail(RLK_ERR_ARG, "bad kept-logits query");
+    *bytes = kept_least(N, H, V, dtype);
     return 0;
 }
 

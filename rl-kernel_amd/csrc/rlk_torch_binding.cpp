@@ -116,7 +116,7 @@ std::vector<at::Tensor> fused_linear_logp_forward_ex(at::Tensor hidden, at::Tens
     }
     if (keep) {
         size_t bytes = 0;
-        TORCH_CHECK(rlk_linear_logp_kept_bytes(n, hd, v, dt, &bytes) == 0, rlk_last_error());
+        TORCH_CHECK(rlk_linear_logp_kept_least_bytes(n, hd, v, dt, &bytes) == 0, rlk_last_error());
         auto kept = at::empty({static_cast<int64_t>(bytes)}, hidden.options().dtype(at::kByte));
         const int rc = rlk_linear_logp_fwd_kept(hidden.data_ptr(), weight.data_ptr(), bias_p, target.data_ptr<int64_t>(),
                                                 logp.data_ptr<float>(), lse.data_ptr<float>(), ws.data_ptr(),

@@ -66,7 +66,7 @@ def fused_linear_logp_grpo_forward(hidden_2d, weight, target_1d, bias, old, ref,
     ws = torch.empty(need.value, device=dev, dtype=torch.uint8)
     bias_f = None if bias is None else bias.detach().to(torch.float32).contiguous()
     p = LL._ptr
-    kept = torch.empty(LL._kept_bytes(hidden_2d, weight), device=dev, dtype=torch.uint8) if keep else None
+    kept = torch.empty(LL._kept_least(hidden_2d, weight), device=dev, dtype=torch.uint8) if keep else None
     rc = lib.rlk_linear_logp_fwd_grpo_kept(
         p(hidden_2d), p(weight), p(bias_f), p(target_1d), p(logp), p(lse), p(ws), ws.numel(), n, h, v,
         0, dt, float(temperature), 0 if ignore_index is None else int(ignore_index),
@@ -87,7 +87,7 @@ class _FusedGRPOStepFunction(torch.autograd.Function):
         w = LL._aligned_contiguous(weight)
         target_1d = marked_ids.reshape(-1).to(device=hidden_2d.device, dtype=torch.long).contiguous()
         seq_len = hidden.shape[-2] if hidden.dim() >= 2 else 1
-        share = LL._share(ctx, w.device, 0 if keep_limit is None else LL._kept_bytes(hidden_2d, w), keep_limit)
+        share = LL._share(ctx, w.device, 0 if keep_limit is None else LL._kept_least(hidden_2d, w), keep_limit)
         with LL._checked_targets(target_1d, w.size(0), IGNORE_INDEX, check_targets):
             logp, lse, _, out3, _, _, dcur, dkl, *kept = fused_linear_logp_grpo_forward(
                 hidden_2d, w, target_1d, bias, old, ref, adv, mask, seq_len=seq_len, clip_eps=clip_eps,

@@ -148,6 +148,16 @@ def _kept_bytes(hidden_2d: torch.Tensor, weight: torch.Tensor, norm: bool = Fals
     return need.value
 
 
+def _kept_least(hidden_2d: torch.Tensor, weight: torch.Tensor, norm: bool = False) -> int:
+    """Bytes of the buffer for them: less than ``_kept_bytes`` for few tokens."""
+    if _kept_bytes(hidden_2d, weight, norm) == 0:
+        return 0
+    need = _native.ctypes.c_size_t(0)
+    _native.check(_native.load().rlk_linear_logp_kept_least_bytes(
+        *hidden_2d.shape, weight.size(0), _DTYPES[hidden_2d.dtype], _native.ctypes.byref(need)), "kept logits query")
+    return need.value
+
+
 _KEPT_BOUND = 800 << 20  # what the library keeps for one call at most
 
 
@@ -254,7 +264,7 @@ def fused_linear_logp_forward(
     ws = torch.empty(max(need.value, 16), device=dev, dtype=torch.uint8)
     bias_f = None if bias is None else bias.detach().to(torch.float32).contiguous()
     if keep:
-        kept = torch.empty(_kept_bytes(hidden_2d, weight), device=dev, dtype=torch.uint8)
+        kept = torch.empty(_kept_least(hidden_2d, weight), device=dev, dtype=torch.uint8)
         rc = lib.rlk_linear_logp_fwd_kept(
             _ptr(hidden_2d), _ptr(weight), _ptr(bias_f), _ptr(target_1d), _ptr(logp), _ptr(lse),
             _ptr(ws), ws.numel(), n, h, v, int(vocab_start), dt, float(temperature),
@@ -350,7 +360,7 @@ def fused_norm_linear_logp_forward(
     ws = torch.empty(max(need.value, 256), device=dev, dtype=torch.uint8)
     bias_f = None if bias is None else bias.detach().to(torch.float32).contiguous()
     if keep:
-        kept = torch.empty(_kept_bytes(x_2d, weight), device=dev, dtype=torch.uint8)
+        kept = torch.empty(_kept_least(x_2d, weight), device=dev, dtype=torch.uint8)
         rc = lib.rlk_linear_logp_rmsnorm_fwd_kept(
             _ptr(x_2d), _ptr(gain), float(eps), _ptr(weight), _ptr(bias_f), _ptr(target_1d), _ptr(logp),
             _ptr(lse), _ptr(ws), ws.numel(), n, h, v, 0, dt, float(temperature),
@@ -588,7 +598,7 @@ class _FusedLinearLogpFunction(torch.autograd.Function):
             ctx.weight_dtype = weight.dtype
             ctx.bias_dtype = bias.dtype if bias is not None else None
             return hidden_2d.new_zeros(hidden.shape[:-1], dtype=torch.float32)
-        share = _share(ctx, w.device, 0 if keep_limit is None else _kept_bytes(hidden_2d, w), keep_limit)
+        share = _share(ctx, w.device, 0 if keep_limit is None else _kept_least(hidden_2d, w), keep_limit)
         with _checked_targets(target_1d, w.size(0), ignore_index, check_targets):
             logp, lse, _, *kept = fused_linear_logp_forward(
                 hidden_2d, w, target_1d, bias, temperature=temperature, ignore_index=ignore_index,
@@ -661,7 +671,7 @@ class _FusedNormLinearLogpFunction(torch.autograd.Function):
         ctx.empty = x_2d.size(0) == 0
         # the gradients that rlk_linear_logp_rmsnorm_bwd_kept always writes have to be wanted
         keeps = keep_limit is not None and ctx.needs_input_grad[0] and ctx.needs_input_grad[2]
-        share = _share(ctx, w.device, _kept_bytes(x_2d, w, norm=True) if keeps else 0, keep_limit)
+        share = _share(ctx, w.device, _kept_least(x_2d, w, norm=True) if keeps else 0, keep_limit)
         with _checked_targets(target_1d, w.size(0), ignore_index, check_targets):
             logp, lse, _, *kept = fused_norm_linear_logp_forward(
                 x_2d, g, w, target_1d, bias, eps=eps, temperature=temperature, ignore_index=ignore_index,

@@ -106,3 +106,19 @@ def test_shares_of_all_threads_stay_within_the_bound():
     others.clear()
     del t, threads
     assert not _KeptShare._alive and _KeptShare.take(here, _KEPT_BOUND) and _KeptShare.take(here, _KEPT_BOUND + 1) is None
+
+
+def test_a_buffer_holds_the_slabs_that_have_tokens():
+    from rl_kernel_amd import _native
+
+    lib, kept, least = _native.load(), ctypes.c_size_t(0), ctypes.c_size_t(0)
+    for n, quarters in ((1, 2), (64, 2), (128, 2), (129, 3), (192, 3), (193, 4), (255, 4), (256, 4), (1000, 4)):
+        for dtype in (0, 1, 2):
+            assert lib.rlk_linear_logp_kept_bytes(n, 4096, 50257, dtype, ctypes.byref(kept)) == 0
+            assert lib.rlk_linear_logp_kept_least_bytes(n, 4096, 50257, dtype, ctypes.byref(least)) == 0
+            assert least.value == (kept.value if dtype == 2 else kept.value * quarters // 4) > 0
+        # one byte less is refused before anything is launched (no pointer is followed)
+        assert lib.rlk_linear_logp_fwd_kept(16, 16, None, 16, 16, 16, 256, 1 << 40, n, 4096, 50257, 0, 1, 1.0, 0, 0, 0,
+                                            None, 16, kept.value * quarters // 4 - 1, None) == -1
+        assert b"buffer too small" in lib.rlk_last_error()
+    assert lib.rlk_linear_logp_kept_least_bytes(100, 64, 5000, 0, ctypes.byref(least)) == 0 and least.value == 0

@@ -57,6 +57,10 @@ def test_unpacked_tensors_may_lie_off_the_16_byte_boundary(dtype, tol, norm):
     (1, 256, 256, torch.bfloat16),
     (17, 320, 257, torch.bfloat16),
     (100, 448, 2300, torch.float16),
+    (128, 512, 1300, torch.bfloat16),
+    (129, 576, 1300, torch.float16),
+    (192, 768, 1300, torch.bfloat16),
+    (193, 832, 1300, torch.bfloat16),
     (255, 1024, 511, torch.bfloat16),
     (256, 1024, 512, torch.float16),
     (300, 1088, 1281, torch.bfloat16),
@@ -168,6 +172,18 @@ def test_many_forwards_before_one_backward_share_one_bound(form):
         op(hidden, weight, ids + v)
     gc.collect()  # the traceback's frames
     assert not LL._KeptShare._alive
+
+
+@pytest.mark.parametrize("n,slabs", [(1, 2), (64, 2), (65, 2), (128, 2), (129, 3), (192, 3), (193, 4), (255, 4)])
+def test_few_tokens_hold_only_the_slabs_they_fill(n, slabs):
+    hidden, weight, bias, ids, grad = inputs(torch.bfloat16, n, 1024, 5000)
+    op = get_op()
+    op(hidden, weight, ids, bias, ignore_index=-100)
+    base = torch.cuda.memory_allocated()
+    logp = op(hidden, weight, ids, bias, ignore_index=-100)
+    held = torch.cuda.memory_allocated() - base
+    assert 20 * slabs * (64 << 10) <= held < 20 * slabs * (64 << 10) + (32 << 10)
+    torch.autograd.grad(logp, [hidden, weight, bias], grad)
 
 
 @pytest.mark.parametrize("norm", [False, True])
