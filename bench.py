@@ -42,13 +42,13 @@ PEAK_HBM_GBS = 8000.0
 # the kernel sources whose digest is recorded with them; with other sources `traffic` is null.
 MEASURED_TRAFFIC = {
     "workload": "llama3-8b-head",
-    "kernel_source_sha16": "51dedae046fdce3b",
-    "measured_at_commit": "19900cc",
+    "kernel_source_sha16": "bc460a3c75fd6b27",
+    "measured_at_commit": "f90a55b",
     "counter_scale": {"FETCH_SIZE": 2.000, "WRITE_SIZE": 1.000},
     "bytes_per_launch": {
-        "linear_logp_fwd_kernel": 57884435200,
-        "linear_logp_dz_kernel": 1942712636,
-        "linear_logp_grads_kernel": 3992529031,
+        "linear_logp_fwd_kernel": 56329095552,
+        "linear_logp_dz_kernel": 1954025774,
+        "linear_logp_grads_kernel": 3980332556,
     },
 }
 
