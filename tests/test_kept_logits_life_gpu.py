@@ -86,6 +86,24 @@ def test_logits_computed_again_give_the_bits_of_kept_ones(n, h, v, dtype):
     assert torch.equal(dh, want[0]) and torch.equal(db, want[2])
 
 
+def test_the_ctypes_route_and_the_compiled_one_are_the_same_calls(monkeypatch):
+    from rl_kernel_amd import _compiled
+    from rl_kernel_amd.ops import linear_logp as LL
+
+    hidden, weight, bias, ids, grad = (t.detach() for t in inputs(n=150))
+
+    def passes():
+        _, lse, _, kept = LL.fused_linear_logp_forward(hidden, weight, ids, bias, keep=True, ignore_index=-100)
+        return [g for as_kept in (False, True) for typed in (False, True)
+                for g in LL.fused_linear_logp_backward(
+                    grad, hidden, weight, ids, lse, bias, ignore_index=-100, typed_weight=typed, as_kept=as_kept,
+                    kept=None if as_kept else kept.clone())]
+
+    want = passes()
+    monkeypatch.setattr(_compiled, "module", lambda: None)
+    assert all(torch.equal(a, b) for a, b in zip(passes(), want))
+
+
 @pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("dtype,h", [(torch.bfloat16, 1024), (torch.float32, 256)])
 def test_a_backward_that_was_left_no_logits_does_not_make_them(dtype, h, norm):
